@@ -99,13 +99,14 @@ __device__ inline double rcp_nr(double x) {
 // the step's own row).  The steps go in 8-wide batches: their mid values
 // load together, then the sums.
 constexpr int kNearGroup = 16;
+constexpr int kFoldBatch = 8;
 __device__ inline void fold_near_group(const double* __restrict__ D, int64_t ld, const double* __restrict__ omega,
                                        int64_t omega_stride, int n0, double* __restrict__ mid, int64_t i, int lo,
                                        int p_lo, int p_hi, bool first) {
     double dv[kNearGroup];
 #pragma unroll
     for (int k = 0; k < kNearGroup; k++) dv[k] = D[(int64_t)(lo + k) * ld + i];
-    constexpr int PB = 8;
+    constexpr int PB = kFoldBatch;
     for (int p0 = p_lo; p0 < p_hi; p0 += PB) {
         double acc[PB];
 #pragma unroll
@@ -244,9 +245,12 @@ constexpr int kGroup = 32;     // history levels per packed group (K of one 16x1
 
 // 1D chunks of the partitioned solve (256 nodes each, N <= 65536)
 constexpr int kMaxChunks = 256;
-// grid exchange of the cooperative 1D launches: per barrier parity, 8 words
-// per reduced row (2 per chunk) and 2 per chunk measure, 8 bytes each
-constexpr size_t kXchBytes = 2 * (size_t)(2 * (8 * kMaxChunks + kMaxChunks)) * 8;
+// grid exchange of the cooperative 1D launches: per barrier parity, one
+// 128-byte line of sixteen tagged words per chunk
+constexpr size_t kXchBytes = 2 * (size_t)kMaxChunks * 16 * 8;
+// row waves (64 nodes each) of a cooperative chunk workgroup: 3 up to 192
+// nodes per chunk, else 4
+__host__ __device__ inline int row_waves(int N, int C) { return (N + C - 1) / C <= 192 ? 3 : 4; }
 
 // Arguments of one 1D step launch (step1d.hip)
 struct Step1DArgs {
@@ -286,7 +290,7 @@ struct Step1DArgs {
     int blk;                  // rows of the history block (far partial and mid rows)
     double* mid;              // near-field groups folded ahead: mid[p - n0][i] = sum over the
                               // folded 16-level groups of the step-p weights times D (null: none)
-    unsigned long long* xch;  // grid exchange words [2 parities][kXchBytes / 16] (tagged halves)
+    unsigned long long* xch;  // grid exchange words [2 parities][kMaxChunks][16] (tagged halves)
     unsigned xtag;            // this launch's tag base: (launch count mod 65535 + 1) << 16
     int* err;                 // [0] set when a grid barrier times out; [1] Picard solves (cooperative launches)
     int64_t wait_ticks;       // a grid barrier gives up after this many ticks of the device's wall clock
@@ -447,7 +451,7 @@ fpde_status launch_gemm_split(int mode, const void* c0, const void* c1, const vo
                               int* splits_out, hipStream_t st, int max_splits = 0);
 fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st);
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st);
-bool step1d_block_supported(int C);
+bool step1d_block_supported(int N, int C);
 bool step1d_batch_supported(int64_t wgs);
 // Batched 3D LOD step: one step of up to kMax3DBatch 3D solves (n <= 128,
 // partitioned sweeps) in one launch per kernel of the step (history combine,

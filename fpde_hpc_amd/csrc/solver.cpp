@@ -433,7 +433,7 @@ fpde_status solver_alloc(fpde_solver* s) {
         // the space-fractional sum needs the whole U^n between two steps: its
         // kernels run between the per-iteration launches (a cooperative form
         // with helper workgroups for the sum measured no faster)
-        s->block_mode = (sp.step_mode == 0) && blocked_history && !space && step1d_block_supported(s->C);
+        s->block_mode = (sp.step_mode == 0) && blocked_history && !space && step1d_block_supported(sp.nodes, s->C);
         s->la = s->block_mode && lookahead_spec(sp);
         if (s->block_mode && s->w.ser_P == 0) DALLOC(s->mid, sizeof(double) * (size_t)sp.block * p.ld);
         DALLOC(s->dmax, sizeof(double) * 2 * s->C);

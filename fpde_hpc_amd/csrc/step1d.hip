@@ -152,11 +152,9 @@ __device__ inline int chunk_solve(double (*pA)[256], double (*pC)[256], double (
 // Far partial sums plus the near levels t in [near_lo, n-2] already in
 // memory, gathered in 32-wide batches of independent loads (a sum over m
 // terms costs ~m/32 memory round trips).  Every load is guarded: omega is
-// read only at n-t-1 >= 1.  With `folded` > 0 the first folded * 16 near
-// levels come as one value of g.mid (fold_near_group) and the loads start after
-// them.
+// read only at n-t-1 >= 1.
 __device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t part_off,
-                                  const double* __restrict__ omega, int folded = 0) {
+                                  const double* __restrict__ omega) {
     constexpr int W = 32;
     double far = 0.0;
     for (int sp0 = 0; sp0 < g.nsplit; sp0 += W) {
@@ -167,9 +165,9 @@ __device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t par
 #pragma unroll
         for (int j = 0; j < W; j++) far += v[j];
     }
-    double nr0 = folded > 0 ? g.mid[(int64_t)(n - g.n0) * g.ld + i] : 0.0, nr1 = 0.0;
+    double nr0 = 0.0, nr1 = 0.0;
     const int t_end = n - 1;   // exclusive: D[n-1] is the newest level, added by the caller
-    for (int t0 = g.near_lo + kNearGroup * folded; t0 < t_end; t0 += W) {
+    for (int t0 = g.near_lo; t0 < t_end; t0 += W) {
         double v[W], w[W];
 #pragma unroll
         for (int j = 0; j < W; j++) {
@@ -509,40 +507,55 @@ __global__ __launch_bounds__(256) void k_step1d(Step1DArgs g) {
 
 // ---------------------------------------------------------------------------
 // Cooperative form: one launch runs the steps [n, n_end) of a history block
-// with every Picard iteration inside, all C workgroups co-resident.  Per
-// iteration each workgroup builds its rows at the iterate (VGM, chunk PCR)
-// and publishes its two reduced rows with the convergence measure of the
-// previous iterate; one grid barrier later every workgroup has the whole
-// reduced system, decides convergence the reference way (stop once
-// max|U^k - U^{k-1}| <= tol, the iterate U^k is the result) and otherwise
-// solves the reduced system and back-substitutes its chunk.  A step's
-// history needs only the workgroup's own nodes (its own earlier writes of D)
-// and the precomputed far partials, so steps follow each other without a
-// barrier; U and D of every step are written as in the per-launch form.
+// with every Picard iteration inside, all C chunk workgroups co-resident.
+// A workgroup has RW row waves (one thread per chunk node: coefficients, rows
+// and the node's history) and one solver wave (the chunk's line solve, the
+// grid exchange, the reduced system).  Per Picard iteration:
+//   row waves    K and 1/C at the iterate (the solver wave: K of the node left
+//                of the chunk), row data to LDS                    -- barrier A
+//   solver wave  chunk rows -> U_i = x_i + y_i U_s + z_i U_s', the separators
+//                s (the chunk's first node) and s' (the next chunk's);
+//                publishes 7 values and the chunk's measure; waits for every
+//                chunk's; decides convergence the reference way (stop once
+//                max|U^k - U^{k-1}| <= tol, the iterate U^k is the result);
+//                solves the C separators' system; U of its nodes to LDS
+//   row waves    meanwhile: the next step's history from memory    -- barrier B
+// A step's history needs only the workgroup's own nodes (its own earlier
+// writes of D) and the precomputed far partials, so steps follow each other
+// without a barrier; U and D of every step are written as in the
+// per-iteration launches.
+//
+// What bounds it: the dependent chain of one iteration (coefficients, line
+// solve, one grid exchange), not memory or arithmetic.  So the line solve sits
+// in ONE wave: 64 lanes of R rows each, the lane's interior rows eliminated in
+// registers, then parallel cyclic reduction over the 64 lanes with no
+// workgroup barrier and (from stride 4 on) no LDS either, since lane
+// 16 (p mod 4) + p/4 holds position p and a stride of 4 q positions is a DPP
+// row shift by q.  One separator per chunk (not both chunk ends) halves the
+// reduced system, whose couplings fall off with the chunk length: its cyclic
+// reduction ends as soon as none exceeds 2^-60.
+// Measured (cycles of one iteration at N = 10^4, 53 chunks, phase timers): row
+// waves 3000 from barrier to barrier (coefficients 1700); solver wave: rows and
+// line solve 2400, publishing 900, waiting for the other chunks 4700,
+// separators and decision 1700, U to LDS 500.  Headline solve (N = 10^4, M =
+// 2 10^4) 373 -> 224 ms, N = 1000 35.7 -> 23.1 ms, six solves in a batch 58.9
+// -> 40.9 ms against the whole workgroup's cyclic reduction over LDS with both
+// chunk ends as separators (five words per row and level, a workgroup barrier
+// per level).
+//
+// The arithmetic is written with explicit fma and contraction off: single
+// and batched launches round alike in every instantiation.
 
-// A grid barrier waits at most `wait_ticks` ticks of the device's constant
-// wall clock (wall_clock64; the host sizes it to 2 s from the clock rate).
-// Workgroups of a cooperative launch can become resident late when other
-// streams' kernels hold CUs at dispatch (the 3D and far-part kernels that
-// advance beside a batch): those finish within micro- to milliseconds, far
-// inside the bound, which exists only so that a launch whose workgroups can
-// never all be resident ends with an error instead of hanging.
-
-// Grid exchange of the chunk workgroups.  Every value a workgroup publishes
-// for the others (its two reduced rows, its convergence measure) travels as
-// two 64-bit words, each holding one 32-bit half of the double and the 32-bit
-// tag of the barrier it belongs to (xtag | (barrier index + 1) mod 2^16; xtag
-// carries the launch count in its upper 16 bits, never 0).  Words are written
-// and read with relaxed agent-scope atomics: each is single-copy atomic and
-// coherent across the XCDs, and a reader takes a word once it carries the
-// barrier's tag, so it holds that barrier's value.  No fence orders one word
-// against another, so a barrier needs no L2 write-back or invalidate (the
-// release/acquire pair of a flag barrier costs more than the exchange).
-// Readers poll the measure words first (thread j < C polls chunk j's: few
-// pollers, little traffic while the last chunks are still computing), then
-// load the rows, which have landed or are about to; polling every word of
-// every row from the start was measured slower (its traffic delays the
-// writers' stores).
+// Grid exchange: the 8 values a chunk publishes per barrier travel as sixteen
+// 64-bit words in one 128-byte line, each holding one 32-bit half of a double
+// and the 32-bit tag of the barrier it belongs to (xtag | (barrier index + 1)
+// mod 2^16; xtag carries the launch count in its upper 16 bits, never 0).
+// Words are written and read with relaxed agent-scope atomics: each is
+// single-copy atomic and coherent across the XCDs, and a reader takes a word
+// once it carries the barrier's tag, so it holds that barrier's value.  No
+// fence orders one word against another, so a barrier needs no L2 write-back
+// or invalidate.  The writer stores its line by one instruction (lanes 0..15),
+// readers load four chunks' lines per instruction and transpose through LDS.
 //  - Words alternate by barrier parity.  A workgroup writes barrier b+1's
 //    words only after it has read every workgroup's barrier-b words, and each
 //    workgroup wrote those after reading its barrier-(b-1) words, so no word
@@ -555,421 +568,785 @@ __global__ __launch_bounds__(256) void k_step1d(Step1DArgs g) {
 //    dispatch, which ends within micro- to milliseconds; the bound exists so
 //    that a launch whose workgroups can never all be resident ends with an
 //    error instead of hanging.
-// Slots (two words each) per parity: value q of reduced row r at 4 r + q
-// (r < 2C), the measure of chunk j at kXchMeasure + j.
-constexpr int kXchMeasure = 8 * kMaxChunks;
-constexpr int kXchWords = 2 * (kXchMeasure + kMaxChunks);       // per parity
-static_assert(2 * kXchWords * 8 <= (int)kXchBytes, "exchange buffer size");
+// Values of chunk j: 0..3 its separator's row with the chunk's own interior
+// eliminated (coupling to the node left of it, diagonal, coupling to the next
+// separator, right-hand side), 4..6 x, y, z of its last node, 7 its measure.
+constexpr int kXchWords = 16;                                   // per chunk and parity
+constexpr int kXchMeasure = 14;                                 // first word of value 7
+constexpr int kXchPad = kXchWords + 2;                          // LDS row: 144 B, 16-byte reads spread over the banks
+static_assert(2 * kMaxChunks * kXchWords * 8 == (int)kXchBytes, "exchange buffer size");
 
-__device__ inline void xput(unsigned long long* x, int slot, unsigned tag, double v) {
-    const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-    const unsigned long long t = (unsigned long long)tag << 32;
-    __hip_atomic_store(x + 2 * slot, t | (b & 0xffffffffull), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_store(x + 2 * slot + 1, t | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+constexpr double kNoCoupling = 0x1p-60;                         // below: no effect on a double of its row's size
+
+// ---- one wave's line solve -------------------------------------------------
+// a double moved within the rows of 16 lanes; lanes without a source take fill
+template <int CTRL>
+__device__ inline double dpp_fill(double v, double fill) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(fill), __double2loint(v), CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(fill), __double2hiint(v), CTRL, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
 }
 
-// History term of step n at node i (levels t < n-1 in memory, the newest
-// difference dnew in a register, the two-level corrections of the oldest
-// intervals from d0m, d1m; Toeplitz weights or the step's own row; the
-// first `folded` near-field groups from g.mid).
-__device__ inline double hist_step(const Step1DArgs& g, int i, int n, double dnew, double d0m, double d1m,
-                                   int folded = 0) {
-    const double* om = g.omega + (int64_t)(n - g.n0) * g.omega_stride;
-    double hm = hist_mem(g, i, n, (int64_t)(n - g.n0) * g.ld, om, folded);
-    return hm + hist_tail(om[0], g.corr[2 * n], g.corr[2 * n + 1], n, g.near_lo, dnew, d0m, d1m);
+__device__ inline int lane_of(int p) { return 16 * (p & 3) + (p >> 2); }
+
+// The value of v at position p + OFF (p: this lane's); fill outside 0..63.
+template <int OFF>
+__device__ inline double at_offset(double v, int p, double fill) {
+    if constexpr (OFF % 4 == 0) {
+        constexpr int Q = OFF / 4;
+        if constexpr (Q > 0) return dpp_fill<0x100 + Q>(v, fill);          // row_shl: from lane + Q
+        else return dpp_fill<0x110 - Q>(v, fill);                          // row_shr: from lane - |Q|
+    } else {
+        const int q = p + OFF;
+        const int src = lane_of(q & 63) << 2;
+        const int lo = __builtin_amdgcn_ds_bpermute(src, __double2loint(v));
+        const int hi = __builtin_amdgcn_ds_bpermute(src, __double2hiint(v));
+        return (q >= 0 && q < 64) ? __hiloint2double(hi, lo) : fill;
+    }
 }
+
+// One level of cyclic reduction over the 64 positions (rows a x_{p-S} + x_p +
+// c x_{p+S} = d).  Past the ends stand the boundary values UL and UR: there a
+// and c stay couplings to them (the partner row "x = U").
+template <int S>
+__device__ inline void pcr_level(double& a, double& c, double& d, int p) {
+#pragma clang fp contract(off)
+    const double am = at_offset<-S>(a, p, -1.0), cm = at_offset<-S>(c, p, 0.0), dm = at_offset<-S>(d, p, 0.0);
+    const double ap = at_offset<S>(a, p, 0.0), cp = at_offset<S>(c, p, -1.0), dp = at_offset<S>(d, p, 0.0);
+    const double inv = rcp_nr(fma(-c, ap, fma(-a, cm, 1.0)));
+    d = fma(-c, dp, fma(-a, dm, d)) * inv;
+    a = -(a * am) * inv;
+    c = -(c * cp) * inv;
+}
+
+// Whether some row still couples to a row S positions away (NaN counts).
+template <int S>
+__device__ inline bool coupled(double a, double c, int p) {
+    const bool l = p >= S && !(fabs(a) <= kNoCoupling), r = p + S < 64 && !(fabs(c) <= kNoCoupling);
+    return __any(l || r);
+}
+
+// Solve the 64 R rows a x_{i-1} + x_i + c x_{i+1} = d of one wave (position p
+// holds rows R p .. R p + R-1) between the boundary values UL (left of row 0)
+// and UR (right of the last): x_i = x + y UL + z UR.  A position's first R-1
+// rows are eliminated against its last one (Thomas with both couplings as
+// right-hand sides), the last ones reduced cyclically.  With EARLY the
+// reduction stops once no coupling between positions exceeds 2^-60 (the
+// boundaries' couplings must be zero: y and z are not formed).
+template <int R, bool EARLY>
+__device__ inline void wave_line(const double (&a)[R], const double (&c)[R], const double (&d)[R], int p,
+                                 double (&x)[R], double (&y)[R], double (&z)[R]) {
+#pragma clang fp contract(off)
+    double A = a[R - 1], Cc = c[R - 1], Dd = d[R - 1];
+    if constexpr (R > 1) {
+        double q[R];                               // c' of the elimination
+        x[0] = d[0];
+        y[0] = -a[0];
+        q[0] = c[0];
+#pragma unroll
+        for (int j = 1; j < R - 1; j++) {
+            const double inv = rcp_nr(fma(-a[j], q[j - 1], 1.0));
+            q[j] = c[j] * inv;
+            x[j] = fma(-a[j], x[j - 1], d[j]) * inv;
+            y[j] = -(a[j] * y[j - 1]) * inv;
+        }
+        z[R - 2] = -q[R - 2];
+#pragma unroll
+        for (int j = R - 3; j >= 0; j--) {
+            x[j] = fma(-q[j], x[j + 1], x[j]);
+            y[j] = fma(-q[j], y[j + 1], y[j]);
+            z[j] = -(q[j] * z[j + 1]);
+        }
+        // the position's last row: its left neighbour and the next position's first row put in
+        const double xn = at_offset<1>(x[0], p, 0.0), yn = at_offset<1>(y[0], p, 0.0), zn = at_offset<1>(z[0], p, 1.0);
+        const double inv = rcp_nr(fma(Cc, yn, fma(A, z[R - 2], 1.0)));
+        Dd = fma(-Cc, xn, fma(-A, x[R - 2], Dd)) * inv;
+        A = (A * y[R - 2]) * inv;
+        Cc = (Cc * zn) * inv;
+    }
+    // (the last position's c goes to UR)
+    if constexpr (EARLY) {
+        if (coupled<1>(A, Cc, p)) {
+            pcr_level<1>(A, Cc, Dd, p);
+            if (coupled<2>(A, Cc, p)) {
+                pcr_level<2>(A, Cc, Dd, p);
+                if (coupled<4>(A, Cc, p)) {
+                    pcr_level<4>(A, Cc, Dd, p);
+                    if (coupled<8>(A, Cc, p)) {
+                        pcr_level<8>(A, Cc, Dd, p);
+                        if (coupled<16>(A, Cc, p)) {
+                            pcr_level<16>(A, Cc, Dd, p);
+                            if (coupled<32>(A, Cc, p)) pcr_level<32>(A, Cc, Dd, p);
+                        }
+                    }
+                }
+            }
+        }
+        x[R - 1] = Dd;
+        y[R - 1] = z[R - 1] = 0.0;
+        if constexpr (R > 1) {
+            const double xl = at_offset<-1>(Dd, p, 0.0);
+#pragma unroll
+            for (int j = 0; j < R - 1; j++) x[j] = fma(z[j], Dd, fma(y[j], xl, x[j]));
+        }
+    } else {
+        pcr_level<1>(A, Cc, Dd, p);
+        pcr_level<2>(A, Cc, Dd, p);
+        pcr_level<4>(A, Cc, Dd, p);
+        pcr_level<8>(A, Cc, Dd, p);
+        pcr_level<16>(A, Cc, Dd, p);
+        pcr_level<32>(A, Cc, Dd, p);
+        x[R - 1] = Dd;
+        y[R - 1] = -A;
+        z[R - 1] = -Cc;
+        if constexpr (R > 1) {
+            // the left neighbour position's last row (row 0's: UL itself)
+            const double xl = at_offset<-1>(x[R - 1], p, 0.0), yl = at_offset<-1>(y[R - 1], p, 1.0),
+                         zl = at_offset<-1>(z[R - 1], p, 0.0);
+#pragma unroll
+            for (int j = 0; j < R - 1; j++) {
+                const double y0 = y[j], z0 = z[j];
+                x[j] = fma(z0, x[R - 1], fma(y0, xl, x[j]));
+                y[j] = fma(z0, y[R - 1], y0 * yl);
+                z[j] = fma(z0, z[R - 1], y0 * zl);
+            }
+        }
+    }
+}
+
+// Row `row` of a solved line in every lane (row is uniform).
+template <int R>
+__device__ inline double line_value(const double (&x)[R], int row) {
+    double v = x[0];
+#pragma unroll
+    for (int j = 1; j < R; j++) {
+        double t = x[j];
+        asm("" : "+v"(t));                          // a select of values, not of places in an array in memory
+        v = (row % R == j) ? t : v;
+    }
+    const int l = __builtin_amdgcn_readfirstlane(lane_of(row / R));
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// LDS operations of one wave complete in order; these keep the compiler from
+// moving them across a hand-over between lanes
+__device__ inline void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+constexpr int kRows = 256;                                      // nodes per chunk at most
+// position of chunk row r in the LDS row arrays: one double of padding per 32
+// keeps the solver wave's reads at stride R doubles free of bank conflicts
+__device__ inline int row_slot(int r) { return r + (r >> 5); }
+constexpr int kRowSlots = kRows + 1 + (kRows >> 5) + 1;
+
+struct Step1DLds {
+    double K[kRowSlots], iC[kRowSlots], d[kRowSlots], u[kRowSlots];
+    double pub[8];
+    double weights[4][128];                                     // per row wave: of a fold or a near field
+    alignas(16) unsigned long long words[kMaxChunks * kXchPad];
+    int status;
+};
+
+enum { kNoCheck = 0, kCheckMet, kCheckPending, kDecide };         // what an exchange decides
+enum { kSolved = 0, kMet, kNotMet, kRollback, kTimeout };         // and what came of it
+
+// Value k of chunk j from its words in LDS.
+__device__ inline double xch_value(const Step1DLds& L, int j, int k) {
+    const ulonglong2 w = *reinterpret_cast<const ulonglong2*>(&L.words[j * kXchPad + 2 * k]);
+    return __longlong_as_double((long long)((w.y << 32) | (w.x & 0xffffffffull)));
+}
+
+// The separators' system: RR rows per lane.  Returns the values at the
+// separators c-1, c and c+1 (0 past the ends).
+template <int RR>
+__device__ inline void solve_separators(const Step1DLds& L, int C, int c, int p, double& xm, double& x0, double& xp) {
+#pragma clang fp contract(off)
+    double a[RR], cc[RR], d[RR], x[RR], y[RR], z[RR];
+#pragma unroll
+    for (int j = 0; j < RR; j++) {
+        const int r = RR * p + j;
+        const bool ok = r < C;
+        const int rr = ok ? r : 0, rl = rr > 0 ? rr - 1 : 0;
+        const double v0 = xch_value(L, rr, 0), v1 = xch_value(L, rr, 1), v2 = xch_value(L, rr, 2),
+                     v3 = xch_value(L, rr, 3);
+        // (row 0 has v0 = 0: what is read for its left neighbour does not enter)
+        const double xl = rr > 0 ? xch_value(L, rl, 4) : 0.0, yl = rr > 0 ? xch_value(L, rl, 5) : 0.0,
+                     zl = rr > 0 ? xch_value(L, rl, 6) : 0.0;
+        const double inv = rcp_nr(fma(v0, zl, v1));
+        a[j] = ok ? (v0 * yl) * inv : 0.0;
+        cc[j] = ok && r + 1 < C ? v2 * inv : 0.0;
+        d[j] = ok ? fma(-v0, xl, v3) * inv : 0.0;
+    }
+    wave_line<RR, true>(a, cc, d, p, x, y, z);
+    xm = c > 0 ? line_value<RR>(x, c - 1) : 0.0;
+    x0 = line_value<RR>(x, c);
+    xp = c + 1 < C ? line_value<RR>(x, c + 1) : 0.0;
+}
+
+// Where a launch stands: step n, Picard iteration k of it, and what the next
+// exchange decides.  Both roles of a workgroup run it on the same results, so
+// it stays uniform.  A step whose last Picard iteration is due (k =
+// picard_max - 1) ends tentatively with U^k when the launch has a next step:
+// its convergence measure goes out with the next step's first iteration, so
+// the exchange that decides it is the one that carries those rows.  If it did
+// not converge, every workgroup restores the step, runs its last iteration,
+// rewrites D[n] and U, and starts the next step again.  Series moments are
+// updated in place, so sum_alg 2 decides convergence before the step ends.
+enum { kGoOn = 0, kStepEnds, kStepEndsTentatively, kGoBack, kLeave };
+struct PicardState {
+    int n, n_end, k, check, picard_max, solves;
+    bool pending, redo, tentative_ok;
+    __device__ inline void begin(int n_, bool pending_) {
+        n = n_;
+        k = 0;
+        redo = false;
+        pending = pending_;
+        check = pending ? kCheckPending : kNoCheck;
+    }
+    __device__ inline int after(int st) {
+        if (st == kSolved) {
+            solves++;
+            k++;
+            pending = false;
+            if (redo || k == picard_max) return kStepEnds;
+            const bool due = k == picard_max - 1;
+            if (due && tentative_ok && n + 1 < n_end) return kStepEndsTentatively;
+            check = due ? kDecide : kCheckMet;     // (due: decided before the last iteration, which it may save)
+            return kGoOn;
+        }
+        if (st == kNotMet) { check = kNoCheck; return kGoOn; }
+        return st == kMet ? kStepEnds : (st == kRollback ? kGoBack : kLeave);
+    }
+    __device__ inline void back(int n_) {          // to the last iteration of step n_
+        n = n_;
+        redo = true;
+        pending = false;
+        check = kNoCheck;
+    }
+};
+
+__device__ inline PicardState picard_state(const Step1DArgs& g) {
+    PicardState ps{};
+    ps.n_end = g.n_end;
+    ps.picard_max = g.picard_max;
+    ps.tentative_ok = g.ser_P == 0;
+    ps.begin(g.n, false);
+    return ps;
+}
+
+// A launch constant kept in vector registers (the two roles have more of them
+// than scalar registers, and a spilled scalar costs two moves per use).
+__device__ inline double in_vgpr(double v) { asm("" : "+v"(v)); return v; }
 
 // Steps [g.n, g.n_end) of one solve by its chunk workgroup c (0 <= c < g.C):
-// the body of the single-solve launch and of the batched one.
-__device__ __forceinline__ void step_block(const Step1DArgs& g, const int c) {
-    __shared__ double rA[2][kMaxRed], rC[2][kMaxRed], rD[2][kMaxRed];
-    __shared__ double pA[2][256], pC[2][256], pX[2][256], pY[2][256], pZ[2][256];
-    __shared__ double sK[258];
-    __shared__ double sdp[4];                  // wave maxima of the last solve's |U^{k+1} - U^k|
-    __shared__ double sMeas[kMaxChunks];       // every chunk's published measure of the last barrier
-    __shared__ int sh_fail;                    // a barrier wait ran out of time
+// a row wave.  Each thread keeps NPT nodes of the chunk, 64 RW apart.
+template <int RW, int NPT>
+__device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step1DLds& L) {
+#pragma clang fp contract(off)
     const int tid = threadIdx.x;
-    const int N = g.N, C = g.C;
-    const int s = (int)(((int64_t)c * N) / C);
-    const int e = (int)(((int64_t)(c + 1) * N) / C) - 1;
-    const int nc = e - s + 1;
-    const int i = s + tid;
-    const bool act = tid < nc;
-    const int R2 = 2 * C;
+    const int s = (int)(((int64_t)c * g.N) / g.C);
+    const int nc = (int)(((int64_t)(c + 1) * g.N) / g.C) - s;
     const bool series = g.ser_P > 0;
-    const int halo_tid = (nc < 256) ? 255 : 0;
-    const bool halo = tid == halo_tid && c > 0;
-    const int wave = tid >> 6, lane = tid & 63;
-    const int ni = nc - 2;
-    const int q = tid - 1;
-    const bool inner = (tid >= 1) && (tid <= nc - 2);
+    const double ksat = in_vgpr(g.ksat);
+    auto row = [&](int q) { return tid + 64 * RW * q; };       // this thread's chunk rows
+    auto act = [&](int q) { return row(q) < nc; };
 
-    // state carried from step to step: U^n and D[n-1] of the own node and of
-    // the halo node s-1 (from memory at the first step of the launch)
+    // state carried from step to step: U^n and D[n-1] of the node (from
+    // memory at the first step of the launch)
     const int n_first = g.n;
-    double un = act ? g.U[i] : 0.0;
-    double dlast = 0.0;
-    if (act && n_first >= 1) dlast = g.D[(series ? ((n_first - 1) & 1) : (n_first - 1)) * g.ld + i];
-    double uh = halo ? g.U[s - 1] : 0.0;
-    double dh = 0.0;
-    if (halo && n_first >= 1) dh = g.D[(series ? ((n_first - 1) & 1) : (n_first - 1)) * g.ld + s - 1];
-    // D[0], D[1] (corrections of the two oldest intervals): from memory when
-    // written by an earlier launch, else taken when this launch makes them
-    double d0m = (!series && act && n_first >= 1) ? g.D[i] : 0.0;
-    double d1m = (!series && act && n_first >= 2) ? g.D[g.ld + i] : 0.0;
-    int bk = 0;                                                    // Picard barriers passed in this launch
-    // Near-field groups of this history block folded into g.mid so far.
-    // The first build of a step s of the block that has a later step in the
-    // block folds every group j (levels near_lo + 16 j ...+15) with
-    // near_lo + 16 j + 17 <= s, i.e. whose levels are final (t <= s - 2)
-    // whatever the previous step's decision; after the steps [n0, s] of the
-    // block that makes (s - near_lo - 1) / 16 groups.  Those of earlier
-    // launches of the block are counted here.
-    int folded = 0;
-    if (g.mid) {
-        const int s_last = min(n_first - 1, g.n0 + g.blk - 2);
-        folded = s_last >= g.n0 ? (s_last - g.near_lo - 1) / kNearGroup : 0;
+    double zi[NPT], un[NPT], dlast[NPT], d0m[NPT], d1m[NPT];
+    double* const Dc = g.D + s + min(tid, nc - 1);             // the first node's column of D (idle threads: the last node's)
+    auto level = [&](int q, int m) { return Dc + 64 * RW * q + (int64_t)(series ? (m & 1) : m) * g.ld; };
+#pragma unroll
+    for (int q = 0; q < NPT; q++) {
+        const bool ok = act(q);
+        zi[q] = in_vgpr((s + row(q)) * g.h);
+        un[q] = ok ? g.U[s + row(q)] : 0.0;
+        dlast[q] = (ok && n_first >= 1) ? *level(q, n_first - 1) : 0.0;
+        // D[0], D[1] (corrections of the two oldest intervals): from memory
+        // when written by an earlier launch, else taken when this launch
+        // makes them
+        d0m[q] = (!series && ok && n_first >= 1) ? *level(q, 0) : 0.0;
+        d1m[q] = (!series && ok && n_first >= 2) ? *level(q, 1) : 0.0;
     }
-    // the exchange words of this workgroup, both parities, zeroed before its
-    // first publication (its rows 2c and 2c+1, its measure)
-    auto xbase = [&](int b) { return g.xch + (size_t)(b & 1) * kXchWords; };
-    auto xtag = [&](int b) { return g.xtag | ((unsigned)(b + 1) & 0xffffu); };
-    if (tid == 0 || tid == nc - 1) {
-        for (int par = 0; par < 2; par++) {
-            unsigned long long* x = g.xch + (size_t)par * kXchWords;
-            const int r = (tid == 0) ? 2 * c : 2 * c + 1;
-            for (int w = 0; w < 8; w++)
-                __hip_atomic_store(x + 8 * r + w, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (tid == 0)
-                for (int w = 0; w < 2; w++)
-                    __hip_atomic_store(x + 2 * (kXchMeasure + c) + w, 0ull, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
-    if (tid == 0) sh_fail = 0;
-    // the words of barrier b: thread j < C the measure of chunk j (into
-    // sMeas), then (rows = true) thread r reduced rows r and r + 256; then a
-    // workgroup barrier.  False when a wait ran out of time (the launch then
-    // ends; the host reports it).
-    auto read_barrier = [&](int b, bool rows, double (*rrow)[4]) -> bool {
-        const unsigned long long* xr = xbase(b);
-        const unsigned tg = xtag(b);
-        const unsigned long long none = (unsigned long long)tg << 32;
-        const int64_t tmax = g.wait_ticks;
-        // load the words the predicate leaves to this thread until all carry
-        // the tag (missing ones reloaded together); false after tmax ticks
-        auto take = [&](unsigned long long* w, int cnt, const unsigned long long* src) -> bool {
-            int64_t t0 = -1;
-            for (;;) {
-                bool all = true;
-                for (int k = 0; k < cnt; k++) all = all && (unsigned)(w[k] >> 32) == tg;
-                if (all) return true;
-                const int64_t now = (int64_t)wall_clock64();
-                if (t0 < 0) t0 = now;
-                else if (now - t0 > tmax) return false;
-                __builtin_amdgcn_s_sleep(1);
-                for (int k = 0; k < cnt; k++)
-                    if ((unsigned)(w[k] >> 32) != tg)
-                        w[k] = __hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // Near-field groups folded ahead into g.mid: group j (levels near_lo + 16 j
+    // ...+15) is final, whatever the pending decision on the previous step,
+    // from step s_j = near_lo + 16 j + 17 on (levels t <= s_j - 2; n0 if that
+    // is later).  The first iteration of step s_j + b folds it for the 8 steps
+    // from s_j + 2 + 8 b on, so a fold is spread over the steps that follow
+    // (done at once for a whole block it stalled the chain: 56 dependent
+    // batches per 128-step block), and step m's history, formed at step m - 1,
+    // finds every group with s_j < m - 1 and sums the other levels itself (at
+    // most 17; near_lo is n0 or up to 31 levels before it).  The schedule
+    // depends on the step alone: launches may end anywhere in a block.
+    auto ready = [&](int j) { return max(g.n0, g.near_lo + kNearGroup * j + kNearGroup + 1); };    // s_j
+    auto groups = [&](int m) { return g.mid && m - 2 >= g.n0 ? (m - 3 - g.near_lo) / kNearGroup : 0; };
+    int fold_done = n_first - 1;                               // (a step done again does not fold again)
+    PicardState ps = picard_state(g);
+    // of a tentatively ended step, what its last iteration still needs
+    double sv_un[NPT], sv_S[NPT];
+    // the in-memory part of the history sum (far partials and near levels
+    // t < n) and the tail weights omega[0], corr[2n], corr[2n+1]: of this step
+    // and of the next one (formed beside this step's first line solve)
+    double hm[NPT], hm_next[NPT];
+    double w0 = 0.0, w1 = 0.0, w2 = 0.0, w0_next = 0.0, w1_next = 0.0, w2_next = 0.0;
+    double S[NPT], it[NPT];
+    double Ln = 0.0;
+#pragma unroll
+    for (int q = 0; q < NPT; q++) sv_un[q] = sv_S[q] = hm[q] = hm_next[q] = 0.0;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    double* const wl = L.weights[wave];
+    // step m's history from memory (levels t < m - 1).  Every load of a node
+    // goes out before the first is used (one memory round trip), the weights
+    // once per wave, through LDS.
+    auto history = [&](int m, double (&h)[NPT], double& a0, double& a1, double& a2) {
+        const double* om = g.omega + (int64_t)(m - g.n0) * g.omega_stride;
+        a0 = om[0];
+        a1 = g.corr[2 * m];
+        a2 = g.corr[2 * m + 1];
+        const int folded = groups(m);
+        const int lo = g.near_lo + kNearGroup * folded;
+        constexpr int W = 16;
+        wl[lane] = om[1 + min(lane, max(m - 2 - lo, 0))];      // wl[k]: weight of level m - 2 - k
+        wave_lds_sync();
+#pragma unroll
+        for (int q = 0; q < NPT; q++) {
+            const int col = act(q) ? 64 * RW * q : 0;          // (idle threads read a column that exists)
+            const double* pt = g.part + (int64_t)(m - g.n0) * g.ld + (Dc - g.D) + col;
+            const double* d = Dc + (int64_t)lo * g.ld + col;
+            double v[W], f0 = 0.0, f1 = 0.0, md = 0.0;
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                v[j] = 0.0;
+                if (lo + j < m - 1) v[j] = *d;
+                d += g.ld;
+                asm("" : "+v"(d));                             // (one running address)
             }
-        };
-        bool ok = true;
-        // first the measures (one pair of words per chunk, the last words a
-        // chunk publishes from its thread 0): few pollers while the others
-        // are still on their way
-        unsigned long long mw[2] = {none, none};
-        if (tid < C) {
-            const unsigned long long* src = xr + 2 * (kXchMeasure + tid);
-            mw[0] = __hip_atomic_load(src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            mw[1] = __hip_atomic_load(src + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ok = take(mw, 2, src);
-        }
-        // then the rows, which have landed or are about to
-        unsigned long long rw[2][8];
-        if (rows) {
-            __syncthreads();
+            if (g.nsplit > 0) f0 = pt[0];
+            if (g.nsplit > 1) f1 = pt[g.part_stride];
+            if (folded > 0) md = g.mid[(int64_t)(m - g.n0) * g.ld + (Dc - g.D) + col];
+            double far = f0 + f1;
+            for (int k = 2; k < g.nsplit; k++) far += pt[(int64_t)k * g.part_stride];
+            double n0 = md, n1 = 0.0;
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const int r = tid + 256 * j;
-#pragma unroll
-                for (int w = 0; w < 8; w++)
-                    rw[j][w] = (r < R2) ? __hip_atomic_load(xr + 8 * r + w, __ATOMIC_RELAXED,
-                                                            __HIP_MEMORY_SCOPE_AGENT)
-                                        : none;
+            for (int j = 0; j < W; j += 2) {
+                n0 = fma(wl[max(m - 2 - lo - j, 0)], v[j], n0);
+                n1 = fma(wl[max(m - 3 - lo - j, 0)], v[j + 1], n1);
             }
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-                if (tid + 256 * j < R2) ok = ok && take(rw[j], 8, xr + 8 * (tid + 256 * j));
+            // levels past the first 16 (a 17th, or a block without g.mid)
+            for (int t = lo + W; t < m - 1; t++) n0 = fma(om[m - 1 - t], Dc[(int64_t)t * g.ld + col], n0);
+            h[q] = far + (n0 + n1);
         }
-        if (!ok) {
-            __hip_atomic_store(g.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            sh_fail = 1;
-        }
-        auto dec = [](unsigned long long lo, unsigned long long hi) {
-            return __longlong_as_double((long long)((hi << 32) | (lo & 0xffffffffull)));
-        };
-        if (tid < C) sMeas[tid] = dec(mw[0], mw[1]);
-        if (rows)
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int qq = 0; qq < 4; qq++) rrow[j][qq] = dec(rw[j][2 * qq], rw[j][2 * qq + 1]);
-        __syncthreads();
-        return sh_fail == 0;
+        wave_lds_sync();
     };
-    // the maximum of the staged measures, formed by every wave itself
-    auto measures_max = [&]() {
-        double dv = 0.0;
-        for (int j = lane; j < C; j += 64) dv = fmax(dv, sMeas[j]);
-        return wave_max(dv);
-    };
-
-    if (tid < 4) sdp[tid] = 0.0;
-    // the chunk's max |U^{k+1} - U^k| of the last solve (thread 0, after a
-    // workgroup barrier that follows that solve)
-    auto last_measure = [&]() { return fmax(fmax(sdp[0], sdp[1]), fmax(sdp[2], sdp[3])); };
-
-    // ---- one Picard build: coefficients at the iterate (uit, uith), rows,
-    // chunk elimination (chunk factors into fx, fy, fz), the two reduced rows
-    // published with the last solve's measure in the convergence slot, then
-    // the grid barrier
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    // the part of the next step's history sum that is already in memory
-    // (far partials and near levels t < n), formed while a barrier is pending
-    double hm_next = 0.0;
-    double tl_next[3] = {0.0, 0.0, 0.0};       // and its tail weights: omega[0], corr[2n], corr[2n+1]
-    auto build = [&](double uit, double uith, double S, double Ln, double un_, int pre_n, int fold_n) -> bool {
-        double K = 0.0, invC = 0.0;
-        if (halo) {
-            double Kl, iCl;
-            vgm_coefs(uith, (s - 1) * g.h, g.ksat, g.coef_mode, Kl, iCl);
-            sK[0] = Kl;
-        }
-        if (act) {
-            vgm_coefs(uit, i * g.h, g.ksat, g.coef_mode, K, invC);
-            sK[tid + 1] = K;
-        }
-        __syncthreads();
-        double ar = 0.0, br = 1.0, cr = 0.0, dr = 0.0;
-        if (act) {
-            if (i == 0) { ar = 0.0; br = 1.0; cr = 0.0; dr = g.utop; }
-            else if (i == N - 1) { ar = -1.0; br = 1.0; cr = 0.0; dr = 0.0; }
-            else {
-                double Km = sK[tid], Kp = sK[tid + 1];
-                double A = Km * invC * g.h2inv;
-                double B = Kp * invC * g.h2inv;
-                double R = invC * (Kp * g.h2inv + Km * g.h2inv) + Ln;
-                ar = A; br = -R; cr = B; dr = -Ln * un_ + S;
-            }
-        }
-        double ib = inner ? rcp_nr(br) : 0.0;
-        const int pp = chunk_solve(pA, pC, pX, pY, pZ, ni, q, inner, (tid == 1) ? 0.0 : ar * ib,
-                                   (tid == nc - 2) ? 0.0 : cr * ib, dr * ib, (tid == 1) ? -ar * ib : 0.0,
-                                   (tid == nc - 2) ? -cr * ib : 0.0);
-        fx = 0.0; fy = 0.0; fz = 0.0;
-        if (inner) { fx = pX[pp][q]; fy = pY[pp][q]; fz = pZ[pp][q]; }
-        unsigned long long* xw = xbase(bk);
-        const unsigned tg = xtag(bk);
-        if (tid == 0) {
-            double x, y, z;
-            if (nc == 2) { x = 0.0; y = 0.0; z = 1.0; }
-            else { x = pX[pp][0]; y = pY[pp][0]; z = pZ[pp][0]; }
-            xput(xw, 4 * (2 * c) + 0, tg, ar);
-            xput(xw, 4 * (2 * c) + 1, tg, br + cr * y);
-            xput(xw, 4 * (2 * c) + 2, tg, cr * z);
-            xput(xw, 4 * (2 * c) + 3, tg, dr - cr * x);
-            xput(xw, kXchMeasure + c, tg, last_measure());
-        }
-        if (tid == nc - 1) {
-            double x, y, z;
-            if (nc == 2) { x = 0.0; y = 1.0; z = 0.0; }
-            else { x = pX[pp][ni - 1]; y = pY[pp][ni - 1]; z = pZ[pp][ni - 1]; }
-            xput(xw, 4 * (2 * c + 1) + 0, tg, ar * y);
-            xput(xw, 4 * (2 * c + 1) + 1, tg, br + ar * z);
-            xput(xw, 4 * (2 * c + 1) + 2, tg, cr);
-            xput(xw, 4 * (2 * c + 1) + 3, tg, dr - ar * x);
-        }
-        // the next near-field group whose levels are final (t <= step - 2)
-        // folded for the later steps of the block, while the exchange is
-        // pending (first build of a step only)
-        if (fold_n >= 0 && g.mid) {
-            while (g.near_lo + kNearGroup * folded + kNearGroup + 1 <= fold_n && fold_n + 1 < g.n0 + g.blk) {
-                if (act)
-                    fold_near_group(g.D, g.ld, g.omega, g.omega_stride, g.n0, g.mid, i,
-                                    g.near_lo + kNearGroup * folded, fold_n + 1, g.n0 + g.blk, folded == 0);
-                folded++;
-            }
-        }
-        if (pre_n >= 0 && act) {
-            const double* om = g.omega + (int64_t)(pre_n - g.n0) * g.omega_stride;
-            tl_next[0] = om[0];
-            tl_next[1] = g.corr[2 * pre_n];
-            tl_next[2] = g.corr[2 * pre_n + 1];
-            hm_next = hist_mem(g, i, pre_n, (int64_t)(pre_n - g.n0) * g.ld, om, folded);
-        }
-        bk++;                                  // the solve reads this barrier's words
-        return true;
-    };
-    // ---- after a build's barrier: the reduced rows; with check != 0 first
-    // the decision on the published convergence slots (check 1: U^k met the
-    // tolerance -> return 1, nothing solved; check 2: the tentatively ended
-    // previous step did not -> return 2, nothing solved); then the reduced
-    // solve and back-substitution (uit, uith updated), return 0.  Every wave
-    // forms the decision's maximum itself, so it is uniform without a
-    // workgroup barrier.  The chunk's max |U^{k+1} - U^k| is left as four
-    // wave maxima in sdp for thread 0, which publishes it with the next build.
-    auto solve = [&](int check, double& uit, double& uith) -> int {
-        double rrow[2][4];
-        if (!read_barrier(bk - 1, true, rrow)) return -1;
-        if (check) {
-            const bool met = measures_max() <= g.tol;
-            if (check == 1 && met) return 1;
-            if (check == 2 && !met) return 2;
-        }
+    // group j of 16 levels into g.mid for the steps [p0, p1), p1 - p0 <= 8
+    auto fold = [&](int j, int p0, int p1) {
+        const int lo = g.near_lo + kNearGroup * j;
+        // weight of level lo + k at step p0 + r: wl[16 r + k]
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int r = tid + 256 * j;
-            if (r < R2) {
-                double ib = rcp_nr(rrow[j][1]);
-                rA[0][r] = rrow[j][0] * ib;
-                rC[0][r] = rrow[j][2] * ib;
-                rD[0][r] = rrow[j][3] * ib;
+        for (int h = 0; h < 2; h++) {
+            const int q = lane + 64 * h, pr = min(p0 + (q >> 4), p1 - 1);
+            wl[q] = g.omega[(int64_t)(pr - g.n0) * g.omega_stride + pr - lo - 1 - (q & 15)];
+        }
+        wave_lds_sync();
+#pragma unroll 1
+        for (int q = 0; q < NPT; q++) {
+            if (!act(q)) break;
+            double dv[kNearGroup], acc[kFoldBatch];
+            const double* d = Dc + (int64_t)lo * g.ld + 64 * RW * q;
+            double* mp = g.mid + (int64_t)(p0 - g.n0) * g.ld + (Dc - g.D) + 64 * RW * q;
+            const double* mr = mp;
+#pragma unroll
+            for (int k = 0; k < kNearGroup; k++) {
+                dv[k] = *d;
+                d += g.ld;
+                asm("" : "+v"(d));
+            }
+#pragma unroll
+            for (int r = 0; r < kFoldBatch; r++) {
+                acc[r] = 0.0;
+                if (j > 0 && p0 + r < p1) acc[r] = *mr;
+                mr += g.ld;
+                asm("" : "+v"(mr));
+            }
+#pragma unroll
+            for (int r = 0; r < kFoldBatch; r++) {
+#pragma unroll
+                for (int k = 0; k < kNearGroup; k++) acc[r] = fma(wl[16 * r + k], dv[k], acc[r]);
+                if (p0 + r < p1) *mp = acc[r];
+                mp += g.ld;
+                asm("" : "+v"(mp));
             }
         }
-        __syncthreads();
-        const double* xs = &rD[pcr_norm(rA, rC, rD, R2)][0];
-        double unew = 0.0;
-        if (act) {
-            if (i == s) unew = xs[2 * c];
-            else if (i == e) unew = xs[2 * c + 1];
-            else unew = fx + fy * xs[2 * c] + fz * xs[2 * c + 1];
-        }
-        double unewh = halo ? xs[2 * c - 1] : 0.0;
-        const double d = wave_max(act ? fabs(unew - uit) : 0.0);
-        if (lane == 0) sdp[wave] = d;
-        uit = unew;
-        uith = unewh;
-        return 0;
+        wave_lds_sync();
     };
-    // ---- end of step m with U^{m+1} = (res, resh): D[m], U, carried state
-    auto finish = [&](int m, double res, double resh) {
-        double dn = res - un;
-        if (act) {
-            g.D[(series ? (m & 1) : m) * g.ld + i] = dn;
-            g.U[i] = res;
+    auto start_step = [&]() {
+        const int n = ps.n;
+        // local coefficient: one, or the step's own (prescribed grid)
+        Ln = g.Lv ? g.Lv[n] : g.L;
+#pragma unroll
+        for (int q = 0; q < NPT; q++) {
+            S[q] = 0.0;
+            if (n >= 1 && act(q))
+                S[q] = series ? series_update(g.H, g.ld, s + row(q), g.ser_P, dlast[q], g.ser_c + (size_t)n * g.ser_P,
+                                              g.ser_v + (size_t)n * g.ser_P)
+                              : hm[q] + hist_tail(w0, w1, w2, n, g.near_lo, dlast[q], d0m[q], d1m[q]);
+            // Picard starts from 2 U^n - U^{n-1} (a single pass: lagged at U^n)
+            it[q] = (g.extrap && n >= 1) ? un[q] + dlast[q] : un[q];
         }
-        dh = resh - uh;
-        uh = resh;
-        dlast = dn;
-        un = res;
-        if (m == 0) d0m = dn;
-        if (m == 1) d1m = dn;
     };
-
-    // A step whose last Picard iteration is due (k = picard_max - 1) ends
-    // tentatively with U^k when the launch has a next step: its convergence
-    // measure goes out in the convergence slots of the next step's first
-    // build, so the barrier that decides it is the one that exchanges those
-    // rows.  If it did not converge, every workgroup (the decision is
-    // uniform) restores the step, runs its last iteration, rewrites D[n] and
-    // U, and starts the next step again.  Series moments are updated in
-    // place, so sum_alg 2 decides convergence before the step ends.
-    bool pending = false;          // the previous step ended tentatively
-    int sv_n = 0;                  // that step's state, for a rollback
-    double sv_un = 0.0, sv_uh = 0.0, sv_dh = 0.0, sv_dlast = 0.0, sv_d0m = 0.0, sv_d1m = 0.0;
-    double sv_S = 0.0, sv_Ln = 0.0, sv_uit = 0.0, sv_uith = 0.0;
-    double hm_cur = 0.0;           // that part for the current step
-    double tl_cur[3] = {0.0, 0.0, 0.0};
-    bool have_hm = false;
-    int nsolve = 0;                // Picard iterations solved (the decisions are uniform)
-    int n = n_first;
-    while (n < g.n_end) {
-        // ---- history term of step n -------------------------------------
-        // weights of step n: one Toeplitz vector, or the step's own row
-        // (prescribed grid); local coefficient likewise
-        const double Ln = g.Lv ? g.Lv[n] : g.L;
-        double S = 0.0;
-        if (n >= 1 && act) {
-            if (series) {
-                S = series_update(g.H, g.ld, i, g.ser_P, dlast, g.ser_c + (size_t)n * g.ser_P,
-                                  g.ser_v + (size_t)n * g.ser_P);
-            } else if (have_hm) {
-                S = hm_cur + hist_tail(tl_cur[0], tl_cur[1], tl_cur[2], n, g.near_lo, dlast, d0m, d1m);
-            } else {
-                S = hist_step(g, i, n, dlast, d0m, d1m, folded);
+    if (!series && n_first >= 1) history(n_first, hm, w0, w1, w2);
+    start_step();
+    bool fresh = true;                                         // the step's first iteration
+    for (;;) {
+        if (ps.check != kDecide) {
+#pragma unroll
+            for (int q = 0; q < NPT; q++) {
+                double K, invC;
+                vgm_coefs(it[q], zi[q], ksat, g.coef_mode, K, invC);
+                if (act(q)) {
+                    const int slot = row_slot(row(q));
+                    L.K[slot] = K;
+                    L.iC[slot] = invC;
+                    L.d[slot] = s + row(q) == 0 ? g.utop : fma(-Ln, un[q], S[q]);
+                }
             }
         }
-        // the next step's in-memory history part goes with this step's first
-        // barrier (levels t < n are written; D[n] enters through the tail)
-        const int pre_n = (!series && n + 1 < g.n_end) ? n + 1 : -1;
-        // Picard starts from 2 U^n - U^{n-1} (a single pass: lagged at U^n)
-        double uit = un, uith = uh;
-        if (g.extrap && n >= 1) { uit = un + dlast; uith = uh + dh; }
-        bool tentative = false, rollback = false;
-        for (int k = 0; k < g.picard_max; k++) {
-            const bool last_due = k >= 1 && k == g.picard_max - 1;
-            if (last_due && !series && n + 1 < g.n_end) {
-                tentative = true;            // U^k ends the step, decided with the next build
-                break;
+        __syncthreads();                                       // A
+        if (fresh && !series) {
+            if (g.mid && ps.n > fold_done) {
+                fold_done = ps.n;
+                for (int j = 0; j < groups(ps.n + 2); j++) {
+                    const int p0 = ready(j) + 2 + kFoldBatch * (ps.n - ready(j)), end = g.n0 + g.blk;
+                    if (p0 < end) fold(j, p0, min(p0 + kFoldBatch, end));
+                }
             }
-            if (last_due) {
-                // the last build is skipped when U^k already met the
-                // tolerance: decide that first (one barrier on the measure)
-                __syncthreads();
-                if (tid == 0) xput(xbase(bk), kXchMeasure + c, xtag(bk), last_measure());
-                bk++;
-                if (!read_barrier(bk - 1, false, nullptr)) return;
-                if (measures_max() <= g.tol) break;           // U^k is the result (uniform decision)
-            }
-            const bool pend_check = k == 0 && pending;
-            if (!build(uit, uith, S, Ln, un, k == 0 ? pre_n : -1, k == 0 ? n : -1)) return;
-            const int r = solve(pend_check ? 2 : ((k >= 1 && !last_due) ? 1 : 0), uit, uith);
-            if (r < 0) return;                                 // a barrier wait ran out of time
-            if (r == 1) break;                                 // U^k is the result
-            if (r == 2) { rollback = true; break; }
-            nsolve++;
-            pending = false;
+            // the next step's history from memory (levels t < n are written;
+            // D[n] enters through the tail)
+            if (ps.n + 1 < g.n_end) history(ps.n + 1, hm_next, w0_next, w1_next, w2_next);
         }
-        if (rollback) {
-            // the tentatively ended step sv_n needs its last iteration
-            un = sv_un; uh = sv_uh; dh = sv_dh; dlast = sv_dlast; d0m = sv_d0m; d1m = sv_d1m;
-            double ruit = sv_uit, ruith = sv_uith;
-            if (!build(ruit, ruith, sv_S, sv_Ln, un, -1, -1)) return;
-            if (solve(0, ruit, ruith) < 0) return;
-            nsolve++;
-            finish(sv_n, ruit, ruith);
-            pending = false;
-            n = sv_n + 1;
+        __syncthreads();                                       // B
+        const int st = __builtin_amdgcn_readfirstlane(L.status);
+        double unew[NPT];
+#pragma unroll
+        for (int q = 0; q < NPT; q++) {
+            unew[q] = L.u[row_slot(row(q))];
+            it[q] = st == kSolved ? unew[q] : it[q];
+        }
+        fresh = false;
+        const int what = ps.after(st);
+        if (what == kGoOn) continue;
+        if (what == kLeave) return;
+        if (what == kGoBack) {
+            // the tentatively ended step n - 1 needs its last iteration (from
+            // its iterate, now in un; dlast, D[0] and D[1] are set at its end)
+#pragma unroll
+            for (int q = 0; q < NPT; q++) { it[q] = un[q]; un[q] = sv_un[q]; S[q] = sv_S[q]; }
+            ps.back(ps.n - 1);
+            Ln = g.Lv ? g.Lv[ps.n] : g.L;
             continue;
         }
-        if (tentative) {
-            sv_n = n; sv_un = un; sv_uh = uh; sv_dh = dh; sv_dlast = dlast; sv_d0m = d0m; sv_d1m = d1m;
-            sv_S = S; sv_Ln = Ln; sv_uit = uit; sv_uith = uith;
-            pending = true;
+        // step n is done: the last iterate is U^{n+1}
+        const int n = ps.n;
+#pragma unroll
+        for (int q = 0; q < NPT; q++) {
+            sv_un[q] = un[q];
+            sv_S[q] = S[q];
+            const double dn = it[q] - un[q];
+            if (act(q)) {
+                *level(q, n) = dn;
+                g.U[s + row(q)] = it[q];
+            }
+            dlast[q] = dn;
+            un[q] = it[q];
+            d0m[q] = n == 0 ? dn : d0m[q];                     // (unconditional: kept in registers)
+            d1m[q] = n == 1 ? dn : d1m[q];
+            hm[q] = ps.redo ? hm[q] : hm_next[q];
         }
-        // ---- step n is done: the last iterate is U^{n+1} -------------------
-        finish(n, uit, uith);
-        hm_cur = hm_next;
-        tl_cur[0] = tl_next[0]; tl_cur[1] = tl_next[1]; tl_cur[2] = tl_next[2];
-        have_hm = pre_n >= 0;
-        n++;
+        if (n + 1 == g.n_end) return;
+        // (after a step done again its successor's history part is at hand)
+        w0 = ps.redo ? w0 : w0_next;
+        w1 = ps.redo ? w1 : w1_next;
+        w2 = ps.redo ? w2 : w2_next;
+        ps.begin(n + 1, what == kStepEndsTentatively);
+        start_step();
+        fresh = true;
     }
-    // the launch's Picard iterations, counted once per solve (err[1])
-    if (c == 0 && tid == 0) __hip_atomic_fetch_add(g.err + 1, nsolve, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ __launch_bounds__(256) void k_step1d_block(Step1DArgs g) { step_block(g, (int)blockIdx.x); }
+// The same steps by the solver wave: R rows per lane, 64 R > chunk nodes - 1.
+// It follows the iterates of its rows and of node s-1 (whose K the
+// separator's row needs), so the chunk's measure max|U^{k+1} - U^k| is formed
+// here, while the row waves evaluate the coefficients.
+template <int R>
+__device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, Step1DLds& L) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    const int N = g.N, C = g.C;
+    const int s = (int)(((int64_t)c * N) / C);
+    const int ni = (int)(((int64_t)(c + 1) * N) / C) - s - 1;  // interior rows s+1 .. e
+    const int pos = 4 * (lane & 15) + (lane >> 4);             // this lane's position in the line solve
+    const int first_row = R * pos;                             // its rows: chunk nodes first_row+1 .. first_row+R
+    const bool series = g.ser_P > 0;
+    const double zh = in_vgpr((s - 1) * g.h), ksat = in_vgpr(g.ksat), h2inv = in_vgpr(g.h2inv);
+    // node r of this lane (r = R: the separator s, r = R + 1: node s-1)
+    auto node = [&](int r) { return r < R ? s + 1 + first_row + r : s + R - r; };
+    auto have = [&](int r) { return r < R ? first_row + r < ni : (r == R || c > 0); };
+    constexpr int NV = R + 2;
+    double un[NV], dlast[NV], it[NV], sv_un[NV];
+    const int n_first = g.n;
+#pragma unroll
+    for (int r = 0; r < NV; r++) {
+        un[r] = have(r) ? g.U[node(r)] : 0.0;
+        dlast[r] = (have(r) && n_first >= 1)
+                       ? g.D[(int64_t)(series ? ((n_first - 1) & 1) : n_first - 1) * g.ld + node(r)]
+                       : 0.0;
+        sv_un[r] = 0.0;
+    }
+    int bk = 0;                                                // grid barriers passed in this launch
+    auto xbase = [&](int b) { return g.xch + (size_t)(b & 1) * kMaxChunks * kXchWords; };
+    auto xtag = [&](int b) { return g.xtag | ((unsigned)(b + 1) & 0xffffu); };
+    // the exchange words of this workgroup, both parities, zeroed before its
+    // first publication (by the lanes that publish them)
+    if (lane < kXchWords)
+        for (int par = 0; par < 2; par++)
+            __hip_atomic_store(xbase(par) + c * kXchWords + lane, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+    auto publish = [&](int b, int lo) {                        // words lo..15 of the values in L.pub
+        wave_lds_sync();
+        const unsigned long long t = (unsigned long long)xtag(b) << 32;
+        if (lane >= lo && lane < kXchWords)
+            __hip_atomic_store(xbase(b) + c * kXchWords + lane,
+                               t | reinterpret_cast<const unsigned*>(L.pub)[lane], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // whether a wait that began at *t0 (-1: now) has run out of time (the
+    // launch then ends; the host reports it)
+    auto timed_out = [&](int64_t* t0) -> bool {
+        const int64_t now = (int64_t)wall_clock64();
+        if (*t0 < 0) *t0 = now;
+        if (now - *t0 <= g.wait_ticks) return false;
+        __hip_atomic_store(g.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return true;
+    };
+    // every chunk's words into L.words once they carry the barrier's tag, 64
+    // chunks per round: load k takes chunks 4 k .. 4 k + 3 of the round
+    auto collect = [&](int b) -> bool {
+        const unsigned tg = xtag(b);
+        int64_t t0 = -1;
+        constexpr int K = 16;
+        for (int j0 = 0; j0 < C; j0 += 64) {
+            unsigned long long w[K];
+            int l = lane;
+            asm volatile("" : "+v"(l));                        // (addresses formed here, not kept across iterations)
+            const unsigned long long* x = xbase(b) + j0 * kXchWords + l;
+            const int kn = min(K, (C - j0 + 3) >> 2);          // loads of this round
+            const int mine = (C - j0 - (l >> 4) + 3) >> 2;     // and those whose chunk exists on this lane
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                w[k] = 0;
+                if (k < kn) w[k] = __hip_atomic_load(x + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            for (;;) {
+                unsigned miss = 0;
+#pragma unroll
+                for (int k = 0; k < K; k++) miss |= k < mine ? (unsigned)(w[k] >> 32) ^ tg : 0u;
+                if (__all(miss == 0)) break;
+                if (timed_out(&t0)) return false;
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                    if (k < mine && (unsigned)(w[k] >> 32) != tg)
+                        w[k] = __hip_atomic_load(x + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            unsigned long long* to = &L.words[(j0 + (l >> 4)) * kXchPad + (l & 15)];
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if (k < mine) to[4 * k * kXchPad] = w[k];
+        }
+        wave_lds_sync();
+        return true;
+    };
+    // the measure words alone
+    auto collect_measures = [&](int b) -> bool {
+        const unsigned tg = xtag(b);
+        int64_t t0 = -1;
+        for (int j0 = 0; j0 < C; j0 += 64) {
+            const int j = min(j0 + lane, C - 1);
+            const unsigned long long* x = xbase(b) + j * kXchWords + kXchMeasure;
+            unsigned long long w[2];
+            for (;;) {
+                for (int k = 0; k < 2; k++) w[k] = __hip_atomic_load(x + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (__all((unsigned)(w[0] >> 32) == tg && (unsigned)(w[1] >> 32) == tg)) break;
+                if (timed_out(&t0)) return false;
+            }
+            for (int k = 0; k < 2; k++) L.words[j * kXchPad + kXchMeasure + k] = w[k];
+        }
+        wave_lds_sync();
+        return true;
+    };
+
+    // Between the barriers of an iteration, K at node s-1 in Kh: kSolved with
+    // the new iterate in L.u and itn; where `check` asks for it, the decision
+    // on the published measures (kCheckMet: U^k met the tolerance -> kMet;
+    // kCheckPending: the tentatively ended previous step did not ->
+    // kRollback; kDecide: the measure alone is exchanged -> kMet or kNotMet);
+    // kTimeout when a wait ran out of time.
+    auto line_solve = [&](int b, int check, double Kh, double Ln, double meas, double (&itn)[NV]) -> int {
+        double x[R], y[R], z[R];
+        const bool decide = check == kDecide;
+        int p = pos;
+        asm volatile("" : "+v"(p));                            // (addresses and masks formed here, not kept across iterations)
+        const int r0 = R * p;
+        if (!decide) {
+            double a[R], cc[R], d[R];
+            double Kv[R + 1], iv[R], dv[R];
+#pragma unroll
+            for (int j = 0; j <= R; j++) Kv[j] = L.K[row_slot(r0 + j)];
+#pragma unroll
+            for (int j = 0; j < R; j++) { iv[j] = L.iC[row_slot(r0 + 1 + j)]; dv[j] = L.d[row_slot(r0 + 1 + j)]; }
+            const double K0 = L.K[0], i0 = L.iC[0], d0 = L.d[0];
+#pragma unroll
+            for (int j = 0; j < R; j++) {
+                const double Km = Kv[j], Kp = Kv[j + 1];
+                const double inv = rcp_nr(-fma(iv[j], Kp * h2inv + Km * h2inv, Ln));
+                a[j] = Km * iv[j] * h2inv * inv;
+                cc[j] = Kp * iv[j] * h2inv * inv;
+                d[j] = dv[j] * inv;
+                // bottom row U_{N-1} = U_{N-2}; rows past the chunk hand on
+                // the next separator's value: x_q = x_{q+1}
+                const bool in = r0 + j < ni, bottom = r0 + j == N - 2 - s;
+                a[j] = in ? (bottom ? -1.0 : a[j]) : 0.0;
+                cc[j] = in ? (bottom ? 0.0 : cc[j]) : -1.0;
+                d[j] = in && !bottom ? d[j] : 0.0;
+            }
+            // the separator's row (node 0: U = u_top)
+            const double as = c > 0 ? Kh * i0 * h2inv : 0.0;
+            const double cs = c > 0 ? K0 * i0 * h2inv : 0.0;
+            const double bs = c > 0 ? -fma(i0, K0 * h2inv + Kh * h2inv, Ln) : 1.0;
+            wave_line<R, false>(a, cc, d, p, x, y, z);
+            if (lane == 0) {
+                L.pub[0] = as;
+                L.pub[1] = fma(cs, y[0], bs);
+                L.pub[2] = cs * z[0];
+                L.pub[3] = fma(-cs, x[0], d0);
+            }
+            // the last node's row: which of the lane's R is launch-uniform
+            double xl = x[0], yl = y[0], zl = z[0];
+#pragma unroll
+            for (int j = 1; j < R; j++) {
+                const bool is = (ni - 1) % R == j;
+                xl = is ? x[j] : xl;
+                yl = is ? y[j] : yl;
+                zl = is ? z[j] : zl;
+            }
+            if (p == (ni - 1) / R) {
+                L.pub[4] = xl;
+                L.pub[5] = yl;
+                L.pub[6] = zl;
+            }
+        }
+        if (lane == 0) L.pub[7] = meas;
+        publish(b, decide ? kXchMeasure : 0);
+        if (!(decide ? collect_measures(b) : collect(b))) return kTimeout;
+        double m = 0.0;
+        for (int j = lane; j < C; j += 64) m = fmax(m, xch_value(L, j, 7));
+        const bool met = wave_max(m) <= g.tol;
+        if (decide) return met ? kMet : kNotMet;
+        double um, us, up;
+        const double xl = c > 0 ? xch_value(L, c - 1, 4) : 0.0, yl = c > 0 ? xch_value(L, c - 1, 5) : 0.0,
+                     zl = c > 0 ? xch_value(L, c - 1, 6) : 0.0;
+        if (C <= 64) solve_separators<1>(L, C, c, p, um, us, up);
+        else solve_separators<4>(L, C, c, p, um, us, up);
+        if (check == kCheckMet && met) return kMet;
+        if (check == kCheckPending && !met) return kRollback;
+#pragma unroll
+        for (int j = 0; j < R; j++) {
+            itn[j] = fma(z[j], up, fma(y[j], us, x[j]));
+            L.u[row_slot(r0 + 1 + j)] = itn[j];
+        }
+        if (lane == 0) L.u[0] = us;
+        itn[R] = us;
+        itn[R + 1] = fma(zl, us, fma(yl, um, xl));             // node s-1 as its own chunk forms it
+        return kSolved;
+    };
+
+    PicardState ps = picard_state(g);
+    double Ln = 0.0, meas = 0.0;
+    auto start_step = [&]() {
+        Ln = g.Lv ? g.Lv[ps.n] : g.L;
+        const bool ex = g.extrap && ps.n >= 1;
+#pragma unroll
+        for (int r = 0; r < NV; r++) it[r] = ex ? un[r] + dlast[r] : un[r];
+    };
+    start_step();
+    for (;;) {
+        double K = 0.0, invC;
+        if (c > 0 && ps.check != kDecide) vgm_coefs(it[R + 1], zh, ksat, g.coef_mode, K, invC);
+        __syncthreads();                                       // A
+        double itn[NV];
+        const int st = line_solve(bk, ps.check, K, Ln, meas, itn);
+        if (lane == 0) L.status = st;
+        __syncthreads();                                       // B
+        bk++;
+        if (st == kSolved) {
+            double m = 0.0;
+#pragma unroll
+            for (int r = 0; r < NV; r++) {
+                if (r <= R) m = fmax(m, have(r) ? fabs(itn[r] - it[r]) : 0.0);
+                it[r] = itn[r];
+            }
+            meas = wave_max(m);
+        }
+        const int what = ps.after(st);
+        if (what == kGoOn) continue;
+        if (what == kLeave) return;
+        if (what == kGoBack) {
+#pragma unroll
+            for (int r = 0; r < NV; r++) { it[r] = un[r]; un[r] = sv_un[r]; }
+            ps.back(ps.n - 1);
+            Ln = g.Lv ? g.Lv[ps.n] : g.L;
+            continue;
+        }
+        const int n = ps.n;
+#pragma unroll
+        for (int r = 0; r < NV; r++) { sv_un[r] = un[r]; dlast[r] = it[r] - un[r]; un[r] = it[r]; }
+        if (n + 1 == g.n_end) break;
+        ps.begin(n + 1, what == kStepEndsTentatively);
+        start_step();
+    }
+    // the launch's Picard iterations, counted once per solve (err[1])
+    if (c == 0 && lane == 0)
+        __hip_atomic_fetch_add(g.err + 1, ps.solves, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The body of the single-solve launch and of the batched one: RW row waves,
+// then the solver wave of R rows per lane.  The roles are compiled apart and
+// keep their control flow flat: together (one loop with the role inside) their
+// launch constants overflowed the scalar registers, and the reloads and
+// branches between two solves cost 2500 of 15000 cycles.
+template <int RW>
+__global__ __launch_bounds__(64 * RW + 64) void k_step1d_block(Step1DArgs g) {
+    __shared__ Step1DLds L;
+    if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) == RW) solver_steps<RW>(g, (int)blockIdx.x, L);
+    else row_steps<RW, 1>(g, (int)blockIdx.x, L);
+}
 
 // Many independent solves in one cooperative launch: workgroups
 // [t.first[j], t.first[j+1]) are the chunks of solve j.  Each solve keeps its
-// own exchange words, convergence slots and Picard decisions, so its arithmetic
+// own exchange words, measures and Picard decisions, so its arithmetic
 // is that of its single-solve launch; the fields that change from block to
-// block come with the launch, the rest from the solve's row of `base`.
-// Registers are held to 256 per lane (a few spills) so that two workgroups
-// share a CU: a batch holds up to 512 chunk workgroups, and the latency-bound
-// waves of two workgroups interleave on each SIMD.  (The single-solve kernel
-// keeps 272 registers and one workgroup per CU, its fastest form.)
-__global__ __launch_bounds__(256, 2) void k_step1d_batch(const Step1DArgs* __restrict__ base, BatchTick t) {
+// block come with the launch, the rest from the solve's row of `base`.  Two
+// row waves of two nodes per thread and the solver wave (whose rows per lane
+// are those of the single-solve launch): two workgroups share a CU at 256
+// registers per lane, so a batch holds up to 512 chunk workgroups, and their
+// latency-bound waves interleave on each SIMD.
+constexpr int kBatchThreads = 192;
+__global__ __launch_bounds__(kBatchThreads, 2) void k_step1d_batch(const Step1DArgs* __restrict__ base, BatchTick t) {
+    __shared__ Step1DLds L;
     const int wg = (int)blockIdx.x;
     int j = 0;
     while (j + 1 < t.count && wg >= t.first[j + 1]) j++;
@@ -982,7 +1359,10 @@ __global__ __launch_bounds__(256, 2) void k_step1d_batch(const Step1DArgs* __res
     g.xtag = t.xtag[j];
     g.part_stride = t.part_stride[j];
     g.part = t.part[j];
-    step_block(g, wg - t.first[j]);
+    const int c = wg - t.first[j];
+    if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) < 2) row_steps<2, 2>(g, c, L);
+    else if (row_waves(g.N, g.C) == 3) solver_steps<3>(g, c, L);
+    else solver_steps<4>(g, c, L);
 }
 
 // Barrier bound in wall-clock ticks: 2 s at the device's wall clock rate
@@ -995,18 +1375,25 @@ int64_t barrier_wait_ticks() {
     return (int64_t)khz * 2000;
 }
 
-static bool coop_fits(const void* kern, int64_t wgs) {
+static bool coop_fits(const void* kern, int threads, int64_t wgs) {
     int dev = 0, coop = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess) return false;
     if (hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev) != hipSuccess || !coop) return false;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return false;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, 0) != hipSuccess) return false;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, threads, 0) != hipSuccess) return false;
     return (int64_t)per_cu * cus >= wgs;
 }
 
+static const void* block_kernel(int rw) {
+    return rw == 3 ? (const void*)k_step1d_block<3> : (const void*)k_step1d_block<4>;
+}
+
 // Whether the C workgroups of a cooperative block launch can be co-resident.
-bool step1d_block_supported(int C) { return coop_fits((const void*)k_step1d_block, C); }
-bool step1d_batch_supported(int64_t wgs) { return coop_fits((const void*)k_step1d_batch, wgs); }
+bool step1d_block_supported(int N, int C) {
+    const int rw = row_waves(N, C);
+    return coop_fits(block_kernel(rw), 64 * rw + 64, C);
+}
+bool step1d_batch_supported(int64_t wgs) { return coop_fits((const void*)k_step1d_batch, kBatchThreads, wgs); }
 
 fpde_status launch_step1d_batch(const Step1DArgs* base, const BatchTick& t, hipStream_t st) {
     if (t.count < 1 || t.count > kMaxBatch) { set_error("batched step: 1 to 32 solves"); return FPDE_ERR_ARG; }
@@ -1017,17 +1404,21 @@ fpde_status launch_step1d_batch(const Step1DArgs* base, const BatchTick& t, hipS
     const Step1DArgs* b = base;
     BatchTick tick = t;
     void* params[] = {&b, &tick};
-    FPDE_HIP_TRY(hipLaunchCooperativeKernel((const void*)k_step1d_batch, dim3(wgs), dim3(256), params, 0, st));
+    FPDE_HIP_TRY(hipLaunchCooperativeKernel((const void*)k_step1d_batch, dim3(wgs), dim3(kBatchThreads), params, 0, st));
     return FPDE_OK;
 }
 
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st) {
-    if (2 * a.C > kMaxRed || a.C > kMaxChunks) { set_error("1D line too long for the reduced system (N <= 65536)"); return FPDE_ERR_ARG; }
+    if (2 * a.C > kMaxRed || a.C > kMaxChunks || (a.N + a.C - 1) / a.C > kRows) {
+        set_error("1D line too long for the reduced system (N <= 65536)");
+        return FPDE_ERR_ARG;
+    }
     if (a.sp_on) { set_error("cooperative step: the space-fractional sum runs with per-iteration launches"); return FPDE_ERR_ARG; }
     if (a.n_end <= a.n) return FPDE_OK;
     Step1DArgs arg = a;
     void* params[] = {&arg};
-    FPDE_HIP_TRY(hipLaunchCooperativeKernel((const void*)k_step1d_block, dim3(a.C), dim3(256), params, 0, st));
+    const int rw = row_waves(a.N, a.C);
+    FPDE_HIP_TRY(hipLaunchCooperativeKernel(block_kernel(rw), dim3(a.C), dim3(64 * rw + 64), params, 0, st));
     return FPDE_OK;
 }
 

@@ -1518,3 +1518,45 @@ def test_autotune_block_picks_a_candidate_that_solves_right(fpde, oracle):
     b3, ms3 = fpde.autotune_block(spec3, v0, trial_steps=280)
     print(f"autotune 3d 24^3: block {b3}, {ms3 * 1e3:.1f} us/step")
     assert b3 in (16, 32, 64, 128) and ms3 > 0.0
+
+
+@pytest.mark.parametrize("nodes,rows", [(5, 0), (192, 0), (193, 0), (256, 256), (257, 256), (2048, 32), (2080, 32),
+                                        (8192, 32), (12288, 0), (12289, 0)])
+@pytest.mark.parametrize("fourier,alpha", [(1.0, 0.9), (40.0, 0.3)])
+def test_wave_line_solve_edges_match_oracle(fpde, oracle, nodes, rows, fourier, alpha):
+    """The cooperative form's line solve at its edges: the smallest line, a
+    chunk that fills the solver wave's rows and one node more (3 and 4 rows per
+    lane), 64 and 65 chunks (one and four separators per lane), 256 chunks; with
+    couplings that fall off within a chunk (the separators' reduction ends
+    early) and that do not (mesh Fourier number 40, alpha 0.3)."""
+    steps = 12
+    u0 = fpde.init_1d(nodes, 7000 + nodes)
+    spec = fpde.make_spec(nodes, steps, 1e-3, alpha=alpha, picard_max=3, picard_tol=1e-12, hist_mode="mfma_f64",
+                          block=16, u_top=u0[0], chunk_rows=rows, fourier=fourier)
+    err = rel_err(fpde.solve(spec, u0), _oracle_1d(oracle, spec, u0, picard_tol=1e-12))
+    print(f"line solve N={nodes} rows={rows} fourier={fourier}: rel err {err:.3e}", flush=True)
+    assert err <= TOL_F64
+
+
+@pytest.mark.parametrize("block", [16, 64, 128])
+@pytest.mark.parametrize("picard", [1, 3])
+def test_launches_that_cut_a_block_give_the_same_bits(fpde, block, picard):
+    """The near field folded ahead follows the step alone: a solve advanced in
+    pieces that end just before, at and after the steps where 16-level groups
+    become final equals the solve advanced at once, bit for bit, alone and in
+    a batch."""
+    nodes, steps = 700, 300
+    u0 = fpde.init_1d(nodes, 93)
+    spec = fpde.make_spec(nodes, steps, 1e-3, alpha=0.7, hist_mode="split_bf16", block=block, picard_max=picard,
+                          picard_tol=1e-12 if picard > 1 else 0.0, u_top=u0[0])
+    whole = fpde.solve(spec, u0)
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b:
+        for s in (a, b):
+            s.set_initial(u0)
+        for piece in (1, 16, 1, 1, 14, 18, 17, 47, 33, 2):
+            a.advance(piece)
+            fpde.advance_batch([b], piece)
+        a.advance(0)
+        fpde.advance_batch([b], 0)
+        np.testing.assert_array_equal(a.solution(), whole)
+        np.testing.assert_array_equal(b.solution(), whole)
