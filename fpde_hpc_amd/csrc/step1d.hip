@@ -535,13 +535,13 @@ __global__ __launch_bounds__(256) void k_step1d(Step1DArgs g) {
 // reduced system, whose couplings fall off with the chunk length: its cyclic
 // reduction ends as soon as none exceeds 2^-60.
 // Measured (cycles of one iteration at N = 10^4, 53 chunks, phase timers): row
-// waves 3000 from barrier to barrier (coefficients 1700); solver wave: rows and
-// line solve 2400, publishing 900, waiting for the other chunks 4700,
-// separators and decision 1700, U to LDS 500.  Headline solve (N = 10^4, M =
-// 2 10^4) 373 -> 224 ms, N = 1000 35.7 -> 23.1 ms, six solves in a batch 58.9
-// -> 40.9 ms against the whole workgroup's cyclic reduction over LDS with both
+// waves 2000 from barrier to barrier (coefficients 640); solver wave: rows and
+// line solve 2500, publishing 900, waiting for the other chunks 4700,
+// separators and decision 1800, U to LDS 500.  Headline solve (N = 10^4, M =
+// 2 10^4) 374 -> 214 ms, N = 1000 35.6 -> 21.7 ms, six solves in a batch 58.9
+// -> 39.5 ms against the whole workgroup's cyclic reduction over LDS with both
 // chunk ends as separators (five words per row and level, a workgroup barrier
-// per level).
+// per level) and coefficients by square roots and divisions (1700 cycles).
 //
 // The arithmetic is written with explicit fma and contraction off: single
 // and batched launches round alike in every instantiation.
@@ -838,6 +838,10 @@ __device__ inline PicardState picard_state(const Step1DArgs& g) {
     return ps;
 }
 
+// s_waitcnt vmcnt(0), the other counters left alone (loads and stores share
+// vmcnt on gfx9)
+constexpr int kDrainVmem = 0x0f70;
+
 // A launch constant kept in vector registers (the two roles have more of them
 // than scalar registers, and a spilled scalar costs two moves per use).
 __device__ inline double in_vgpr(double v) { asm("" : "+v"(v)); return v; }
@@ -851,7 +855,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
     const int s = (int)(((int64_t)c * g.N) / g.C);
     const int nc = (int)(((int64_t)(c + 1) * g.N) / g.C) - s;
     const bool series = g.ser_P > 0;
-    const double ksat = in_vgpr(g.ksat);
+    const double ksat = in_vgpr(g.ksat), L0 = in_vgpr(g.L), utop = in_vgpr(g.utop);
     auto row = [&](int q) { return tid + 64 * RW * q; };       // this thread's chunk rows
     auto act = [&](int q) { return row(q) < nc; };
 
@@ -895,7 +899,8 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
     double hm[NPT], hm_next[NPT];
     double w0 = 0.0, w1 = 0.0, w2 = 0.0, w0_next = 0.0, w1_next = 0.0, w2_next = 0.0;
     double S[NPT], it[NPT];
-    double Ln = 0.0;
+    // local coefficient: one, or the step's own (prescribed grid)
+    double Ln = g.Lv ? g.Lv[n_first] : L0, Ln_prev = Ln, Ln_next = Ln;
 #pragma unroll
     for (int q = 0; q < NPT; q++) sv_un[q] = sv_S[q] = hm[q] = hm_next[q] = 0.0;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -986,8 +991,6 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
     };
     auto start_step = [&]() {
         const int n = ps.n;
-        // local coefficient: one, or the step's own (prescribed grid)
-        Ln = g.Lv ? g.Lv[n] : g.L;
 #pragma unroll
         for (int q = 0; q < NPT; q++) {
             S[q] = 0.0;
@@ -1002,6 +1005,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
     if (!series && n_first >= 1) history(n_first, hm, w0, w1, w2);
     start_step();
     bool fresh = true;                                         // the step's first iteration
+    __builtin_amdgcn_s_waitcnt(kDrainVmem);
     for (;;) {
         if (ps.check != kDecide) {
 #pragma unroll
@@ -1012,7 +1016,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
                     const int slot = row_slot(row(q));
                     L.K[slot] = K;
                     L.iC[slot] = invC;
-                    L.d[slot] = s + row(q) == 0 ? g.utop : fma(-Ln, un[q], S[q]);
+                    L.d[slot] = s + row(q) == 0 ? utop : fma(-Ln, un[q], S[q]);
                 }
             }
         }
@@ -1029,12 +1033,21 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
             // D[n] enters through the tail)
             if (ps.n + 1 < g.n_end) history(ps.n + 1, hm_next, w0_next, w1_next, w2_next);
         }
+        if (fresh && g.Lv && ps.n + 1 < g.n_end) Ln_next = g.Lv[ps.n + 1];
+        // memory drained here, beside the solver wave: from barrier B to the
+        // next A only the stores of D and U are under way, and no load's wait
+        // has to sit out their way to memory
+        __builtin_amdgcn_s_waitcnt(kDrainVmem);
         __syncthreads();                                       // B
-        const int st = __builtin_amdgcn_readfirstlane(L.status);
         double unew[NPT];
 #pragma unroll
         for (int q = 0; q < NPT; q++) {
             unew[q] = L.u[row_slot(row(q))];
+            asm volatile("" : "+v"(unew[q]));                  // (read beside the status, not after it)
+        }
+        const int st = __builtin_amdgcn_readfirstlane(L.status);
+#pragma unroll
+        for (int q = 0; q < NPT; q++) {
             it[q] = st == kSolved ? unew[q] : it[q];
         }
         fresh = false;
@@ -1047,11 +1060,14 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
 #pragma unroll
             for (int q = 0; q < NPT; q++) { it[q] = un[q]; un[q] = sv_un[q]; S[q] = sv_S[q]; }
             ps.back(ps.n - 1);
-            Ln = g.Lv ? g.Lv[ps.n] : g.L;
+            Ln_next = Ln;
+            Ln = Ln_prev;
             continue;
         }
         // step n is done: the last iterate is U^{n+1}
         const int n = ps.n;
+        Ln_prev = Ln;
+        Ln = Ln_next;
 #pragma unroll
         for (int q = 0; q < NPT; q++) {
             sv_un[q] = un[q];
@@ -1092,7 +1108,8 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
     const int pos = 4 * (lane & 15) + (lane >> 4);             // this lane's position in the line solve
     const int first_row = R * pos;                             // its rows: chunk nodes first_row+1 .. first_row+R
     const bool series = g.ser_P > 0;
-    const double zh = in_vgpr((s - 1) * g.h), ksat = in_vgpr(g.ksat), h2inv = in_vgpr(g.h2inv);
+    const double zh = in_vgpr((s - 1) * g.h), ksat = in_vgpr(g.ksat), h2inv = in_vgpr(g.h2inv), tol = in_vgpr(g.tol);
+    const double L0 = in_vgpr(g.L);
     // node r of this lane (r = R: the separator s, r = R + 1: node s-1)
     auto node = [&](int r) { return r < R ? s + 1 + first_row + r : s + R - r; };
     auto have = [&](int r) { return r < R ? first_row + r < ni : (r == R || c > 0); };
@@ -1189,15 +1206,17 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         return true;
     };
 
-    // Between the barriers of an iteration, K at node s-1 in Kh: kSolved with
-    // the new iterate in L.u and itn; where `check` asks for it, the decision
+    // Between the barriers of an iteration (Kh: K at node s-1, `change`: the
+    // lane's share of the chunk's measure): kSolved with the new iterate in
+    // L.u and itn; where `check` asks for it, the decision
     // on the published measures (kCheckMet: U^k met the tolerance -> kMet;
     // kCheckPending: the tentatively ended previous step did not ->
     // kRollback; kDecide: the measure alone is exchanged -> kMet or kNotMet);
     // kTimeout when a wait ran out of time.
-    auto line_solve = [&](int b, int check, double Kh, double Ln, double meas, double (&itn)[NV]) -> int {
+    auto line_solve = [&](int b, int check, double Kh, double Ln, double change, double (&itn)[NV]) -> int {
         double x[R], y[R], z[R];
         const bool decide = check == kDecide;
+        double meas;
         int p = pos;
         asm volatile("" : "+v"(p));                            // (addresses and masks formed here, not kept across iterations)
         const int r0 = R * p;
@@ -1209,6 +1228,7 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
 #pragma unroll
             for (int j = 0; j < R; j++) { iv[j] = L.iC[row_slot(r0 + 1 + j)]; dv[j] = L.d[row_slot(r0 + 1 + j)]; }
             const double K0 = L.K[0], i0 = L.iC[0], d0 = L.d[0];
+            meas = wave_max(change);
 #pragma unroll
             for (int j = 0; j < R; j++) {
                 const double Km = Kv[j], Kp = Kv[j + 1];
@@ -1248,13 +1268,15 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
                 L.pub[5] = yl;
                 L.pub[6] = zl;
             }
+        } else {
+            meas = wave_max(change);
         }
         if (lane == 0) L.pub[7] = meas;
         publish(b, decide ? kXchMeasure : 0);
         if (!(decide ? collect_measures(b) : collect(b))) return kTimeout;
         double m = 0.0;
         for (int j = lane; j < C; j += 64) m = fmax(m, xch_value(L, j, 7));
-        const bool met = wave_max(m) <= g.tol;
+        const bool met = __builtin_amdgcn_readfirstlane(wave_max(m) <= tol ? 1 : 0) != 0;     // (uniform)
         if (decide) return met ? kMet : kNotMet;
         double um, us, up;
         const double xl = c > 0 ? xch_value(L, c - 1, 4) : 0.0, yl = c > 0 ? xch_value(L, c - 1, 5) : 0.0,
@@ -1275,31 +1297,30 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
     };
 
     PicardState ps = picard_state(g);
-    double Ln = 0.0, meas = 0.0;
+    double Ln = 0.0, change = 0.0;
     auto start_step = [&]() {
-        Ln = g.Lv ? g.Lv[ps.n] : g.L;
+        Ln = g.Lv ? g.Lv[ps.n] : L0;
         const bool ex = g.extrap && ps.n >= 1;
 #pragma unroll
         for (int r = 0; r < NV; r++) it[r] = ex ? un[r] + dlast[r] : un[r];
     };
     start_step();
     for (;;) {
-        double K = 0.0, invC;
-        if (c > 0 && ps.check != kDecide) vgm_coefs(it[R + 1], zh, ksat, g.coef_mode, K, invC);
+        double Kh, iCh;
+        vgm_coefs(it[R + 1], zh, ksat, g.coef_mode, Kh, iCh);
         __syncthreads();                                       // A
         double itn[NV];
-        const int st = line_solve(bk, ps.check, K, Ln, meas, itn);
+        const int st = __builtin_amdgcn_readfirstlane(line_solve(bk, ps.check, Kh, Ln, change, itn));
         if (lane == 0) L.status = st;
         __syncthreads();                                       // B
         bk++;
         if (st == kSolved) {
-            double m = 0.0;
+            change = 0.0;
 #pragma unroll
             for (int r = 0; r < NV; r++) {
-                if (r <= R) m = fmax(m, have(r) ? fabs(itn[r] - it[r]) : 0.0);
+                if (r <= R) change = fmax(change, have(r) ? fabs(itn[r] - it[r]) : 0.0);
                 it[r] = itn[r];
             }
-            meas = wave_max(m);
         }
         const int what = ps.after(st);
         if (what == kGoOn) continue;
@@ -1308,7 +1329,7 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
 #pragma unroll
             for (int r = 0; r < NV; r++) { it[r] = un[r]; un[r] = sv_un[r]; }
             ps.back(ps.n - 1);
-            Ln = g.Lv ? g.Lv[ps.n] : g.L;
+            Ln = g.Lv ? g.Lv[ps.n] : L0;
             continue;
         }
         const int n = ps.n;
