@@ -21,6 +21,10 @@ using namespace fpde;
 struct fpde_cl_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
+    // partial rows of "Sum" launches, used in the order of the stream; grown
+    // and launched under the mutex
+    std::mutex mu;
+    ScratchLease scratch;
 };
 
 struct fpde_cl_buf {
@@ -415,8 +419,16 @@ fpde_status fpde_cl_launch(fpde_cl_ctx* ctx, fpde_cl_kernel* k, int ndims, const
         set_error("kb/tau buffers too small");
         return FPDE_ERR_ARG;
     }
+    std::lock_guard<std::mutex> lock(ctx->mu);
+    const int splits = ref_sum_splits(nodes, old_size - 1);
+    const size_t need = splits > 1 ? sizeof(double) * (size_t)splits * nodes : 0;
+    if (need > ctx->scratch.bytes()) {
+        FPDE_HIP_TRY(hipStreamSynchronize(ctx->stream));     // earlier launches are done with what it gives back
+        if ((rc = ctx->scratch.take(need)) != FPDE_OK) return rc;
+    }
     rc = launch_ref_sum((double*)S->ptr, (const double*)old->ptr, old_size, os, nodes, (const double*)tau->ptr,
-                        (const double*)kb->ptr, sum_alg, sum_param, k->prog->bs, ctx->stream);
+                        (const double*)kb->ptr, sum_alg, sum_param, k->prog->bs, (double*)ctx->scratch.ptr(),
+                        ctx->stream);
     if (rc != FPDE_OK) return rc;
     FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
@@ -436,10 +448,16 @@ fpde_status fpde_reference_sum(double* S, const double* old, int64_t old_size, i
         return FPDE_ERR_ARG;
     }
     if (sum_alg != 0 && sum_alg != 1) { set_error("sum_alg must be 0 or 1"); return FPDE_ERR_ARG; }
-    fpde_status rc = launch_ref_sum(S, old, old_size, os, nodes, tau, kb, sum_alg, sum_param, 16, 0);
+    ScratchLease scratch;
+    const int splits = ref_sum_splits(nodes, old_size - 1);
+    fpde_status rc = FPDE_OK;
+    if (splits > 1 && (rc = scratch.take(sizeof(double) * (size_t)splits * nodes)) != FPDE_OK) return rc;
+    rc = launch_ref_sum(S, old, old_size, os, nodes, tau, kb, sum_alg, sum_param, 16, (double*)scratch.ptr(), 0);
     if (rc != FPDE_OK) return rc;
-    FPDE_HIP_TRY(hipGetLastError());
-    FPDE_HIP_TRY(hipDeviceSynchronize());
+    hipError_t e = hipGetLastError();
+    const hipError_t done = hipDeviceSynchronize();          // (before the scratch memory is given back)
+    if (e == hipSuccess) e = done;
+    if (e != hipSuccess) { set_error(hipGetErrorString(e)); return FPDE_ERR_HIP; }
     return FPDE_OK;
 }
 
@@ -455,16 +473,17 @@ fpde_status fpde_history_sum_f64(double* S, const double* D, int64_t n, int64_t 
         return FPDE_OK;
     }
     // partials then one combine pass
-    double* part = nullptr;
-    FPDE_HIP_TRY(hipMalloc(&part, sizeof(double) * 64 * (size_t)ld));
+    ScratchLease scratch;
+    fpde_status rc = scratch.take(sizeof(double) * kPlainMaxSplits * (size_t)ld);
+    if (rc != FPDE_OK) return rc;
+    double* part = (double*)scratch.ptr();
     int splits = 0;
-    fpde_status rc = launch_hist_plain(D, ld, (int)nodes, (int)n, (int)n, omega, part, &splits, 0);
+    rc = launch_hist_plain(D, ld, (int)nodes, (int)n, (int)n, omega, part, &splits, 0);
     if (rc == FPDE_OK) {
         // combine: S = sum of partial rows (no near levels, no corrections)
         rc = launch_hist_combine(S, part, splits, ld, 0, D, ld, nodes, 0, 0, omega, 0, 0, 0, nullptr, nullptr, 1.0, 0);
     }
     hipError_t e = hipDeviceSynchronize();
-    hipFree(part);
     if (rc != FPDE_OK) return rc;
     if (e != hipSuccess) { set_error(hipGetErrorString(e)); return FPDE_ERR_HIP; }
     return FPDE_OK;

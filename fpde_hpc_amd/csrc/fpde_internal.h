@@ -472,8 +472,12 @@ constexpr int kPlainMaxSplits = 64;
 int hist_plain_plan(int nodes, int t_hi, int* chunk_out);
 fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int t_hi, const double* omega,
                               double* part, int* splits_out, hipStream_t st);
+// The reference Sum (sum_alg 0/1): the intervals go in ref_sum_splits(nodes,
+// intervals) parts, whose partial rows need as many rows of `nodes` doubles in
+// `part` (one part: none).
+int ref_sum_splits(int64_t nodes, int64_t intervals);
 fpde_status launch_ref_sum(double* S, const double* old, int64_t old_size, int64_t os, int64_t nodes,
-                           const double* tau, const double* kb, int sum_alg, double sum_param, int bs,
+                           const double* tau, const double* kb, int sum_alg, double sum_param, int bs, double* part,
                            hipStream_t st);
 fpde_status launch_ref_series(double* S, const double* old, int64_t old_size, int64_t os, int64_t nodes,
                               const double* tau, int tstep, double* Htmp, const double* coef, int P, double gtj,
@@ -583,6 +587,26 @@ private:
     std::vector<std::pair<char*, size_t>> segs_;
     std::map<char*, Block> free_, live_;
 };
+
+// Device scratch memory leased from the library's pool (scratch.cpp).  The
+// holder gives it back (or lets the lease go) only when the device has
+// finished with it.
+class ScratchLease {
+public:
+    ScratchLease() = default;
+    ScratchLease(const ScratchLease&) = delete;
+    ScratchLease& operator=(const ScratchLease&) = delete;
+    ~ScratchLease() { give(); }
+    fpde_status take(size_t bytes);     // in place of what it held; on the current device
+    void give();
+    void* ptr() const { return ptr_; }
+    size_t bytes() const { return ptr_ ? bytes_ : 0; }
+private:
+    void* ptr_ = nullptr;
+    size_t bytes_ = 0;
+    int dev_ = 0;
+};
+bool scratch_shutdown();                // frees what is not leased
 
 // A solver whose device buffers come from `arena` and whose launches go to
 // `stream` (both owned by the caller, the request server): destroying it

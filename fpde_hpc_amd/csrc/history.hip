@@ -16,6 +16,7 @@
 //                    (hi+lo or hi+mid+lo) with fp32 MFMA accumulation flushed
 //                    to fp64 after every 32-level group.
 #include "fpde_internal.h"
+#include <algorithm>
 
 namespace fpde {
 
@@ -70,32 +71,112 @@ __global__ __launch_bounds__(256) void k_hist_plain(const double* __restrict__ D
 
 // ---------------------------------------------------------------------------
 // The reference Sum kernel, sum_alg 0/1 (fpde_hpc_1d.cpp:1247-1284): newest
-// interval first, chunks of BS levels; sum_alg 1 stops after the first chunk whose
-// weights are all below sum_param in magnitude.  One thread per node.
-__global__ __launch_bounds__(256) void k_ref_sum(double* __restrict__ S, const double* __restrict__ old,
-                                                 int64_t old_size, int64_t os, int64_t nodes,
-                                                 const double* __restrict__ tau,
-                                                 const double* __restrict__ kb, int sum_alg,
-                                                 double sum_param, int bs) {
-    int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (id >= nodes) return;
-    double time_sum = 0.0;
-    if (old_size >= 2) {
-        for (int64_t t = old_size - 2; t >= 0; t -= bs) {
-            int br = 0, cnt = 0;
-            for (int tt = 0; tt < bs && t - tt >= 0; tt++) {
-                int64_t l = t - tt;
-                double kv = kb[l];
-                double diff = old[(l + 1) * os + id] - old[l * os + id];
-                time_sum += kv * diff / tau[l];
-                if (fabs(kv) < sum_param) br++;
-                cnt++;
+// interval first, in chunks of BS levels; sum_alg 1 stops after the first full
+// chunk whose weights are all below sum_param in magnitude (the test is on the
+// weights alone, so every workgroup finds the cut `lo` first and the sum runs
+// over [lo, n)).
+// HBM bound: each level is read once (16 bytes per thread and load, 8 levels
+// in flight), its difference to the next newer one formed in registers, kb/tau
+// divided once per workgroup into LDS windows.  The intervals are split over
+// the grid's y as the plain stream's levels are: one thread walking the whole
+// history of a node leaves 10^4 nodes on 40 workgroups, each with one load
+// in flight (4000 levels x 10^4 nodes: 1775 us, 0.18 TB/s; split: 54 + 4 us,
+// 5.9 TB/s).
+// Partial rows out[ks * out_stride + i], added newest first by k_ref_combine.
+constexpr int kRefWin = 1024;
+template <int V>
+__global__ __launch_bounds__(256) void k_ref_sum(double* __restrict__ out, int64_t out_stride,
+                                                 const double* __restrict__ old, int64_t n, int64_t os, int64_t nodes,
+                                                 const double* __restrict__ tau, const double* __restrict__ kb,
+                                                 int sum_alg, double sum_param, int bs, int64_t chunk) {
+    __shared__ double w[kRefWin];                          // w[l - w0] = kb[l] / tau[l]
+    __shared__ unsigned long long cut;                     // first chunk (newest first) wholly below sum_param
+    const int tid = threadIdx.x;
+    int64_t lo = 0;
+    if (sum_alg == 1) {
+        const int64_t full = n / bs;
+        if (tid == 0) cut = (unsigned long long)full;
+        __syncthreads();
+        for (int64_t m0 = 0; m0 < full; m0 += 256) {
+            const int64_t m = m0 + tid;
+            bool below = m < full;
+            for (int k = 0; k < bs && below; k++) below = fabs(kb[n - 1 - m * bs - k]) < sum_param;
+            if (below) atomicMin(&cut, (unsigned long long)m);
+            __syncthreads();
+            const bool found = cut < (unsigned long long)(m0 + 256);
+            __syncthreads();
+            if (found) break;
+        }
+        if (cut < (unsigned long long)full) lo = n - ((int64_t)cut + 1) * bs;
+    }
+    const int64_t t0 = max(lo, (int64_t)blockIdx.y * chunk), t1 = min(n, ((int64_t)blockIdx.y + 1) * chunk);
+    const int64_t i = ((int64_t)blockIdx.x * 256 + tid) * V;
+    const bool ok = i < nodes;                             // the other threads still stage weights
+    double acc[V], prev[V];
+    auto level = [&](int64_t l, double (&v)[V]) {
+        if constexpr (V == 2) {
+            const double2 d = *reinterpret_cast<const double2*>(old + l * os + i);
+            v[0] = d.x;
+            v[1] = d.y;
+        } else {
+            v[0] = old[l * os + i];
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < V; k++) acc[k] = prev[k] = 0.0;
+    if (ok && t1 > t0) level(t1, prev);
+    for (int64_t w1 = t1; w1 > t0; w1 -= kRefWin) {
+        const int64_t w0 = max(t0, w1 - kRefWin);
+        __syncthreads();
+        for (int q = tid; q < (int)(w1 - w0); q += 256) w[q] = kb[w0 + q] / tau[w0 + q];
+        __syncthreads();
+        if (!ok) continue;
+        int64_t l = w1 - 1;
+        for (; l - 7 >= w0; l -= 8) {
+            double v[8][V];
+#pragma unroll
+            for (int j = 0; j < 8; j++) level(l - j, v[j]);
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const double wj = w[l - j - w0];
+#pragma unroll
+                for (int k = 0; k < V; k++) {
+                    acc[k] = fma(wj, prev[k] - v[j][k], acc[k]);
+                    prev[k] = v[j][k];
+                }
             }
-            if (sum_alg == 1 && br == bs) break;
-            (void)cnt;
+        }
+        for (; l >= w0; l--) {
+            double v[V];
+            level(l, v);
+#pragma unroll
+            for (int k = 0; k < V; k++) {
+                acc[k] = fma(w[l - w0], prev[k] - v[k], acc[k]);
+                prev[k] = v[k];
+            }
         }
     }
-    S[id] = time_sum;
+    if (!ok) return;
+#pragma unroll
+    for (int k = 0; k < V; k++)
+        if (i + k < nodes) out[(int64_t)blockIdx.y * out_stride + i + k] = acc[k];
+}
+
+// S[i] = the parts' sums, newest part first.
+__global__ __launch_bounds__(256) void k_ref_combine(double* __restrict__ S, const double* __restrict__ part,
+                                                     int splits, int64_t nodes) {
+    constexpr int W = 16;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= nodes) return;
+    double s = 0.0;
+    for (int k0 = splits - 1; k0 >= 0; k0 -= W) {
+        double v[W];
+#pragma unroll
+        for (int j = 0; j < W; j++) v[j] = k0 >= j ? part[(int64_t)(k0 - j) * nodes + i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < W; j++) s += v[j];
+    }
+    S[i] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -597,14 +678,42 @@ fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int
     return FPDE_OK;
 }
 
+// Parts of the reference Sum: about 2048 workgroups with the 512-node tiles
+// (8 per CU; 512 to 4096 measured alike), each walking at least 64 intervals:
+// whole calls of 4000 x 10^4 took 71, 71 and 67 us with at least 16, 32 and 64,
+// of 8000 x 300 41, 29 and 24 us (fewer partial rows to add), of 500 x 5000
+// 18.5, 18.3 and 19.6 us.
+int ref_sum_splits(int64_t nodes, int64_t intervals) {
+    const int64_t tiles = (nodes + 511) / 512;
+    int64_t s = std::min<int64_t>((2048 + tiles - 1) / tiles, intervals / 64);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(s, kPlainMaxSplits));
+}
+
 fpde_status launch_ref_sum(double* S, const double* old, int64_t old_size, int64_t os,
                            int64_t nodes, const double* tau, const double* kb, int sum_alg,
-                           double sum_param, int bs, hipStream_t st) {
+                           double sum_param, int bs, double* part, hipStream_t st) {
     if (nodes <= 0) return FPDE_OK;
-    dim3 grid((unsigned)((nodes + 255) / 256));
     if (bs < 1) bs = 1;
-    hipLaunchKernelGGL(k_ref_sum, grid, dim3(256), 0, st, S, old, old_size, os, nodes, tau, kb,
-                       sum_alg, sum_param, bs);
+    const int64_t n = old_size >= 2 ? old_size - 1 : 0;
+    int splits = ref_sum_splits(nodes, n);
+    if (splits > 1 && !part) { set_error("reference sum: no room for the partial rows"); return FPDE_ERR_ARG; }
+    const int64_t chunk = std::max<int64_t>((n + splits - 1) / splits, 1);
+    splits = (int)std::max<int64_t>((n + chunk - 1) / chunk, 1);
+    double* out = splits > 1 ? part : S;
+    // two nodes per thread where every level's rows are 16-byte aligned and the
+    // last pair stays inside the level
+    const bool pairs = os % 2 == 0 && ((uintptr_t)old & 15) == 0;
+    const int64_t per = pairs ? 512 : 256;
+    const dim3 grid((unsigned)((nodes + per - 1) / per), (unsigned)splits);
+    if (pairs)
+        hipLaunchKernelGGL(k_ref_sum<2>, grid, dim3(256), 0, st, out, nodes, old, n, os, nodes, tau, kb, sum_alg,
+                           sum_param, bs, chunk);
+    else
+        hipLaunchKernelGGL(k_ref_sum<1>, grid, dim3(256), 0, st, out, nodes, old, n, os, nodes, tau, kb, sum_alg,
+                           sum_param, bs, chunk);
+    if (splits > 1)
+        hipLaunchKernelGGL(k_ref_combine, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, st, S, part, splits,
+                           nodes);
     return FPDE_OK;
 }
 

@@ -1172,6 +1172,7 @@ fpde_status fpde_shutdown(void) {
         kv.second = nullptr;
     }
     g_rows_tab.clear();
+    if (!scratch_shutdown()) rc = FPDE_ERR_HIP;
     if (have_dev) {
         (void)hipSetDevice(cur);
         if (hipDeviceSynchronize() != hipSuccess) rc = FPDE_ERR_HIP;

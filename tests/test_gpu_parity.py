@@ -1560,3 +1560,42 @@ def test_launches_that_cut_a_block_give_the_same_bits(fpde, block, picard):
         fpde.advance_batch([b], 0)
         np.testing.assert_array_equal(a.solution(), whole)
         np.testing.assert_array_equal(b.solution(), whole)
+
+
+@pytest.mark.parametrize("nodes,os_,levels", [(1, 1, 2), (2, 2, 1), (3, 3, 64), (511, 512, 33), (513, 513, 1100),
+                                              (1025, 1026, 2081), (5000, 5000, 130)])
+@pytest.mark.parametrize("keep", [None, 0.0, 0.3, 1.0])
+def test_reference_sum_parts_match_the_reference_loop(fpde, oracle, nodes, os_, levels, keep):
+    """fpde_reference_sum over its forms: one part and several, whole weight
+    windows and remainders, odd level strides (one node per thread) and even
+    ones (two); sum_alg 0 (keep None) and sum_alg 1 with the cut at the newest
+    chunk, inside, and nowhere; against the reference loop (newest interval
+    first, chunks of 16, the first full chunk below the threshold is the last
+    one added)."""
+    L = fpde.lib()
+    rng = np.random.default_rng(nodes + levels)
+    old = np.cumsum(rng.standard_normal((levels, os_)) * 1e-3, 0)
+    n = levels - 1
+    tau = 1e-3 * (1.0 + rng.random(max(n, 1)))
+    kb = np.sort(rng.random(max(n, 1)) + 0.1)
+    cut = 0.0 if keep is None or n == 0 else (10.0 if keep == 0.0 else float(kb[int((1 - keep) * (n - 1))]))
+    ref = np.zeros(nodes)
+    t = n - 1
+    while t >= 0:
+        lo = max(t - 15, 0)
+        for l in range(t, lo - 1, -1):
+            ref += kb[l] * (old[l + 1, :nodes] - old[l, :nodes]) / tau[l]
+        if keep is not None and t >= 15 and np.all(np.abs(kb[lo:t + 1]) < cut):
+            break
+        t -= 16
+    dv = Dev(L)
+    try:
+        bS, bo, bt, bk = dv.put(np.full(nodes, 7.0)), dv.put(old), dv.put(tau), dv.put(kb)
+        rc = L.fpde_reference_sum(dv.ptr(bS), dv.ptr(bo), levels, os_, nodes, dv.ptr(bt), dv.ptr(bk),
+                                  0 if keep is None else 1, cut)
+        assert rc == 0, L.fpde_last_error()
+        got = dv.get(bS, nodes)
+    finally:
+        dv.close()
+    scale = np.max(np.abs(ref)) if n else 1.0
+    assert np.max(np.abs(got - ref)) <= 1e-12 * scale
