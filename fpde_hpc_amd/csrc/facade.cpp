@@ -546,41 +546,22 @@ fpde_status fpde_history_block_gemm(int mode, const double* D, int64_t ld, int64
     }
     bool split = mode >= 2;
     if (split && tc % kGroup) { set_error("split modes need tc % 32 == 0"); return FPDE_ERR_ARG; }
-    int ks = gemm_max_splits(nodes);
-    double* part = nullptr;
-    void* comp[3] = {nullptr, nullptr, nullptr};
-    float* scale = nullptr;
-    void* afrag = nullptr;
-    double* ainv = nullptr;
-    fpde_status rc = FPDE_OK;
+    // partial rows of the K splits, then the block's weight fragments (split forms)
+    const size_t part_bytes = sizeof(double) * (size_t)gemm_max_splits(nodes) * block * ld;
+    const size_t frag_bytes = split ? split_afrag_bytes(mode, block, tc / kGroup) : 0;
+    const size_t inv_bytes = split ? sizeof(double) * (size_t)(tc / kGroup) * (block / 16) : 0;
+    ScratchLease scratch;
+    fpde_status rc = scratch.take(part_bytes + frag_bytes + inv_bytes);
+    if (rc != FPDE_OK) return rc;
+    double* part = (double*)scratch.ptr();
+    void* afrag = (char*)scratch.ptr() + part_bytes;
+    double* ainv = (double*)((char*)afrag + frag_bytes);
     int splits = 0;
-    int64_t lv = ((levels + kGroup - 1) / kGroup) * kGroup;
-    hipError_t e = hipMalloc(&part, sizeof(double) * (size_t)ks * block * ld);
-    if (e == hipSuccess && split) {
-        for (int c = 0; c < 3 && e == hipSuccess; c++) e = hipMalloc(&comp[c], 2 * (size_t)lv * ld);
-        if (e == hipSuccess) e = hipMalloc(&scale, sizeof(float) * (size_t)(lv / kGroup) * ld);
-        if (e == hipSuccess) e = hipMalloc(&afrag, split_afrag_bytes(mode, block, (int)(lv / kGroup)));
-        if (e == hipSuccess) e = hipMalloc(&ainv, sizeof(double) * (size_t)(lv / kGroup) * (block / 16));
-    }
-    if (e != hipSuccess) { rc = FPDE_ERR_NOMEM; set_error("hipMalloc failed"); }
-    if (rc == FPDE_OK && split) rc = launch_pack_split(mode, D, ld, (int)nodes, 0, tc / kGroup, comp[0], comp[1], comp[2], scale, 0);
-    if (rc == FPDE_OK) {
-        if (split) rc = launch_gemm_split(mode, comp[0], comp[1], comp[2], scale, ld, (int)nodes, n0, tc, block, omega, nullptr, 0, afrag, ainv, part, &splits, 0);
-        else rc = launch_gemm_f64(D, ld, (int)nodes, n0, tc, block, omega, part, &splits, 0);
-    }
-    if (rc == FPDE_OK) {
-        // P[r] = sum over K splits (combine kernel, one row at a time)
-        for (int r = 0; r < block && rc == FPDE_OK; r++)
-            rc = launch_hist_combine(P + (size_t)r * ld, part, splits, (int64_t)block * ld, (int64_t)r * ld, D, ld,
-                                     nodes, 0, 0, omega, 0, 0, 0, nullptr, nullptr, 1.0, 0);
-    }
-    e = hipDeviceSynchronize();
+    if (split) rc = launch_gemm_split_direct(mode, D, ld, (int)nodes, n0, tc, block, omega, afrag, ainv, part, &splits, 0);
+    else rc = launch_gemm_f64(D, ld, (int)nodes, n0, tc, block, omega, part, &splits, 0);
+    if (rc == FPDE_OK) rc = launch_part_sum(P, part, splits, block, ld, (int)nodes, 0);
+    const hipError_t e = hipDeviceSynchronize();
     if (rc == FPDE_OK && e != hipSuccess) { rc = FPDE_ERR_HIP; set_error(hipGetErrorString(e)); }
-    hipFree(part);
-    for (int c = 0; c < 3; c++) hipFree(comp[c]);
-    hipFree(scale);
-    hipFree(afrag);
-    hipFree(ainv);
     return rc;
 }
 

@@ -504,6 +504,13 @@ fpde_status launch_gemm_split(int mode, const void* c0, const void* c1, const vo
                               int64_t ld, int nodes, int n0, int tc, int block, const double* omega,
                               const double* W, int64_t ldw, void* afrag, double* ainv, double* P,
                               int* splits_out, hipStream_t st, int max_splits = 0);
+// the same GEMM from the FP64 levels themselves (no packed components), and
+// the sum of its partial rows into P [rows][ld]
+fpde_status launch_gemm_split_direct(int mode, const double* D, int64_t ld, int nodes, int n0, int tc, int block,
+                                     const double* omega, void* afrag, double* ainv, double* P, int* splits_out,
+                                     hipStream_t st);
+fpde_status launch_part_sum(double* P, const double* part, int splits, int rows, int64_t ld, int nodes,
+                            hipStream_t st);
 fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st);
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st);
 bool step1d_block_supported(int N, int C);

@@ -484,6 +484,28 @@ __global__ __launch_bounds__(256) void k_afrag_split(int n0, const double* __res
     }
 }
 
+// The products of one 32-level group, components a (weights) and b (history),
+// hi first: one fp32 chain, hi*hi, then the smaller cross products (their
+// rounding is 2^-24 of the group sum).
+template <typename T, int NS>
+__device__ __forceinline__ f4_t split_products(const typename SplitTraits<T>::vec (&a)[NS],
+                                               const typename SplitTraits<T>::vec (&b)[NS]) {
+    f4_t p = {0.f, 0.f, 0.f, 0.f};
+    auto add = [&](int i, int j) {
+        if constexpr (SplitTraits<T>::scaled) p = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], p, 0, 0, 0);
+        else p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], p, 0, 0, 0);
+    };
+    add(0, 0);
+    add(0, 1);
+    add(1, 0);
+    if constexpr (NS == 3) {
+        add(0, 2);
+        add(1, 1);
+        add(2, 0);
+    }
+    return p;
+}
+
 // Split GEMM.  Grid: x = 64-node tiles, y = K splits.  Per 32-level group:
 // wave w (nodes 16w..16w+15) loads its B fragments (one 16-B load per
 // component), the A fragments (k_afrag_split) come from LDS, where the block
@@ -566,38 +588,15 @@ __global__ __launch_bounds__(256) void k_gemm_split(const T* __restrict__ c0, co
         for (int gi = 0; gi < GB; gi++) {
             int g = gb0 + gi;
             if (g >= ghi) break;
-            const vec_t bh = bfr[gi][0], bm = bfr[gi][1];
+            vec_t b[NS];
+#pragma unroll
+            for (int c = 0; c < NS; c++) b[c] = bfr[gi][c];
 #pragma unroll
             for (int rt = 0; rt < RT; rt++) {
-                vec_t ah = afrag[0][gi][rt][lane];
-                vec_t am = afrag[1][gi][rt][lane];
-                // one fp32 chain per group: hi*hi first, then the smaller
-                // cross products (their rounding is 2^-24 of the group sum)
-                f4_t z = {0.f, 0.f, 0.f, 0.f};
-                f4_t p;
-                if constexpr (SplitTraits<T>::scaled) {
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bh, z, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bm, p, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bh, p, 0, 0, 0);
-                    if (NS == 3) {
-                        vec_t al = afrag[NS - 1][gi][rt][lane];
-                        vec_t bl = bfr[gi][NS - 1];
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, bl, p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_f16(am, bm, p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh, p, 0, 0, 0);
-                    }
-                } else {
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bh, z, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bm, p, 0, 0, 0);
-                    p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bh, p, 0, 0, 0);
-                    if (NS == 3) {
-                        vec_t al = afrag[NS - 1][gi][rt][lane];
-                        vec_t bl = bfr[gi][NS - 1];
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ah, bl, p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(am, bm, p, 0, 0, 0);
-                        p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(al, bh, p, 0, 0, 0);
-                    }
-                }
+                vec_t a[NS];
+#pragma unroll
+                for (int c = 0; c < NS; c++) a[c] = afrag[c][gi][rt][lane];
+                const f4_t p = split_products<T, NS>(a, b);
                 double scr = SplitTraits<T>::scaled ? bsc[gi] * ainv[gi][rt] : 1.0;
 #pragma unroll
                 for (int v = 0; v < 4; v++) acc[rt][v] = fma(scr, (double)p[v], acc[rt][v]);
@@ -614,6 +613,160 @@ __global__ __launch_bounds__(256) void k_gemm_split(const T* __restrict__ c0, co
             }
         }
     }
+}
+
+// The split GEMM straight from the FP64 history, for one block of steps (the
+// direct call): the levels are split into their 16-bit components in the
+// registers of the wave that multiplies them, in the values and the order of
+// k_pack_split and k_gemm_split, so the results are theirs bit for bit.  One
+// pass over 8 B per level and node instead of packing them (8 read, 4 or 6
+// written) and reading the components back; where a history serves many
+// blocks, as in a solve, packing once is the cheaper way.  HBM bound: a lane's
+// 8 levels x 4 groups are in flight while the previous 4 groups' are split and
+// multiplied (levels 8 (l/16) + e of the group at node l%16 are just its B
+// operand, so nothing goes through LDS but the weights' fragments).
+// 9984 levels x 10^4 nodes, B = 64, bf16: 182-201 us (4.2 TB/s) and 13 us for the
+// sum of 13 splits, against 259 us packing, 105 us GEMM, 64 sums of 3.5 us and
+// about 17 ms of allocating and freeing the components; whole call 19.1 -> 0.20 ms.
+template <typename T, int NS, int BR>
+__global__ __launch_bounds__(256) void k_gemm_split_direct(const double* __restrict__ D, int64_t ld, int nodes, int tc,
+                                                           int kchunk,
+                                                           const typename SplitTraits<T>::vec* __restrict__ afrag_g,
+                                                           const double* __restrict__ ainv_g,
+                                                           double* __restrict__ P) {
+    typedef typename SplitTraits<T>::vec vec_t;
+    constexpr int RT = BR / 16;
+    constexpr int GB = 2;                                  // groups per batch
+    __shared__ vec_t afrag[NS][GB][RT][64];
+    __shared__ double ainv[GB][RT];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int ks = blockIdx.y;
+    const int glo = (ks * kchunk) / kGroup;
+    const int ghi = min(tc, ks * kchunk + kchunk) / kGroup;
+    const int node = blockIdx.x * 64 + wave * 16 + (lane & 15);
+    const bool node_ok = node < nodes;
+    const double* col = D + (node_ok ? node : 0) + (int64_t)(8 * (lane >> 4)) * ld;
+    d4_t acc[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) acc[rt] = (d4_t){0.0, 0.0, 0.0, 0.0};
+    constexpr int AE = (GB * RT * 64 + 255) / 256;         // A entries per thread per batch
+    double dn[GB][8];
+    vec_t an[AE][NS];
+    double ain[AE];
+    auto load_batch = [&](int gb0) {
+#pragma unroll
+        for (int gi = 0; gi < GB; gi++) {
+            const double* d = col + (int64_t)min(gb0 + gi, ghi - 1) * kGroup * ld;
+#pragma unroll
+            for (int e = 0; e < 8; e++) dn[gi][e] = d[(int64_t)e * ld];
+        }
+#pragma unroll
+        for (int k = 0; k < AE; k++) {
+            const int f = min((int)threadIdx.x + 256 * k, GB * RT * 64 - 1);
+            const int fl = f & 63, frt = (f >> 6) % RT, fgb = f / (64 * RT);
+            const int g = min(gb0 + fgb, ghi - 1);          // groups past ghi are never used
+            const size_t base = ((size_t)g * NS * RT + frt) * 64 + fl;
+            an[k][0] = afrag_g[base];
+            an[k][1] = afrag_g[base + RT * 64];
+            if (NS == 3) an[k][NS - 1] = afrag_g[base + 2 * RT * 64];
+            ain[k] = ainv_g[g * RT + frt];
+        }
+    };
+    if (glo < ghi) load_batch(glo);
+    for (int gb0 = glo; gb0 < ghi; gb0 += GB) {
+        double dv[GB][8];
+#pragma unroll
+        for (int gi = 0; gi < GB; gi++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) dv[gi][e] = node_ok ? dn[gi][e] : 0.0;
+        __syncthreads();                       // the previous batch is done with the LDS fragments
+#pragma unroll
+        for (int k = 0; k < AE; k++) {
+            const int f = threadIdx.x + 256 * k;
+            const int fl = f & 63, frt = (f >> 6) % RT, fgb = f / (64 * RT);
+            if (f < GB * RT * 64) {
+#pragma unroll
+                for (int c = 0; c < NS; c++) afrag[c][fgb][frt][fl] = an[k][c];
+                if (fl == 0) ainv[fgb][frt] = ain[k];
+            }
+        }
+        if (gb0 + GB < ghi) load_batch(gb0 + GB);
+        __syncthreads();
+#pragma unroll
+        for (int gi = 0; gi < GB; gi++) {
+            if (gb0 + gi >= ghi) break;
+            // this lane's levels in components (k_pack_split)
+            double sc = 1.0;
+            if constexpr (SplitTraits<T>::scaled) {
+                double mx = 0.0;
+#pragma unroll
+                for (int e = 0; e < 8; e++) mx = fmax(mx, fabs(dv[gi][e]));
+                mx = fmax(mx, __shfl_xor(mx, 16));          // the group's other 24 levels of the node
+                mx = fmax(mx, __shfl_xor(mx, 32));
+                if (mx > 0.0) sc = ldexp(1.0, ilogb(mx) - 14);
+            }
+            const double inv = 1.0 / sc;
+            vec_t b[NS];
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const double x = dv[gi][e] * inv;
+                const T h = (T)(float)x;
+                const double r = x - (double)(float)h;
+                const T m = (T)(float)r;
+                b[0][e] = h;
+                b[1][e] = m;
+                if (NS == 3) b[NS - 1][e] = (T)(float)(r - (double)(float)m);
+            }
+            const double bsc = SplitTraits<T>::scaled ? (node_ok ? (double)(float)sc : 0.0) : 1.0;
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) {
+                vec_t a[NS];
+#pragma unroll
+                for (int c = 0; c < NS; c++) a[c] = afrag[c][gi][rt][lane];
+                const f4_t p = split_products<T, NS>(a, b);
+                const double scr = SplitTraits<T>::scaled ? bsc * ainv[gi][rt] : 1.0;
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[rt][v] = fma(scr, (double)p[v], acc[rt][v]);
+            }
+        }
+    }
+    if (node_ok) {
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                int r = rt * 16 + 4 * (lane >> 4) + v;
+                P[((int64_t)ks * BR + r) * ld + node] = acc[rt][v];
+            }
+        }
+    }
+}
+
+// P[r][i] = the K splits' partial rows added in split order (as the 3D history
+// combine adds them), for every row of a block at once.
+__global__ __launch_bounds__(256) void k_part_sum(double* __restrict__ P, const double* __restrict__ part, int splits,
+                                                  int rows, int64_t ld, int nodes) {
+    constexpr int W = 16;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int r = blockIdx.y;
+    if (i >= nodes) return;
+    double s = 0.0;
+    for (int k0 = 0; k0 < splits; k0 += W) {
+        double v[W];
+#pragma unroll
+        for (int j = 0; j < W; j++) v[j] = (k0 + j < splits) ? part[((int64_t)(k0 + j) * rows + r) * ld + i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < W; j++) s += v[j];
+    }
+    P[(int64_t)r * ld + i] = s;
+}
+
+fpde_status launch_part_sum(double* P, const double* part, int splits, int rows, int64_t ld, int nodes,
+                            hipStream_t st) {
+    hipLaunchKernelGGL(k_part_sum, dim3((unsigned)((nodes + 255) / 256), (unsigned)rows), dim3(256), 0, st, P, part,
+                       splits, rows, ld, nodes);
+    FPDE_HIP_TRY(hipGetLastError());
+    return FPDE_OK;
 }
 
 // ---------------------------------------------------------------------------
@@ -819,6 +972,48 @@ static fpde_status gemm_split_b(int block, dim3 grid, hipStream_t st, const void
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
     return FPDE_OK;
+}
+
+template <typename T, int NS, int BR>
+static void gemm_direct_t(dim3 grid, hipStream_t st, const double* D, int64_t ld, int nodes, int n0, int tc, int kchunk,
+                          const double* omega, void* afrag, double* ainv, double* P) {
+    typedef typename SplitTraits<T>::vec vec_t;
+    hipLaunchKernelGGL((k_afrag_split<T, NS, BR, false>), dim3(tc / kGroup), dim3(256), 0, st, n0, omega, (const double*)nullptr,
+                       (int64_t)0, (vec_t*)afrag, ainv);
+    hipLaunchKernelGGL((k_gemm_split_direct<T, NS, BR>), grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk,
+                       (const vec_t*)afrag, (const double*)ainv, P);
+}
+
+template <typename T, int NS>
+static fpde_status gemm_direct_b(int block, dim3 grid, hipStream_t st, const double* D, int64_t ld, int nodes, int n0,
+                                 int tc, int kchunk, const double* omega, void* afrag, double* ainv, double* P) {
+    switch (block) {
+        case 16: gemm_direct_t<T, NS, 16>(grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        case 32: gemm_direct_t<T, NS, 32>(grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        case 64: gemm_direct_t<T, NS, 64>(grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        case 128: gemm_direct_t<T, NS, 128>(grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
+    }
+    return FPDE_OK;
+}
+
+fpde_status launch_gemm_split_direct(int mode, const double* D, int64_t ld, int nodes, int n0, int tc, int block,
+                                     const double* omega, void* afrag, double* ainv, double* P, int* splits_out,
+                                     hipStream_t st) {
+    if (tc <= 0) { *splits_out = 0; return FPDE_OK; }
+    if (tc % kGroup != 0) { set_error("split GEMM needs a group-aligned cut"); return FPDE_ERR_ARG; }
+    int kchunk, splits;
+    gemm_split_plan(tc, nodes, &kchunk, &splits, 0);
+    const dim3 grid((nodes + 63) / 64, splits);
+    fpde_status rc;
+    switch (mode) {
+        case HIST_SPLIT_BF16: rc = gemm_direct_b<__bf16, 2>(block, grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        case HIST_SPLIT_F16: rc = gemm_direct_b<_Float16, 2>(block, grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        case HIST_SPLIT_BF16X3: rc = gemm_direct_b<__bf16, 3>(block, grid, st, D, ld, nodes, n0, tc, kchunk, omega, afrag, ainv, P); break;
+        default: set_error("bad split mode"); return FPDE_ERR_ARG;
+    }
+    *splits_out = splits;
+    return rc;
 }
 
 size_t split_afrag_bytes(int mode, int block, int groups) {

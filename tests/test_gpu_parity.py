@@ -1599,3 +1599,39 @@ def test_reference_sum_parts_match_the_reference_loop(fpde, oracle, nodes, os_, 
         dv.close()
     scale = np.max(np.abs(ref)) if n else 1.0
     assert np.max(np.abs(got - ref)) <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+@pytest.mark.parametrize("nodes,tc,block", [(1, 32, 16), (63, 0, 32), (65, 96, 128), (130, 32 * 37, 64),
+                                            (2000, 32 * 17, 32)])
+def test_block_gemm_edges_exact(fpde, mode, nodes, tc, block):
+    """The direct block product at its edges (one node, tiles with a remainder,
+    no level at all, one group, odd group counts, several K splits; a group of
+    zeros, a node at zero in another, one group far below the others, which
+    moves the fp16 scale) on data that every form represents and adds exactly:
+    levels of 16 significant bits (two 8-bit components), weights 3, 2, 1, so a
+    32-level group sums within 24 bits.  No rounding, so equality."""
+    L = fpde.lib()
+    rng = np.random.default_rng(nodes + tc)
+    ld = -(-nodes // 64) * 64
+    D = np.zeros((tc + 32, ld))
+    D[:tc, :nodes] = rng.integers(-2 ** 15, 2 ** 15, (tc, nodes)) / 1024.0
+    if tc >= 96:
+        D[:32] = 0.0
+        D[32:64, 0] = 0.0
+        D[64:96] *= 2.0 ** -20
+    n0 = tc + 3
+    omega = np.zeros(n0 + block + 600)
+    omega[: n0 + block] = np.sort(rng.integers(1, 4, n0 + block))[::-1]
+    W = np.array([[omega[n0 + r - t - 1] for t in range(tc)] for r in range(block)]).reshape(block, tc)
+    ref = W @ D[:tc, :nodes]
+    dv = Dev(L)
+    try:
+        bD, bw, bP = dv.put(D), dv.put(omega), dv.put(np.full(block * ld, 7.0))
+        rc = L.fpde_history_block_gemm(mode, dv.ptr(bD), ld, nodes, tc + 32, n0, tc, block, dv.ptr(bw), dv.ptr(bP))
+        assert rc == 0, L.fpde_last_error()
+        P = dv.get(bP, block * ld).reshape(block, ld)
+    finally:
+        dv.close()
+    np.testing.assert_array_equal(P[:, :nodes], ref)
+    assert np.all(P[:, nodes:] == 7.0)
