@@ -773,9 +773,8 @@ __device__ inline void solve_separators(const Step1DLds& L, int C, int c, int p,
         const int rr = ok ? r : 0, rl = rr > 0 ? rr - 1 : 0;
         const double v0 = xch_value(L, rr, 0), v1 = xch_value(L, rr, 1), v2 = xch_value(L, rr, 2),
                      v3 = xch_value(L, rr, 3);
-        // (row 0 has v0 = 0: what is read for its left neighbour does not enter)
-        const double xl = rr > 0 ? xch_value(L, rl, 4) : 0.0, yl = rr > 0 ? xch_value(L, rl, 5) : 0.0,
-                     zl = rr > 0 ? xch_value(L, rl, 6) : 0.0;
+        // (row 0 has v0 = 0: the values read for a left neighbour, its own chunk's, do not enter)
+        const double xl = xch_value(L, rl, 4), yl = xch_value(L, rl, 5), zl = xch_value(L, rl, 6);
         const double inv = rcp_nr(fma(v0, zl, v1));
         a[j] = ok ? (v0 * yl) * inv : 0.0;
         cc[j] = ok && r + 1 < C ? v2 * inv : 0.0;
@@ -1151,8 +1150,10 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         return true;
     };
     // every chunk's words into L.words once they carry the barrier's tag, 64
-    // chunks per round: load k takes chunks 4 k .. 4 k + 3 of the round
-    auto collect = [&](int b) -> bool {
+    // chunks per round: load k takes chunks 4 k .. 4 k + 3 of the round; the
+    // largest measure on the way (its halves sit in lanes 14 and 15 of each
+    // row of 16)
+    auto collect = [&](int b, double& largest) -> bool {
         const unsigned tg = xtag(b);
         int64_t t0 = -1;
         constexpr int K = 16;
@@ -1180,15 +1181,24 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
                         w[k] = __hip_atomic_load(x + 64 * k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             unsigned long long* to = &L.words[(j0 + (l >> 4)) * kXchPad + (l & 15)];
+            double m = 0.0;
 #pragma unroll
-            for (int k = 0; k < K; k++)
+            for (int k = 0; k < K; k++) {
                 if (k < mine) to[4 * k * kXchPad] = w[k];
+                // lane 15 of a row: its own half above lane 14's
+                const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)w[k], 0x111, 0xf, 0xf, false);
+                m = fmax(m, k < mine ? __hiloint2double((int)(unsigned)w[k], lo) : 0.0);
+            }
+#pragma unroll
+            for (int r = 15; r < 64; r += 16)
+                largest = fmax(largest, __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(m), r),
+                                                         __builtin_amdgcn_readlane(__double2loint(m), r)));
         }
         wave_lds_sync();
         return true;
     };
     // the measure words alone
-    auto collect_measures = [&](int b) -> bool {
+    auto collect_measures = [&](int b, double& largest) -> bool {
         const unsigned tg = xtag(b);
         int64_t t0 = -1;
         for (int j0 = 0; j0 < C; j0 += 64) {
@@ -1200,9 +1210,8 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
                 if (__all((unsigned)(w[0] >> 32) == tg && (unsigned)(w[1] >> 32) == tg)) break;
                 if (timed_out(&t0)) return false;
             }
-            for (int k = 0; k < 2; k++) L.words[j * kXchPad + kXchMeasure + k] = w[k];
+            largest = fmax(largest, wave_max(__longlong_as_double((long long)((w[1] << 32) | (w[0] & 0xffffffffull)))));
         }
-        wave_lds_sync();
         return true;
     };
 
@@ -1273,10 +1282,9 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         }
         if (lane == 0) L.pub[7] = meas;
         publish(b, decide ? kXchMeasure : 0);
-        if (!(decide ? collect_measures(b) : collect(b))) return kTimeout;
-        double m = 0.0;
-        for (int j = lane; j < C; j += 64) m = fmax(m, xch_value(L, j, 7));
-        const bool met = __builtin_amdgcn_readfirstlane(wave_max(m) <= tol ? 1 : 0) != 0;     // (uniform)
+        double largest = 0.0;
+        if (!(decide ? collect_measures(b, largest) : collect(b, largest))) return kTimeout;
+        const bool met = __builtin_amdgcn_readfirstlane(largest <= tol ? 1 : 0) != 0;     // (uniform)
         if (decide) return met ? kMet : kNotMet;
         double um, us, up;
         const double xl = c > 0 ? xch_value(L, c - 1, 4) : 0.0, yl = c > 0 ? xch_value(L, c - 1, 5) : 0.0,
