@@ -323,9 +323,8 @@ struct Step1DArgs {
     int near_lo;              // near terms t in [near_lo, n)
     double* Sbuf;             // history term of step n, reused by Picard iterations
     double* xyz;              // [3][ld] chunk factors
-    double* red;              // [2][2*C][4]
+    double* red;              // [2][C][8] the chunks' values of the separators' system, by launch parity
     double* Uit;              // Picard iterate (for the convergence test)
-    double* dmax;             // [2][C] per-chunk max |U^k - U^{k-1}|
     int* flags;               // unused
     double tol;
     int64_t omega_stride;     // per-step weight rows (prescribed grid): omega + (n - n0) * stride
@@ -444,6 +443,14 @@ __device__ inline void space_unit(const double* __restrict__ F, int N, const dou
     const double sum = (L.red[0][v][l] + L.red[1][v][l]) + (L.red[2][v][l] + L.red[3][v][l]);
     const int64_t i = (int64_t)kSpTile * t + 16 * (l & 15) + 4 * v + (l >> 4);
     P[(int64_t)y * ldp + i] = sum;
+}
+
+// F of an interior row (Om1 equation 0, fpde_hpc_1d.cpp:4176-4179): K_j and
+// K_{j-1}, U_{j-1}, U_j, U_{j+1}; one division, no product of U lost to the
+// difference, and the same bits in the flux kernel and in a finalize launch
+__device__ inline double space_flux(double Km, double Kj, double um, double u0, double up, double h) {
+#pragma clang fp contract(off)
+    return fma(Kj, up - u0, -(Km * (u0 - um))) / (h * h);
 }
 
 // E_i of an interior row i (1 <= i <= N-2) from the partials and the two

@@ -203,7 +203,6 @@ struct fpde_solver {
     double* red = nullptr;
     double* part = nullptr;
     double* Uit = nullptr;
-    double* dmax = nullptr;
     double* mid = nullptr;     // near-field groups folded ahead [block][ld] (1D cooperative launches, 3D combine)
     double* H = nullptr;       // sum_alg 2 moments [P][ld]
     double* Uit0 = nullptr;    // initial Picard iterate
@@ -402,7 +401,7 @@ fpde_status solver_alloc(fpde_solver* s) {
     if (sp.dims == 1) {
         s->C = chunk_count(sp);
         DALLOC(s->xyz, sizeof(double) * 3 * p.ld);
-        DALLOC(s->red, sizeof(double) * 2 * 2 * s->C * 4);
+        DALLOC(s->red, sizeof(double) * 2 * s->C * 8);
         DALLOC(s->Uit, sizeof(double) * p.ld);
         DALLOC(s->Uit0, sizeof(double) * p.ld);
         DALLOC(s->uend, sizeof(double) * 2 * 2 * s->C);
@@ -436,7 +435,6 @@ fpde_status solver_alloc(fpde_solver* s) {
         s->block_mode = (sp.step_mode == 0) && blocked_history && !space && step1d_block_supported(sp.nodes, s->C);
         s->la = s->block_mode && lookahead_spec(sp);
         if (s->block_mode && s->w.ser_P == 0) DALLOC(s->mid, sizeof(double) * (size_t)sp.block * p.ld);
-        DALLOC(s->dmax, sizeof(double) * 2 * s->C);
         DALLOC(s->flags, sizeof(int) * 16);
     } else {
         int n = sp.nodes;
@@ -742,7 +740,6 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
     a.xyz = s->xyz;
     a.red = s->red;
     a.Uit = s->Uit;
-    a.dmax = s->dmax;
     a.flags = s->flags;
     a.tol = sp.picard_tol;
     a.prev_k = s->last_k;
@@ -854,7 +851,6 @@ Step1DArgs block_args(fpde_solver* s, int n, int n_end, int n0, int nsplit, int6
     a.part_stride = stride;
     a.near_lo = near_lo;
     a.red = s->red;
-    a.dmax = s->dmax;
     a.xch = s->xch;
     a.xtag = launch_tag(s);
     a.err = s->err;

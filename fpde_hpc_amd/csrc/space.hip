@@ -27,8 +27,7 @@ __global__ __launch_bounds__(256) void k_space_flux(const double* __restrict__ U
         double Km, Kj, iC;
         vgm_coefs(um, (double)(j - 1) * h, ksat, mode, Km, iC);
         vgm_coefs(u0, (double)j * h, ksat, mode, Kj, iC);
-        const double hh = h * h;
-        f = Kj * up / hh - (Kj / hh + Km / hh) * u0 + Km * um / hh;
+        f = space_flux(Km, Kj, um, u0, up, h);
     }
     F[j] = f;
 }

@@ -5,16 +5,16 @@
 // sequential sweep of 1e4 rows is latency bound, so the line is cut into C
 // chunks of <= 256 nodes, one workgroup each (partitioned / SPIKE-style
 // solve):
-//  - inside a chunk the interior rows are solved by parallel cyclic reduction
-//    in LDS for three right-hand sides, giving U_i = x_i + y_i U_s + z_i U_e
-//    in terms of the chunk's end nodes s, e;
-//  - the end-node rows then form a tridiagonal "reduced" system of 2C rows,
-//    written to global memory;
-//  - the NEXT launch solves the reduced system redundantly in every
-//    workgroup (PCR in LDS) and back-substitutes its chunk.
-// So one launch = [finish the previous solve] + [history term, coefficients,
-// rows, chunk elimination of this solve]: one launch per Picard iteration and
-// no grid-wide barrier.  Rows (fpde_hpc_1d.cpp:3095-3142 with Dg=1, gamma=1):
+//  - a chunk's first node s is its separator; the rows after it are solved by
+//    one wave for three right-hand sides, giving U_i = x_i + y_i U_s + z_i U_s'
+//    in terms of the separators s and s' (the next chunk's);
+//  - the separators' rows, with the chunks put in, form a tridiagonal system of
+//    C rows, which every workgroup solves redundantly before it substitutes
+//    back.
+// The separators' values pass between the workgroups through an exchange in
+// memory within one cooperative launch, or from one launch to the next
+// (k_step1d: one launch per Picard iteration and no grid-wide barrier).
+// Rows (fpde_hpc_1d.cpp:3095-3142 with Dg=1, gamma=1):
 //   A_i U_{i-1} - R_i U_i + B_i U_{i+1} = Om_i,
 //   A_i = K_{i-1}/C_i/h^2, B_i = K_i/C_i/h^2, R_i = (K_i+K_{i-1})/C_i/h^2 + L,
 //   Om_i = -L U^n_i + S_n[i]      (Om1, :4165-4268; S_n = Da*history sum)
@@ -23,131 +23,6 @@
 #include "fpde_internal.h"
 
 namespace fpde {
-
-constexpr int kMaxRed = 512;   // reduced rows (2C) per launch: N <= 65536
-
-// Parallel cyclic reduction on rows normalised to b = 1 (row r: a_r x_{r-1}
-// + x_r + c_r x_{r+1} = d_r), 256 threads, two rows per thread kept in
-// registers, ping-pong LDS buffers for the partners, so each level costs one
-// barrier and one reciprocal per row.  Rows outside [0,n) are identity rows.
-// Returns the buffer holding x in D.
-__device__ inline int pcr_norm(double (*A)[kMaxRed], double (*Cc)[kMaxRed], double (*Dd)[kMaxRed], int n) {
-    const int tid = threadIdx.x;
-    double ar[2], cr[2], dr[2];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int r = tid + 256 * j;
-        ar[j] = r < n ? A[0][r] : 0.0;
-        cr[j] = r < n ? Cc[0][r] : 0.0;
-        dr[j] = r < n ? Dd[0][r] : 0.0;
-    }
-    int p = 0;
-    for (int delta = 1; delta < n; delta <<= 1) {
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int r = tid + 256 * j;
-            if (r < n) {
-                double am = 0.0, cm = 0.0, dm = 0.0, ap = 0.0, cp = 0.0, dp = 0.0;
-                if (r - delta >= 0) { am = A[p][r - delta]; cm = Cc[p][r - delta]; dm = Dd[p][r - delta]; }
-                if (r + delta < n) { ap = A[p][r + delta]; cp = Cc[p][r + delta]; dp = Dd[p][r + delta]; }
-                double inv = rcp_nr(1.0 - ar[j] * cm - cr[j] * ap);
-                dr[j] = (dr[j] - ar[j] * dm - cr[j] * dp) * inv;
-                ar[j] = -ar[j] * am * inv;
-                cr[j] = -cr[j] * cp * inv;
-                A[1 - p][r] = ar[j];
-                Cc[1 - p][r] = cr[j];
-                Dd[1 - p][r] = dr[j];
-            }
-        }
-        __syncthreads();
-        p = 1 - p;
-    }
-    return p;
-}
-
-// The same reduction by one wave on its own LDS slice (A/Cc/Dd: [2][128]),
-// for n <= 128 rows (rows r = lane, lane + 64).  Every wave of the block
-// solves the reduced system redundantly, so no workgroup barrier is needed:
-// LDS operations of one wave complete in order, and the wavefront fences
-// keep the compiler from moving them across a level.
-__device__ inline int pcr_wave(double* A, double* Cc, double* Dd, int n) {
-    const int lane = threadIdx.x & 63;
-    int p = 0;
-    for (int delta = 1; delta < n; delta <<= 1) {
-        double na[2], nc[2], nd[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int r = lane + 64 * j;
-            na[j] = 0.0; nc[j] = 0.0; nd[j] = 0.0;
-            if (r < n) {
-                const double* a = A + p * 128;
-                const double* cc = Cc + p * 128;
-                const double* d = Dd + p * 128;
-                double ar = a[r], cr = cc[r], dr = d[r];
-                double am = 0.0, cm = 0.0, dm = 0.0, ap = 0.0, cp = 0.0, dp = 0.0;
-                if (r - delta >= 0) { am = a[r - delta]; cm = cc[r - delta]; dm = d[r - delta]; }
-                if (r + delta < n) { ap = a[r + delta]; cp = cc[r + delta]; dp = d[r + delta]; }
-                double inv = rcp_nr(1.0 - ar * cm - cr * ap);
-                na[j] = -ar * am * inv;
-                nc[j] = -cr * cp * inv;
-                nd[j] = (dr - ar * dm - cr * dp) * inv;
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            int r = lane + 64 * j;
-            if (r < n) {
-                A[(1 - p) * 128 + r] = na[j];
-                Cc[(1 - p) * 128 + r] = nc[j];
-                Dd[(1 - p) * 128 + r] = nd[j];
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        p = 1 - p;
-    }
-    return p;
-}
-
-// Chunk elimination: the interior rows q in [0, ni) of a chunk, normalised
-// to b = 1 (a_q x_{q-1} + x_q + c_q x_{q+1} = d_q) and held by thread q + 1
-// in registers, for three right-hand sides (x: the row's own; y, z: unit
-// values at the chunk ends), by parallel cyclic reduction: each thread keeps
-// its own row in registers and reads its two partners of the level from the
-// LDS ping-pong buffers.  Returns the buffer holding the solution of every
-// row.
-__device__ inline int chunk_solve(double (*pA)[256], double (*pC)[256], double (*pX)[256], double (*pY)[256],
-                                  double (*pZ)[256], int ni, int q, bool inner, double aq, double cq, double xq,
-                                  double yq, double zq) {
-    if (inner) { pA[0][q] = aq; pC[0][q] = cq; pX[0][q] = xq; pY[0][q] = yq; pZ[0][q] = zq; }
-    __syncthreads();
-    int pp = 0;
-    for (int delta = 1; delta < ni; delta <<= 1) {
-        if (inner) {
-            double am = 0, cm = 0, xm = 0, ym = 0, zm = 0, ap = 0, cp = 0, xp = 0, yp = 0, zp = 0;
-            if (q - delta >= 0) {
-                am = pA[pp][q - delta]; cm = pC[pp][q - delta];
-                xm = pX[pp][q - delta]; ym = pY[pp][q - delta]; zm = pZ[pp][q - delta];
-            }
-            if (q + delta < ni) {
-                ap = pA[pp][q + delta]; cp = pC[pp][q + delta];
-                xp = pX[pp][q + delta]; yp = pY[pp][q + delta]; zp = pZ[pp][q + delta];
-            }
-            const double inv = rcp_nr(1.0 - aq * cm - cq * ap);
-            const double na = -aq * am * inv, nc = -cq * cp * inv;
-            xq = (xq - aq * xm - cq * xp) * inv;
-            yq = (yq - aq * ym - cq * yp) * inv;
-            zq = (zq - aq * zm - cq * zp) * inv;
-            aq = na;
-            cq = nc;
-            pA[1 - pp][q] = aq; pC[1 - pp][q] = cq; pX[1 - pp][q] = xq; pY[1 - pp][q] = yq; pZ[1 - pp][q] = zq;
-        }
-        __syncthreads();
-        pp = 1 - pp;
-    }
-    return pp;
-}
 
 // Far partial sums plus the near levels t in [near_lo, n-2] already in
 // memory, gathered in 32-wide batches of independent loads (a sum over m
@@ -199,312 +74,6 @@ __device__ inline double hist_tail(double om0, double c0, double c1, int n, int 
     return fma(w0, dnew, cr);
 }
 
-// max over the 256 threads of a block (wave maxima + LDS across the 4 waves)
-__device__ inline double block_max(double v, double* sh) {
-    v = wave_max(v);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
-    __syncthreads();
-    return v;
-}
-
-__global__ __launch_bounds__(256) void k_step1d(Step1DArgs g) {
-    __shared__ double rA[2][kMaxRed], rC[2][kMaxRed], rD[2][kMaxRed];
-    __shared__ double pA[2][256], pC[2][256], pX[2][256], pY[2][256], pZ[2][256];
-    __shared__ double sK[258];
-    __shared__ double sred[4];
-    const int tid = threadIdx.x;
-    const int c = blockIdx.x;
-    const int N = g.N, C = g.C;
-    const int s = (int)(((int64_t)c * N) / C);
-    const int e = (int)(((int64_t)(c + 1) * N) / C) - 1;
-    const int nc = e - s + 1;
-    const int i = s + tid;
-    const bool act = tid < nc;
-    const int R2 = 2 * C;
-    const int n = g.n;
-    const bool first = g.k <= 0;          // first Picard iteration of step n (or finalize)
-
-    // reduced systems of up to 128 rows are solved by every wave on its own
-    // LDS slice (no workgroup barrier), larger ones by the whole block
-    const bool wave_red = R2 <= 128;
-    const int wave = tid >> 6, lane = tid & 63;
-
-    // ---- 0. loads that do not depend on the pending solve (one round trip) ---
-    double rrow[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        int r = wave_red ? lane + 64 * j : tid + 256 * j;
-        bool ok = g.recover && r < R2;
-        const double* red = g.red + (size_t)(1 - g.parity) * R2 * 4 + 4 * r;
-#pragma unroll
-        for (int q = 0; q < 4; q++) rrow[j][q] = ok ? red[q] : 0.0;
-    }
-    const bool inner_node = act && i != s && i != e;
-    double fx = 0.0, fy = 0.0, fz = 0.0;
-    if (g.recover && inner_node) { fx = g.xyz[i]; fy = g.xyz[g.ld + i]; fz = g.xyz[2 * g.ld + i]; }
-    double uold = act ? g.U[i] : 0.0;                    // U^{n-1} (recovering, k=0) or U^n
-    double Sk = (!first && act) ? g.Sbuf[i] : 0.0;
-    const bool series = g.ser_P > 0;
-    const int64_t drow = series ? ((n - 1) & 1) : (n - 1);    // row of D[n-1]
-    double dmem = (first && !g.recover && act && n >= 1) ? g.D[drow * g.ld + i] : 0.0;
-    double d0m = (first && !series && act && n >= 2) ? g.D[i] : 0.0;
-    double d1m = (first && !series && act && n >= 3) ? g.D[g.ld + i] : 0.0;
-    // Picard convergence of the previous launch (decided one launch late: the
-    // test needs the max over every chunk): dmax of the previous launch and the
-    // iterate it stored
-    const bool check_conv = g.recover && g.prev_k >= 1;
-    double dprev = (check_conv && tid < C) ? g.dmax[(size_t)(1 - g.parity) * C + tid] : 0.0;
-    // previous iterate: the initial one for iteration 1, else the stored one
-    double uitp = 0.0;
-    if ((check_conv || g.k >= 1) && act) uitp = (g.k == 1) ? g.Uit0[i] : g.Uit[i];
-    // halo node s-1 (owned by chunk c-1, whose workgroup rewrites U and D in
-    // this launch): the converged iterate and U^{n-1} come from buffers that
-    // no workgroup writes in this launch
-    const int halo_tid = (nc < 256) ? 255 : 0;
-    const bool halo = tid == halo_tid && c > 0;
-    const bool extrap0 = first && g.k == 0 && g.extrap && n >= 1;
-    double uit_halo = (halo && check_conv) ? g.Uit[s - 1] : 0.0;
-    double uprev_halo = (halo && extrap0) ? g.uend[(size_t)((n - 1) & 1) * R2 + 2 * c - 1] : 0.0;
-    double hm = (first && !series && g.k == 0 && act && n >= 1) ? hist_mem(g, i, n, g.part_off, g.omega) : 0.0;
-
-    // ---- 1. finish the previous solve: reduced system, then back-substitute --
-    double val = 0.0;
-    const double* xs = nullptr;          // solution of the reduced system
-    if (g.recover) {
-        if (wave_red) {
-            double* A = &rA[0][0] + wave * 256;
-            double* Cc = &rC[0][0] + wave * 256;
-            double* Dd = &rD[0][0] + wave * 256;
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                int r = lane + 64 * j;
-                if (r < R2) {
-                    double ib = rcp_nr(rrow[j][1]);
-                    A[r] = rrow[j][0] * ib;
-                    Cc[r] = rrow[j][2] * ib;
-                    Dd[r] = rrow[j][3] * ib;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            int pr = pcr_wave(A, Cc, Dd, R2);
-            xs = Dd + pr * 128;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                int r = tid + 256 * j;
-                if (r < R2) {
-                    double ib = rcp_nr(rrow[j][1]);
-                    rA[0][r] = rrow[j][0] * ib;
-                    rC[0][r] = rrow[j][2] * ib;
-                    rD[0][r] = rrow[j][3] * ib;
-                }
-            }
-            __syncthreads();
-            int pr = pcr_norm(rA, rC, rD, R2);
-            xs = &rD[pr][0];
-        }
-        if (act) {
-            if (i == s) val = xs[2 * c];
-            else if (i == e) val = xs[2 * c + 1];
-            else val = fx + fy * xs[2 * c] + fz * xs[2 * c + 1];
-        }
-    }
-    // the previous Picard iterate met the tolerance: it is the step's result
-    bool conv = false;
-    if (check_conv) conv = block_max(dprev, sred) <= g.tol;
-    if (conv) val = uitp;
-
-    // ---- 2. advance the state -----------------------------------------------
-    double un = 0.0, uit = 0.0, S = 0.0;
-    if (first) {
-        if (act) {
-            un = uold;
-            double dnew = dmem;
-            if (g.recover) {                     // val = U^n, uold = U^{n-1}
-                dnew = val - uold;
-                g.D[drow * g.ld + i] = dnew;
-                g.U[i] = val;
-                un = val;
-            }
-            if (g.k >= 0 && n >= 1 && series) {
-                // moments += newest interval, then the series (sum_alg 2)
-                S = series_update(g.H, g.ld, i, g.ser_P, dnew, g.ser_c, g.ser_v);
-            } else if (g.k >= 0 && n >= 1) {
-                // S_n = far + near (in memory) + newest level + two-level corrections
-                S = hm + hist_tail(g.omega[0], g.corr[2 * n], g.corr[2 * n + 1], n, g.near_lo, dnew, d0m, d1m);
-            }
-            if (g.k >= 0) g.Sbuf[i] = S;
-            // Picard starts from the extrapolation 2 U^n - U^{n-1}; the
-            // iterate is kept for the convergence test of the next launch and
-            // the chunk ends of U^n for the next step's halo
-            uit = un;
-            if (g.extrap && g.k == 0) {
-                if (n >= 1) uit = un + dnew;
-                g.Uit0[i] = uit;
-                double* ue = g.uend + (size_t)(n & 1) * R2;
-                if (i == s) ue[2 * c] = un;
-                if (i == e) ue[2 * c + 1] = un;
-            }
-        }
-    } else if (act) {
-        un = uold;
-        S = Sk;
-        uit = val;
-    }
-    if (g.k < 0) {                               // finalize only (uniform)
-        // space-fractional scheme: F of U^n for this chunk's rows (Om1
-        // equation 0, fpde_hpc_1d.cpp:4176-4179), the arithmetic of
-        // k_space_flux.  The neighbours s-1 and e+1 are chunk ends of the
-        // reduced solution (or of the converged iterate), so the next step
-        // needs no flux launch.
-        if (g.sp_on && g.recover) {
-            double* sU = &pA[0][0];              // U^n of nodes s-1 .. e+1
-            double* sKf = &pC[0][0];             // K at U^n of nodes s-1 .. e
-            if (act) {
-                double k, icv;
-                vgm_coefs(un, i * g.h, g.ksat, g.coef_mode, k, icv);
-                sU[tid + 1] = un;
-                sKf[tid + 1] = k;
-            }
-            if (tid == halo_tid) {
-                if (c > 0) {
-                    const double ul = conv ? uit_halo : xs[2 * c - 1];
-                    double k, icv;
-                    vgm_coefs(ul, (s - 1) * g.h, g.ksat, g.coef_mode, k, icv);
-                    sU[0] = ul;
-                    sKf[0] = k;
-                }
-                if (c < C - 1) sU[nc + 1] = conv ? g.Uit[e + 1] : xs[2 * c + 2];
-            }
-            __syncthreads();
-            if (act) {
-                double f = 0.0;
-                if (i >= 1 && i <= N - 2) {
-                    const double um = sU[tid], u0 = sU[tid + 1], up = sU[tid + 2];
-                    const double Km = sKf[tid], Kj = sKf[tid + 1];
-                    const double hh = g.h * g.h;
-                    f = Kj * up / hh - (Kj / hh + Km / hh) * u0 + Km * um / hh;
-                }
-                g.sp_F[i] = f;
-            }
-        }
-        return;
-    }
-
-    if (!first) {
-        double* dm = g.dmax + (size_t)g.parity * C;
-        if (conv) {
-            // converged: hand the iterate on unchanged through an identity
-            // reduced system and x = U, y = z = 0 (dmax 0 keeps later launches
-            // of this step passing it on)
-            double* redw = g.red + (size_t)g.parity * R2 * 4;
-            if (act && i != s && i != e) { g.xyz[i] = uit; g.xyz[g.ld + i] = 0.0; g.xyz[2 * g.ld + i] = 0.0; }
-            if (tid == 0) {
-                redw[4 * (2 * c) + 0] = 0.0; redw[4 * (2 * c) + 1] = 1.0;
-                redw[4 * (2 * c) + 2] = 0.0; redw[4 * (2 * c) + 3] = uit;
-                dm[c] = 0.0;
-            }
-            if (tid == nc - 1) {
-                redw[4 * (2 * c + 1) + 0] = 0.0; redw[4 * (2 * c + 1) + 1] = 1.0;
-                redw[4 * (2 * c + 1) + 2] = 0.0; redw[4 * (2 * c + 1) + 3] = uit;
-            }
-            return;                              // uniform: conv is block-wide
-        }
-        // |U^{k} - U^{k-1}| over the chunk; U^0 of the step is the initial
-        // iterate stored by the k = 0 launch
-        double d = act ? fabs(uit - uitp) : 0.0;
-        d = block_max(d, sred);
-        if (tid == 0) dm[c] = d;
-        if (act) g.Uit[i] = uit;
-    }
-
-    // ---- 3. coefficients at the iterate ------------------------------------
-    double K = 0.0, invC = 0.0;
-    // K of the node left of the chunk, on a thread without a node of its own
-    // when there is one (else thread 0 does both evaluations), at the same
-    // iterate as the chunk's own nodes
-    if (halo) {
-        double ulo = g.recover ? (conv ? uit_halo : xs[2 * c - 1]) : g.U[s - 1];
-        if (extrap0) ulo += ulo - uprev_halo;
-        double Kl, iCl;
-        vgm_coefs(ulo, (s - 1) * g.h, g.ksat, g.coef_mode, Kl, iCl);
-        sK[0] = Kl;
-    }
-    if (act) {
-        vgm_coefs(uit, i * g.h, g.ksat, g.coef_mode, K, invC);
-        sK[tid + 1] = K;
-    }
-    __syncthreads();
-
-    // ---- 4. rows -------------------------------------------------------------
-    // (space-fractional scheme: the diffusion part of A_/B/R scaled by
-    // Dg kb(gamma,i-1,i,i) and Om1's explicit sum -inv_dw_dh E_i, :4182-4189;
-    // E of step n is formed by its first launch and reused by the others)
-    double ar = 0.0, br = 1.0, cr = 0.0, dr = 0.0;
-    if (act) {
-        if (i == 0) { ar = 0.0; br = 1.0; cr = 0.0; dr = g.utop; }
-        else if (i == N - 1) { ar = -1.0; br = 1.0; cr = 0.0; dr = 0.0; }
-        else {
-            const double kap = g.sp_on ? g.sp_kap : 1.0;
-            double Km = sK[tid], Kp = sK[tid + 1];
-            double A = Km * invC * g.h2inv * kap;
-            double B = Kp * invC * g.h2inv * kap;
-            double R = invC * (Kp * g.h2inv + Km * g.h2inv) * kap + g.L;
-            ar = A; br = -R; cr = B; dr = -g.L * un + S;
-            if (g.sp_on) {
-                double E;
-                if (first) {
-                    E = space_sum(g.sp_P, g.sp_ldp, g.sp_corr, g.sp_F, i);
-                    g.sp_E[i] = E;
-                } else {
-                    E = g.sp_E[i];
-                }
-                dr -= invC * E;
-            }
-        }
-    }
-
-    // ---- 5. chunk elimination: interior rows 1..nc-2, three right-hand sides
-    // (x: the row's own RHS; y, z: unit values at the chunk ends s and e) ---
-    const int ni = nc - 2;
-    const int q = tid - 1;
-    const bool inner = (tid >= 1) && (tid <= nc - 2);
-    double ib = inner ? rcp_nr(br) : 0.0;
-    const int pp = chunk_solve(pA, pC, pX, pY, pZ, ni, q, inner, (tid == 1) ? 0.0 : ar * ib,
-                               (tid == nc - 2) ? 0.0 : cr * ib, dr * ib, (tid == 1) ? -ar * ib : 0.0,
-                               (tid == nc - 2) ? -cr * ib : 0.0);
-    if (inner) {
-        g.xyz[i] = pX[pp][q];
-        g.xyz[g.ld + i] = pY[pp][q];
-        g.xyz[2 * g.ld + i] = pZ[pp][q];
-    }
-
-    // ---- 6. reduced rows of the chunk ends ----------------------------------
-    double* redw = g.red + (size_t)g.parity * R2 * 4;
-    if (tid == 0) {
-        double x, y, z;
-        if (nc == 2) { x = 0.0; y = 0.0; z = 1.0; }
-        else { x = pX[pp][0]; y = pY[pp][0]; z = pZ[pp][0]; }
-        redw[4 * (2 * c) + 0] = ar;
-        redw[4 * (2 * c) + 1] = br + cr * y;
-        redw[4 * (2 * c) + 2] = cr * z;
-        redw[4 * (2 * c) + 3] = dr - cr * x;
-    }
-    if (tid == nc - 1) {
-        double x, y, z;
-        if (nc == 2) { x = 0.0; y = 1.0; z = 0.0; }
-        else { x = pX[pp][ni - 1]; y = pY[pp][ni - 1]; z = pZ[pp][ni - 1]; }
-        redw[4 * (2 * c + 1) + 0] = ar * y;
-        redw[4 * (2 * c + 1) + 1] = br + ar * z;
-        redw[4 * (2 * c + 1) + 2] = cr;
-        redw[4 * (2 * c + 1) + 3] = dr - ar * x;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Cooperative form: one launch runs the steps [n, n_end) of a history block
 // with every Picard iteration inside, all C chunk workgroups co-resident.
@@ -537,9 +106,9 @@ __global__ __launch_bounds__(256) void k_step1d(Step1DArgs g) {
 // Measured (cycles of one iteration at N = 10^4, 53 chunks, phase timers): row
 // waves 2000 from barrier to barrier (coefficients 640); solver wave: rows and
 // line solve 2500, publishing 900, waiting for the other chunks 4700,
-// separators and decision 1800, U to LDS 500.  Headline solve (N = 10^4, M =
-// 2 10^4) 374 -> 214 ms, N = 1000 35.6 -> 21.7 ms, six solves in a batch 58.9
-// -> 39.5 ms against the whole workgroup's cyclic reduction over LDS with both
+// decision 150, separators 1100, U to LDS 500.  Headline solve (N = 10^4, M =
+// 2 10^4) 374 -> 206 ms, N = 1000 35.7 -> 21.5 ms, six solves in a batch 59.0
+// -> 38.9 ms against the whole workgroup's cyclic reduction over LDS with both
 // chunk ends as separators (five words per row and level, a workgroup barrier
 // per level) and coefficients by square roots and divisions (1700 cycles).
 //
@@ -760,30 +329,320 @@ __device__ inline double xch_value(const Step1DLds& L, int j, int k) {
     return __longlong_as_double((long long)((w.y << 32) | (w.x & 0xffffffffull)));
 }
 
-// The separators' system: RR rows per lane.  Returns the values at the
-// separators c-1, c and c+1 (0 past the ends).
+// The separators' system: RR rows per lane, row r of it from chunk r's values
+// 0..3 in v[..][0..3] and the left chunk's 4..6 in v[..][4..6] (any finite
+// values for a row without one).  Returns the values at the separators c-1, c
+// and c+1 (0 past the ends).
 template <int RR>
-__device__ inline void solve_separators(const Step1DLds& L, int C, int c, int p, double& xm, double& x0, double& xp) {
+__device__ inline void solve_separators(const double (&v)[RR][7], int C, int c, int p, double& xm, double& x0,
+                                        double& xp) {
 #pragma clang fp contract(off)
     double a[RR], cc[RR], d[RR], x[RR], y[RR], z[RR];
 #pragma unroll
     for (int j = 0; j < RR; j++) {
         const int r = RR * p + j;
         const bool ok = r < C;
-        const int rr = ok ? r : 0, rl = rr > 0 ? rr - 1 : 0;
-        const double v0 = xch_value(L, rr, 0), v1 = xch_value(L, rr, 1), v2 = xch_value(L, rr, 2),
-                     v3 = xch_value(L, rr, 3);
         // (row 0 has v0 = 0: the values read for a left neighbour, its own chunk's, do not enter)
-        const double xl = xch_value(L, rl, 4), yl = xch_value(L, rl, 5), zl = xch_value(L, rl, 6);
-        const double inv = rcp_nr(fma(v0, zl, v1));
-        a[j] = ok ? (v0 * yl) * inv : 0.0;
-        cc[j] = ok && r + 1 < C ? v2 * inv : 0.0;
-        d[j] = ok ? fma(-v0, xl, v3) * inv : 0.0;
+        const double inv = rcp_nr(fma(v[j][0], v[j][6], v[j][1]));
+        a[j] = ok ? (v[j][0] * v[j][5]) * inv : 0.0;
+        cc[j] = ok && r + 1 < C ? v[j][2] * inv : 0.0;
+        d[j] = ok ? fma(-v[j][0], v[j][4], v[j][3]) * inv : 0.0;
     }
     wave_line<RR, true>(a, cc, d, p, x, y, z);
     xm = c > 0 ? line_value<RR>(x, c - 1) : 0.0;
     x0 = line_value<RR>(x, c);
     xp = c + 1 < C ? line_value<RR>(x, c + 1) : 0.0;
+}
+
+template <int RR>
+__device__ inline void separator_rows(const Step1DLds& L, int C, int p, double (&v)[RR][7]) {
+#pragma unroll
+    for (int j = 0; j < RR; j++) {
+        const int r = RR * p + j, rr = r < C ? r : 0, rl = rr > 0 ? rr - 1 : 0;
+#pragma unroll
+        for (int k = 0; k < 7; k++) v[j][k] = xch_value(L, k < 4 ? rr : rl, k);
+    }
+}
+
+// One wave's elimination of a chunk: interior rows s+1 .. e (ni of them, R per
+// lane) from the chunk's K, 1/C and right-hand sides in LDS; U_i = x + y U_s +
+// z U_s' with the separators s and s'.  Values 0..6 of the chunk to pub.  Kh:
+// K at node s-1.
+template <int R>
+__device__ __forceinline__ void chunk_line(const double* K, const double* iC, const double* dr, int N, int s, int ni,
+                                           int c, int p, double Kh, double Ln, double h2inv, double (&x)[R],
+                                           double (&y)[R], double (&z)[R], double* pub) {
+#pragma clang fp contract(off)
+    const int r0 = R * p;
+    double a[R], cc[R], d[R];
+    double Kv[R + 1], iv[R], dv[R];
+#pragma unroll
+    for (int j = 0; j <= R; j++) Kv[j] = K[row_slot(r0 + j)];
+#pragma unroll
+    for (int j = 0; j < R; j++) { iv[j] = iC[row_slot(r0 + 1 + j)]; dv[j] = dr[row_slot(r0 + 1 + j)]; }
+    const double K0 = K[0], i0 = iC[0], d0 = dr[0];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const double Km = Kv[j], Kp = Kv[j + 1];
+        const double inv = rcp_nr(-fma(iv[j], Kp * h2inv + Km * h2inv, Ln));
+        a[j] = Km * iv[j] * h2inv * inv;
+        cc[j] = Kp * iv[j] * h2inv * inv;
+        d[j] = dv[j] * inv;
+        // bottom row U_{N-1} = U_{N-2}; rows past the chunk hand on the next
+        // separator's value: x_q = x_{q+1}
+        const bool in = r0 + j < ni, bottom = r0 + j == N - 2 - s;
+        a[j] = in ? (bottom ? -1.0 : a[j]) : 0.0;
+        cc[j] = in ? (bottom ? 0.0 : cc[j]) : -1.0;
+        d[j] = in && !bottom ? d[j] : 0.0;
+    }
+    // the separator's row (node 0: U = u_top)
+    const double as = c > 0 ? Kh * i0 * h2inv : 0.0;
+    const double cs = c > 0 ? K0 * i0 * h2inv : 0.0;
+    const double bs = c > 0 ? -fma(i0, K0 * h2inv + Kh * h2inv, Ln) : 1.0;
+    wave_line<R, false>(a, cc, d, p, x, y, z);
+    if (p == 0) {
+        pub[0] = as;
+        pub[1] = fma(cs, y[0], bs);
+        pub[2] = cs * z[0];
+        pub[3] = fma(-cs, x[0], d0);
+    }
+    // the last node's row: which of the lane's R is launch-uniform
+    double xl = x[0], yl = y[0], zl = z[0];
+#pragma unroll
+    for (int j = 1; j < R; j++) {
+        const bool is = (ni - 1) % R == j;
+        xl = is ? x[j] : xl;
+        yl = is ? y[j] : yl;
+        zl = is ? z[j] : zl;
+    }
+    if (p == (ni - 1) / R) {
+        pub[4] = xl;
+        pub[5] = yl;
+        pub[6] = zl;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Per-iteration form (plain history, space-fractional scheme, step_mode 1,
+// captured steps): one launch is [finish the previous solve] + [history term,
+// coefficients, rows, chunk elimination of this solve].  The chunks' values of
+// the separators' system (red: per launch parity, 8 doubles per chunk: 0..6 as
+// in the exchange above, 7 the chunk's max |U^k - U^{k-1}|) are written by one
+// launch and solved by every wave of the next, redundantly and without a
+// barrier; the nodes' x, y, z stay in xyz for its back-substitution.  The
+// launch order stands in for the grid barrier.
+// What bounds it: the dependent chain again (one memory trip, the separators,
+// the coefficients, one barrier, the line in wave 0), so it has the cooperative
+// form's wave-level solves: at N = 3001 a launch takes 7.8 us against 11.8 us
+// with the whole workgroup's cyclic reduction over LDS and both chunk ends as
+// separators.
+template <int RW, int RR>
+__global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
+#pragma clang fp contract(off)
+    __shared__ double sK[kRowSlots], sC[kRowSlots], sR[kRowSlots], pub[8], wmax[RW];
+    __shared__ double sKh;
+    constexpr int T = 64 * RW;
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int p = 4 * (lane & 15) + (lane >> 4);
+    const int c = blockIdx.x;
+    const int N = g.N, C = g.C;
+    const int s = (int)(((int64_t)c * N) / C);
+    const int nc = (int)(((int64_t)(c + 1) * N) / C) - s;
+    const int i = s + tid;
+    const bool act = tid < nc;
+    const int n = g.n;
+    const bool first = g.k <= 0;          // first Picard iteration of step n (or finalize)
+
+    // ---- 0. loads that do not depend on the pending solve (one round trip) ---
+    const double* const red = g.red + (size_t)(1 - g.parity) * C * 8;
+    double v[RR][7], dprev = 0.0, xh = 0.0, yh = 0.0, zh = 0.0;   // h: node s-1 of the chunk to the left
+    // Picard convergence of the previous launch (decided one launch late: the
+    // test needs the max over every chunk): the measures it left and the
+    // iterate it stored
+    const bool check_conv = g.recover && g.prev_k >= 1;
+    if (g.recover) {
+#pragma unroll
+        for (int j = 0; j < RR; j++) {
+            const int r = RR * p + j, rr = r < C ? r : 0, rl = rr > 0 ? rr - 1 : 0;
+#pragma unroll
+            for (int k = 0; k < 7; k++) v[j][k] = red[8 * (k < 4 ? rr : rl) + k];
+            if (check_conv) dprev = fmax(dprev, red[8 * rr + 7]);
+        }
+        if (c > 0) { xh = red[8 * c - 4]; yh = red[8 * c - 3]; zh = red[8 * c - 2]; }
+    }
+    double fx = 0.0, fy = 0.0, fz = 0.0;
+    if (g.recover && act && tid > 0) { fx = g.xyz[i]; fy = g.xyz[g.ld + i]; fz = g.xyz[2 * g.ld + i]; }
+    double uold = act ? g.U[i] : 0.0;                    // U^{n-1} (recovering, k=0) or U^n
+    double Sk = (!first && act) ? g.Sbuf[i] : 0.0;
+    const bool series = g.ser_P > 0;
+    const int64_t drow = series ? ((n - 1) & 1) : (n - 1);    // row of D[n-1]
+    double dmem = (first && !g.recover && act && n >= 1) ? g.D[drow * g.ld + i] : 0.0;
+    double d0m = (first && !series && act && n >= 2) ? g.D[i] : 0.0;
+    double d1m = (first && !series && act && n >= 3) ? g.D[g.ld + i] : 0.0;
+    // previous iterate: the initial one for iteration 1, else the stored one
+    double uitp = 0.0;
+    if ((check_conv || g.k >= 1) && act) uitp = (g.k == 1) ? g.Uit0[i] : g.Uit[i];
+    // halo node s-1 (owned by chunk c-1, whose workgroup rewrites U and D in
+    // this launch): the converged iterate and U^{n-1} come from buffers that
+    // no workgroup writes in this launch; on a thread without a node of its
+    // own when there is one (else thread 0 does both evaluations)
+    const int halo_tid = (nc < T) ? T - 1 : 0;
+    const bool halo = tid == halo_tid && c > 0;
+    const bool extrap0 = first && g.k == 0 && g.extrap && n >= 1;
+    double uit_halo = (halo && check_conv) ? g.Uit[s - 1] : 0.0;
+    double u_halo = (halo && !g.recover) ? g.U[s - 1] : 0.0;
+    double uprev_halo = (halo && extrap0) ? g.uend[(size_t)((n - 1) & 1) * 2 * C + 2 * c - 1] : 0.0;
+    double hm = (first && !series && g.k == 0 && act && n >= 1) ? hist_mem(g, i, n, g.part_off, g.omega) : 0.0;
+
+    // space-fractional scheme: Om1's explicit sum -inv_dw_dh E_i (:4182-4189);
+    // E of step n is formed by its first launch and reused by the others
+    double E = 0.0;
+    if (g.sp_on && g.k >= 0 && i > 0 && i < N - 1 && act) {
+        E = first ? space_sum(g.sp_P, g.sp_ldp, g.sp_corr, g.sp_F, i) : g.sp_E[i];
+        if (first) g.sp_E[i] = E;
+    }
+
+    // ---- 1. finish the previous solve: separators, then back-substitute ------
+    double val = 0.0, um = 0.0, us = 0.0, up = 0.0;
+    bool conv = false;
+    if (g.recover) {
+        solve_separators<RR>(v, C, c, p, um, us, up);
+        val = tid == 0 ? us : fma(fz, up, fma(fy, us, fx));
+        // node s-1 as its own chunk forms it (a chunk of one node: its separator)
+        u_halo = fma(zh, us, fma(yh, um, xh));
+        // the previous Picard iterate met the tolerance: it is the step's result
+        if (check_conv) conv = wave_max(dprev) <= g.tol;
+        if (conv) { val = uitp; u_halo = uit_halo; }
+    }
+
+    // ---- 2. advance the state -----------------------------------------------
+    double un = 0.0, uit = 0.0, S = 0.0;
+    if (first) {
+        if (act) {
+            un = uold;
+            double dnew = dmem;
+            if (g.recover) {                     // val = U^n, uold = U^{n-1}
+                dnew = val - uold;
+                g.D[drow * g.ld + i] = dnew;
+                g.U[i] = val;
+                un = val;
+            }
+            if (g.k >= 0 && n >= 1 && series) {
+                // moments += newest interval, then the series (sum_alg 2)
+                S = series_update(g.H, g.ld, i, g.ser_P, dnew, g.ser_c, g.ser_v);
+            } else if (g.k >= 0 && n >= 1) {
+                // S_n = far + near (in memory) + newest level + two-level corrections
+                S = hm + hist_tail(g.omega[0], g.corr[2 * n], g.corr[2 * n + 1], n, g.near_lo, dnew, d0m, d1m);
+            }
+            if (g.k >= 0) g.Sbuf[i] = S;
+            // Picard starts from the extrapolation 2 U^n - U^{n-1}; the
+            // iterate is kept for the convergence test of the next launch and
+            // the chunk ends of U^n for the next step's halo
+            uit = un;
+            if (g.extrap && g.k == 0) {
+                if (n >= 1) uit = un + dnew;
+                g.Uit0[i] = uit;
+                double* ue = g.uend + (size_t)(n & 1) * 2 * C;
+                if (tid == nc - 1) ue[2 * c + 1] = un;
+            }
+        }
+    } else if (act) {
+        un = uold;
+        S = Sk;
+        uit = val;
+    }
+    if (g.k < 0) {                               // finalize only (uniform)
+        // space-fractional scheme: F of U^n for this chunk's rows (Om1
+        // equation 0, fpde_hpc_1d.cpp:4176-4179), the arithmetic of
+        // k_space_flux.  The neighbours s-1 and e+1 come from the separators
+        // (or the converged iterate), so the next step needs no flux launch.
+        if (g.sp_on && g.recover) {
+            double* sU = sR;                     // U^n of nodes s-1 .. e+1
+            double* sKf = sK;                    // K at U^n of nodes s-1 .. e
+            double k, icv;
+            if (act) {
+                vgm_coefs(un, i * g.h, g.ksat, g.coef_mode, k, icv);
+                sU[tid + 1] = un;
+                sKf[tid + 1] = k;
+            }
+            if (tid == halo_tid) {
+                if (c > 0) {
+                    vgm_coefs(u_halo, (s - 1) * g.h, g.ksat, g.coef_mode, k, icv);
+                    sU[0] = u_halo;
+                    sKf[0] = k;
+                }
+                if (c < C - 1) sU[nc + 1] = conv ? g.Uit[s + nc] : up;
+            }
+            __syncthreads();
+            if (act) {
+                double f = 0.0;
+                if (i >= 1 && i <= N - 2) {
+                    const double ul = sU[tid], u0 = sU[tid + 1], ur = sU[tid + 2];
+                    const double Km = sKf[tid], Kj = sKf[tid + 1];
+                    f = space_flux(Km, Kj, ul, u0, ur, g.h);
+                }
+                g.sp_F[i] = f;
+            }
+        }
+        return;
+    }
+
+    double* const mine = g.red + ((size_t)g.parity * C + c) * 8;
+    if (!first && conv) {
+        // converged: hand the iterate on unchanged, x = U, y = z = 0 and the
+        // separator's row "U_s = U" (measure 0 keeps later launches of this
+        // step passing it on)
+        if (act && tid > 0) { g.xyz[i] = uit; g.xyz[g.ld + i] = 0.0; g.xyz[2 * g.ld + i] = 0.0; }
+        if (tid == 0) { mine[0] = 0.0; mine[1] = 1.0; mine[2] = 0.0; mine[3] = uit; mine[7] = 0.0; }
+        if (tid == nc - 1) { mine[4] = uit; mine[5] = 0.0; mine[6] = 0.0; }
+        return;                                  // uniform: every wave forms conv alike
+    }
+    if (!first) {
+        // |U^{k} - U^{k-1}| over the chunk; U^0 of the step is the initial
+        // iterate stored by the k = 0 launch
+        const double d = wave_max(act ? fabs(uit - uitp) : 0.0);
+        if (lane == 0) wmax[wave] = d;
+        if (act) g.Uit[i] = uit;
+    }
+
+    // ---- 3. coefficients at the iterate, right-hand sides -------------------
+    // (space-fractional scheme: the diffusion part of A_/B/R scaled by
+    // Dg kb(gamma,i-1,i,i))
+    const double kap = g.sp_on ? g.sp_kap : 1.0;
+    if (extrap0) u_halo += u_halo - uprev_halo;
+    const bool spare = halo && !act;             // (in the same evaluation as the wave's own nodes)
+    double K, invC;
+    vgm_coefs(spare ? u_halo : uit, (spare ? s - 1 : i) * g.h, g.ksat, g.coef_mode, K, invC);
+    if (spare) sKh = K * kap;
+    if (act) {
+        const int slot = row_slot(tid);
+        sK[slot] = K * kap;
+        sC[slot] = invC;
+        sR[slot] = i == 0 ? g.utop : fma(-invC, E, fma(-g.L, un, S));
+    }
+    if (halo && act) {
+        vgm_coefs(u_halo, (s - 1) * g.h, g.ksat, g.coef_mode, K, invC);
+        sKh = K * kap;
+    }
+    __syncthreads();
+    if (wave > 0) return;
+
+    // ---- 4. the chunk's elimination, in wave 0 ------------------------------
+    double x[RW], y[RW], z[RW];
+    chunk_line<RW>(sK, sC, sR, N, s, nc - 1, c, p, c > 0 ? sKh : 0.0, g.L, g.h2inv, x, y, z, pub);
+    double* const to = g.xyz + s + 1 + RW * p;
+#pragma unroll
+    for (int j = 0; j < RW; j++)
+        if (RW * p + j < nc - 1) { to[j] = x[j]; to[g.ld + j] = y[j]; to[2 * g.ld + j] = z[j]; }
+    if (p == 0) {
+        double d = 0.0;
+        if (!first)
+#pragma unroll
+            for (int w = 0; w < RW; w++) d = fmax(d, wmax[w]);
+        pub[7] = d;
+    }
+    wave_lds_sync();
+    if (lane < 8) mine[lane] = pub[lane];
 }
 
 // Where a launch stands: step n, Picard iteration k of it, and what the next
@@ -1225,61 +1084,12 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
     auto line_solve = [&](int b, int check, double Kh, double Ln, double change, double (&itn)[NV]) -> int {
         double x[R], y[R], z[R];
         const bool decide = check == kDecide;
-        double meas;
         int p = pos;
         asm volatile("" : "+v"(p));                            // (addresses and masks formed here, not kept across iterations)
         const int r0 = R * p;
-        if (!decide) {
-            double a[R], cc[R], d[R];
-            double Kv[R + 1], iv[R], dv[R];
-#pragma unroll
-            for (int j = 0; j <= R; j++) Kv[j] = L.K[row_slot(r0 + j)];
-#pragma unroll
-            for (int j = 0; j < R; j++) { iv[j] = L.iC[row_slot(r0 + 1 + j)]; dv[j] = L.d[row_slot(r0 + 1 + j)]; }
-            const double K0 = L.K[0], i0 = L.iC[0], d0 = L.d[0];
-            meas = wave_max(change);
-#pragma unroll
-            for (int j = 0; j < R; j++) {
-                const double Km = Kv[j], Kp = Kv[j + 1];
-                const double inv = rcp_nr(-fma(iv[j], Kp * h2inv + Km * h2inv, Ln));
-                a[j] = Km * iv[j] * h2inv * inv;
-                cc[j] = Kp * iv[j] * h2inv * inv;
-                d[j] = dv[j] * inv;
-                // bottom row U_{N-1} = U_{N-2}; rows past the chunk hand on
-                // the next separator's value: x_q = x_{q+1}
-                const bool in = r0 + j < ni, bottom = r0 + j == N - 2 - s;
-                a[j] = in ? (bottom ? -1.0 : a[j]) : 0.0;
-                cc[j] = in ? (bottom ? 0.0 : cc[j]) : -1.0;
-                d[j] = in && !bottom ? d[j] : 0.0;
-            }
-            // the separator's row (node 0: U = u_top)
-            const double as = c > 0 ? Kh * i0 * h2inv : 0.0;
-            const double cs = c > 0 ? K0 * i0 * h2inv : 0.0;
-            const double bs = c > 0 ? -fma(i0, K0 * h2inv + Kh * h2inv, Ln) : 1.0;
-            wave_line<R, false>(a, cc, d, p, x, y, z);
-            if (lane == 0) {
-                L.pub[0] = as;
-                L.pub[1] = fma(cs, y[0], bs);
-                L.pub[2] = cs * z[0];
-                L.pub[3] = fma(-cs, x[0], d0);
-            }
-            // the last node's row: which of the lane's R is launch-uniform
-            double xl = x[0], yl = y[0], zl = z[0];
-#pragma unroll
-            for (int j = 1; j < R; j++) {
-                const bool is = (ni - 1) % R == j;
-                xl = is ? x[j] : xl;
-                yl = is ? y[j] : yl;
-                zl = is ? z[j] : zl;
-            }
-            if (p == (ni - 1) / R) {
-                L.pub[4] = xl;
-                L.pub[5] = yl;
-                L.pub[6] = zl;
-            }
-        } else {
-            meas = wave_max(change);
-        }
+        if (!decide)
+            chunk_line<R>(L.K, L.iC, L.d, N, s, ni, c, p, Kh, Ln, h2inv, x, y, z, L.pub);
+        const double meas = wave_max(change);
         if (lane == 0) L.pub[7] = meas;
         publish(b, decide ? kXchMeasure : 0);
         double largest = 0.0;
@@ -1289,8 +1099,15 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         double um, us, up;
         const double xl = c > 0 ? xch_value(L, c - 1, 4) : 0.0, yl = c > 0 ? xch_value(L, c - 1, 5) : 0.0,
                      zl = c > 0 ? xch_value(L, c - 1, 6) : 0.0;
-        if (C <= 64) solve_separators<1>(L, C, c, p, um, us, up);
-        else solve_separators<4>(L, C, c, p, um, us, up);
+        if (C <= 64) {
+            double v[1][7];
+            separator_rows<1>(L, C, p, v);
+            solve_separators<1>(v, C, c, p, um, us, up);
+        } else {
+            double v[4][7];
+            separator_rows<4>(L, C, p, v);
+            solve_separators<4>(v, C, c, p, um, us, up);
+        }
         if (check == kCheckMet && met) return kMet;
         if (check == kCheckPending && !met) return kRollback;
 #pragma unroll
@@ -1438,7 +1255,7 @@ fpde_status launch_step1d_batch(const Step1DArgs* base, const BatchTick& t, hipS
 }
 
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st) {
-    if (2 * a.C > kMaxRed || a.C > kMaxChunks || (a.N + a.C - 1) / a.C > kRows) {
+    if (a.C > kMaxChunks || (a.N + a.C - 1) / a.C > kRows) {
         set_error("1D line too long for the reduced system (N <= 65536)");
         return FPDE_ERR_ARG;
     }
@@ -1452,8 +1269,13 @@ fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st) {
 }
 
 fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st) {
-    if (2 * a.C > kMaxRed) { set_error("1D line too long for the reduced system (N <= 65536)"); return FPDE_ERR_ARG; }
-    hipLaunchKernelGGL(k_step1d, dim3(a.C), dim3(256), 0, st, a);
+    if (a.C > kMaxChunks || (a.N + a.C - 1) / a.C > kRows) {
+        set_error("1D line too long for the reduced system (N <= 65536)");
+        return FPDE_ERR_ARG;
+    }
+    const bool three = row_waves(a.N, a.C) == 3, few = a.C <= 64;
+    auto* const kern = three ? (few ? k_step1d<3, 1> : k_step1d<3, 4>) : (few ? k_step1d<4, 1> : k_step1d<4, 4>);
+    hipLaunchKernelGGL(kern, dim3(a.C), dim3(three ? 192 : 256), 0, st, a);
     return FPDE_OK;
 }
 

@@ -1538,6 +1538,26 @@ def test_wave_line_solve_edges_match_oracle(fpde, oracle, nodes, rows, fourier, 
     assert err <= TOL_F64
 
 
+@pytest.mark.parametrize("nodes,rows,gamma", [(5, 0, 1.0), (192, 0, 1.0), (193, 0, 0.8), (256, 256, 1.0),
+                                              (512, 256, 0.8), (2048, 32, 1.0), (2080, 32, 0.8), (12289, 0, 1.0)])
+@pytest.mark.parametrize("picard", [1, 4])
+def test_per_iteration_launch_edges_match_oracle(fpde, oracle, nodes, rows, gamma, picard):
+    """The per-iteration launch at its edges: the smallest line, full chunks of
+    three and four waves (no spare thread for the node left of the chunk) and
+    one node more, 64 and 65 chunks (one and four separators per lane); a step
+    that ends on the Picard tolerance, and the fused flux of the
+    space-fractional scheme across chunk ends."""
+    steps = 12
+    u0 = fpde.init_1d(nodes, 7100 + nodes)
+    spec = fpde.make_spec(nodes, steps, 1e-3, alpha=0.7, picard_max=picard, picard_tol=1e-9 if picard > 1 else 0.0,
+                          hist_mode="mfma_f64", block=16, u_top=u0[0], chunk_rows=rows, gamma=gamma, step_mode=1)
+    u = fpde.solve(spec, u0)
+    ref = _oracle_space(oracle, spec, u0) if gamma < 1.0 else _oracle_1d(oracle, spec, u0, picard_tol=spec.picard_tol)
+    err = rel_err(u, ref)
+    print(f"per-iteration N={nodes} rows={rows} gamma={gamma} picard={picard}: rel err {err:.3e}", flush=True)
+    assert err <= TOL_F64
+
+
 @pytest.mark.parametrize("block", [16, 64, 128])
 @pytest.mark.parametrize("picard", [1, 3])
 def test_launches_that_cut_a_block_give_the_same_bits(fpde, block, picard):
