@@ -5,6 +5,7 @@
 #include <cstddef>
 #include <string>
 #include <map>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/fpde_hip.h"
@@ -333,6 +334,11 @@ struct Step1DArgs {
     int extrap;               // Picard starts from 2 U^n - U^{n-1} (picard_max > 1)
     double* Uit0;             // that initial iterate (convergence test of iteration 1)
     double* uend;             // [2][2C] U^n at the chunk ends, by step parity
+    // per-iteration form: the plain history of the next step, streamed by
+    // ahead_tiles * ahead_splits more workgroups of the launch (0: none): its
+    // levels [ahead_lo, ahead_hi), none of them written by this launch
+    int ahead_lo, ahead_hi, ahead_chunk, ahead_tiles, ahead_splits;
+    double* ahead_part;
     // cooperative block form (k_step1d_block): steps [n, n_end) in one launch
     int n_end;
     int picard_max;
@@ -464,6 +470,57 @@ __device__ inline double space_sum(const double* __restrict__ P, int64_t ldp, co
     return fma(corr[2 * (i - 1) + 1], F[2], e);
 }
 
+// Plain FP64 stream of one workgroup of T threads: part[ks*ld + i] = sum_{t in
+// chunk ks, t < t_hi} omega[n-t-1] * D[t*ld + i] for the 2 T nodes of a tile.
+// Two nodes per thread (16-B loads), DEPTH levels in flight; the weights of
+// the chunk are staged in LDS windows of kPlainWin levels (wave-uniform reads,
+// one barrier pair per window).  Even and odd levels of a window's groups of
+// four are summed apart, whatever T and DEPTH.
+constexpr int kPlainWin = 1024;
+template <int T, int DEPTH>
+__device__ inline void plain_stream(const double* __restrict__ D, int64_t ld, int nodes, int n, int t_hi, int chunk,
+                                    const double* __restrict__ omega, double* __restrict__ part, int tile, int ks,
+                                    double* wwin /* [kPlainWin]: omega[n - t - 1] at t - w0 */) {
+    const int i2 = (tile * T + (int)threadIdx.x) * 2;
+    const bool ok = i2 < nodes;                       // threads past the nodes still stage weights
+    const int t0 = ks * chunk;
+    const int t1 = min(t_hi, t0 + chunk);
+    double a0 = 0.0, a1 = 0.0, b0 = 0.0, b1 = 0.0;
+    for (int w0 = t0; w0 < t1; w0 += kPlainWin) {
+        const int w1 = min(t1, w0 + kPlainWin);
+        __syncthreads();
+        for (int q = threadIdx.x; q < w1 - w0; q += T) wwin[q] = omega[n - (w0 + q) - 1];
+        __syncthreads();
+        if (!ok) continue;
+        int t = w0;
+        auto levels = [&](auto depth) {
+            constexpr int W = decltype(depth)::value;
+            double2 d[W];
+#pragma unroll
+            for (int j = 0; j < W; j++) d[j] = *reinterpret_cast<const double2*>(D + (int64_t)(t + j) * ld + i2);
+            const double* w = wwin + (t - w0);
+#pragma unroll
+            for (int j = 0; j < W; j += 2) {
+                a0 = fma(w[j], d[j].x, a0); a1 = fma(w[j], d[j].y, a1);
+                b0 = fma(w[j + 1], d[j + 1].x, b0); b1 = fma(w[j + 1], d[j + 1].y, b1);
+            }
+        };
+        for (; t + DEPTH <= w1; t += DEPTH) levels(std::integral_constant<int, DEPTH>{});
+        if constexpr (DEPTH > 4)
+            for (; t + 4 <= w1; t += 4) levels(std::integral_constant<int, 4>{});
+        for (; t < w1; t++) {
+            const double2 d0 = *reinterpret_cast<const double2*>(D + (int64_t)t * ld + i2);
+            const double x0 = wwin[t - w0];
+            a0 = fma(x0, d0.x, a0); a1 = fma(x0, d0.y, a1);
+        }
+    }
+    if (!ok) return;
+    double2 r;
+    r.x = a0 + b0;
+    r.y = a1 + b1;
+    *reinterpret_cast<double2*>(part + (int64_t)ks * ld + i2) = r;
+}
+
 // Kernel launchers (weights.hip, history.hip, space.hip, step1d.hip, lod3d.hip)
 fpde_status launch_weights(const fpde_spec& s, DeviceWeights& w, hipStream_t st);
 fpde_status launch_space_weights(const fpde_spec& s, DeviceWeights& w, double h, hipStream_t st);
@@ -476,9 +533,9 @@ fpde_status launch_space_reduce(double* V, const double* P, const double* F, con
 // plain FP64 stream over t < t_hi: partial rows part[ks*ld + i], ks < the
 // returned row count of hist_plain_plan (at most kPlainMaxSplits)
 constexpr int kPlainMaxSplits = 64;
-int hist_plain_plan(int nodes, int t_hi, int* chunk_out);
+int hist_plain_plan(int nodes, int t_hi, int* chunk_out, int max_splits = kPlainMaxSplits);
 fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int t_hi, const double* omega,
-                              double* part, int* splits_out, hipStream_t st);
+                              double* part, int* splits_out, hipStream_t st, int max_splits = kPlainMaxSplits);
 // The reference Sum (sum_alg 0/1): the intervals go in ref_sum_splits(nodes,
 // intervals) parts, whose partial rows need as many rows of `nodes` doubles in
 // `part` (one part: none).

@@ -252,6 +252,7 @@ struct fpde_solver {
     bool initialized = false;
     // GEMM block state
     int n0 = -1, tc = 0, gsplits = 0, packed_groups = 0;
+    int ahead_step = -1;         // step whose plain history the last step's launch streamed (within one call)
     double* part_cur = nullptr;  // partial rows the current block's steps read
     // far part one block ahead (1D cooperative form, lookahead_spec): the
     // older levels [0, tc of this block) of the next block's GEMM run on
@@ -584,6 +585,34 @@ fpde_status lookahead_drain(fpde_solver* s) {
     return FPDE_OK;
 }
 
+// Plain history of 1D step n streamed by the launch of step n - 1, beside its
+// chain (one launch per step instead of two dependent ones): the levels t <
+// n - 2, which that launch does not write, into one half of the partial rows
+// by step parity; the step's own launch adds the last two levels.  The split
+// depends on n alone, so the first step of a call, which streams by itself,
+// rounds alike.  At most 32 partial rows, which the chain reads in one memory
+// trip.  N = 3001: 11.6 -> 7.2 us per step over 1500 steps; N = 10^4: 26.7 ->
+// 20.0 over 3000 steps, 44.6 -> 41.6 over 6000, 89 -> 85 over 12000: 5 to 7 us
+// a step at any length.  A history beyond kAheadBytes streams for over 90 us,
+// of which that is 5%: it keeps its own launch (64 partial rows), which the
+// profile's history class times.
+constexpr int kAheadSplits = 32;
+constexpr double kAheadBytes = 512e6;
+bool plain_ahead(const fpde_solver* s, int n) {
+    const fpde_spec& sp = s->spec;
+    return sp.dims == 1 && sp.hist_mode == HIST_PLAIN_F64 && sp.sum_alg != 2 && !s->w.grid &&
+           8.0 * n * (double)s->plan.nodes <= kAheadBytes;
+}
+struct AheadStream { int lo, hi, chunk, splits; int64_t off; };
+AheadStream ahead_stream(const fpde_solver* s, int n) {
+    AheadStream h{};
+    h.lo = std::max(0, n - s->w.jmax);             // restricted summing: lags above jmax have zero weight
+    h.hi = std::max(n - 2, 0);
+    h.splits = hist_plain_plan((int)s->plan.nodes, h.hi - h.lo, &h.chunk, kAheadSplits);
+    h.off = (int64_t)(n & 1) * kAheadSplits * s->plan.ld;
+    return h;
+}
+
 // far part of the history for step n (GEMM modes: start a new block when due)
 fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_t* off, int* near_lo) {
     const fpde_spec& sp = s->spec;
@@ -597,6 +626,27 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
     }
     // levels available in memory: t < avail
     int avail = s->pending ? n - 1 : n;
+    if (sp.hist_mode == HIST_PLAIN_F64 && plain_ahead(s, n)) {
+        const AheadStream h = ahead_stream(s, n);
+        if (s->ahead_step != n && h.splits > 0) {
+            size_t slot = 0;
+            int ns = 0;
+            ev_begin(s, 0, &slot);
+            fpde_status rc = launch_hist_plain(s->D + (size_t)h.lo * p.ld, p.ld, (int)p.nodes, n - h.lo, h.hi - h.lo,
+                                               s->w.omega, s->part + h.off, &ns, s->stream, kAheadSplits);
+            ev_end(s, slot);
+            if (rc != FPDE_OK) return rc;
+            s->stats.history_launches++;
+            s->stats.history_alg_bytes += 8.0 * (h.hi - h.lo) * (double)p.nodes;
+            s->stats.history_alg_flops += 2.0 * (h.hi - h.lo) * (double)p.nodes;
+        }
+        s->omega_cur = s->w.omega;
+        *nsplit = h.splits;
+        *stride = p.ld;
+        *off = h.off;
+        *near_lo = std::max(h.lo, h.hi);
+        return FPDE_OK;
+    }
     if (sp.hist_mode == HIST_PLAIN_F64) {
         int ns = 0;
         size_t slot = 0;
@@ -711,7 +761,8 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
     return FPDE_OK;
 }
 
-fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, int64_t off, int near_lo) {
+fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, int64_t off, int near_lo,
+                      bool ahead = false) {
     const fpde_spec& sp = s->spec;
     Step1DArgs a{};
     a.N = sp.nodes;
@@ -737,6 +788,14 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
     a.part_off = off;
     a.near_lo = near_lo;
     a.Sbuf = s->S;
+    if (ahead && plain_ahead(s, n + 1)) {
+        const AheadStream h = ahead_stream(s, n + 1);
+        a.ahead_lo = h.lo;
+        a.ahead_hi = h.hi;
+        a.ahead_chunk = h.chunk;
+        a.ahead_splits = h.splits;
+        a.ahead_part = s->part + h.off;
+    }
     a.xyz = s->xyz;
     a.red = s->red;
     a.Uit = s->Uit;
@@ -795,7 +854,9 @@ fpde_status space_part(fpde_solver* s) {
     return FPDE_OK;
 }
 
-fpde_status enqueue_1d_step(fpde_solver* s, int n) {
+// Step n of a per-iteration solver; `more`: step n + 1 follows in this call,
+// so the launch may stream its plain history beside the chain.
+fpde_status enqueue_1d_step(fpde_solver* s, int n, bool more) {
     int nsplit = 0, near_lo = 0;
     int64_t stride = 0, off = 0;
     if (s->w.sp_on) {
@@ -805,9 +866,15 @@ fpde_status enqueue_1d_step(fpde_solver* s, int n) {
     fpde_status rc = far_part(s, n, &nsplit, &stride, &off, &near_lo);
     if (rc != FPDE_OK) return rc;
     for (int k = 0; k < s->spec.picard_max; k++) {
-        rc = launch_1d(s, n, k, nsplit, stride, off, near_lo);
+        rc = launch_1d(s, n, k, nsplit, stride, off, near_lo, more && k == 0);
         if (rc != FPDE_OK) return rc;
         s->stats.picard_iters_total++;
+    }
+    s->ahead_step = -1;
+    if (more && plain_ahead(s, n + 1)) {
+        const AheadStream h = ahead_stream(s, n + 1);
+        s->ahead_step = n + 1;
+        s->stats.step_alg_bytes += 8.0 * std::max(0, h.hi - h.lo) * (double)s->plan.nodes;
     }
     count_steps(s, n, n + 1, near_lo);
     return FPDE_OK;
@@ -1297,7 +1364,7 @@ fpde_status fpde_solver_advance(fpde_solver* s, int nsteps) {
         return FPDE_OK;
     }
     for (int n = s->step; n < end; n++) {
-        fpde_status rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n) : enqueue_3d_step(s, n);
+        fpde_status rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n, n + 1 < end) : enqueue_3d_step(s, n);
         if (rc != FPDE_OK) return rc;
         s->step = n + 1;
     }
@@ -1492,7 +1559,7 @@ fpde_status fpde_solver_advance_graph(fpde_solver* s, int nsteps, int steps_per_
         hipError_t e = hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal);
         if (e != hipSuccess) { set_error(std::string("hipStreamBeginCapture: ") + hipGetErrorString(e)); rc = FPDE_ERR_HIP; break; }
         for (int n = s->step; n < g_end && rc == FPDE_OK; n++) {
-            rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n) : enqueue_3d_step(s, n);
+            rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n, n + 1 < g_end) : enqueue_3d_step(s, n);
             if (rc == FPDE_OK) s->step = n + 1;
         }
         if (rc == FPDE_OK && s->spec.dims == 1 && s->step == M) rc = finalize_1d(s);
@@ -1541,7 +1608,7 @@ fpde_status fpde_solver_advance_tau(fpde_solver* s, double tau) {
     s->w.hLv[n] = grid_local(s->spec, s->Time_h[n], s->Time_h[n + 1]);
     fpde_status rc = launch_set_grid_point(s->w, n, s->Time_h[n + 1], tau, s->w.hLv[n], s->stream);
     if (rc != FPDE_OK) return rc;
-    rc = enqueue_1d_step(s, n);
+    rc = enqueue_1d_step(s, n, false);
     if (rc != FPDE_OK) return rc;
     s->step = n + 1;
     rc = finalize_1d(s);

@@ -25,24 +25,31 @@
 namespace fpde {
 
 // Far partial sums plus the near levels t in [near_lo, n-2] already in
-// memory, gathered in 32-wide batches of independent loads (a sum over m
-// terms costs ~m/32 memory round trips).  Every load is guarded: omega is
-// read only at n-t-1 >= 1.
+// memory, gathered in batches of independent loads (up to 32 partial rows and
+// the first two levels in one memory round trip, a sum over m more levels in
+// ~m/32).  omega is read only at n-t-1 >= 1.
 __device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t part_off,
                                   const double* __restrict__ omega) {
     constexpr int W = 32;
-    double far = 0.0;
-    for (int sp0 = 0; sp0 < g.nsplit; sp0 += W) {
-        double v[W];
-#pragma unroll
-        for (int j = 0; j < W; j++)
-            v[j] = (sp0 + j < g.nsplit) ? g.part[(int64_t)(sp0 + j) * g.part_stride + part_off + i] : 0.0;
-#pragma unroll
-        for (int j = 0; j < W; j++) far += v[j];
-    }
-    double nr0 = 0.0, nr1 = 0.0;
     const int t_end = n - 1;   // exclusive: D[n-1] is the newest level, added by the caller
-    for (int t0 = g.near_lo; t0 < t_end; t0 += W) {
+    double v0 = 0.0, v1 = 0.0, w0 = 0.0, w1 = 0.0;
+    if (g.near_lo < t_end) { v0 = g.D[(int64_t)g.near_lo * g.ld + i]; w0 = omega[n - g.near_lo - 1]; }
+    if (g.near_lo + 1 < t_end) { v1 = g.D[(int64_t)(g.near_lo + 1) * g.ld + i]; w1 = omega[n - g.near_lo - 2]; }
+    double far = 0.0;
+    const double* const part = g.part + part_off + i;
+    auto rows = [&](int r0, auto width) {          // (rows past the last: the last again, not added)
+        constexpr int V = decltype(width)::value;
+        double v[V];
+#pragma unroll
+        for (int j = 0; j < V; j++) v[j] = part[(int64_t)min(r0 + j, g.nsplit - 1) * g.part_stride];
+#pragma unroll
+        for (int j = 0; j < V; j++) far += r0 + j < g.nsplit ? v[j] : 0.0;
+    };
+    if (g.nsplit > 0 && g.nsplit <= 8) rows(0, std::integral_constant<int, 8>{});
+    else
+        for (int r0 = 0; r0 < g.nsplit; r0 += W) rows(r0, std::integral_constant<int, W>{});
+    double nr0 = w0 * v0, nr1 = w1 * v1;
+    for (int t0 = g.near_lo + 2; t0 < t_end; t0 += W) {
         double v[W], w[W];
 #pragma unroll
         for (int j = 0; j < W; j++) {
@@ -435,7 +442,10 @@ __device__ __forceinline__ void chunk_line(const double* K, const double* iC, co
 // the coefficients, one barrier, the line in wave 0), so it has the cooperative
 // form's wave-level solves: at N = 3001 a launch takes 7.8 us against 11.8 us
 // with the whole workgroup's cyclic reduction over LDS and both chunk ends as
-// separators.
+// separators.  Workgroups past the chunks stream the next step's plain history
+// meanwhile, 16 levels in flight per thread; with them, and the partial rows
+// and last levels loaded in one trip, the launch takes 7.3 us and no launch of
+// the stream (4.4 us) stands between two steps.
 template <int RW, int RR>
 __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
 #pragma clang fp contract(off)
@@ -446,6 +456,13 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
     const int p = 4 * (lane & 15) + (lane >> 4);
     const int c = blockIdx.x;
     const int N = g.N, C = g.C;
+    if (c >= C) {                         // the next step's history
+        __shared__ double wwin[kPlainWin];
+        const int b = c - C;
+        plain_stream<T, 16>(g.D + (int64_t)g.ahead_lo * g.ld, g.ld, N, g.n + 1 - g.ahead_lo, g.ahead_hi - g.ahead_lo,
+                            g.ahead_chunk, g.omega, g.ahead_part, b % g.ahead_tiles, b / g.ahead_tiles, wwin);
+        return;
+    }
     const int s = (int)(((int64_t)c * N) / C);
     const int nc = (int)(((int64_t)(c + 1) * N) / C) - s;
     const int i = s + tid;
@@ -1275,7 +1292,10 @@ fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st) {
     }
     const bool three = row_waves(a.N, a.C) == 3, few = a.C <= 64;
     auto* const kern = three ? (few ? k_step1d<3, 1> : k_step1d<3, 4>) : (few ? k_step1d<4, 1> : k_step1d<4, 4>);
-    hipLaunchKernelGGL(kern, dim3(a.C), dim3(three ? 192 : 256), 0, st, a);
+    Step1DArgs arg = a;
+    const int T = three ? 192 : 256;
+    arg.ahead_tiles = (a.N + 2 * T - 1) / (2 * T);
+    hipLaunchKernelGGL(kern, dim3(a.C + arg.ahead_tiles * a.ahead_splits), dim3(T), 0, st, arg);
     return FPDE_OK;
 }
 

@@ -1558,6 +1558,32 @@ def test_per_iteration_launch_edges_match_oracle(fpde, oracle, nodes, rows, gamm
     assert err <= TOL_F64
 
 
+@pytest.mark.parametrize("nodes,steps,picard,extra", [
+    (5, 40, 1, {}), (384, 130, 3, {}), (385, 1100, 1, {}), (1537, 200, 1, {"sum_alg": 1, "sum_param": 1e-2}),
+    (700, 90, 2, {"gamma": 0.8}), (65536, 985, 1, {})])
+def test_plain_history_streamed_ahead(fpde, nodes, steps, picard, extra):
+    """The plain history streamed by the previous step's launch: a solve
+    advanced at once, in pieces and as graph replays gives the same bits, and
+    agrees with the FP64 block form; two steps and less of history, tiles of
+    384 nodes, restricted summing, one level per part and more, and a history
+    that outgrows the limit (N = 65536 beyond 976 steps)."""
+    u0 = fpde.init_1d(nodes, 95)
+    kw = dict(alpha=0.7, picard_max=picard, picard_tol=1e-12 if picard > 1 else 0.0, u_top=u0[0], **extra)
+    spec = fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw)
+    whole = fpde.solve(spec, u0)
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b:
+        a.set_initial(u0)
+        b.set_initial(u0)
+        for piece in (1, 1, 2, 3, 11, 0):
+            a.advance(piece)
+        b.advance_graph(0, 7)
+        assert np.array_equal(a.solution(), whole)
+        assert np.array_equal(b.solution(), whole)
+    err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="mfma_f64", block=16, **kw), u0))
+    print(f"plain ahead N={nodes} M={steps}: rel err {err:.3e}", flush=True)
+    assert err <= TOL_F64
+
+
 @pytest.mark.parametrize("block", [16, 64, 128])
 @pytest.mark.parametrize("picard", [1, 3])
 def test_launches_that_cut_a_block_give_the_same_bits(fpde, block, picard):
