@@ -503,7 +503,7 @@ fpde_status fpde_space_sum(double* V, const double* F, int64_t nodes, double h, 
     sp.weight_mode = weight_mode;
     sp.series_eps = series_eps;
     const int64_t ldp = (nodes + kSpTile - 1) / kSpTile * kSpTile;
-    const size_t chunks = (size_t)space_chunks((int)(ldp / kSpTile) - 1);
+    const size_t chunks = (size_t)space_chunks((int)(ldp / kSpTile) - 1, ldp);
     DeviceWeights w;
     double *Fp = nullptr, *P = nullptr;
     fpde_status rc = FPDE_OK;

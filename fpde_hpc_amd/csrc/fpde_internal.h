@@ -383,11 +383,17 @@ struct BatchTick {
 // ---------------------------------------------------------------------------
 // Space-fractional sum (space.hip): rows are cut into tiles of kSpTile rows
 // (16 blocks of 16) and the 16-wide block diagonals d of the lower-triangular
-// Toeplitz matrix into chunks of kSpDiag; a tile t has block diagonals
-// d < 16 (t + 1) and space_chunks(t) partial rows.
+// Toeplitz matrix into chunks of space_diag(ldp); a tile t has block diagonals
+// d < 16 (t + 1) and space_chunks(t, ldp) partial rows.  Chunks of 64 leave a
+// short line on few workgroups (N = 4000: 40, whose waves each do 64 FP64 MFMA
+// one after the other), of 16 make as many rows of partial sums as tiles; up to
+// 8192 rows these are 32 rows at most.
 constexpr int kSpTile = 256;
 constexpr int kSpDiag = 64;
-__host__ __device__ inline int space_chunks(int t) { return (16 * (t + 1) + kSpDiag - 1) / kSpDiag; }
+__host__ __device__ inline int space_diag(int64_t ldp) { return ldp <= 8192 ? 16 : kSpDiag; }
+__host__ __device__ inline int space_chunks(int t, int64_t ldp) {
+    return (16 * (t + 1) + space_diag(ldp) - 1) / space_diag(ldp);
+}
 
 typedef double sd4_t __attribute__((ext_vector_type(4)));
 
@@ -402,11 +408,12 @@ struct SpaceUnitLds {
 };
 
 // One work unit of the spatial sum: P[y][i] = sum over the block diagonals d
-// in [kSpDiag y, kSpDiag y + kSpDiag) of row tile t (rows i = 256 t + 16 I'
+// in [W y, W y + W), W = space_diag, of row tile t (rows i = 256 t + 16 I'
 // + p) of sum_q w(16 d + p - q) F[16 (I0 + I' - d) + q], I0 = 16 t, with
 // w(m) = om[m-1] for 1 <= m <= N, else 0 (om: the Toeplitz lag vector).
-// Wave w takes 16 of the diagonals; the four waves' results are added
-// through LDS.  v_mfma_f64_16x16x4f64 layout (as in the history GEMM): A
+// Wave w takes a quarter of the diagonals; the four waves' results are added
+// through LDS.  Latency bound: all of a thread's loads of F and w go out
+// together (one by one they took 5 of the 8 us of N = 4000).  v_mfma_f64_16x16x4f64 layout (as in the history GEMM): A
 // lane l = A[l%16][l/16], B lane l = B[l/16][l%16], result v of lane l =
 // D[4v + l/16][l%16]; M index p, N index I', K index q.  Called by all 256
 // threads of a workgroup (it synchronises the workgroup).
@@ -414,27 +421,34 @@ __device__ inline void space_unit(const double* __restrict__ F, int N, const dou
                                   double* __restrict__ P, int64_t ldp, int t, int y, SpaceUnitLds& L) {
     const int tid = threadIdx.x;
     const int I0 = 16 * t;
-    const int d_lo = kSpDiag * y;
-    const int d_hi = min(d_lo + kSpDiag, I0 + 16);
+    const int W = space_diag(ldp);
+    const int d_lo = W * y;
+    const int d_hi = min(d_lo + W, I0 + 16);
     const int Jb = I0 - d_hi + 1;
     const int nfb = d_hi - d_lo + 15;
     const int mb = 16 * d_lo - 15;
     const int nw = 16 * (d_hi - d_lo) + 15;
     __syncthreads();                                   // LDS free (a previous unit may still read it)
-    for (int q = tid; q < nfb * 16; q += 256) {
-        const int b = q >> 4, c = q & 15;
-        const int64_t j = (int64_t)(Jb + b) * 16 + c;
-        L.Fs[b * 17 + c] = (j >= 0 && j < ldp) ? F[j] : 0.0;
+    constexpr int K = (16 * (kSpDiag + 15) + 255) / 256;   // loads per thread: nfb * 16 and nw are at most 256 K
+    double fv[K], wv[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int q = tid + 256 * k, m = mb + q;
+        const int64_t j = (int64_t)Jb * 16 + q;
+        fv[k] = (q < nfb * 16 && j >= 0 && j < ldp) ? F[j] : 0.0;
+        wv[k] = (q < nw && m >= 1 && m <= N) ? om[m - 1] : 0.0;
     }
-    for (int q = tid; q < nw; q += 256) {
-        const int m = mb + q;
-        L.Ws[q] = (m >= 1 && m <= N) ? om[m - 1] : 0.0;
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int q = tid + 256 * k;
+        if (q < nfb * 16) L.Fs[(q >> 4) * 17 + (q & 15)] = fv[k];
+        if (q < nw) L.Ws[q] = wv[k];
     }
     __syncthreads();
     const int lane = tid & 63, wave = tid >> 6;
     const int r16 = lane & 15, k4 = lane >> 4;
     sd4_t acc = {0.0, 0.0, 0.0, 0.0};
-    const int dw_lo = d_lo + 16 * wave, dw_hi = min(dw_lo + 16, d_hi);
+    const int dw_lo = d_lo + W / 4 * wave, dw_hi = min(dw_lo + W / 4, d_hi);
     for (int d = dw_lo; d < dw_hi; d++) {
         const int fb = (r16 + d_hi - 1 - d) * 17 + k4;   // F block I0 + I' - d, element 4 kq + k4
         const int wb = 16 * d + r16 - k4 - mb;           // w(16 d + p - q), q = 4 kq + k4
@@ -463,9 +477,16 @@ __device__ inline double space_flux(double Km, double Kj, double um, double u0, 
 // surface-interval corrections
 __device__ inline double space_sum(const double* __restrict__ P, int64_t ldp, const double* __restrict__ corr,
                                    const double* __restrict__ F, int i) {
-    const int ny = space_chunks(i / kSpTile);
+    const int ny = space_chunks(i / kSpTile, ldp);
     double e = 0.0;
-    for (int y = 0; y < ny; y++) e += P[(int64_t)y * ldp + i];
+    constexpr int B = 16;                               // rows loaded together
+    for (int y0 = 0; y0 < ny; y0 += B) {
+        double v[B];
+#pragma unroll
+        for (int j = 0; j < B; j++) v[j] = P[(int64_t)min(y0 + j, ny - 1) * ldp + i];
+#pragma unroll
+        for (int j = 0; j < B; j++) e += y0 + j < ny ? v[j] : 0.0;
+    }
     e = fma(corr[2 * (i - 1)], F[1], e);
     return fma(corr[2 * (i - 1) + 1], F[2], e);
 }

@@ -176,7 +176,7 @@ size_t footprint_bytes(const fpde_spec& s) {
     if (s.gamma > 0.0 && s.gamma < 1.0) {                            // space-fractional sum
         b += sizeof(double) * (3 * (size_t)s.nodes + p.ld);
         size_t ldp = (size_t)round_up(s.nodes, kSpTile);
-        if (s.dims == 1) b += sizeof(double) * ldp * (1 + space_chunks((int)(ldp / kSpTile) - 1));
+        if (s.dims == 1) b += sizeof(double) * ldp * (1 + space_chunks((int)(ldp / kSpTile) - 1, (int64_t)ldp));
     }
     if (s.taus || s.var_tau || s.fk) {                               // grid, weight rows
         size_t M = (size_t)s.steps, B = (size_t)s.block;
@@ -427,7 +427,7 @@ fpde_status solver_alloc(fpde_solver* s) {
             DALLOC(s->w.sp_omega, sizeof(double) * (size_t)sp.nodes);
             DALLOC(s->w.sp_corr, sizeof(double) * 2 * (size_t)sp.nodes);
             DALLOC(s->spF, sizeof(double) * (size_t)s->sp_ldp);
-            DALLOC(s->spP, sizeof(double) * (size_t)s->sp_ldp * space_chunks((int)(s->sp_ldp / kSpTile) - 1));
+            DALLOC(s->spP, sizeof(double) * (size_t)s->sp_ldp * space_chunks((int)(s->sp_ldp / kSpTile) - 1, s->sp_ldp));
             DALLOC(s->spE, sizeof(double) * p.ld);
         }
         // the space-fractional sum needs the whole U^n between two steps: its

@@ -10,7 +10,7 @@
 // d = I - J, so a tile of 256 rows (I = I0 .. I0+15) accumulates, per block
 // diagonal d, T_d (A operand, 16 x 16) times the 16 x 16 matrix of F blocks
 // F_{I-d} (B operand) in four 4-deep v_mfma_f64_16x16x4f64 steps.  Row tiles
-// x chunks of kSpDiag block diagonals form the grid; the chunks' partial
+// x chunks of space_diag block diagonals form the grid; the chunks' partial
 // sums are added by the consumer (space_sum).
 #include "fpde_internal.h"
 
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(256) void k_space_apply(const double* __restrict__ 
                                                      int64_t ldp) {
     __shared__ SpaceUnitLds lds;
     const int t = blockIdx.x, y = blockIdx.y;
-    if (y >= space_chunks(t)) return;                  // uniform over the block
+    if (y >= space_chunks(t, ldp)) return;                  // uniform over the block
     space_unit(F, N, om, P, ldp, t, y, lds);
 }
 
@@ -175,7 +175,7 @@ fpde_status launch_space_apply(const double* F, int N, const double* sp_omega, d
                                hipStream_t st) {
     if (ldp < N || ldp % kSpTile) { set_error("space sum: bad padded length"); return FPDE_ERR_ARG; }
     const int T = (int)(ldp / kSpTile);
-    hipLaunchKernelGGL(k_space_apply, dim3(T, space_chunks(T - 1)), dim3(256), 0, st, F, N, sp_omega, P, ldp);
+    hipLaunchKernelGGL(k_space_apply, dim3(T, space_chunks(T - 1, ldp)), dim3(256), 0, st, F, N, sp_omega, P, ldp);
     FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
 }

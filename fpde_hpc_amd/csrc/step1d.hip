@@ -445,8 +445,9 @@ __device__ __forceinline__ void chunk_line(const double* K, const double* iC, co
 // separators.  Workgroups past the chunks stream the next step's plain history
 // meanwhile, 16 levels in flight per thread; with them, and the partial rows
 // and last levels loaded in one trip, the launch takes 7.3 us and no launch of
-// the stream (4.4 us) stands between two steps.
-template <int RW, int RR>
+// the stream (4.4 us) stands between two steps.  SPACE: the space-fractional
+// scheme (compiled apart: its code in the other form cost 9% of the step).
+template <int RW, int RR, bool SPACE>
 __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
 #pragma clang fp contract(off)
     __shared__ double sK[kRowSlots], sC[kRowSlots], sR[kRowSlots], pub[8], wmax[RW];
@@ -514,7 +515,7 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
     // space-fractional scheme: Om1's explicit sum -inv_dw_dh E_i (:4182-4189);
     // E of step n is formed by its first launch and reused by the others
     double E = 0.0;
-    if (g.sp_on && g.k >= 0 && i > 0 && i < N - 1 && act) {
+    if (SPACE && g.k >= 0 && i > 0 && i < N - 1 && act) {
         E = first ? space_sum(g.sp_P, g.sp_ldp, g.sp_corr, g.sp_F, i) : g.sp_E[i];
         if (first) g.sp_E[i] = E;
     }
@@ -573,7 +574,7 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
         // equation 0, fpde_hpc_1d.cpp:4176-4179), the arithmetic of
         // k_space_flux.  The neighbours s-1 and e+1 come from the separators
         // (or the converged iterate), so the next step needs no flux launch.
-        if (g.sp_on && g.recover) {
+        if (SPACE && g.recover) {
             double* sU = sR;                     // U^n of nodes s-1 .. e+1
             double* sKf = sK;                    // K at U^n of nodes s-1 .. e
             double k, icv;
@@ -625,7 +626,7 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
     // ---- 3. coefficients at the iterate, right-hand sides -------------------
     // (space-fractional scheme: the diffusion part of A_/B/R scaled by
     // Dg kb(gamma,i-1,i,i))
-    const double kap = g.sp_on ? g.sp_kap : 1.0;
+    const double kap = SPACE ? g.sp_kap : 1.0;
     if (extrap0) u_halo += u_halo - uprev_halo;
     const bool spare = halo && !act;             // (in the same evaluation as the wave's own nodes)
     double K, invC;
@@ -1291,7 +1292,10 @@ fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st) {
         return FPDE_ERR_ARG;
     }
     const bool three = row_waves(a.N, a.C) == 3, few = a.C <= 64;
-    auto* const kern = three ? (few ? k_step1d<3, 1> : k_step1d<3, 4>) : (few ? k_step1d<4, 1> : k_step1d<4, 4>);
+    auto* const kern = a.sp_on ? (three ? (few ? k_step1d<3, 1, true> : k_step1d<3, 4, true>)
+                                        : (few ? k_step1d<4, 1, true> : k_step1d<4, 4, true>))
+                               : (three ? (few ? k_step1d<3, 1, false> : k_step1d<3, 4, false>)
+                                        : (few ? k_step1d<4, 1, false> : k_step1d<4, 4, false>));
     Step1DArgs arg = a;
     const int T = three ? 192 : 256;
     arg.ahead_tiles = (a.N + 2 * T - 1) / (2 * T);

@@ -1265,6 +1265,25 @@ def test_space_sum_kernel_matches_oracle(fpde, oracle, n, wm):
         assert V[1] == 0.0 and abs(V[2] - ref[2]) <= 1e-12 * abs(ref[2])
 
 
+@pytest.mark.parametrize("n", [769, 1024, 8192, 8193])
+def test_space_sum_chunk_widths(fpde, oracle, n):
+    """The widths of the block-diagonal chunks: 16 up to 8192 rows, 64 beyond
+    (the last row of the one, the first of the other, and the last tile of each
+    with a single row).  Each element is a sum of at most n products rounded in
+    double, so 1e-12 of the largest holds whatever the split."""
+    F = np.random.default_rng(5 * n).standard_normal(n)
+    h, gam = 1.0 / (n - 1), 0.8
+    ref = oracle.space_v(F, h, gam, weight_mode=0)
+    L = fpde.lib()
+    dv = Dev(L)
+    try:
+        bF, bV = dv.put(F), dv.put(np.zeros(n))
+        assert L.fpde_space_sum(dv.ptr(bV), dv.ptr(bF), n, h, gam, 0, 1e-5) == 0, L.fpde_last_error()
+        assert rel_err(dv.get(bV, n), ref) <= 1e-12
+    finally:
+        dv.close()
+
+
 def _oracle_space(oracle, spec, u0):
     p = oracle.make_params(spec.nodes, spec.steps, spec.tau, spec.alpha, ksat=spec.ksat,
                            coef_mode=spec.coef_mode, picard_max=spec.picard_max, picard_tol=spec.picard_tol,
