@@ -607,7 +607,7 @@ bool step1d_batch_supported(int64_t wgs);
 // row holds what its single-solve launches take.
 constexpr int kMax3DBatch = 8;
 struct Lod3DRow {
-    double *U, *S, *Uprev, *Dlev;
+    double *U, *S, *V, *Dlev;
     const double *part, *D, *omega, *corr, *utop;
     int64_t part_stride, part_off, ld, nodes;
     int n, nsplit, step, near_lo, coef_mode, split;
@@ -629,12 +629,11 @@ struct Lod3DRow {
 struct Lod3DBatch {
     int count;
     int first_node[kMax3DBatch + 1];   // 256-node blocks (history combine, coefficients)
-    int first_lat[kMax3DBatch + 1];    // 32-line blocks (lateral sweeps)
-    int first_z[kMax3DBatch + 1];      // 16-line blocks (depth sweep)
+    int first_line[kMax3DBatch + 1];   // groups of kLinesHost3D lines (sweeps)
     Lod3DRow row[kMax3DBatch];
 };
 fpde_status launch_lod3d_batch(const Lod3DBatch& b, hipStream_t st);
-constexpr int kZLinesHost = 16;      // depth lines per workgroup of the partitioned z sweep
+constexpr int kLinesHost3D = 16;     // lines per workgroup of the partitioned sweeps
 bool solver_3d_batchable(const fpde_solver* s);
 fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps);
 // 3D solves in batched LOD steps (groups of kMax3DBatch), the rest on their own streams
@@ -709,13 +708,13 @@ fpde_status launch_coef3d(const double* U, int n, double h, double ksat, int mod
                           hipStream_t st);
 // K, iC null: the partitioned sweep (lateral3d_partitioned) evaluates the
 // coefficients at U itself; the one-thread-per-line sweep needs them
-fpde_status launch_lateral3d(double* U, const double* K, const double* iC, const double* H, int n, int axis,
+fpde_status launch_lateral3d(const double* Uin, double* Uout, const double* K, const double* iC, const double* H, int n, int axis,
                              double h2inv, double L, double* Al, double* Bt, double kap, const double* E,
                              double h, double ksat, int mode, hipStream_t st);
 inline bool lateral3d_partitioned(int n, double L) { return n <= 128 && L > 0.0; }
 // K, iC: the coefficients at U when a coefficient pass already formed them
 // (else nullptr: the sweep evaluates them itself)
-fpde_status launch_zline3d(double* U, double* Uprev, const double* utop, int n, double h, double h2inv,
+fpde_status launch_zline3d(const double* V, double* U, const double* utop, int n, double h, double h2inv,
                            double ksat, int mode, double L, double* Dlev, double kap, const double* E,
                            const double* K, const double* iC, const double* H, hipStream_t st);
 fpde_status launch_space3d(const double* U, const double* K, int n, int axis, double h, const double* sp_omega,

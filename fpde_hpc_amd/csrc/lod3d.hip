@@ -15,6 +15,7 @@
 // With the space-fractional scheme every sweep also takes kap and the line
 // sums E of its own axis (space.hip, k_space3d).
 #include "fpde_internal.h"
+#include <algorithm>
 
 namespace fpde {
 
@@ -44,7 +45,7 @@ __global__ __launch_bounds__(256) void k_coef3d(const double* __restrict__ U, in
 // Space-fractional scheme (E != nullptr): the diffusion part of the rows is
 // scaled by kap = Dg kb(gamma,i-1,i,i) and Om carries -inv_dw_dh E (E: the
 // line sums of k_space3d), as in the 1D rows.
-__global__ __launch_bounds__(256) void k_lateral3d(double* __restrict__ U, const double* __restrict__ K,
+__global__ __launch_bounds__(256) void k_lateral3d(const double* U, double* Uout, const double* __restrict__ K,
                                                    const double* __restrict__ iC,
                                                    const double* __restrict__ H, int n, int axis,
                                                    double h2inv, double L, double* __restrict__ Al,
@@ -100,7 +101,7 @@ __global__ __launch_bounds__(256) void k_lateral3d(double* __restrict__ U, const
     double uN;
     if (fabs(bt) > 1e-15) uN = (fabs(1.0 - al) > 1e-15) ? bt / (1.0 - al) : U[base + stride * (N - 1)];
     else uN = (fabs(1.0 - al) > 1e-15) ? 0.0 : U[base + stride * (N - 1)];
-    U[base + stride * N] = uN;
+    Uout[base + stride * N] = uN;
     double u = uN;
     for (int i1 = N - 1; i1 >= 0; i1 -= R) {
         double aa[R], bb[R];
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(256) void k_lateral3d(double* __restrict__ U, const
             int i = i1 - j;
             if (i >= 0) {
                 u = aa[j] * u + bb[j];
-                U[base + stride * i] = u;
+                Uout[base + stride * i] = u;
             }
         }
     }
@@ -125,9 +126,9 @@ __global__ __launch_bounds__(256) void k_lateral3d(double* __restrict__ U, const
 
 // Depth sweep: block = one z line, one node per thread (blockDim = n rounded
 // up to 64, n <= 256).  PCR on rows normalised to b = 1 with ping-pong LDS
-// buffers (one barrier and one reciprocal per level).  Writes U^{n+1}, the
-// history level D[t] = U^{n+1} - Uprev and refreshes Uprev.
-__global__ __launch_bounds__(256) void k_zline3d(double* __restrict__ U, double* __restrict__ Uprev,
+// buffers (one barrier and one reciprocal per level).  From V; writes U^{n+1}
+// over U^n and the history level D[t] = U^{n+1} - U^n.
+__global__ __launch_bounds__(256) void k_zline3d(const double* __restrict__ V, double* __restrict__ U,
                                                  const double* __restrict__ utop, int n, double h,
                                                  double h2inv, double ksat, int mode, double L,
                                                  double* __restrict__ Dlev, double kap,
@@ -140,8 +141,8 @@ __global__ __launch_bounds__(256) void k_zline3d(double* __restrict__ U, double*
     const bool act = tid < n;
     double u = 0.0, k = 0.0, ic = 0.0, uprev = 0.0;
     if (act) {
-        u = U[base + tid];
-        uprev = Uprev[base + tid];
+        u = V[base + tid];
+        uprev = U[base + tid];
         vgm_coefs(u, tid * h, ksat, mode, k, ic);
         sK[tid] = k;
     }
@@ -183,306 +184,258 @@ __global__ __launch_bounds__(256) void k_zline3d(double* __restrict__ U, double*
         int64_t id = base + tid;
         U[id] = un;
         Dlev[id] = un - uprev;
-        Uprev[id] = un;
     }
 }
 
-// Lateral (y or x) sweep as a partitioned solve: each line's n nodes are cut
-// into kLatSeg segments of at most S rows, one thread each (32 lines x 8
-// segments per workgroup; the 32 lines are consecutive z, so every row load
-// is coalesced).  The line's system is the reference one: zero flux at both
-// ends (U_0 = U_1: Al_1 = 1, Bt_1 = 0, fpde_hpc_1d.cpp:4021, :4511; U_N =
-// U_{N-1}: the bottom of U1, :4704-4720) and the rows of A_/B/R/Om between.
-//  1. A segment [lo, hi] moves its couplings to U_{lo-1} and U_{hi+1} to two
-//     right-hand sides (a_lo e_1, c_hi e_last) and runs the Thomas
-//     recurrences for the three: U_i = x_i + y_i U_{lo-1} + z_i U_{hi+1}.
-//  2. One barrier publishes the segments' end rows; every thread runs the
-//     recursion over the segments (f_s = U_lo, l_s = U_hi: l_{s-1} = P + Q f_s
-//     forward, f_s = F_s + G_s f_{s+1} back) and back-substitutes its rows.
-// Same system as the one-thread-per-line sweeps (k_lateral3d*).  The
-// reference's 1e-15 guards on the bottom row act on singular lines (|1 -
-// Al_N| <= 1e-15, which L > 0 rules out: every row is diagonally dominant)
-// and on a bottom value within 1e-15 of zero, where the two differ by less
-// than that absolute amount.
-// K, iC: the coefficients at U from a coefficient pass, or nullptr: then the
-// sweep evaluates them itself, at the rows it solves and the node before its
-// first row (every node of a lateral line has the same depth z0 h), the same
-// values the pass would store.
-constexpr int kLatSeg = 8;
-static_assert(16 * kLatSeg == 128, "lateral3d_partitioned: 8 segments of at most 16 rows");
-template <int S>
-__device__ __forceinline__ void lateral3d_seg_body(double* __restrict__ U, const double* __restrict__ K,
-                                                   const double* __restrict__ iC, const double* __restrict__ H,
-                                                   int n, int axis, double h2inv, double L, double kap,
-                                                   const double* __restrict__ E, double h, double ksat, int mode,
+// Partitioned sweeps (n <= 128, L > 0): a workgroup takes kLineGroup lines and
+// cuts each into segments of kSegRows rows, one thread each (thread = line +
+// kLineGroup * segment, so that the lateral axes' loads are coalesced over the
+// 16 consecutive z).  The line's system is the reference one (lateral: zero
+// flux at both ends, U_0 = U_1: Al_1 = 1, Bt_1 = 0, fpde_hpc_1d.cpp:4021,
+// :4511; U_N = U_{N-1}: the bottom of U1, :4704-4720; depth: U_0 = u_top) and
+// the rows of A_/B/R/Om between.  The reference's 1e-15 guards on the bottom
+// row act on singular lines (|1 - Al_N| <= 1e-15, which L > 0 rules out: every
+// row is diagonally dominant) and on a bottom value within 1e-15 of zero,
+// where the two differ by less than that absolute amount.
+//
+// What bounds them: FP64 issue (VGM coefficients and row eliminations, about
+// half of the time) and memory, one after the other unless several workgroups
+// of a CU are in different phases.  So the rows per thread are few enough for
+// 4 waves per SIMD: segments of 8 rows with their last rows reduced cyclically
+// over the segments (4 levels, one reciprocal each, through LDS) instead of
+// segments of 16 with every thread walking all segments' ends (256 registers,
+// 2 waves per SIMD, a reciprocal per segment).  n = 128: lateral sweep 23.0 ->
+// 16.4 us, depth sweep 34 -> 21.3 us.
+constexpr int kSegRows = 8, kSegMax = 16, kLineGroup = kLinesHost3D;
+struct Line3DLds { double v[2][3][kSegMax][kLineGroup]; };
+
+// Solve the lines of a workgroup, rows a x_{i-1} + b x_i + c x_{i+1} = d of
+// segment sg (of W; a = 0 on the line's first row, c = 0 on its last) of line l:
+// a segment's first rows are eliminated against its last one (two couplings as
+// right-hand sides), the last ones reduced cyclically.  Called by all threads;
+// L.v[0] is free on entry.
+__device__ __forceinline__ void line3d_solve(const double (&a)[kSegRows], const double (&b)[kSegRows],
+                                             const double (&c)[kSegRows], const double (&d)[kSegRows], int l, int sg,
+                                             int W, Line3DLds& L, double (&x)[kSegRows]) {
+#pragma clang fp contract(off)
+    constexpr int S = kSegRows;
+    double q[S - 1], y[S - 1];                      // q: c' of the elimination, then z
+    {
+        const double inv = rcp_nr(b[0]);
+        q[0] = c[0] * inv;
+        x[0] = d[0] * inv;
+        y[0] = -a[0] * inv;
+    }
+#pragma unroll
+    for (int j = 1; j < S - 1; j++) {
+        const double inv = rcp_nr(fma(-a[j], q[j - 1], b[j]));
+        q[j] = c[j] * inv;
+        x[j] = fma(-a[j], x[j - 1], d[j]) * inv;
+        y[j] = -(a[j] * y[j - 1]) * inv;
+    }
+    q[S - 2] = -q[S - 2];
+#pragma unroll
+    for (int j = S - 3; j >= 0; j--) {
+        x[j] = fma(-q[j], x[j + 1], x[j]);
+        y[j] = fma(-q[j], y[j + 1], y[j]);
+        q[j] = -(q[j] * q[j + 1]);
+    }
+    L.v[0][0][sg][l] = x[0];
+    L.v[0][1][sg][l] = y[0];
+    L.v[0][2][sg][l] = q[0];
+    __syncthreads();
+    double xn = 0.0, yn = 0.0, zn = 0.0;
+    if (sg + 1 < W) { xn = L.v[0][0][sg + 1][l]; yn = L.v[0][1][sg + 1][l]; zn = L.v[0][2][sg + 1][l]; }
+    double A = a[S - 1], C = c[S - 1], D;
+    {
+        const double inv = rcp_nr(fma(C, yn, fma(A, q[S - 2], b[S - 1])));
+        D = fma(-C, xn, fma(-A, x[S - 2], d[S - 1])) * inv;
+        A = (A * y[S - 2]) * inv;
+        C = (C * zn) * inv;
+    }
+    int par = 1;
+    for (int s = 1; s < W; s <<= 1) {
+        L.v[par][0][sg][l] = A;
+        L.v[par][1][sg][l] = C;
+        L.v[par][2][sg][l] = D;
+        __syncthreads();
+        double am = 0.0, cm = 0.0, dm = 0.0, ap = 0.0, cp = 0.0, dp = 0.0;
+        if (sg >= s) { am = L.v[par][0][sg - s][l]; cm = L.v[par][1][sg - s][l]; dm = L.v[par][2][sg - s][l]; }
+        if (sg + s < W) { ap = L.v[par][0][sg + s][l]; cp = L.v[par][1][sg + s][l]; dp = L.v[par][2][sg + s][l]; }
+        const double inv = rcp_nr(fma(-C, ap, fma(-A, cm, 1.0)));
+        D = fma(-C, dp, fma(-A, dm, D)) * inv;
+        A = -(A * am) * inv;
+        C = -(C * cp) * inv;
+        par ^= 1;
+    }
+    L.v[par][0][sg][l] = D;
+    __syncthreads();
+    const double xl = sg > 0 ? L.v[par][0][sg - 1][l] : 0.0;
+    x[S - 1] = D;
+#pragma unroll
+    for (int j = 0; j < S - 1; j++) x[j] = fma(q[j], D, fma(y[j], xl, x[j]));
+}
+
+// Rows of a segment from its U, K, 1/C and the right-hand sides' other terms
+// rhs = H - E/C (row i = 8 sg + j); rows past the line are x = 0, coupled to
+// nothing.  K of the segment to the left comes through LDS.
+__device__ __forceinline__ void line3d_rows(const double (&u)[kSegRows], const double (&K)[kSegRows],
+                                            const double (&iC)[kSegRows], const double (&rhs)[kSegRows], int n, int l,
+                                            int sg, double h2inv, double lam, double kap, bool depth, double top,
+                                            Line3DLds& L, double (&a)[kSegRows], double (&b)[kSegRows],
+                                            double (&c)[kSegRows], double (&d)[kSegRows]) {
+#pragma clang fp contract(off)
+    L.v[1][0][sg][l] = K[kSegRows - 1];
+    __syncthreads();
+    double Km = sg > 0 ? L.v[1][0][sg - 1][l] : 0.0;
+#pragma unroll
+    for (int j = 0; j < kSegRows; j++) {
+        const int i = kSegRows * sg + j;
+        const bool inner = i >= 1 && i < n - 1;
+        const double g = iC[j] * h2inv * kap;
+        a[j] = inner ? Km * g : (i == n - 1 ? -1.0 : 0.0);
+        c[j] = inner ? K[j] * g : (i == 0 && !depth ? -1.0 : 0.0);
+        b[j] = inner ? -fma(g, K[j] + Km, lam) : 1.0;
+        d[j] = inner ? fma(-lam, u[j], rhs[j]) : (i == 0 ? top : 0.0);
+        Km = K[j];
+    }
+}
+
+// Lateral (y or x) sweep from Uin to Uout (the same field or another).
+// K, iC: the coefficients at Uin from a coefficient pass, or nullptr: then the
+// sweep evaluates them itself (every node of a lateral line has the same depth
+// z0 h), the same values the pass would store.
+__device__ __forceinline__ void lateral3d_seg_body(const double* Uin, double* Uout, const double* K, const double* iC,
+                                                   const double* H, int n, int axis, double h2inv, double lam,
+                                                   double kap, const double* E, double h, double ksat, int mode,
                                                    int bid) {
-    __shared__ double sEnd[kLatSeg][32][7];    // x, y, z of the first and the last row
+#pragma clang fp contract(off)
+    __shared__ Line3DLds L;
     const int tid = threadIdx.x;
-    const int l = tid & 31, sg = tid >> 5;
-    const int line = bid * 32 + l;
-    const bool ok_line = line < n * n;
-    const int ln = ok_line ? line : 0;
+    const int l = tid % kLineGroup, sg = tid / kLineGroup;
+    const int line = bid * kLineGroup + l;
+    const int ln = min(line, n * n - 1);
     const int z0 = ln % n, o = ln / n;
     int64_t base, stride;
     if (axis == 2) { base = z0 + (int64_t)n * o; stride = (int64_t)n * n; }   // (z,x=o), along y
     else { base = z0 + (int64_t)n * n * o; stride = n; }                        // (z,y=o), along x
-    const int N = n - 1;
-    const int Sg = (n + kLatSeg - 1) / kLatSeg;      // rows per segment (<= S)
-    const int W = (n + Sg - 1) / Sg;                 // segments present
-    const int lo = sg * Sg, hi = min(n, lo + Sg) - 1;
-    const bool act = ok_line && lo <= hi;
-    // 1. Thomas on the segment: cp = c', x/y the modified right-hand sides
-    // (straight-line code: rows past hi and the two end rows by selects)
-    double cp[S], xs[S], ys[S];
-    double zl = 0.0;                                 // z of the last row
-    double cprev = 0.0, xprev = 0.0, yprev = 0.0;
+    const int W = (n + kSegRows - 1) / kSegRows;
     const double zd = z0 * h;
-    double Km = 0.0;
-    if (act && lo >= 1) {
-        if (K) {
-            Km = K[base + stride * (lo - 1)];
-        } else {
-            double icm;
-            vgm_coefs(U[base + stride * (lo - 1)], zd, ksat, mode, Km, icm);
-        }
-    }
-    // the rows' coefficients first (independent evaluations that the
-    // scheduler interleaves), then the recurrence
-    double Kr[S], ir[S], ur[S];
+    auto at = [&](int j) { return base + stride * min(kSegRows * sg + j, n - 1); };   // (rows past the line: its last)
+    double u[kSegRows], r[kSegRows], k[kSegRows], ic[kSegRows];
 #pragma unroll
-    for (int j = 0; j < S; j++) {
-        const int i = lo + j;
-        const bool inner = act && i <= hi && i >= 1 && i <= N - 1;
-        const int64_t id = base + stride * (inner ? i : 0);
-        ur[j] = inner ? U[id] : 0.0;
-        if (K) {
-            Kr[j] = inner ? K[id] : 0.0;
-            ir[j] = inner ? iC[id] : 0.0;
-        } else {
-            double kv = 0.0, iv = 0.0;
-            if (inner) vgm_coefs(ur[j], zd, ksat, mode, kv, iv);
-            Kr[j] = kv;
-            ir[j] = iv;
-        }
-    }
+    for (int j = 0; j < kSegRows; j++) u[j] = Uin[at(j)];
 #pragma unroll
-    for (int j = 0; j < S; j++) {
-        const int i = lo + j;
-        const bool valid = act && i <= hi;
-        const bool inner = valid && i >= 1 && i <= N - 1;
-        const int64_t id = base + stride * (inner ? i : 0);
-        const double Kp = Kr[j];
-        const double icv = ir[j];
-        const double uv = ur[j];
-        const double hv = (inner && H) ? H[id] : 0.0;
-        const double ev = (inner && E) ? E[id] : 0.0;
-        const double a = inner ? Km * icv * h2inv * kap : (i == N ? -1.0 : 0.0);
-        const double c = inner ? Kp * icv * h2inv * kap : (i == 0 ? -1.0 : 0.0);
-        const double b = inner ? -(icv * ((Kp * h2inv) + (Km * h2inv)) * kap + L) : 1.0;
-        const double d = inner ? -L * uv + hv - icv * ev : 0.0;
-        Km = Kp;
-        const double inv = rcp_nr(j == 0 ? b : b - a * cprev);
-        cp[j] = (valid && i < hi) ? c * inv : 0.0;
-        xs[j] = valid ? (j == 0 ? d : d - a * xprev) * inv : 0.0;
-        ys[j] = valid ? (j == 0 ? -a : -a * yprev) * inv : 0.0;
-        if (valid && i == hi) zl = -c * inv;
-        cprev = cp[j]; xprev = xs[j]; yprev = ys[j];
-    }
-    // back: x, y in place, z_i = -c'_i z_{i+1} into cp (rows past hi stay 0)
-    double xn = 0.0, yn = 0.0, zn = 0.0;
+    for (int j = 0; j < kSegRows; j++) r[j] = H ? H[at(j)] : 0.0;
 #pragma unroll
-    for (int j = S - 1; j >= 0; j--) {
-        const int i = lo + j;
-        const bool valid = act && i <= hi;
-        const bool last = valid && i == hi;
-        xn = last ? xs[j] : xs[j] - cp[j] * xn;
-        yn = last ? ys[j] : ys[j] - cp[j] * yn;
-        zn = last ? zl : -cp[j] * zn;
-        xs[j] = xn; ys[j] = yn; cp[j] = zn;
-        if (valid && j == 0) { sEnd[sg][l][0] = xn; sEnd[sg][l][1] = yn; sEnd[sg][l][2] = zn; }
-        if (last) { sEnd[sg][l][3] = xn; sEnd[sg][l][4] = yn; sEnd[sg][l][5] = zn; }
+    for (int j = 0; j < kSegRows; j++) {
+        if (K) { k[j] = K[at(j)]; ic[j] = iC[at(j)]; }
+        else vgm_coefs(u[j], zd, ksat, mode, k[j], ic[j]);
+        if (E) r[j] = fma(-ic[j], E[at(j)], r[j]);
     }
-    __syncthreads();
-    if (!act) return;
-    // 2. the segments' end values: forward l_{s-1} = P + Q f_s, back f_s = F_s + G_s f_{s+1}
-    double Fv[kLatSeg], Gv[kLatSeg], Pv[kLatSeg], Qv[kLatSeg];
-    double pv = 0.0, qv = 0.0;
+    double a[kSegRows], b[kSegRows], c[kSegRows], d[kSegRows], x[kSegRows];
+    line3d_rows(u, k, ic, r, n, l, sg, h2inv, lam, kap, false, 0.0, L, a, b, c, d);
+    line3d_solve(a, b, c, d, l, sg, W, L, x);
+    if (line >= n * n) return;
 #pragma unroll
-    for (int k = 0; k < kLatSeg; k++) {
-        if (k < W) {
-            const double Xf = sEnd[k][l][0], Yf = sEnd[k][l][1], Zf = sEnd[k][l][2];
-            const double Xl = sEnd[k][l][3], Yl = sEnd[k][l][4], Zl = sEnd[k][l][5];
-            const double inv = rcp_nr(1.0 - Yf * qv);
-            Fv[k] = (Xf + Yf * pv) * inv;
-            Gv[k] = Zf * inv;
-            const double yq = Yl * qv;
-            pv = Xl + Yl * pv + yq * Fv[k];
-            qv = yq * Gv[k] + Zl;
-            Pv[k] = pv; Qv[k] = qv;
-        }
-    }
-    double fr = 0.0, vr = 0.0, vl = 0.0;             // f_{k+1}; this segment's right and left values
-#pragma unroll
-    for (int k = kLatSeg - 1; k >= 0; k--) {
-        if (k < W) {
-            if (k == sg) vr = fr;
-            if (k == sg - 1) vl = Pv[k] + Qv[k] * fr;    // l_{sg-1}
-            fr = Fv[k] + Gv[k] * fr;
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < S; j++) {
-        const int i = lo + j;
-        if (i <= hi) U[base + stride * i] = xs[j] + ys[j] * vl + cp[j] * vr;
-    }
+    for (int j = 0; j < kSegRows; j++)
+        if (kSegRows * sg + j < n) Uout[at(j)] = x[j];
 }
-template <int S>
-__global__ __launch_bounds__(256, 2) void k_lateral3d_seg(double* __restrict__ U, const double* __restrict__ K,
-                                                      const double* __restrict__ iC,
-                                                      const double* __restrict__ H, int n, int axis,
-                                                      double h2inv, double L, double kap,
-                                                      const double* __restrict__ E, double h, double ksat,
-                                                      int mode) {
-    lateral3d_seg_body<S>(U, K, iC, H, n, axis, h2inv, L, kap, E, h, ksat, mode, blockIdx.x);
+constexpr int kSegThreads = kSegMax * kLineGroup;
+__global__ __launch_bounds__(kSegThreads, 4) void k_lateral3d_seg(const double* Uin, double* Uout, const double* K,
+                                                                  const double* iC, const double* H, int n, int axis,
+                                                                  double h2inv, double lam, double kap,
+                                                                  const double* E, double h, double ksat, int mode) {
+    lateral3d_seg_body(Uin, Uout, K, iC, H, n, axis, h2inv, lam, kap, E, h, ksat, mode, blockIdx.x);
 }
 
-
-// Depth (z) sweep as a partitioned solve over 16 contiguous lines per
-// workgroup: the lines' U, their VGM coefficients at U and the right-hand
-// sides are staged in LDS by coalesced loads, then each line's n nodes are
-// cut into kZSeg segments of at most 8 rows (one thread each) and solved as
-// in k_lateral3d_seg (Thomas per segment with the two coupling right-hand
-// sides, one barrier, the recursion over the segments).  Rows: Dirichlet top
-// U_0 = u_top, the rows of A_/B/R/Om, zero-flux bottom U_{n-1} = U_{n-2};
-// the new U, D[n] = U - Uprev and Uprev go out through LDS, coalesced.
-constexpr int kZSeg = 16, kZLines = 16, kZThreads = kZSeg * kZLines;
-static_assert(kZLines == kZLinesHost, "the host's block count of the depth sweep");
-__device__ __forceinline__ void zline3d_seg_body(double* __restrict__ U, double* __restrict__ Uprev,
-                                                 const double* __restrict__ utop, int n, double h, double h2inv,
-                                                 double ksat, int mode, double L, double* __restrict__ Dlev,
-                                                 double kap, const double* __restrict__ E,
-                                                 const double* __restrict__ Kin, const double* __restrict__ iCin,
-                                                 const double* __restrict__ H, int bid) {
-    constexpr int LD = 129;                      // odd row stride: the 16 lines hit distinct banks
-    __shared__ double sK[kZLines][LD], sIC[kZLines][LD], sD[kZLines][LD];
-    __shared__ double sEnd[kZSeg][kZLines][7];
-    const int tid = threadIdx.x;
-    const int nlines = n * n;
-    const int line0 = bid * kZLines;
-    const int nl = min(kZLines, nlines - line0);        // lines of this group
+// Depth (z) sweep from V: the new U over U^n, D[n] = U - U^n.  The lines are
+// contiguous, so rows go between memory (coalesced) and the threads' segments
+// through LDS.
+__device__ __forceinline__ void zline3d_seg_body(const double* V, double* U, const double* utop, int n, double h,
+                                                 double h2inv, double ksat, int mode, double lam, double* Dlev,
+                                                 double kap, const double* E, const double* Kin, const double* iCin,
+                                                 const double* H, int bid) {
+#pragma clang fp contract(off)
+    constexpr int LD = kSegRows * kSegMax + 1;          // odd row stride: the 16 lines hit distinct banks
+    __shared__ Line3DLds L;
+    __shared__ double sU[kLineGroup][LD];
+    const int tid = threadIdx.x, T = blockDim.x;
+    const int l = tid % kLineGroup, sg = tid / kLineGroup;
+    const int line0 = bid * kLineGroup;
+    const int nl = min(kLineGroup, n * n - line0);        // lines of this group
     const int64_t base0 = (int64_t)n * line0;
-    // stage: K, 1/C and the right-hand side -L U - E/C of every node (four
-    // nodes in flight per thread: the VGM chains are latency bound); K and
-    // 1/C come from memory when a coefficient pass already formed them at U
-#pragma unroll 4
-    for (int q = tid; q < nl * n; q += kZThreads) {
-        const int l = q / n, i = q % n;
-        const double u = U[base0 + q];
-        double k, ic;
-        if (Kin) { k = Kin[base0 + q]; ic = iCin[base0 + q]; }
-        else vgm_coefs(u, i * h, ksat, mode, k, ic);
-        sK[l][i] = k;
-        sIC[l][i] = ic;
-        sD[l][i] = (-L * u + (H ? H[base0 + q] : 0.0)) - (E ? ic * E[base0 + q] : 0.0);
-    }
-    __syncthreads();
-    const int l = tid & (kZLines - 1), sg = tid / kZLines;
-    const int N = n - 1;
-    const int Sg = (n + kZSeg - 1) / kZSeg;             // rows per segment (<= 8)
-    const int W = (n + Sg - 1) / Sg;
-    const int lo = sg * Sg, hi = min(n, lo + Sg) - 1;
-    const bool act = l < nl && lo <= hi;
-    const double top = (act && lo == 0) ? utop[line0 + l] : 0.0;
-    constexpr int S = 8;
-    double cp[S], xs[S], ys[S];
-    double zl = 0.0, cprev = 0.0, xprev = 0.0, yprev = 0.0;
+    const int W = (n + kSegRows - 1) / kSegRows;
+    const int total = nl * n;                             // <= kSegRows T
+    // this thread's elements tid + T k of the group's rows, line and row of each
+    const int dl = T / n, di = T % n, l_first = tid / n, i_first = tid % n;
+    auto elements = [&](auto&& f) {
+        int ll = l_first, ii = i_first;
 #pragma unroll
-    for (int j = 0; j < S; j++) {
-        const int i = lo + j;
-        const bool valid = act && i <= hi;
-        const bool inner = valid && i >= 1 && i <= N - 1;
-        const int ii = inner ? i : 1;
-        const double Km = inner ? sK[l][ii - 1] : 0.0, Kp = inner ? sK[l][ii] : 0.0;
-        const double icv = inner ? sIC[l][ii] : 0.0;
-        const double a = inner ? Km * icv * h2inv * kap : (i == N ? -1.0 : 0.0);
-        const double c = inner ? Kp * icv * h2inv * kap : 0.0;
-        const double b = inner ? -(icv * ((Kp * h2inv) + (Km * h2inv)) * kap + L) : 1.0;
-        const double d = inner ? sD[l][ii] : (i == 0 ? top : 0.0);
-        const double inv = rcp_nr(j == 0 ? b : b - a * cprev);
-        cp[j] = (valid && i < hi) ? c * inv : 0.0;
-        xs[j] = valid ? (j == 0 ? d : d - a * xprev) * inv : 0.0;
-        ys[j] = valid ? (j == 0 ? -a : -a * yprev) * inv : 0.0;
-        if (valid && i == hi) zl = -c * inv;
-        cprev = cp[j]; xprev = xs[j]; yprev = ys[j];
-    }
-    double xn = 0.0, yn = 0.0, zn = 0.0;
-#pragma unroll
-    for (int j = S - 1; j >= 0; j--) {
-        const int i = lo + j;
-        const bool valid = act && i <= hi;
-        const bool last = valid && i == hi;
-        xn = last ? xs[j] : xs[j] - cp[j] * xn;
-        yn = last ? ys[j] : ys[j] - cp[j] * yn;
-        zn = last ? zl : -cp[j] * zn;
-        xs[j] = xn; ys[j] = yn; cp[j] = zn;
-        if (valid && j == 0) { sEnd[sg][l][0] = xn; sEnd[sg][l][1] = yn; sEnd[sg][l][2] = zn; }
-        if (last) { sEnd[sg][l][3] = xn; sEnd[sg][l][4] = yn; sEnd[sg][l][5] = zn; }
-    }
-    __syncthreads();
-    if (act) {
-        double Fv[kZSeg], Gv[kZSeg], Pv[kZSeg], Qv[kZSeg];
-        double pv = 0.0, qv = 0.0;
-#pragma unroll
-        for (int k = 0; k < kZSeg; k++) {
-            if (k < W) {
-                const double Xf = sEnd[k][l][0], Yf = sEnd[k][l][1], Zf = sEnd[k][l][2];
-                const double Xl = sEnd[k][l][3], Yl = sEnd[k][l][4], Zl = sEnd[k][l][5];
-                const double inv = rcp_nr(1.0 - Yf * qv);
-                Fv[k] = (Xf + Yf * pv) * inv;
-                Gv[k] = Zf * inv;
-                const double yq = Yl * qv;
-                pv = Xl + Yl * pv + yq * Fv[k];
-                qv = yq * Gv[k] + Zl;
-                Pv[k] = pv; Qv[k] = qv;
-            }
+        for (int k = 0; k < kSegRows; k++) {
+            if (tid + T * k < total) f(k, ll, ii);
+            ll += dl;
+            ii += di;
+            if (ii >= n) { ii -= n; ll++; }
         }
-        double fr = 0.0, vr = 0.0, vl = 0.0;
+    };
+    // a field's values of this thread's rows (rows past the line and lines past
+    // the group: of the last one)
+    auto stage = [&](const double* src, double (&to)[kSegRows]) {
+        double t[kSegRows];
+        elements([&](int k, int, int) { t[k] = src[base0 + tid + T * k]; });
+        elements([&](int k, int ll, int ii) { sU[ll][ii] = t[k]; });
+        __syncthreads();
 #pragma unroll
-        for (int k = kZSeg - 1; k >= 0; k--) {
-            if (k < W) {
-                if (k == sg) vr = fr;
-                if (k == sg - 1) vl = Pv[k] + Qv[k] * fr;
-                fr = Fv[k] + Gv[k] * fr;
-            }
-        }
-        // this thread's rows of sD are read by no other thread: overwrite
-        // them with the solution
+        for (int j = 0; j < kSegRows; j++) to[j] = sU[min(l, nl - 1)][min(kSegRows * sg + j, n - 1)];
+    };
+    double u[kSegRows], r[kSegRows], k[kSegRows], ic[kSegRows], uold[kSegRows];
+    stage(V, u);
+    elements([&](int q, int, int) { uold[q] = U[base0 + tid + T * q]; });
+    if (Kin) {
+        __syncthreads();
+        stage(Kin, k);
+        __syncthreads();
+        stage(iCin, ic);
+    } else {
 #pragma unroll
-        for (int j = 0; j < S; j++) {
-            const int i = lo + j;
-            if (i <= hi) sD[l][i] = xs[j] + ys[j] * vl + cp[j] * vr;
-        }
+        for (int j = 0; j < kSegRows; j++)
+            vgm_coefs(u[j], min(kSegRows * sg + j, n - 1) * h, ksat, mode, k[j], ic[j]);
     }
+#pragma unroll
+    for (int j = 0; j < kSegRows; j++) r[j] = 0.0;
+    if (H) {
+        __syncthreads();
+        stage(H, r);
+    }
+    if (E) {
+        double e[kSegRows];
+        __syncthreads();
+        stage(E, e);
+#pragma unroll
+        for (int j = 0; j < kSegRows; j++) r[j] = fma(-ic[j], e[j], r[j]);
+    }
+    const double top = utop[line0 + min(l, nl - 1)];
+    double a[kSegRows], b[kSegRows], c[kSegRows], d[kSegRows], x[kSegRows];
+    line3d_rows(u, k, ic, r, n, l, sg, h2inv, lam, kap, true, top, L, a, b, c, d);
+    line3d_solve(a, b, c, d, l, sg, W, L, x);
+    // (every thread has read its staged rows: line3d_rows and line3d_solve synchronise)
+#pragma unroll
+    for (int j = 0; j < kSegRows; j++)
+        if (l < nl && kSegRows * sg + j < n) sU[l][kSegRows * sg + j] = x[j];
     __syncthreads();
-    for (int q = tid; q < nl * n; q += kZThreads) {
-        const int ll = q / n, i = q % n;
-        const double un = sD[ll][i];
-        const int64_t id = base0 + q;
-        const double up = Uprev[id];
-        U[id] = un;
-        Dlev[id] = un - up;
-        Uprev[id] = un;
-    }
+    elements([&](int q, int ll, int ii) {
+        const double un = sU[ll][ii];
+        U[base0 + tid + T * q] = un;
+        Dlev[base0 + tid + T * q] = un - uold[q];
+    });
 }
-__global__ __launch_bounds__(kZThreads, 2) void k_zline3d_seg(double* __restrict__ U, double* __restrict__ Uprev,
-                                                       const double* __restrict__ utop, int n, double h,
-                                                       double h2inv, double ksat, int mode, double L,
-                                                       double* __restrict__ Dlev, double kap,
-                                                       const double* __restrict__ E,
-                                                       const double* __restrict__ Kin,
-                                                       const double* __restrict__ iCin,
-                                                       const double* __restrict__ H) {
-    zline3d_seg_body(U, Uprev, utop, n, h, h2inv, ksat, mode, L, Dlev, kap, E, Kin, iCin, H, blockIdx.x);
+__global__ __launch_bounds__(kSegThreads, 4) void k_zline3d_seg(const double* V, double* U, const double* utop, int n,
+                                                                double h, double h2inv, double ksat, int mode,
+                                                                double lam, double* Dlev, double kap, const double* E,
+                                                                const double* Kin, const double* iCin,
+                                                                const double* H) {
+    zline3d_seg_body(V, U, utop, n, h, h2inv, ksat, mode, lam, Dlev, kap, E, Kin, iCin, H, blockIdx.x);
 }
 
 
@@ -589,33 +542,43 @@ __global__ __launch_bounds__(256) void k_hist_combine_batch(Lod3DBatch b) {
 
 // y sweep (axis 2) carries the history term; the x sweep (axis 1) a third of
 // it with split3d odd
-__global__ __launch_bounds__(256, 2) void k_lateral3d_batch(Lod3DBatch b, int axis) {
-    const int j = batch_slot(b.first_lat, b.count, blockIdx.x);
+__global__ __launch_bounds__(kSegThreads, 4) void k_lateral3d_batch(Lod3DBatch b, int axis) {
+    const int j = batch_slot(b.first_line, b.count, blockIdx.x);
     const Lod3DRow& r = b.row[j];
-    lateral3d_seg_body<16>(r.U, r.Kl, r.iCl, (axis == 2 || r.split) ? r.S : nullptr, r.n, axis, r.h2inv, r.L,
-                           r.kap, r.E, r.h, r.ksat, r.coef_mode, (int)blockIdx.x - b.first_lat[j]);
+    lateral3d_seg_body(axis == 2 ? r.U : r.V, r.V, r.Kl, r.iCl, (axis == 2 || r.split) ? r.S : nullptr, r.n, axis, r.h2inv, r.L,
+                           r.kap, r.E, r.h, r.ksat, r.coef_mode, (int)blockIdx.x - b.first_line[j]);
 }
 
-__global__ __launch_bounds__(kZThreads, 2) void k_zline3d_batch(Lod3DBatch b) {
-    const int j = batch_slot(b.first_z, b.count, blockIdx.x);
+__global__ __launch_bounds__(kSegThreads, 4) void k_zline3d_batch(Lod3DBatch b) {
+    const int j = batch_slot(b.first_line, b.count, blockIdx.x);
     const Lod3DRow& r = b.row[j];
-    zline3d_seg_body(r.U, r.Uprev, r.utop, r.n, r.h, r.h2inv, r.ksat, r.coef_mode, r.L, r.Dlev, r.kap, r.E,
-                     r.Kz, r.iCz, r.split ? r.S : nullptr, (int)blockIdx.x - b.first_z[j]);
+    zline3d_seg_body(r.V, r.U, r.utop, r.n, r.h, r.h2inv, r.ksat, r.coef_mode, r.L, r.Dlev, r.kap, r.E,
+                     r.Kz, r.iCz, r.split ? r.S : nullptr, (int)blockIdx.x - b.first_line[j]);
 }
+
+// threads of a workgroup of the partitioned sweeps (whole waves)
+static int seg_threads(int n) {
+    const int t = (n + kSegRows - 1) / kSegRows * kLineGroup;
+    return (t + 63) / 64 * 64;
+}
+static int seg_groups(int n) { return (n * n + kLineGroup - 1) / kLineGroup; }
 
 fpde_status launch_lod3d_batch(const Lod3DBatch& b, hipStream_t st) {
     if (b.count < 1 || b.count > kMax3DBatch) { set_error("batched 3D step: 1 to 8 solves"); return FPDE_ERR_ARG; }
-    for (int j = 0; j < b.count; j++)
-        if (b.row[j].n > 16 * kLatSeg || !(b.row[j].L > 0.0)) {
+    int T = 0;                                            // threads of the longest lines' segments
+    for (int j = 0; j < b.count; j++) {
+        if (!lateral3d_partitioned(b.row[j].n, b.row[j].L)) {
             set_error("batched 3D step: partitioned sweeps only (n <= 128)");
             return FPDE_ERR_ARG;
         }
-    const int gn = b.first_node[b.count], gl = b.first_lat[b.count], gz = b.first_z[b.count];
+        T = std::max(T, seg_threads(b.row[j].n));
+    }
+    const int gn = b.first_node[b.count], gl = b.first_line[b.count];
     // the lateral sweeps evaluate their coefficients themselves (rows' Kl, iCl null)
     hipLaunchKernelGGL(k_hist_combine_batch, dim3(gn), dim3(256), 0, st, b);
-    hipLaunchKernelGGL(k_lateral3d_batch, dim3(gl), dim3(256), 0, st, b, 2);
-    hipLaunchKernelGGL(k_lateral3d_batch, dim3(gl), dim3(256), 0, st, b, 1);
-    hipLaunchKernelGGL(k_zline3d_batch, dim3(gz), dim3(kZThreads), 0, st, b);
+    hipLaunchKernelGGL(k_lateral3d_batch, dim3(gl), dim3(T), 0, st, b, 2);
+    hipLaunchKernelGGL(k_lateral3d_batch, dim3(gl), dim3(T), 0, st, b, 1);
+    hipLaunchKernelGGL(k_zline3d_batch, dim3(gl), dim3(T), 0, st, b);
     FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
 }
@@ -634,33 +597,33 @@ fpde_status launch_coef3d(const double* U, int n, double h, double ksat, int mod
     return FPDE_OK;
 }
 
-fpde_status launch_lateral3d(double* U, const double* K, const double* iC, const double* H, int n,
+fpde_status launch_lateral3d(const double* Uin, double* Uout, const double* K, const double* iC, const double* H, int n,
                              int axis, double h2inv, double L, double* Al, double* Bt, double kap,
                              const double* E, double h, double ksat, int mode, hipStream_t st) {
     int nl = n * n;
-    if (lateral3d_partitioned(n, L)) {   // 8 segments of <= 16 rows per line
-        hipLaunchKernelGGL(k_lateral3d_seg<16>, dim3((nl + 31) / 32), dim3(256), 0, st, U, K, iC, H, n, axis, h2inv,
-                           L, kap, E, h, ksat, mode);
+    if (lateral3d_partitioned(n, L)) {
+        hipLaunchKernelGGL(k_lateral3d_seg, dim3(seg_groups(n)), dim3(seg_threads(n)), 0, st, Uin, Uout, K, iC, H, n,
+                           axis, h2inv, L, kap, E, h, ksat, mode);
         return FPDE_OK;
     }
     if (!K || !iC) { set_error("3D lateral sweep over 128 nodes needs the coefficient pass"); return FPDE_ERR_ARG; }
-    hipLaunchKernelGGL(k_lateral3d, dim3((nl + 255) / 256), dim3(256), 0, st, U, K, iC, H, n, axis, h2inv, L, Al, Bt,
-                       kap, E);
+    hipLaunchKernelGGL(k_lateral3d, dim3((nl + 255) / 256), dim3(256), 0, st, Uin, Uout, K, iC, H, n, axis, h2inv, L,
+                       Al, Bt, kap, E);
     return FPDE_OK;
 }
 
-fpde_status launch_zline3d(double* U, double* Uprev, const double* utop, int n, double h, double h2inv,
+fpde_status launch_zline3d(const double* V, double* U, const double* utop, int n, double h, double h2inv,
                            double ksat, int mode, double L, double* Dlev, double kap, const double* E,
                            const double* K, const double* iC, const double* H, hipStream_t st) {
     if (n > 256) { set_error("3D grid: at most 256 nodes per axis"); return FPDE_ERR_ARG; }
-    if (n <= 8 * kZSeg && L > 0.0) {        // partitioned: 16 lines per workgroup, 16 segments of <= 8 rows
-        hipLaunchKernelGGL(k_zline3d_seg, dim3((n * n + kZLines - 1) / kZLines), dim3(kZThreads), 0, st, U, Uprev, utop, n,
-                           h, h2inv, ksat, mode, L, Dlev, kap, E, K, iC, H);
+    if (lateral3d_partitioned(n, L)) {
+        hipLaunchKernelGGL(k_zline3d_seg, dim3(seg_groups(n)), dim3(seg_threads(n)), 0, st, V, U, utop, n, h, h2inv,
+                           ksat, mode, L, Dlev, kap, E, K, iC, H);
         return FPDE_OK;
     }
     int bs = ((n + 63) / 64) * 64;
-    hipLaunchKernelGGL(k_zline3d, dim3(n * n), dim3(bs), 0, st, U, Uprev, utop, n, h, h2inv, ksat, mode, L, Dlev,
-                       kap, E, H);
+    hipLaunchKernelGGL(k_zline3d, dim3(n * n), dim3(bs), 0, st, V, U, utop, n, h, h2inv, ksat, mode, L, Dlev, kap, E,
+                       H);
     return FPDE_OK;
 }
 

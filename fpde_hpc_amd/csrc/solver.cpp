@@ -166,7 +166,7 @@ size_t footprint_bytes(const fpde_spec& s) {
     b += sizeof(double) * (size_t)p.ld * 8;                      // U, S, xyz, ...
     if (s.hist_mode != HIST_PLAIN_F64 && s.sum_alg != 2)
         b += sizeof(double) * (size_t)s.block * p.ld;                 // folded near-field groups
-    if (s.dims == 3) b += sizeof(double) * (size_t)p.ld * 6;     // Uprev, K, iC, Al, Bt
+    if (s.dims == 3) b += sizeof(double) * (size_t)p.ld * 6;     // V, K, iC, Al, Bt
     b += sizeof(double) * (size_t)(s.steps + 512) * 3;           // weights
     if (s.sum_alg == 2) {
         size_t P = (size_t)s.sum_param;
@@ -234,7 +234,7 @@ struct fpde_solver {
     void* afrag = nullptr;       // A fragments of a split GEMM block
     double* ainv = nullptr;
     // 3D
-    double* Uprev = nullptr;
+    double* V = nullptr;      // the field between the sweeps of a 3D step
     double* utop = nullptr;
     double* K = nullptr;
     double* iC = nullptr;
@@ -444,7 +444,7 @@ fpde_status solver_alloc(fpde_solver* s) {
             DALLOC(s->w.sp_corr, sizeof(double) * 2 * (size_t)n);
             DALLOC(s->spE, sizeof(double) * p.ld);
         }
-        DALLOC(s->Uprev, sizeof(double) * p.ld);
+        DALLOC(s->V, sizeof(double) * p.ld);
         DALLOC(s->utop, sizeof(double) * (size_t)n * n);
         DALLOC(s->K, sizeof(double) * p.ld);
         DALLOC(s->iC, sizeof(double) * p.ld);
@@ -1054,8 +1054,8 @@ fpde_status enqueue_3d_step(fpde_solver* s, int n) {
     const bool space = s->w.sp_on;
     const double kap = space ? s->w.sp_kap : 1.0;
     double* E = space ? s->spE : nullptr;
-    auto space_sums = [&](int axis) {
-        return space ? launch_space3d(s->U, s->K, nn, axis, s->h, s->w.sp_omega, s->w.sp_corr, s->spE, s->stream)
+    auto space_sums = [&](const double* field, int axis) {
+        return space ? launch_space3d(field, s->K, nn, axis, s->h, s->w.sp_omega, s->w.sp_corr, s->spE, s->stream)
                      : FPDE_OK;
     };
     // local coefficient of this step: per step on a grid (generalized kernel)
@@ -1066,23 +1066,25 @@ fpde_status enqueue_3d_step(fpde_solver* s, int n) {
     const bool pass = space || !lateral3d_partitioned(nn, Lc);
     const double* Kc = pass ? s->K : nullptr;
     const double* iCc = pass ? s->iC : nullptr;
-    auto coef_pass = [&]() {
-        return pass ? launch_coef3d(s->U, nn, s->h, sp.ksat, sp.coef_mode, s->K, s->iC, s->stream) : FPDE_OK;
+    auto coef_pass = [&](const double* field) {
+        return pass ? launch_coef3d(field, nn, s->h, sp.ksat, sp.coef_mode, s->K, s->iC, s->stream) : FPDE_OK;
     };
-    if ((rc = coef_pass()) != FPDE_OK) return rc;
-    if ((rc = space_sums(2)) != FPDE_OK) return rc;
-    if ((rc = launch_lateral3d(s->U, Kc, iCc, s->S, nn, 2, h2inv, Lc, s->Al, s->Bt, kap, E, s->h, sp.ksat,
+    // the y sweep goes from U to V, the x sweep stays in V, the depth sweep
+    // returns to U, which holds U^n until then
+    if ((rc = coef_pass(s->U)) != FPDE_OK) return rc;
+    if ((rc = space_sums(s->U, 2)) != FPDE_OK) return rc;
+    if ((rc = launch_lateral3d(s->U, s->V, Kc, iCc, s->S, nn, 2, h2inv, Lc, s->Al, s->Bt, kap, E, s->h, sp.ksat,
                                sp.coef_mode, s->stream)) != FPDE_OK) return rc;
-    if ((rc = coef_pass()) != FPDE_OK) return rc;
-    if ((rc = space_sums(1)) != FPDE_OK) return rc;
-    if ((rc = launch_lateral3d(s->U, Kc, iCc, split ? s->S : nullptr, nn, 1, h2inv, Lc, s->Al, s->Bt, kap, E, s->h,
+    if ((rc = coef_pass(s->V)) != FPDE_OK) return rc;
+    if ((rc = space_sums(s->V, 1)) != FPDE_OK) return rc;
+    if ((rc = launch_lateral3d(s->V, s->V, Kc, iCc, split ? s->S : nullptr, nn, 1, h2inv, Lc, s->Al, s->Bt, kap, E, s->h,
                                sp.ksat, sp.coef_mode, s->stream)) != FPDE_OK) return rc;
     if (space) {
-        if ((rc = launch_coef3d(s->U, nn, s->h, sp.ksat, sp.coef_mode, s->K, s->iC, s->stream)) != FPDE_OK) return rc;
-        if ((rc = space_sums(0)) != FPDE_OK) return rc;
+        if ((rc = launch_coef3d(s->V, nn, s->h, sp.ksat, sp.coef_mode, s->K, s->iC, s->stream)) != FPDE_OK) return rc;
+        if ((rc = space_sums(s->V, 0)) != FPDE_OK) return rc;
     }
     // the depth sweep reuses the coefficient pass of the space-fractional sums
-    if ((rc = launch_zline3d(s->U, s->Uprev, s->utop, nn, s->h, h2inv, sp.ksat, sp.coef_mode, Lc,
+    if ((rc = launch_zline3d(s->V, s->U, s->utop, nn, s->h, h2inv, sp.ksat, sp.coef_mode, Lc,
                              s->D + (size_t)(series ? (n & 1) : n) * p.ld, kap, E, space ? s->K : nullptr,
                              space ? s->iC : nullptr, split ? s->S : nullptr, s->stream)) != FPDE_OK) return rc;
     ev_end(s, slot);
@@ -1149,7 +1151,7 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
             s->stream = own;
             if (rc != FPDE_OK) break;
             Lod3DRow& r = b.row[k];
-            r.U = s->U; r.S = s->S; r.Uprev = s->Uprev;
+            r.U = s->U; r.S = s->S; r.V = s->V;
             r.Dlev = s->D + (size_t)n * p.ld;
             r.part = s->part; r.D = s->D;
             const HistRows hr = hist_rows(s, n);
@@ -1164,8 +1166,7 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
             r.kap = 1.0; r.E = nullptr; r.Kz = nullptr; r.iCz = nullptr; r.Kl = nullptr; r.iCl = nullptr;
             const int lines = sp.nodes * sp.nodes;
             b.first_node[k + 1] = b.first_node[k] + (int)((p.nodes + 255) / 256);
-            b.first_lat[k + 1] = b.first_lat[k] + (lines + 31) / 32;
-            b.first_z[k + 1] = b.first_z[k] + (lines + kZLinesHost - 1) / kZLinesHost;
+            b.first_line[k + 1] = b.first_line[k] + (lines + kLinesHost3D - 1) / kLinesHost3D;
             k++;
         }
         if (rc != FPDE_OK || k == 0) break;
@@ -1321,7 +1322,6 @@ fpde_status fpde_solver_set_initial(fpde_solver* s, const double* u0) {
         std::vector<double> top((size_t)n * n);
         for (int y = 0; y < n; y++)
             for (int x = 0; x < n; x++) top[(size_t)y * n + x] = u0[(size_t)n * (x + (size_t)n * y)];
-        FPDE_HIP_TRY(hipMemcpyAsync(s->Uprev, s->U, sizeof(double) * p.ld, hipMemcpyDeviceToDevice, s->stream));
         FPDE_HIP_TRY(hipMemcpyAsync(s->utop, top.data(), sizeof(double) * top.size(), hipMemcpyHostToDevice, s->stream));
         s->u0_h.assign(u0, u0 + p.nodes);
     }

@@ -743,6 +743,21 @@ def test_advance_batch_refuses_what_does_not_fit(fpde):
             s.close()
 
 
+@pytest.mark.parametrize("n", [4, 7, 8, 9, 16, 17, 63, 65, 120, 121, 128])
+def test_partitioned_sweeps_edges_match_oracle(fpde, oracle, n):
+    """The partitioned sweeps at their edges: one segment of 8 rows and less,
+    a last segment of one row and of all, the last group of 16 lines cut short,
+    16 segments, and coefficients from a pass (space-fractional)."""
+    u0 = fpde.init_3d(n, 1100 + n)
+    for gamma in (0.0, 0.7):
+        spec = fpde.make_spec(n, 4, 1e-3, alpha=0.85, dims=3, hist_mode="plain", u_top=u0[0], gamma=gamma)
+        ref = _oracle_space3d(oracle, spec, u0) if gamma else oracle.solve_3d(
+            oracle.make_params(n, 4, 1e-3, 0.85, ksat=spec.ksat), u0)
+        err = rel_err(fpde.solve(spec, u0), ref)
+        print(f"3D sweeps n={n} gamma={gamma}: rel err {err:.3e}", flush=True)
+        assert err <= TOL_F64
+
+
 def test_batched_3d_steps_equal_solo(fpde):
     """3D solves of different sizes, orders, history forms and block sizes
     (one with split3d odd, one with the generalized kernel FK 3) advance in
