@@ -481,7 +481,7 @@ fpde_status fpde_history_sum_f64(double* S, const double* D, int64_t n, int64_t 
     rc = launch_hist_plain(D, ld, (int)nodes, (int)n, (int)n, omega, part, &splits, 0);
     if (rc == FPDE_OK) {
         // combine: S = sum of partial rows (no near levels, no corrections)
-        rc = launch_hist_combine(S, part, splits, ld, 0, D, ld, nodes, 0, 0, omega, 0, 0, 0, nullptr, nullptr, 1.0, 0);
+        rc = launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, 0);
     }
     hipError_t e = hipDeviceSynchronize();
     if (rc != FPDE_OK) return rc;

@@ -142,47 +142,13 @@ __host__ __device__ inline void vgm_coefs(double u, double z, double ksat, int m
     }
 }
 
-// Near-field history folded ahead in groups of 16 levels (1D cooperative
-// step, 3D history combine): the group [lo, lo + 16) of node i goes into
-// mid for the steps p in [p_lo, p_hi) of the history block that starts at
-// step n0:
-//   mid[p - n0][i] = (first ? 0 : mid[p - n0][i]) + sum_k w_p[p - lo - k - 1] D[lo + k][i],
-// w_p = omega + (p - n0) * omega_stride (one Toeplitz vector, stride 0, or
-// the step's own row).  The steps go in 8-wide batches: their mid values
-// load together, then the sums.
+// Near-field history folded ahead by the 1D cooperative step in groups of 16
+// levels: group [lo, lo + 16) of node i goes into mid for steps p of the
+// history block that starts at step n0,
+//   mid[p - n0][i] += sum_k w_p[p - lo - k - 1] D[lo + k][i],
+// kFoldBatch steps at a time.
 constexpr int kNearGroup = 16;
 constexpr int kFoldBatch = 8;
-__device__ inline void fold_near_group(const double* __restrict__ D, int64_t ld, const double* __restrict__ omega,
-                                       int64_t omega_stride, int n0, double* __restrict__ mid, int64_t i, int lo,
-                                       int p_lo, int p_hi, bool first) {
-    double dv[kNearGroup];
-#pragma unroll
-    for (int k = 0; k < kNearGroup; k++) dv[k] = D[(int64_t)(lo + k) * ld + i];
-    constexpr int PB = kFoldBatch;
-    for (int p0 = p_lo; p0 < p_hi; p0 += PB) {
-        double acc[PB];
-#pragma unroll
-        for (int j = 0; j < PB; j++) {
-            const int p = p0 + j;
-            acc[j] = (!first && p < p_hi) ? mid[(int64_t)(p - n0) * ld + i] : 0.0;
-        }
-#pragma unroll
-        for (int j = 0; j < PB; j++) {
-            const int p = p0 + j;
-            if (p < p_hi) {
-                const double* om = omega + (int64_t)(p - n0) * omega_stride + (p - lo - 1);
-#pragma unroll
-                for (int k = 0; k < kNearGroup; k++) acc[j] = fma(om[-k], dv[k], acc[j]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < PB; j++) {
-            const int p = p0 + j;
-            if (p < p_hi) mid[(int64_t)(p - n0) * ld + i] = acc[j];
-        }
-    }
-}
-
 // one DPP move of a double (both 32-bit halves) inside the rows of 16 lanes
 template <int CTRL>
 __device__ inline double dpp_move(double v) {
@@ -573,13 +539,15 @@ fpde_status launch_ref_series(double* S, const double* old, int64_t old_size, in
 // has folded them into P[0].
 fpde_status launch_gemm_f64(const double* D, int64_t ld, int nodes, int n0, int tc, int block,
                             const double* omega, double* P, int* splits_out, hipStream_t st,
-                            int max_splits = 0);
+                            int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);
 fpde_status launch_part_reduce(double* P, int splits, int rows, int64_t ld, int nodes, hipStream_t st);
 fpde_status launch_pack_split(int mode, const double* D, int64_t ld, int nodes, int g_lo, int g_hi, void* c0,
                               void* c1, void* c2, float* scale, hipStream_t st);
 fpde_status launch_gemm_f64_dense(const double* D, int64_t ld, int nodes, int tc, int block, const double* W,
                                   int64_t ldw, double* P, int* splits_out, hipStream_t st,
-                                  int max_splits = 0);
+                                  int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);
+// corr (of the block's first step, with D0 the first two levels): the two-level
+// corrections added to the rows as well.
 // W != nullptr: dense weight rows W[r][t] (leading dimension ldw >= tc) of a
 // prescribed grid in place of the Toeplitz vector omega.  afrag / ainv:
 // workspace of split_afrag_bytes(mode, block, tc / 32) bytes and
@@ -588,7 +556,7 @@ size_t split_afrag_bytes(int mode, int block, int groups);
 fpde_status launch_gemm_split(int mode, const void* c0, const void* c1, const void* c2, const float* scale,
                               int64_t ld, int nodes, int n0, int tc, int block, const double* omega,
                               const double* W, int64_t ldw, void* afrag, double* ainv, double* P,
-                              int* splits_out, hipStream_t st, int max_splits = 0);
+                              int* splits_out, hipStream_t st, int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);
 // the same GEMM from the FP64 levels themselves (no packed components), and
 // the sum of its partial rows into P [rows][ld]
 fpde_status launch_gemm_split_direct(int mode, const double* D, int64_t ld, int nodes, int n0, int tc, int block,
@@ -600,6 +568,28 @@ fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st);
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st);
 bool step1d_block_supported(int N, int C);
 bool step1d_batch_supported(int64_t wgs);
+// History term of a 3D step: S = partial rows + near levels [lo, n) + two-level
+// corrections (corr: of step n; null where the partial rows hold them).
+struct Hist3D {
+    const double* part;        // this step's row of K split 0
+    int64_t part_stride;
+    int rows;                  // partial rows
+    const double* D;
+    int64_t ld;
+    int n, lo;
+    const double* omega;       // of step n: weight of level t at n - t - 1
+    const double* corr;        // at 2 n
+};
+// One fold of near levels [lo, lo + len) into the partial rows of the steps
+// [p_lo, p_hi) (first: nothing in those rows yet)
+struct Fold3D {
+    const double* D;
+    int64_t ld, nodes;
+    const double* omega;       // weight row of the block's first step n0
+    int64_t omega_stride;
+    double* part;              // row of step n0
+    int n0, lo, len, p_lo, p_hi, first;
+};
 // Batched 3D LOD step: one step of up to kMax3DBatch 3D solves (n <= 128,
 // partitioned sweeps) in one launch per kernel of the step (history combine,
 // coefficients, y sweep, coefficients, x sweep, z sweep).  Workgroups
@@ -608,13 +598,10 @@ bool step1d_batch_supported(int64_t wgs);
 constexpr int kMax3DBatch = 8;
 struct Lod3DRow {
     double *U, *S, *V, *Dlev;
-    const double *part, *D, *omega, *corr, *utop;
-    int64_t part_stride, part_off, ld, nodes;
-    int n, nsplit, step, near_lo, coef_mode, split;
-    // history block: first step, rows, weight-row stride, folded near groups
-    int n0, blk;
-    int64_t omega_stride;
-    double* mid;
+    const double* utop;
+    Hist3D hist;
+    int64_t nodes;
+    int n, coef_mode, split;
     double h, h2inv, ksat, L, hscale;
     // arguments the solo sweeps take that a batched solve leaves at their
     // neutral values: kap = 1 and no line sums E (no space-fractional term),
@@ -631,6 +618,11 @@ struct Lod3DBatch {
     int first_node[kMax3DBatch + 1];   // 256-node blocks (history combine, coefficients)
     int first_line[kMax3DBatch + 1];   // groups of kLinesHost3D lines (sweeps)
     Lod3DRow row[kMax3DBatch];
+};
+struct Fold3DBatch {
+    int count;
+    int first[kMax3DBatch + 1];        // 256-node blocks
+    Fold3D row[kMax3DBatch];
 };
 fpde_status launch_lod3d_batch(const Lod3DBatch& b, hipStream_t st);
 constexpr int kLinesHost3D = 16;     // lines per workgroup of the partitioned sweeps
@@ -721,15 +713,9 @@ fpde_status launch_space3d(const double* U, const double* K, int n, int axis, do
                            const double* sp_corr, double* E, hipStream_t st);
 fpde_status launch_series3d(double* S, double* H, int P, const double* dnew, const double* ser_c,
                             const double* ser_v, int64_t nodes, int64_t ld, double hscale, hipStream_t st);
-// 3D history term of step n (far partials, near levels [near_lo, n),
-// corrections); omega is the weight row of the block's first step n0 (rows
-// omega_stride apart on a prescribed grid, else one Toeplitz vector); with
-// mid (a block of blk rows) the near levels go in 16-level groups folded
-// ahead, each at the step that completes it.
-fpde_status launch_hist_combine(double* S, const double* part, int nsplit, int64_t part_stride, int64_t part_off,
-                                const double* D, int64_t ld, int64_t nodes, int n, int near_lo,
-                                const double* omega, int64_t omega_stride, int n0, int blk, double* mid,
-                                const double* corr, double hscale, hipStream_t st);
+// 3D history term of a step, and the folds that go before it
+fpde_status launch_hist_combine(double* S, const Hist3D& h, int64_t nodes, double hscale, hipStream_t st);
+fpde_status launch_fold3d(const Fold3DBatch& b, hipStream_t st);
 int gemm_max_splits(int64_t nodes);
 
 }  // namespace fpde

@@ -194,6 +194,21 @@ typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
 
+// The two-level corrections corr[2 (n0+r)] D[0] + corr[2 (n0+r)+1] D[1] of a
+// block's rows, added to the partial rows of K split 0 (3D: the step then
+// reads neither level; corr null: the step kernel adds them itself).
+struct GemmCorr {
+    const double* corr;        // at 2 n0
+    double d0, d1;
+    __device__ GemmCorr(const double* c, const double* D0, int64_t ld, int ks, int64_t node, bool ok)
+        : corr(ks == 0 ? c : nullptr), d0(0.0), d1(0.0) {
+        if (corr && ok) { d0 = D0[node]; d1 = D0[ld + node]; }
+    }
+    __device__ double operator()(int r, double acc) const {
+        return corr ? fma(corr[2 * r + 1], d1, fma(corr[2 * r], d0, acc)) : acc;
+    }
+};
+
 // FP64 time-block GEMM.  Grid: x = 64-node tiles, y = K splits (t-chunks).
 // Block 256 = 4 waves; wave w owns nodes [16w,16w+16) of the tile and all BR
 // rows (BR/16 MFMA tiles).  v_mfma_f64_16x16x4f64 operand layout (checked
@@ -204,7 +219,8 @@ template <int BR>
 __global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, int64_t ld, int nodes,
                                                   int n0, int tc, int kchunk,
                                                   const double* __restrict__ omega,
-                                                  double* __restrict__ P) {
+                                                  double* __restrict__ P,
+                                                    const double* __restrict__ corr, const double* __restrict__ D0) {
     constexpr int RT = BR / 16;
     constexpr int SLAB = 1024;                  // t-values per LDS weight window
     __shared__ double win[BR + SLAB];
@@ -255,13 +271,14 @@ __global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, 
             }
         }
     }
+    const GemmCorr add(corr, D0, ld, ks, node, node_ok);
     if (node_ok) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 int r = rt * 16 + 4 * v + (lane >> 4);
-                P[((int64_t)ks * BR + r) * ld + node] = acc[rt][v];
+                P[((int64_t)ks * BR + r) * ld + node] = add(r, acc[rt][v]);
             }
         }
     }
@@ -274,7 +291,8 @@ __global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, 
 template <int BR>
 __global__ __launch_bounds__(256) void k_gemm_f64_dense(const double* __restrict__ D, int64_t ld, int nodes,
                                                         int tc, int kchunk, const double* __restrict__ W,
-                                                        int64_t ldw, double* __restrict__ P) {
+                                                        int64_t ldw, double* __restrict__ P,
+                                                    const double* __restrict__ corr, const double* __restrict__ D0) {
     constexpr int RT = BR / 16;
     constexpr int SL = 64;
     __shared__ double win[BR][SL + 1];
@@ -316,13 +334,14 @@ __global__ __launch_bounds__(256) void k_gemm_f64_dense(const double* __restrict
             }
         }
     }
+    const GemmCorr add(corr, D0, ld, ks, node, node_ok);
     if (node_ok) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 int r = rt * 16 + 4 * v + (lane >> 4);
-                P[((int64_t)ks * BR + r) * ld + node] = acc[rt][v];
+                P[((int64_t)ks * BR + r) * ld + node] = add(r, acc[rt][v]);
             }
         }
     }
@@ -480,7 +499,8 @@ __global__ __launch_bounds__(256) void k_gemm_split(const T* __restrict__ c0, co
                                                     int nodes, int tc, int kchunk,
                                                     const typename SplitTraits<T>::vec* __restrict__ afrag_g,
                                                     const double* __restrict__ ainv_g,
-                                                    double* __restrict__ P) {
+                                                    double* __restrict__ P,
+                                                    const double* __restrict__ corr, const double* __restrict__ D0) {
     typedef typename SplitTraits<T>::vec vec_t;
     constexpr int RT = BR / 16;
     constexpr int GB = 4;                                  // groups per LDS batch
@@ -565,13 +585,14 @@ __global__ __launch_bounds__(256) void k_gemm_split(const T* __restrict__ c0, co
             }
         }
     }
+    const GemmCorr add(corr, D0, ld, ks, node, node_ok);
     if (node_ok) {
 #pragma unroll
         for (int rt = 0; rt < RT; rt++) {
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 int r = rt * 16 + 4 * (lane >> 4) + v;
-                P[((int64_t)ks * BR + r) * ld + node] = acc[rt][v];
+                P[((int64_t)ks * BR + r) * ld + node] = add(r, acc[rt][v]);
             }
         }
     }
@@ -851,16 +872,17 @@ static void gemm_split_plan(int tc, int64_t nodes, int* kchunk, int* splits, int
 }
 
 fpde_status launch_gemm_f64_dense(const double* D, int64_t ld, int nodes, int tc, int block, const double* W,
-                                  int64_t ldw, double* P, int* splits_out, hipStream_t st, int max_splits) {
+                                  int64_t ldw, double* P, int* splits_out, hipStream_t st, int max_splits, const double* corr,
+                              const double* D0) {
     if (tc <= 0) { *splits_out = 0; return FPDE_OK; }
     int kchunk, splits;
     gemm_split_plan(tc, nodes, &kchunk, &splits, max_splits);
     dim3 grid((unsigned)((nodes + 63) / 64), (unsigned)splits);
     switch (block) {
-        case 16: hipLaunchKernelGGL(k_gemm_f64_dense<16>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P); break;
-        case 32: hipLaunchKernelGGL(k_gemm_f64_dense<32>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P); break;
-        case 64: hipLaunchKernelGGL(k_gemm_f64_dense<64>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P); break;
-        case 128: hipLaunchKernelGGL(k_gemm_f64_dense<128>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P); break;
+        case 16: hipLaunchKernelGGL(k_gemm_f64_dense<16>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P, corr, D0); break;
+        case 32: hipLaunchKernelGGL(k_gemm_f64_dense<32>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P, corr, D0); break;
+        case 64: hipLaunchKernelGGL(k_gemm_f64_dense<64>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P, corr, D0); break;
+        case 128: hipLaunchKernelGGL(k_gemm_f64_dense<128>, grid, dim3(256), 0, st, D, ld, nodes, tc, kchunk, W, ldw, P, corr, D0); break;
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
     *splits_out = splits;
@@ -869,17 +891,18 @@ fpde_status launch_gemm_f64_dense(const double* D, int64_t ld, int nodes, int tc
 }
 
 fpde_status launch_gemm_f64(const double* D, int64_t ld, int nodes, int n0, int tc, int block,
-                            const double* omega, double* P, int* splits_out, hipStream_t st, int max_splits) {
+                            const double* omega, double* P, int* splits_out, hipStream_t st, int max_splits, const double* corr,
+                              const double* D0) {
     if (tc <= 0) { *splits_out = 0; return FPDE_OK; }
     int kchunk, splits;
     gemm_split_plan(tc, nodes, &kchunk, &splits, max_splits);
     dim3 grid((nodes + 63) / 64, splits);
     size_t lds = 0;
     switch (block) {
-        case 16: hipLaunchKernelGGL(k_gemm_f64<16>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P); break;
-        case 32: hipLaunchKernelGGL(k_gemm_f64<32>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P); break;
-        case 64: hipLaunchKernelGGL(k_gemm_f64<64>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P); break;
-        case 128: hipLaunchKernelGGL(k_gemm_f64<128>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P); break;
+        case 16: hipLaunchKernelGGL(k_gemm_f64<16>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P, corr, D0); break;
+        case 32: hipLaunchKernelGGL(k_gemm_f64<32>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P, corr, D0); break;
+        case 64: hipLaunchKernelGGL(k_gemm_f64<64>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P, corr, D0); break;
+        case 128: hipLaunchKernelGGL(k_gemm_f64<128>, grid, dim3(256), lds, st, D, ld, nodes, n0, tc, kchunk, omega, P, corr, D0); break;
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
     *splits_out = splits;
@@ -909,7 +932,8 @@ fpde_status launch_pack_split(int mode, const double* D, int64_t ld, int nodes, 
 template <typename T, int NS, int BR>
 static void gemm_split_t(dim3 grid, hipStream_t st, const void* c0, const void* c1, const void* c2,
                          const float* scale, int64_t ld, int nodes, int n0, int tc, int kchunk,
-                         const double* omega, const double* W, int64_t ldw, void* afrag, double* ainv, double* P) {
+                         const double* omega, const double* W, int64_t ldw, void* afrag, double* ainv, double* P,
+                         const double* corr, const double* D0) {
     typedef typename SplitTraits<T>::vec vec_t;
     if (W)
         hipLaunchKernelGGL((k_afrag_split<T, NS, BR, true>), dim3(tc / kGroup), dim3(256), 0, st, n0, omega, W, ldw,
@@ -918,19 +942,19 @@ static void gemm_split_t(dim3 grid, hipStream_t st, const void* c0, const void* 
         hipLaunchKernelGGL((k_afrag_split<T, NS, BR, false>), dim3(tc / kGroup), dim3(256), 0, st, n0, omega, W, ldw,
                            (vec_t*)afrag, ainv);
     hipLaunchKernelGGL((k_gemm_split<T, NS, BR>), grid, dim3(256), 0, st, (const T*)c0, (const T*)c1, (const T*)c2,
-                       scale, ld, nodes, tc, kchunk, (const vec_t*)afrag, (const double*)ainv, P);
+                       scale, ld, nodes, tc, kchunk, (const vec_t*)afrag, (const double*)ainv, P, corr, D0);
 }
 
 template <typename T, int NS>
 static fpde_status gemm_split_b(int block, dim3 grid, hipStream_t st, const void* c0, const void* c1,
                                 const void* c2, const float* scale, int64_t ld, int nodes, int n0,
                                 int tc, int kchunk, const double* omega, const double* W, int64_t ldw,
-                                void* afrag, double* ainv, double* P) {
+                                void* afrag, double* ainv, double* P, const double* corr, const double* D0) {
     switch (block) {
-        case 16: gemm_split_t<T, NS, 16>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
-        case 32: gemm_split_t<T, NS, 32>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
-        case 64: gemm_split_t<T, NS, 64>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
-        case 128: gemm_split_t<T, NS, 128>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
+        case 16: gemm_split_t<T, NS, 16>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
+        case 32: gemm_split_t<T, NS, 32>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
+        case 64: gemm_split_t<T, NS, 64>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
+        case 128: gemm_split_t<T, NS, 128>(grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
     return FPDE_OK;
@@ -986,7 +1010,8 @@ size_t split_afrag_bytes(int mode, int block, int groups) {
 fpde_status launch_gemm_split(int mode, const void* c0, const void* c1, const void* c2,
                               const float* scale, int64_t ld, int nodes, int n0, int tc, int block,
                               const double* omega, const double* W, int64_t ldw, void* afrag, double* ainv,
-                              double* P, int* splits_out, hipStream_t st, int max_splits) {
+                              double* P, int* splits_out, hipStream_t st, int max_splits, const double* corr,
+                              const double* D0) {
     if (tc <= 0) { *splits_out = 0; return FPDE_OK; }
     if (tc % kGroup != 0) { set_error("split GEMM needs a group-aligned cut"); return FPDE_ERR_ARG; }
     if (W && ldw < tc) { set_error("split GEMM: dense weight rows shorter than the cut"); return FPDE_ERR_ARG; }
@@ -996,9 +1021,9 @@ fpde_status launch_gemm_split(int mode, const void* c0, const void* c1, const vo
     dim3 grid((nodes + 63) / 64, splits);
     fpde_status rc;
     switch (mode) {
-        case HIST_SPLIT_BF16: rc = gemm_split_b<__bf16, 2>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
-        case HIST_SPLIT_F16: rc = gemm_split_b<_Float16, 2>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
-        case HIST_SPLIT_BF16X3: rc = gemm_split_b<__bf16, 3>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P); break;
+        case HIST_SPLIT_BF16: rc = gemm_split_b<__bf16, 2>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
+        case HIST_SPLIT_F16: rc = gemm_split_b<_Float16, 2>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
+        case HIST_SPLIT_BF16X3: rc = gemm_split_b<__bf16, 3>(block, grid, st, c0, c1, c2, scale, ld, nodes, n0, tc, kchunk, omega, W, ldw, afrag, ainv, P, corr, D0); break;
         default: set_error("bad split mode"); return FPDE_ERR_ARG;
     }
     *splits_out = splits;

@@ -439,74 +439,143 @@ __global__ __launch_bounds__(kSegThreads, 4) void k_zline3d_seg(const double* V,
 }
 
 
-// S[i] = sum of far partials + near levels [near_lo, n) + two-level corrections,
-// times hscale (1, or 1/3 when every sweep carries a third of the term).
-// omega is the weight row of the block's first step n0 (rows omega_stride
-// apart).  With mid, the 16-level groups [near_lo + 16 j, +16) of the near
-// field are folded into mid for the steps [s, n0 + blk) at the step s that
-// completes them (the block's first step folds those already complete), and
-// step n takes the complete groups as one mid value plus the levels after
-// them.
-__device__ __forceinline__ void hist_combine_body(double* __restrict__ S, const double* __restrict__ part,
-                                                  int nsplit, int64_t part_stride, int64_t part_off,
-                                                  const double* __restrict__ D, int64_t ld, int64_t nodes, int n,
-                                                  int near_lo, const double* __restrict__ omega_blk,
-                                                  int64_t omega_stride, int n0, int blk, double* __restrict__ mid,
-                                                  const double* __restrict__ corr, double hscale, int bid) {
-    const double* __restrict__ omega = omega_blk + (int64_t)(n - n0) * omega_stride;
-    int64_t i = (int64_t)bid * 256 + threadIdx.x;
-    if (i >= nodes) return;
-    constexpr int W = 16;      // independent loads per batch
-    double far = 0.0;
-    for (int sp0 = 0; sp0 < nsplit; sp0 += W) {
-        double v[W];
+// History term of NV nodes (id: their indexes): the partial rows, the near
+// levels, W of them loaded together, the corrections; the same order of sums
+// whatever NV and W.
+template <int NV, int W>
+__device__ __forceinline__ void hist3d_sum(const Hist3D& h, const int64_t (&id)[NV], double (&S)[NV]) {
+#pragma clang fp contract(off)
+    double far[NV], nr0[NV], nr1[NV];
 #pragma unroll
-        for (int j = 0; j < W; j++) v[j] = (sp0 + j < nsplit) ? part[(sp0 + j) * part_stride + part_off + i] : 0.0;
+    for (int q = 0; q < NV; q++) far[q] = nr0[q] = nr1[q] = 0.0;
+    for (int r0 = 0; r0 < h.rows; r0 += W) {
+        double v[W][NV];
 #pragma unroll
-        for (int j = 0; j < W; j++) far += v[j];
+        for (int j = 0; j < W; j++)
+#pragma unroll
+            for (int q = 0; q < NV; q++) v[j][q] = r0 + j < h.rows ? h.part[(r0 + j) * h.part_stride + id[q]] : 0.0;
+#pragma unroll
+        for (int j = 0; j < W; j++)
+#pragma unroll
+            for (int q = 0; q < NV; q++) far[q] += v[j][q];
     }
-    double nr0 = 0.0, nr1 = 0.0;
-    int lo = near_lo;
-    if (mid) {
-        const int done = n > near_lo ? (n - near_lo) / kNearGroup : 0;       // groups complete by now
-        const int before = (n > n0 && n - 1 > near_lo) ? (n - 1 - near_lo) / kNearGroup : 0;
-        for (int j = before; j < done; j++)
-            fold_near_group(D, ld, omega_blk, omega_stride, n0, mid, i, near_lo + kNearGroup * j, n, n0 + blk,
-                            j == 0);
-        if (done > 0) {
-            nr0 = mid[(int64_t)(n - n0) * ld + i];
-            lo = near_lo + kNearGroup * done;
-        }
-    }
-    for (int t0 = lo; t0 < n; t0 += W) {
-        double v[W], w[W];
+    for (int t0 = h.lo; t0 < h.n; t0 += W) {
+        double v[W][NV], w[W];
 #pragma unroll
         for (int j = 0; j < W; j++) {
-            int t = t0 + j;
-            bool ok = t < n;
-            v[j] = ok ? D[(int64_t)t * ld + i] : 0.0;
-            w[j] = ok ? omega[n - t - 1] : 0.0;
+            const bool ok = t0 + j < h.n;
+#pragma unroll
+            for (int q = 0; q < NV; q++) v[j][q] = ok ? h.D[(int64_t)(t0 + j) * h.ld + id[q]] : 0.0;
+            w[j] = ok ? h.omega[h.n - t0 - j - 1] : 0.0;
         }
 #pragma unroll
-        for (int j = 0; j < W; j += 2) {
-            nr0 = fma(w[j], v[j], nr0);
-            nr1 = fma(w[j + 1], v[j + 1], nr1);
-        }
+        for (int j = 0; j < W; j += 2)
+#pragma unroll
+            for (int q = 0; q < NV; q++) {
+                nr0[q] = fma(w[j], v[j][q], nr0[q]);
+                nr1[q] = fma(w[j + 1], v[j + 1][q], nr1[q]);
+            }
     }
-    double cr = 0.0;
-    if (n >= 1) cr = corr[2 * n] * D[i];
-    if (n >= 2) cr = fma(corr[2 * n + 1], D[ld + i], cr);
-    S[i] = (far + (nr0 + nr1) + cr) * hscale;
+    const double c0 = h.corr && h.n >= 1 ? h.corr[0] : 0.0, c1 = h.corr && h.n >= 2 ? h.corr[1] : 0.0;
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        double cr = 0.0;
+        if (h.corr && h.n >= 1) cr = c0 * h.D[id[q]];
+        if (h.corr && h.n >= 2) cr = fma(c1, h.D[h.ld + id[q]], cr);
+        S[q] = (far[q] + (nr0[q] + nr1[q])) + cr;
+    }
 }
-__global__ __launch_bounds__(256) void k_hist_combine(double* __restrict__ S, const double* __restrict__ part,
-                                                      int nsplit, int64_t part_stride, int64_t part_off,
-                                                      const double* __restrict__ D, int64_t ld, int64_t nodes,
-                                                      int n, int near_lo, const double* __restrict__ omega,
-                                                      int64_t omega_stride, int n0, int blk,
-                                                      double* __restrict__ mid,
-                                                      const double* __restrict__ corr, double hscale) {
-    hist_combine_body(S, part, nsplit, part_stride, part_off, D, ld, nodes, n, near_lo, omega, omega_stride, n0,
-                      blk, mid, corr, hscale, blockIdx.x);
+
+// S of every node, times hscale (1, or 1/3 when every sweep carries a third of
+// the term): HBM bound, one pass over the rows and levels of hist3d_sum.
+__device__ __forceinline__ void hist_combine_body(double* __restrict__ S, const Hist3D& h, int64_t nodes,
+                                                  double hscale, int bid) {
+    const int64_t id[1] = {(int64_t)bid * 256 + threadIdx.x};
+    if (id[0] >= nodes) return;
+    double s[1];
+    hist3d_sum<1, 8>(h, id, s);
+    S[id[0]] = s[0] * hscale;
+}
+__global__ __launch_bounds__(256) void k_hist_combine(double* __restrict__ S, Hist3D h, int64_t nodes, double hscale) {
+    hist_combine_body(S, h, nodes, hscale, blockIdx.x);
+}
+
+// Near levels folded ahead, at most 32 at a time: every level of the range is
+// read once and added to the partial rows of the steps that follow, so a step
+// reads one row and at most 7 levels.  HBM bound.  Ranges and targets: when
+// c levels of the near field are complete, 2^k the lowest bit of c (2^k >= 8),
+// the last 2^k levels go to the next 2^k steps, so that at any step the binary
+// digits of c name the ranges its row holds.  Per step of a 64-step block 4.5
+// rows and levels move here and 3.5 levels are read directly (16-level groups
+// folded for the rest of the block: 4 and 7.5, and a row of their own).  128^3,
+// per step: folds 14 us (5.3 TB/s) and history term 17.9 us against 49 us.
+// The weights of a batch of targets stand in the lanes of one register (a
+// Toeplitz vector) or one per target (the steps' own rows) and are broadcast
+// from there: one scalar load per weight and target took 200 cycles each.
+__device__ inline double lane_value(double v, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                            __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+template <int LEN, bool TOEPLITZ>
+__device__ __forceinline__ void fold3d_levels(const Fold3D& f, int64_t i, bool ok, int lo, bool first) {
+#pragma clang fp contract(off)
+    constexpr int PB = 8;
+    const int lane = threadIdx.x & 63;
+    double dv[LEN], row[PB];
+#pragma unroll
+    for (int k = 0; k < LEN; k++) dv[k] = f.D[(int64_t)(lo + k) * f.ld + i];
+    auto load = [&](int p0) {
+#pragma unroll
+        for (int j = 0; j < PB; j++)
+            row[j] = !first && p0 + j < f.p_hi ? f.part[(int64_t)(p0 + j - f.n0) * f.ld + i] : 0.0;
+    };
+    load(f.p_lo);
+    for (int p0 = f.p_lo; p0 < f.p_hi; p0 += PB) {
+        double acc[PB], wv[TOEPLITZ ? 1 : PB];
+        // weight of level lo + k at step p0 + j: lane LEN - 1 + j - k of wv[0], or lane k of wv[j]
+        if constexpr (TOEPLITZ) {
+            wv[0] = f.omega[min(p0 - lo - LEN + lane, f.p_hi - lo - 2)];
+        } else {
+#pragma unroll
+            for (int j = 0; j < PB; j++) {
+                const int p = min(p0 + j, f.p_hi - 1);
+                wv[j] = f.omega[(int64_t)(p - f.n0) * f.omega_stride + p - lo - 1 - min(lane, LEN - 1)];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < PB; j++) acc[j] = row[j];
+        if (p0 + PB < f.p_hi) load(p0 + PB);
+#pragma unroll
+        for (int k = 0; k < LEN; k++)
+#pragma unroll
+            for (int j = 0; j < PB; j++)
+                acc[j] = fma(TOEPLITZ ? lane_value(wv[0], LEN - 1 + j - k) : lane_value(wv[TOEPLITZ ? 0 : j], k), dv[k],
+                             acc[j]);
+#pragma unroll
+        for (int j = 0; j < PB; j++)
+            if (ok && p0 + j < f.p_hi) f.part[(int64_t)(p0 + j - f.n0) * f.ld + i] = acc[j];
+    }
+}
+__device__ inline int batch_slot(const int* first, int count, int bid) {
+    int j = 0;
+    while (j + 1 < count && bid >= first[j + 1]) j++;
+    return j;
+}
+__global__ __launch_bounds__(256) void k_fold3d(Fold3DBatch b) {
+    const int j = batch_slot(b.first, b.count, blockIdx.x);
+    const Fold3D& f = b.row[j];
+    const int64_t i0 = (int64_t)((int)blockIdx.x - b.first[j]) * 256 + threadIdx.x;
+    const bool ok = i0 < f.nodes;                      // (idle lanes still hold weights)
+    const int64_t i = ok ? i0 : 0;
+    auto fold = [&](auto toeplitz) {
+        constexpr bool T = decltype(toeplitz)::value;
+        if (f.len == 8) fold3d_levels<8, T>(f, i, ok, f.lo, f.first);
+        else if (f.len == 16) fold3d_levels<16, T>(f, i, ok, f.lo, f.first);
+        else
+            for (int q = 0; q < f.len; q += 32) fold3d_levels<32, T>(f, i, ok, f.lo + q, f.first && q == 0);
+    };
+    if (f.omega_stride == 0) fold(std::true_type{});
+    else fold(std::false_type{});
 }
 
 // Series-compressed history (sum_alg 2): add the newest interval dnew to the
@@ -526,18 +595,10 @@ __global__ __launch_bounds__(256) void k_series3d(double* __restrict__ S, double
 // ---------------------------------------------------------------------------
 // Batched step of several 3D solves: the same bodies, each workgroup mapped to
 // (solve j, its local block) by the prefix counts of the table.
-__device__ inline int batch_slot(const int* first, int count, int bid) {
-    int j = 0;
-    while (j + 1 < count && bid >= first[j + 1]) j++;
-    return j;
-}
-
 __global__ __launch_bounds__(256) void k_hist_combine_batch(Lod3DBatch b) {
     const int j = batch_slot(b.first_node, b.count, blockIdx.x);
     const Lod3DRow& r = b.row[j];
-    hist_combine_body(r.S, r.part, r.nsplit, r.part_stride, r.part_off, r.D, r.ld, r.nodes, r.step, r.near_lo,
-                      r.omega, r.omega_stride, r.n0, r.blk, r.mid, r.corr, r.hscale,
-                      (int)blockIdx.x - b.first_node[j]);
+    hist_combine_body(r.S, r.hist, r.nodes, r.hscale, (int)blockIdx.x - b.first_node[j]);
 }
 
 // y sweep (axis 2) carries the history term; the x sweep (axis 1) a third of
@@ -627,13 +688,18 @@ fpde_status launch_zline3d(const double* V, double* U, const double* utop, int n
     return FPDE_OK;
 }
 
-fpde_status launch_hist_combine(double* S, const double* part, int nsplit, int64_t part_stride,
-                                int64_t part_off, const double* D, int64_t ld, int64_t nodes, int n,
-                                int near_lo, const double* omega, int64_t omega_stride, int n0, int blk,
-                                double* mid, const double* corr, double hscale, hipStream_t st) {
-    hipLaunchKernelGGL(k_hist_combine, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, st, S, part,
-                       nsplit, part_stride, part_off, D, ld, nodes, n, near_lo, omega, omega_stride, n0, blk, mid,
-                       corr, hscale);
+fpde_status launch_hist_combine(double* S, const Hist3D& h, int64_t nodes, double hscale, hipStream_t st) {
+    hipLaunchKernelGGL(k_hist_combine, dim3((unsigned)((nodes + 255) / 256)), dim3(256), 0, st, S, h, nodes, hscale);
+    return FPDE_OK;
+}
+
+fpde_status launch_fold3d(const Fold3DBatch& b, hipStream_t st) {
+    if (b.count < 1) return FPDE_OK;
+    for (int j = 0; j < b.count; j++) {
+        const int len = b.row[j].len;
+        if (len != 8 && len != 16 && (len < 32 || len % 32)) { set_error("3D fold: 8, 16 or whole 32 levels"); return FPDE_ERR_ARG; }
+    }
+    hipLaunchKernelGGL(k_fold3d, dim3(b.first[b.count]), dim3(256), 0, st, b);
     return FPDE_OK;
 }
 

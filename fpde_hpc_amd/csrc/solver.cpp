@@ -164,7 +164,7 @@ size_t footprint_bytes(const fpde_spec& s) {
     }
     b += sizeof(double) * (size_t)p.part_rows * p.part_bufs * p.ld;   // partial sums
     b += sizeof(double) * (size_t)p.ld * 8;                      // U, S, xyz, ...
-    if (s.hist_mode != HIST_PLAIN_F64 && s.sum_alg != 2)
+    if (s.dims == 1 && s.hist_mode != HIST_PLAIN_F64 && s.sum_alg != 2)
         b += sizeof(double) * (size_t)s.block * p.ld;                 // folded near-field groups
     if (s.dims == 3) b += sizeof(double) * (size_t)p.ld * 6;     // V, K, iC, Al, Bt
     b += sizeof(double) * (size_t)(s.steps + 512) * 3;           // weights
@@ -252,6 +252,7 @@ struct fpde_solver {
     bool initialized = false;
     // GEMM block state
     int n0 = -1, tc = 0, gsplits = 0, packed_groups = 0;
+    bool corr_in_part = false;   // 3D: the block's partial rows hold the two-level corrections
     int ahead_step = -1;         // step whose plain history the last step's launch streamed (within one call)
     double* part_cur = nullptr;  // partial rows the current block's steps read
     // far part one block ahead (1D cooperative form, lookahead_spec): the
@@ -450,9 +451,6 @@ fpde_status solver_alloc(fpde_solver* s) {
         DALLOC(s->iC, sizeof(double) * p.ld);
         DALLOC(s->Al, sizeof(double) * (size_t)(n + 1) * n * n);
         DALLOC(s->Bt, sizeof(double) * (size_t)(n + 1) * n * n);
-        // the history combine folds its near field in 16-level groups (GEMM forms)
-        if (sp.hist_mode != HIST_PLAIN_F64 && s->w.ser_P == 0)
-            DALLOC(s->mid, sizeof(double) * (size_t)sp.block * p.ld);
     }
     s->h = sp.length / (sp.nodes - 1);
     fpde_status rc = launch_weights(sp, s->w, s->stream);
@@ -701,6 +699,9 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
         int t_lo = std::max(0, n - s->w.jmax);
         if (is_split(sp.hist_mode)) t_lo = (t_lo / kGroup) * kGroup;
         t_lo = std::min(t_lo, tc);
+        // 3D: the rows take the two-level corrections with them
+        s->corr_in_part = sp.dims == 3 && tc >= 2 && tc > t_lo;
+        const double* corr = s->corr_in_part ? s->w.corr + 2 * (size_t)n : nullptr;
         size_t slot = 0;
         ev_begin(s, 0, &slot);
         fpde_status rc = FPDE_OK;
@@ -725,7 +726,7 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
                 rc = launch_gemm_split(sp.hist_mode, cp(0), cp(1), cp(2), s->scale + (size_t)(t_lo / kGroup) * p.ld,
                                        p.ld, (int)p.nodes, n - t_lo, tc - t_lo, B, s->w.omega,
                                        s->w.grid ? s->Wfar : nullptr, s->ldwf, s->afrag, s->ainv, s->part,
-                                       &s->gsplits, s->stream);
+                                       &s->gsplits, s->stream, 0, corr, s->D);
         } else if (s->w.grid) {
             // prescribed grid: dense weights of the block, far (t < tc) and
             // near (t in [tc, n), one reversed row per step)
@@ -734,10 +735,10 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
                 rc = launch_weights_grid(sp, s->w, n, B, B + 32, tc, 1, s->Wnear, s->ldwn, s->stream);
             if (rc == FPDE_OK)
                 rc = launch_gemm_f64_dense(s->D, p.ld, (int)p.nodes, tc, B, s->Wfar, s->ldwf, s->part, &s->gsplits,
-                                           s->stream);
+                                           s->stream, 0, corr, s->D);
         } else {
             rc = launch_gemm_f64(s->D + (size_t)t_lo * p.ld, p.ld, (int)p.nodes, n - t_lo, tc - t_lo, B, s->w.omega,
-                                 s->part, &s->gsplits, s->stream);
+                                 s->part, &s->gsplits, s->stream, 0, corr, s->D);
         }
         // 1D: the step kernels read one far value per node (K splits folded
         // here); 3D: the history combine adds the splits itself
@@ -1020,6 +1021,49 @@ HistRows hist_rows(const fpde_solver* s, int n) {
     return HistRows{(s->w.grid && s->omega_cur) ? s->omega_cur : s->w.omega, 0, n};
 }
 
+// History term of a 3D step from far_part's rows, and the folds of near levels
+// that come before it (GEMM forms; the plain form has no near field).
+Hist3D hist_3d(const fpde_solver* s, int n, int nsplit, int64_t stride, int64_t off, int near_lo) {
+    const HistRows hr = hist_rows(s, n);
+    const bool blocked = s->spec.hist_mode != HIST_PLAIN_F64;
+    const int c = n - near_lo;                         // near levels
+    Hist3D h{};
+    h.part = s->part + off;
+    h.part_stride = stride;
+    h.rows = blocked && c >= 8 ? std::max(nsplit, 1) : nsplit;
+    h.D = s->D;
+    h.ld = s->plan.ld;
+    h.n = n;
+    h.lo = blocked ? near_lo + c / 8 * 8 : near_lo;
+    h.omega = hr.omega + (int64_t)(n - hr.n0) * hr.stride;
+    h.corr = blocked && s->corr_in_part ? nullptr : s->w.corr + 2 * (size_t)n;
+    return h;
+}
+std::vector<Fold3D> folds_3d(const fpde_solver* s, int n, int nsplit, int near_lo) {
+    std::vector<Fold3D> v;
+    if (s->spec.hist_mode == HIST_PLAIN_F64 || s->w.ser_P > 0) return v;
+    const HistRows hr = hist_rows(s, n);
+    const int c = n - near_lo;
+    auto add = [&](int pos, int len) {                 // levels near_lo + [pos, pos + len)
+        const int lo = near_lo + pos;
+        const int p_lo = std::max(lo + len, s->n0), p_hi = std::min(lo + 2 * len, s->n0 + s->spec.block);
+        if (p_lo < p_hi)
+            v.push_back(Fold3D{s->D, s->plan.ld, s->plan.nodes, hr.omega, hr.stride, s->part, s->n0, lo, len, p_lo,
+                               p_hi, nsplit == 0 && pos == 0});
+    };
+    if (n == s->n0) {
+        // a block that starts with near levels: the ranges its first step's digits name
+        int pos = 0;
+        for (int len = 1 << 20; len >= 8; len >>= 1)
+            if (c & len) { add(pos, len); pos += len; }
+    } else if (c > 0 && c % 8 == 0) {
+        const int len = c & -c;
+        add(c - len, len);
+    }
+    return v;
+}
+int node_blocks(const fpde_solver* s) { return (int)((s->plan.nodes + 255) / 256); }
+
 fpde_status enqueue_3d_step(fpde_solver* s, int n) {
     const fpde_spec& sp = s->spec;
     const Plan& p = s->plan;
@@ -1042,9 +1086,14 @@ fpde_status enqueue_3d_step(fpde_solver* s, int n) {
         rc = launch_series3d(s->S, s->H, s->w.ser_P, dnew, s->w.ser_c + row, s->w.ser_v + row, p.nodes, p.ld,
                              hscale, s->stream);
     } else {
-        const HistRows hr = hist_rows(s, n);
-        rc = launch_hist_combine(s->S, s->part, nsplit, stride, off, s->D, p.ld, p.nodes, n, near_lo, hr.omega,
-                                 hr.stride, hr.n0, sp.block, s->mid, s->w.corr, hscale, s->stream);
+        for (const Fold3D& f : folds_3d(s, n, nsplit, near_lo)) {
+            Fold3DBatch fb{};
+            fb.count = 1;
+            fb.first[1] = node_blocks(s);
+            fb.row[0] = f;
+            if ((rc = launch_fold3d(fb, s->stream)) != FPDE_OK) return rc;
+        }
+        rc = launch_hist_combine(s->S, hist_3d(s, n, nsplit, stride, off, near_lo), p.nodes, hscale, s->stream);
     }
     ev_end(s, slot);
     if (rc != FPDE_OK) return rc;
@@ -1136,6 +1185,7 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
         if (v[j]->stream != bst && hip_ok(hipEventRecord(ev[j], v[j]->stream))) hip_ok(hipStreamWaitEvent(bst, ev[j], 0));
     while (rc == FPDE_OK) {
         Lod3DBatch b{};
+        std::vector<Fold3D> folds[kMax3DBatch];
         int k = 0;
         for (int j = 0; j < count && rc == FPDE_OK; j++) {
             fpde_solver* s = v[j];
@@ -1153,12 +1203,10 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
             Lod3DRow& r = b.row[k];
             r.U = s->U; r.S = s->S; r.V = s->V;
             r.Dlev = s->D + (size_t)n * p.ld;
-            r.part = s->part; r.D = s->D;
-            const HistRows hr = hist_rows(s, n);
-            r.omega = hr.omega; r.omega_stride = hr.stride; r.n0 = hr.n0; r.blk = sp.block; r.mid = s->mid;
-            r.corr = s->w.corr; r.utop = s->utop;
-            r.part_stride = stride; r.part_off = off; r.ld = p.ld; r.nodes = p.nodes;
-            r.n = sp.nodes; r.nsplit = nsplit; r.step = n; r.near_lo = near_lo; r.coef_mode = sp.coef_mode;
+            r.hist = hist_3d(s, n, nsplit, stride, off, near_lo);
+            folds[k] = folds_3d(s, n, nsplit, near_lo);
+            r.nodes = p.nodes; r.utop = s->utop;
+            r.n = sp.nodes; r.coef_mode = sp.coef_mode;
             r.split = (sp.split3d & 1) ? 1 : 0;
             r.h = s->h; r.h2inv = 1.0 / (s->h * s->h); r.ksat = sp.ksat;
             r.L = (s->w.grid && n < sp.steps) ? s->w.hLv[n] : s->w.local;
@@ -1171,6 +1219,18 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
         }
         if (rc != FPDE_OK || k == 0) break;
         b.count = k;
+        // the q-th fold of every solve that has one
+        for (size_t q = 0; rc == FPDE_OK; q++) {
+            Fold3DBatch fb{};
+            for (int j = 0; j < k; j++)
+                if (q < folds[j].size()) {
+                    fb.first[fb.count + 1] = fb.first[fb.count] + b.first_node[j + 1] - b.first_node[j];
+                    fb.row[fb.count++] = folds[j][q];
+                }
+            if (fb.count == 0) break;
+            rc = launch_fold3d(fb, bst);
+        }
+        if (rc != FPDE_OK) break;
         rc = launch_lod3d_batch(b, bst);
         if (rc != FPDE_OK) break;
         for (int j = 0; j < count; j++) {

@@ -758,6 +758,26 @@ def test_partitioned_sweeps_edges_match_oracle(fpde, oracle, n):
         assert err <= TOL_F64
 
 
+@pytest.mark.parametrize("mode,tol", [("mfma_f64", TOL_F64), ("split_bf16", TOL_MIXED)])
+@pytest.mark.parametrize("block,kw", [(16, {}), (64, {}), (128, {}), (128, {"weight_mode": 0, "fk": 3, "fp": 0.9}),
+                                      (32, {"sum_alg": 1, "sum_param": 1e-2})])
+def test_3d_near_field_folds_match_oracle(fpde, oracle, mode, tol, block, kw):
+    """Near levels of a 3D history block folded ahead in ranges of 8 to 64
+    levels, from the first block (nothing in the partial rows yet) on, with one
+    weight vector and with the steps' own rows, and the two-level corrections
+    in the rows of the later blocks."""
+    n, steps = 5, 290
+    u0 = fpde.init_3d(n, 1200 + block)
+    spec = fpde.make_spec(n, steps, 1e-3, alpha=0.85, dims=3, hist_mode=mode, block=block, u_top=u0[0], **kw)
+    u = fpde.solve(spec, u0)
+    plain = fpde.solve(fpde.make_spec(n, steps, 1e-3, alpha=0.85, dims=3, hist_mode="plain", u_top=u0[0], **kw), u0)
+    err = rel_err(u, plain)
+    if not kw:
+        err = max(err, rel_err(u, oracle.solve_3d(oracle.make_params(n, steps, 1e-3, 0.85, ksat=spec.ksat), u0)))
+    print(f"3D folds {mode} block={block} {kw}: rel err {err:.3e}", flush=True)
+    assert err <= tol
+
+
 def test_batched_3d_steps_equal_solo(fpde):
     """3D solves of different sizes, orders, history forms and block sizes
     (one with split3d odd, one with the generalized kernel FK 3) advance in
