@@ -135,6 +135,8 @@ fpde_status validate(const fpde_spec& s) {
     return FPDE_OK;
 }
 
+constexpr int kOlderSplits = 4;     // K splits of a lookahead solve's older far part
+
 Plan make_plan(const fpde_spec& s) {
     Plan p;
     p.nodes = (s.dims == 1) ? s.nodes : (int64_t)s.nodes * s.nodes * s.nodes;
@@ -145,9 +147,8 @@ Plan make_plan(const fpde_spec& s) {
     int rows_gemm = (s.hist_mode == HIST_PLAIN_F64) ? 0 : gemm_max_splits(p.nodes) * s.block;
     p.part_rows = (s.sum_alg == 2) ? 1 : std::max(rows_plain, rows_gemm);
     if (lookahead_spec(s)) {
-        // the older part's K splits, folded into the first B rows, then the
-        // newer part's single split in the next B rows
-        p.part_rows = std::max(p.part_rows, 2 * s.block);
+        // the older part's K splits of B rows, then the newer part's single one
+        p.part_rows = std::max(p.part_rows, (std::min(gemm_max_splits(p.nodes), kOlderSplits) + 1) * s.block);
         p.part_bufs = 2;
     }
     return p;
@@ -263,8 +264,9 @@ struct fpde_solver {
     hipStream_t side = nullptr;
     hipEvent_t ev_far = nullptr;   // main: this block's far part is enqueued
     hipEvent_t ev_side = nullptr;  // side: the next block's older part is done
+    bool batched = false;          // within a batched advance: far parts on the batch's stream, none ahead
     int la_n0 = -1;                // the block the pending older part is for
-    int la_tc = 0;                 // its cut (levels [0, la_tc))
+    int la_tc = 0, la_splits = 0;  // its cut (levels [0, la_tc)) and K splits
     int la_par = 0;                // parity of the current block's buffer
     // profiling
     int prof = 0;
@@ -482,11 +484,13 @@ fpde_status gemm_range(fpde_solver* s, int n0, int t_lo, int t_hi, double* P, in
                            s->w.omega, P, splits, st, max_splits);
 }
 
-// The older part of block n0's far sums, levels [0, tcA), folded into the
-// first B rows of P; returns its split count (0 or 1).  The split forms pack
-// the levels it needs first (those not packed yet), on the same stream.
-// (With a single K split, to draw HBM more slowly beside a step launch, the
-// FP64 GEMM lost its occupancy and the split one gained nothing.)
+// The older part of block n0's far sums, levels [0, tcA), as up to
+// kOlderSplits splits of B rows in P.  The split forms pack the levels it
+// needs first (those not packed yet), on the same stream.
+// The step launch adds the splits itself, beside its chain: fourteen splits
+// (N = 10^4) and a pass that added them wrote and read 72 MB more per block and
+// solve, 2 to 6 splits measured alike; six solves of N = 10^4, 2000 steps, in a
+// batch 38.9 -> 35.3 ms.
 fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t st, int* splits) {
     const fpde_spec& sp = s->spec;
     fpde_status rc = FPDE_OK;
@@ -497,10 +501,7 @@ fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t s
         s->packed_groups = ghi;
         if (rc != FPDE_OK) return rc;
     }
-    int sp_ = 0;
-    rc = gemm_range(s, n0, 0, tcA, P, 0, &sp_, st);
-    if (rc == FPDE_OK && sp_ > 1) rc = launch_part_reduce(P, sp_, s->spec.block, s->plan.ld, (int)s->plan.nodes, st);
-    *splits = sp_ > 0 ? 1 : 0;
+    rc = gemm_range(s, n0, 0, tcA, P, kOlderSplits, splits, st);
     if (rc == FPDE_OK && tcA > 0) {
         s->stats.history_launches++;
         s->stats.history_alg_bytes += 8.0 * tcA * (double)s->plan.nodes * s->spec.block;
@@ -523,7 +524,7 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     const Plan& p = s->plan;
     const int B = sp.block;
     fpde_status rc = FPDE_OK;
-    if (!s->ev_far) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_far, hipEventDisableTiming));
+    if (!s->batched && !s->ev_far) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_far, hipEventDisableTiming));
     const bool ahead = s->la_n0 == n0 && s->la_tc == tcA;
     if (s->la_n0 >= 0) {
         // the side stream's work is this block's older part, or stale: either
@@ -535,7 +536,7 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     double* P = s->part + (size_t)s->la_par * p.part_rows * p.ld;
     size_t slot = 0;
     ev_begin(s, 0, &slot);
-    int spA = (ahead && tcA > 0) ? 1 : 0;
+    int spA = ahead ? s->la_splits : 0;
     if (!ahead) rc = older_part(s, n0, tcA, P, s->stream, &spA);
     int spB = 0;
     if (rc == FPDE_OK) rc = gemm_range(s, n0, tcA, tc, P + (size_t)spA * B * p.ld, 1, &spB, s->stream, true);
@@ -548,7 +549,9 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     }
     s->gsplits = spA + spB;
     s->part_cur = P;
-    FPDE_HIP_TRY(hipEventRecord(s->ev_far, s->stream));     // the levels [0, tcA) are in memory
+    // the levels [0, tcA) are in memory (a batched advance issues nothing
+    // ahead, and has finished when it returns)
+    if (!s->batched) FPDE_HIP_TRY(hipEventRecord(s->ev_far, s->stream));
     return FPDE_OK;
 }
 
@@ -573,6 +576,7 @@ fpde_status lookahead_issue(fpde_solver* s, int n_next) {
     FPDE_HIP_TRY(hipEventRecord(s->ev_side, s->side));
     s->la_n0 = n_next;
     s->la_tc = s->tc;
+    s->la_splits = spA;
     return FPDE_OK;
 }
 
@@ -1492,8 +1496,11 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
     std::vector<Step1DArgs> rows(B);
     for (int j = 0; j < B; j++) rows[j] = block_args(blk[j], blk[j]->step, blk[j]->step, 0, 0, 0, 0);
     for (fpde_solver* s : blk) FPDE_HIP_TRY(hipStreamSynchronize(s->stream));
-    std::vector<hipEvent_t> ev(B + 1, nullptr);
     fpde_status rc = FPDE_OK;
+    // everything of the batch goes on the first solve's stream, the far parts
+    // too: the other streams are idle until this call returns, and the waits
+    // between six streams and the batch's cost more (130 us a block) than six
+    // far parts side by side gained
     hipStream_t bst = blk[0]->stream;
     auto hip_ok = [&](hipError_t e) {
         if (e == hipSuccess) return true;
@@ -1503,9 +1510,7 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
     };
     // the previous batch's launches have finished: that call synchronised
     // its streams before returning
-    if (hip_ok(hipMemcpy(drows, rows.data(), sizeof(Step1DArgs) * B, hipMemcpyHostToDevice))) {
-        for (int j = 0; j <= B && rc == FPDE_OK; j++) hip_ok(hipEventCreateWithFlags(&ev[j], hipEventDisableTiming));
-    }
+    hip_ok(hipMemcpy(drows, rows.data(), sizeof(Step1DArgs) * B, hipMemcpyHostToDevice));
     while (rc == FPDE_OK) {
         BatchTick t{};
         t.count = B;
@@ -1517,7 +1522,12 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
             if (s->step >= ends[j]) continue;                // done: no workgroups
             int nsplit = 0, near_lo = 0, n_end = 0, n0 = 0;
             int64_t stride = 0, off = 0;
+            hipStream_t own = s->stream;
+            s->stream = bst;
+            s->batched = true;
             rc = far_part(s, s->step, &nsplit, &stride, &off, &near_lo);
+            s->stream = own;
+            s->batched = false;
             if (rc != FPDE_OK) break;
             next_block(s, s->step, ends[j], &n_end, &n0);
             t.n_end[j] = n_end;
@@ -1528,18 +1538,15 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
             t.part[j] = s->part_cur;
             t.xtag[j] = launch_tag(s);
             first += s->C;
-            if (s->stream != bst && hip_ok(hipEventRecord(ev[j], s->stream))) hip_ok(hipStreamWaitEvent(bst, ev[j], 0));
         }
         if (rc != FPDE_OK) break;
         t.first[B] = first;
         if (first == 0) break;
         rc = launch_step1d_batch(drows, t, bst);
         if (rc != FPDE_OK) break;
-        if (!hip_ok(hipEventRecord(ev[B], bst))) break;
         for (int j = 0; j < B; j++) {
             fpde_solver* s = blk[j];
             if (t.n_end[j] == t.n[j]) continue;
-            if (s->stream != bst && !hip_ok(hipStreamWaitEvent(s->stream, ev[B], 0))) break;
             s->launches++;
             s->coop_launches++;
             s->stats.step_launches++;
@@ -1555,8 +1562,6 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         hipError_t e = hipStreamSynchronize(solvers[i]->stream);
         if (rc == FPDE_OK) hip_ok(e);
     }
-    for (hipEvent_t e : ev)
-        if (e) hipEventDestroy(e);
     if (rc != FPDE_OK) return rc;
     for (fpde_solver* s : blk) {
         rc = check_barrier(s);

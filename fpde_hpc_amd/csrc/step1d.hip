@@ -799,7 +799,8 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
             const int col = act(q) ? 64 * RW * q : 0;          // (idle threads read a column that exists)
             const double* pt = g.part + (int64_t)(m - g.n0) * g.ld + (Dc - g.D) + col;
             const double* d = Dc + (int64_t)lo * g.ld + col;
-            double v[W], f0 = 0.0, f1 = 0.0, md = 0.0;
+            constexpr int F = 5;                               // partial rows loaded together
+            double v[W], f[F], md = 0.0;
 #pragma unroll
             for (int j = 0; j < W; j++) {
                 v[j] = 0.0;
@@ -807,11 +808,18 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
                 d += g.ld;
                 asm("" : "+v"(d));                             // (one running address)
             }
-            if (g.nsplit > 0) f0 = pt[0];
-            if (g.nsplit > 1) f1 = pt[g.part_stride];
+#pragma unroll
+            for (int k = 0; k < F; k++) {
+                f[k] = 0.0;
+                if (k < g.nsplit) f[k] = *pt;
+                pt += g.part_stride;
+                asm("" : "+v"(pt));
+            }
             if (folded > 0) md = g.mid[(int64_t)(m - g.n0) * g.ld + (Dc - g.D) + col];
-            double far = f0 + f1;
-            for (int k = 2; k < g.nsplit; k++) far += pt[(int64_t)k * g.part_stride];
+            double far = f[0] + f[1];
+#pragma unroll
+            for (int k = 2; k < F; k++) far += f[k];
+            for (int k = F; k < g.nsplit; k++) { far += *pt; pt += g.part_stride; }
             double n0 = md, n1 = 0.0;
 #pragma unroll
             for (int j = 0; j < W; j += 2) {
