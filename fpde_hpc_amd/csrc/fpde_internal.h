@@ -540,6 +540,16 @@ fpde_status launch_ref_series(double* S, const double* old, int64_t old_size, in
 fpde_status launch_gemm_f64(const double* D, int64_t ld, int nodes, int n0, int tc, int block,
                             const double* omega, double* P, int* splits_out, hipStream_t st,
                             int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);
+// one K split over [0, tc) each, `block` rows, in one launch
+struct GemmF64Job {
+    const double* D;
+    int64_t ld;
+    int nodes, n0, tc;
+    const double* omega;
+    double* P;
+};
+struct GemmF64Jobs { GemmF64Job job[kMaxBatch]; };
+fpde_status launch_gemm_f64_jobs(const GemmF64Jobs& b, int count, int block, hipStream_t st);
 fpde_status launch_part_reduce(double* P, int splits, int rows, int64_t ld, int nodes, hipStream_t st);
 fpde_status launch_pack_split(int mode, const double* D, int64_t ld, int nodes, int g_lo, int g_hi, void* c0,
                               void* c1, void* c2, float* scale, hipStream_t st);

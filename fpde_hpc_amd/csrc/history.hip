@@ -216,19 +216,17 @@ struct GemmCorr {
 // four results of lane l are D[4v + l/16][l%16], v=0..3 (rows interleaved,
 // unlike the f32-output MFMAs where lane l holds rows 4(l/16)+v).
 template <int BR>
-__global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, int64_t ld, int nodes,
-                                                  int n0, int tc, int kchunk,
-                                                  const double* __restrict__ omega,
-                                                  double* __restrict__ P,
-                                                    const double* __restrict__ corr, const double* __restrict__ D0) {
+__device__ __forceinline__ void gemm_f64_body(const double* __restrict__ D, int64_t ld, int nodes, int n0, int tc,
+                                              int kchunk, const double* __restrict__ omega, double* __restrict__ P,
+                                              const double* __restrict__ corr, const double* __restrict__ D0, int bx,
+                                              int ks) {
     constexpr int RT = BR / 16;
     constexpr int SLAB = 1024;                  // t-values per LDS weight window
     __shared__ double win[BR + SLAB];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int ks = blockIdx.y;
     const int tlo = ks * kchunk;
     const int thi = min(tc, tlo + kchunk);
-    const int node = blockIdx.x * 64 + wave * 16 + (lane & 15);
+    const int node = bx * 64 + wave * 16 + (lane & 15);
     const bool node_ok = node < nodes;
     const int kk = lane >> 4;          // k index within the 4-deep MFMA
     d4_t acc[RT];
@@ -282,6 +280,24 @@ __global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, 
             }
         }
     }
+}
+template <int BR>
+__global__ __launch_bounds__(256) void k_gemm_f64(const double* __restrict__ D, int64_t ld, int nodes, int n0, int tc,
+                                                  int kchunk, const double* __restrict__ omega,
+                                                  double* __restrict__ P, const double* __restrict__ corr,
+                                                  const double* __restrict__ D0) {
+    gemm_f64_body<BR>(D, ld, nodes, n0, tc, kchunk, omega, P, corr, D0, blockIdx.x, blockIdx.y);
+}
+
+// Several solves' GEMMs of one K split in one launch (y: the solve): the newest
+// levels of a batch's solves stand between two step launches, where a launch
+// each cost 14 us (8 us and a gap), or 45 us on the hardware queue that shares
+// its pipe with the cooperative launches'; six of N = 10^4 in one: 17 us (33).
+template <int BR>
+__global__ __launch_bounds__(256) void k_gemm_f64_jobs(GemmF64Jobs b) {
+    const GemmF64Job& j = b.job[blockIdx.y];
+    if ((int)blockIdx.x * 64 >= j.nodes) return;
+    gemm_f64_body<BR>(j.D, j.ld, j.nodes, j.n0, j.tc, j.tc, j.omega, j.P, nullptr, nullptr, blockIdx.x, 0);
 }
 
 // FP64 time-block GEMM with dense weights (a prescribed non-uniform grid,
@@ -906,6 +922,22 @@ fpde_status launch_gemm_f64(const double* D, int64_t ld, int nodes, int n0, int 
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
     *splits_out = splits;
+    return FPDE_OK;
+}
+
+fpde_status launch_gemm_f64_jobs(const GemmF64Jobs& b, int count, int block, hipStream_t st) {
+    int nodes = 0;
+    if (count < 1) return FPDE_OK;
+    if (count > kMaxBatch) { set_error("GEMM jobs: at most 32"); return FPDE_ERR_ARG; }
+    for (int j = 0; j < count; j++) nodes = std::max(nodes, b.job[j].nodes);
+    const dim3 grid((unsigned)((nodes + 63) / 64), (unsigned)count);
+    switch (block) {
+        case 16: hipLaunchKernelGGL(k_gemm_f64_jobs<16>, grid, dim3(256), 0, st, b); break;
+        case 32: hipLaunchKernelGGL(k_gemm_f64_jobs<32>, grid, dim3(256), 0, st, b); break;
+        case 64: hipLaunchKernelGGL(k_gemm_f64_jobs<64>, grid, dim3(256), 0, st, b); break;
+        case 128: hipLaunchKernelGGL(k_gemm_f64_jobs<128>, grid, dim3(256), 0, st, b); break;
+        default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
+    }
     return FPDE_OK;
 }
 

@@ -264,7 +264,9 @@ struct fpde_solver {
     hipStream_t side = nullptr;
     hipEvent_t ev_far = nullptr;   // main: this block's far part is enqueued
     hipEvent_t ev_side = nullptr;  // side: the next block's older part is done
-    bool batched = false;          // within a batched advance: far parts on the batch's stream, none ahead
+    bool batched = false;          // within a batched advance: far parts on the batch's streams,
+    GemmF64Job newer{};            // the newer part left to the batch (tc 0: none)
+    hipEvent_t la_done = nullptr;  // when the pending older part is there (null: it is)
     int la_n0 = -1;                // the block the pending older part is for
     int la_tc = 0, la_splits = 0;  // its cut (levels [0, la_tc)) and K splits
     int la_par = 0;                // parity of the current block's buffer
@@ -339,7 +341,13 @@ void ev_collect(fpde_solver* s) {
 fpde_status solver_alloc(fpde_solver* s) {
     const fpde_spec& sp = s->spec;
     const Plan& p = s->plan;
-    if (!s->stream) FPDE_HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
+    if (!s->stream) {
+        // created next to each other, the two streams get hardware queues of
+        // their own; sharing one, the work ahead waits for the step launch (a
+        // batch of six N = 10^4 solves, 2000 steps: 29.4 ms against 27.4)
+        FPDE_HIP_TRY(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
+        if (lookahead_spec(sp)) FPDE_HIP_TRY(hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking));
+    }
     int M = sp.steps;
     s->w.M = M;
     if (sp.var_tau) {
@@ -510,6 +518,14 @@ fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t s
     return rc;
 }
 
+// The stream and the events of the work ahead.
+fpde_status side_stream(fpde_solver* s) {
+    if (!s->side) FPDE_HIP_TRY(hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking));
+    if (!s->ev_far) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_far, hipEventDisableTiming));
+    if (!s->ev_side) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_side, hipEventDisableTiming));
+    return FPDE_OK;
+}
+
 // Block n0 starts (cut tc; the previous block's cut tcA <= tc): its far sums
 // are the older part [0, tcA) -- computed ahead on the side stream during
 // the previous block's step launch when lookahead_issue ran for n0, else
@@ -524,12 +540,11 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     const Plan& p = s->plan;
     const int B = sp.block;
     fpde_status rc = FPDE_OK;
-    if (!s->batched && !s->ev_far) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_far, hipEventDisableTiming));
     const bool ahead = s->la_n0 == n0 && s->la_tc == tcA;
     if (s->la_n0 >= 0) {
         // the side stream's work is this block's older part, or stale: either
         // way it must be done before this block's buffers are written or read
-        FPDE_HIP_TRY(hipStreamWaitEvent(s->stream, s->ev_side, 0));
+        if (s->la_done) FPDE_HIP_TRY(hipStreamWaitEvent(s->stream, s->la_done, 0));
         s->la_n0 = -1;
     }
     s->la_par ^= 1;
@@ -539,7 +554,13 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     int spA = ahead ? s->la_splits : 0;
     if (!ahead) rc = older_part(s, n0, tcA, P, s->stream, &spA);
     int spB = 0;
-    if (rc == FPDE_OK) rc = gemm_range(s, n0, tcA, tc, P + (size_t)spA * B * p.ld, 1, &spB, s->stream, true);
+    double* Pn = P + (size_t)spA * B * p.ld;
+    if (s->batched) {                        // with the other solves' newer parts, in one launch
+        spB = tc > tcA ? 1 : 0;
+        s->newer = GemmF64Job{s->D + (size_t)tcA * p.ld, p.ld, (int)p.nodes, n0 - tcA, tc - tcA, s->w.omega, Pn};
+    } else if (rc == FPDE_OK) {
+        rc = gemm_range(s, n0, tcA, tc, Pn, 1, &spB, s->stream, true);
+    }
     ev_end(s, slot);
     if (rc != FPDE_OK) return rc;
     if (tc > tcA) {
@@ -549,31 +570,33 @@ fpde_status far_block_lookahead(fpde_solver* s, int n0, int tc, int tcA) {
     }
     s->gsplits = spA + spB;
     s->part_cur = P;
-    // the levels [0, tcA) are in memory (a batched advance issues nothing
-    // ahead, and has finished when it returns)
-    if (!s->batched) FPDE_HIP_TRY(hipEventRecord(s->ev_far, s->stream));
+    // the levels [0, tc) are in memory (a batched advance records that once
+    // for all of its solves)
+    if (!s->batched) {
+        fpde_status e = side_stream(s);
+        if (e != FPDE_OK) return e;
+        FPDE_HIP_TRY(hipEventRecord(s->ev_far, s->stream));
+    }
     return FPDE_OK;
 }
 
 // After the launch of block s->n0 (cut s->tc), ending at n_next = s->n0 + B:
-// the older part of block n_next, levels [0, s->tc), on the side stream, into
-// the other parity's buffer, while the step launch runs.
-fpde_status lookahead_issue(fpde_solver* s, int n_next) {
-    if (!s->la || s->tc <= 0 || n_next >= s->spec.steps || !s->ev_far) return FPDE_OK;
-    if (!s->side) FPDE_HIP_TRY(hipStreamCreateWithFlags(&s->side, hipStreamNonBlocking));
-    if (!s->ev_side) FPDE_HIP_TRY(hipEventCreateWithFlags(&s->ev_side, hipEventDisableTiming));
-    FPDE_HIP_TRY(hipStreamWaitEvent(s->side, s->ev_far, 0));
+// the older part of block n_next, levels [0, s->tc), on stream `side`, into
+// the other parity's buffer, while the step launch runs.  The stream has been
+// made to wait for those levels; the caller records `done` after it.
+fpde_status lookahead_issue(fpde_solver* s, int n_next, hipStream_t side, hipEvent_t done) {
+    if (!s->la || s->tc <= 0 || n_next >= s->spec.steps) return FPDE_OK;
     double* P = s->part + (size_t)(s->la_par ^ 1) * s->plan.part_rows * s->plan.ld;
     hipStream_t main = s->stream;
-    s->stream = s->side;                      // profiling events go on the side stream
+    s->stream = side;                         // profiling events go on the side stream
     size_t slot = 0;
     ev_begin(s, 0, &slot);
     int spA = 0;
-    fpde_status rc = older_part(s, n_next, s->tc, P, s->side, &spA);
+    fpde_status rc = older_part(s, n_next, s->tc, P, side, &spA);
     ev_end(s, slot);
     s->stream = main;
     if (rc != FPDE_OK) return rc;
-    FPDE_HIP_TRY(hipEventRecord(s->ev_side, s->side));
+    s->la_done = done;
     s->la_n0 = n_next;
     s->la_tc = s->tc;
     s->la_splits = spA;
@@ -990,7 +1013,12 @@ fpde_status enqueue_1d_blocks(fpde_solver* s, int n, int end) {
         if (rc != FPDE_OK) return rc;
         // the block is complete: the next one's older far part starts now,
         // beside this launch
-        if (s->la && n_end == s->n0 + s->spec.block && (rc = lookahead_issue(s, n_end)) != FPDE_OK) return rc;
+        if (s->la && s->side && s->ev_far && n_end == s->n0 + s->spec.block) {
+            FPDE_HIP_TRY(hipStreamWaitEvent(s->side, s->ev_far, 0));
+            rc = lookahead_issue(s, n_end, s->side, s->ev_side);
+            if (rc != FPDE_OK) return rc;
+            FPDE_HIP_TRY(hipEventRecord(s->ev_side, s->side));
+        }
         n = n_end;
         s->step = n;
     }
@@ -1496,7 +1524,8 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
     std::vector<Step1DArgs> rows(B);
     for (int j = 0; j < B; j++) rows[j] = block_args(blk[j], blk[j]->step, blk[j]->step, 0, 0, 0, 0);
     for (fpde_solver* s : blk) FPDE_HIP_TRY(hipStreamSynchronize(s->stream));
-    fpde_status rc = FPDE_OK;
+    fpde_status rc = side_stream(blk[0]);
+    if (rc != FPDE_OK) return rc;
     // everything of the batch goes on the first solve's stream, the far parts
     // too: the other streams are idle until this call returns, and the waits
     // between six streams and the batch's cost more (130 us a block) than six
@@ -1515,6 +1544,16 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         BatchTick t{};
         t.count = B;
         int first = 0;
+        // the work ahead of every solve, usually one event for all of them
+        hipEvent_t waited = nullptr;
+        for (fpde_solver* s : blk) {
+            if (s->la_n0 >= 0 && s->la_done && s->la_done != waited) {
+                waited = s->la_done;
+                if (!hip_ok(hipStreamWaitEvent(bst, waited, 0))) break;
+            }
+            s->la_done = nullptr;
+        }
+        if (rc != FPDE_OK) break;
         for (int j = 0; j < B && rc == FPDE_OK; j++) {
             fpde_solver* s = blk[j];
             t.first[j] = first;
@@ -1542,8 +1581,22 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         if (rc != FPDE_OK) break;
         t.first[B] = first;
         if (first == 0) break;
+        // the newer far parts of the blocks that start, in one launch per block size
+        for (int bs = 16; bs <= 128 && rc == FPDE_OK; bs *= 2) {
+            GemmF64Jobs jobs{};
+            int nj = 0;
+            for (fpde_solver* s : blk)
+                if (s->spec.block == bs && s->newer.tc > 0) {
+                    jobs.job[nj++] = s->newer;
+                    s->newer.tc = 0;
+                }
+            rc = launch_gemm_f64_jobs(jobs, nj, bs, bst);
+        }
+        if (rc != FPDE_OK) break;
+        if (!hip_ok(hipEventRecord(blk[0]->ev_far, bst))) break;
         rc = launch_step1d_batch(drows, t, bst);
         if (rc != FPDE_OK) break;
+        if (!hip_ok(hipStreamWaitEvent(blk[0]->side, blk[0]->ev_far, 0))) break;
         for (int j = 0; j < B; j++) {
             fpde_solver* s = blk[j];
             if (t.n_end[j] == t.n[j]) continue;
@@ -1552,11 +1605,21 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
             s->stats.step_launches++;
             count_steps(s, t.n[j], t.n_end[j], t.near_lo[j]);
             s->step = t.n_end[j];
-            // (no far part ahead here: beside a batched launch, which already
-            // fills the GPU, the solves' side GEMMs slowed the batch more than
-            // they hid: 6 x N=1e4 took 0.097 s against 0.087 s)
+            // the next block's older far parts one after the other on one side
+            // stream (on the solves' own six at once they slowed the launch by
+            // what they hid: 6 x N = 10^4, 2000 steps, 31.2 ms without work
+            // ahead, 32.4 with six side streams, 27.6 with one)
+            if (s->la && t.n_end[j] == s->n0 + s->spec.block)
+                rc = lookahead_issue(s, t.n_end[j], blk[0]->side, blk[0]->ev_side);
+            if (rc != FPDE_OK) break;
         }
+        if (rc == FPDE_OK) hip_ok(hipEventRecord(blk[0]->ev_side, blk[0]->side));
     }
+    // the side stream's last work is for a later call: finished here, since the
+    // buffers it writes belong to solves that may be destroyed first
+    hipError_t side_done = hipStreamSynchronize(blk[0]->side);
+    if (rc == FPDE_OK) hip_ok(side_done);
+    for (fpde_solver* s : blk) s->la_done = nullptr;
     // the argument rows stay alive until the last launch has run
     for (int i = 0; i < count; i++) {
         hipError_t e = hipStreamSynchronize(solvers[i]->stream);
