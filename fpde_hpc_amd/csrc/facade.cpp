@@ -472,17 +472,11 @@ fpde_status fpde_history_sum_f64(double* S, const double* D, int64_t n, int64_t 
         FPDE_HIP_TRY(hipDeviceSynchronize());
         return FPDE_OK;
     }
-    // partials then one combine pass
     ScratchLease scratch;
     fpde_status rc = scratch.take(sizeof(double) * kPlainMaxSplits * (size_t)ld);
     if (rc != FPDE_OK) return rc;
     double* part = (double*)scratch.ptr();
-    int splits = 0;
-    rc = launch_hist_plain(D, ld, (int)nodes, (int)n, (int)n, omega, part, &splits, 0);
-    if (rc == FPDE_OK) {
-        // combine: S = sum of partial rows (no near levels, no corrections)
-        rc = launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, 0);
-    }
+    rc = launch_hist_sum(S, D, ld, (int)nodes, (int)n, omega, part, 0);
     hipError_t e = hipDeviceSynchronize();
     if (rc != FPDE_OK) return rc;
     if (e != hipSuccess) { set_error(hipGetErrorString(e)); return FPDE_ERR_HIP; }

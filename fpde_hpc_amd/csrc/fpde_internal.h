@@ -723,6 +723,8 @@ fpde_status launch_space3d(const double* U, const double* K, int n, int axis, do
                            const double* sp_corr, double* E, hipStream_t st);
 fpde_status launch_series3d(double* S, double* H, int P, const double* dnew, const double* ser_c,
                             const double* ser_v, int64_t nodes, int64_t ld, double hscale, hipStream_t st);
+fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
+                            double* part, hipStream_t st);
 // 3D history term of a step, and the folds that go before it
 fpde_status launch_hist_combine(double* S, const Hist3D& h, int64_t nodes, double hscale, hipStream_t st);
 fpde_status launch_fold3d(const Fold3DBatch& b, hipStream_t st);

@@ -32,6 +32,62 @@ __global__ __launch_bounds__(256) void k_hist_plain(const double* __restrict__ D
 }
 
 // ---------------------------------------------------------------------------
+// The whole sum of a short history in one launch: S[i] = sum_t omega[n-t-1]
+// D[t][i], a workgroup's 16 waves each taking a sixteenth of the levels of the
+// same 128 nodes, the waves' sums added through LDS in level order.  Bound by
+// latency: one launch instead of the stream's and the sum of its parts, and a
+// wave's levels in flight together, 8 at a time, the first beside the weights.
+// Whole calls: 64 levels x 1000 nodes 15.9 -> 14.3 us, 256 x 1000 16.6 -> 15.7,
+// 256 x 20000 20.4 -> 18.2; 512 levels 17.0 against 17.9 us (N = 1000), so longer
+// histories keep the split over more workgroups.
+constexpr int kShortLevels = 256, kShortWaves = 16;
+__global__ __launch_bounds__(64 * kShortWaves) void k_hist_short(double* __restrict__ S, const double* __restrict__ D,
+                                                                 int64_t ld, int nodes, int n, int t_hi,
+                                                                 const double* __restrict__ omega) {
+    __shared__ double w[kShortLevels];                     // w[t] = omega[n-t-1]
+    __shared__ double sums[kShortWaves][128];
+    constexpr int W = 8;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int i2 = (blockIdx.x * 64 + lane) * 2;
+    const double* const col = D + (i2 < nodes ? i2 : 0);   // (threads past the nodes still stage weights)
+    const int c = (t_hi + kShortWaves - 1) / kShortWaves;
+    const int t0 = min(wave * c, t_hi), t1 = min(t0 + c, t_hi);
+    double2 d[W];
+    auto load = [&](int t) {
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            d[j] = {0.0, 0.0};
+            if (t + j < t1) d[j] = *reinterpret_cast<const double2*>(col + (int64_t)(t + j) * ld);
+        }
+    };
+    load(t0);
+    for (int q = tid; q < t_hi; q += 64 * kShortWaves) w[q] = omega[n - q - 1];
+    __syncthreads();
+    double a0 = 0.0, a1 = 0.0;
+    for (int t = t0; t < t1; t += W) {
+        double2 e[W];
+#pragma unroll
+        for (int j = 0; j < W; j++) e[j] = d[j];
+        load(t + W);
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const double x = t + j < t1 ? w[t + j] : 0.0;
+            a0 = fma(x, e[j].x, a0);
+            a1 = fma(x, e[j].y, a1);
+        }
+    }
+    sums[wave][2 * lane] = a0;
+    sums[wave][2 * lane + 1] = a1;
+    __syncthreads();
+    const int i = blockIdx.x * 128 + tid;
+    if (tid >= 128 || i >= nodes) return;
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < kShortWaves; k++) s += sums[k][tid];
+    S[i] = s;
+}
+
+// ---------------------------------------------------------------------------
 // The reference Sum kernel, sum_alg 0/1 (fpde_hpc_1d.cpp:1247-1284): newest
 // interval first, in chunks of BS levels; sum_alg 1 stops after the first full
 // chunk whose weights are all below sum_param in magnitude (the test is on the
@@ -828,6 +884,22 @@ fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int
     dim3 grid(tiles, splits);
     hipLaunchKernelGGL(k_hist_plain, grid, dim3(256), 0, st, D, ld, nodes, n, t_hi, chunk, omega, part);
     return FPDE_OK;
+}
+
+// S[i] = sum_{t < n} omega[n-t-1] D[t][i]; part: kPlainMaxSplits rows of ld.
+fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
+                            double* part, hipStream_t st) {
+    if (n <= kShortLevels) {
+        if (nodes > 0)
+            hipLaunchKernelGGL(k_hist_short, dim3((unsigned)((nodes + 127) / 128)), dim3(64 * kShortWaves), 0, st, S, D,
+                               ld, nodes, n, n, omega);
+        return FPDE_OK;
+    }
+    int splits = 0;
+    fpde_status rc = launch_hist_plain(D, ld, nodes, n, n, omega, part, &splits, st);
+    if (rc != FPDE_OK) return rc;
+    // no near levels, no corrections: the partial rows added
+    return launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, st);
 }
 
 // Parts of the reference Sum: about 2048 workgroups with the 512-node tiles

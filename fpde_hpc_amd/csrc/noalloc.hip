@@ -67,17 +67,12 @@ extern "C" fpde_status fpde_history_sum_f64_noalloc(double* S, const double* D, 
     double* part = nullptr;
     fpde_status rc = scratch_of_current_device(&part);
     if (rc != FPDE_OK) return rc;
-    // the same kernels as fpde_history_sum_f64: partial rows of <= 64
-    // t-chunks, then one combine pass (with no levels, n = 0, the combine
-    // writes S = 0)
+    // the same launches as fpde_history_sum_f64 (with no levels, n = 0, S = 0)
     if (hist_plain_plan((int)nodes, (int)n, nullptr) > kNoAllocRows) {
         set_error("partial rows exceed the scratch array");
         return FPDE_ERR_STATE;
     }
-    int splits = 0;
-    rc = launch_hist_plain(D, ld, (int)nodes, (int)n, (int)n, omega, part, &splits, 0);
-    if (rc != FPDE_OK) return rc;
-    rc = launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, 0);
+    rc = launch_hist_sum(S, D, ld, (int)nodes, (int)n, omega, part, 0);
     if (rc != FPDE_OK) return rc;
     FPDE_HIP_TRY(hipGetLastError());
     FPDE_HIP_TRY(hipDeviceSynchronize());

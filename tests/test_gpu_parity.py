@@ -1735,3 +1735,28 @@ def test_block_gemm_edges_exact(fpde, mode, nodes, tc, block):
         dv.close()
     np.testing.assert_array_equal(P[:, :nodes], ref)
     assert np.all(P[:, nodes:] == 7.0)
+
+
+@pytest.mark.parametrize("nodes", [1, 127, 128, 129, 1001])
+@pytest.mark.parametrize("levels", [1, 15, 17, 128, 129, 255, 256, 257])
+def test_short_history_sum_edges(fpde, nodes, levels):
+    """The one-launch sum of a short history and the first length past it:
+    remainders of its 16 parts, of the 8 levels in flight and of the 128-node
+    tile.  Products of magnitude <= 1 summed in double: the error is at most
+    (levels + 16) roundings of the sum of magnitudes."""
+    rng = np.random.default_rng(17 * nodes + levels)
+    ld = (nodes + 63) // 64 * 64
+    D, w = rng.uniform(-1.0, 1.0, (levels, ld)), rng.uniform(-1.0, 1.0, levels)
+    ref = np.longdouble(w[::-1, None] * np.longdouble(D[:, :nodes])).sum(axis=0)
+    bound = (levels + 16) * np.finfo(float).eps * (np.abs(w[::-1, None] * D[:, :nodes]).sum(axis=0) + 1e-300)
+    L = fpde.lib()
+    dv = Dev(L)
+    try:
+        bD, bw, bS = dv.put(D), dv.put(w), dv.put(np.full(nodes + 1, 7.0))
+        for fn in (L.fpde_history_sum_f64, L.fpde_history_sum_f64_noalloc):
+            assert fn(dv.ptr(bS), dv.ptr(bD), levels, nodes, ld, dv.ptr(bw)) == 0, L.fpde_last_error()
+            S = dv.get(bS, nodes + 1)
+            assert S[nodes] == 7.0                      # nothing past the nodes
+            assert (np.abs(S[:nodes] - ref) <= bound).all()
+    finally:
+        dv.close()
