@@ -300,11 +300,16 @@ struct Step1DArgs {
     int extrap;               // Picard starts from 2 U^n - U^{n-1} (picard_max > 1)
     double* Uit0;             // that initial iterate (convergence test of iteration 1)
     double* uend;             // [2][2C] U^n at the chunk ends, by step parity
-    // per-iteration form: the plain history of the next step, streamed by
-    // ahead_tiles * ahead_splits more workgroups of the launch (0: none): its
-    // levels [ahead_lo, ahead_hi), none of them written by this launch
+    // per-iteration form: the history of the next step, but its last two levels,
+    // summed by more workgroups of the launch into ahead_part (null: none).
+    // Plain: ahead_tiles * ahead_splits of them stream its levels [ahead_lo,
+    // ahead_hi).  GEMM forms (ahead_splits 0): ahead_rows far rows (ahead_far,
+    // part_stride apart) and the near levels from ahead_lo on, with the weights
+    // ahead_omega, into one row.
     int ahead_lo, ahead_hi, ahead_chunk, ahead_tiles, ahead_splits;
     double* ahead_part;
+    int ahead_rows;
+    const double *ahead_far, *ahead_omega;
     // cooperative block form (k_step1d_block): steps [n, n_end) in one launch
     int n_end;
     int picard_max;

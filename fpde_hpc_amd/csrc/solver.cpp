@@ -146,6 +146,7 @@ Plan make_plan(const fpde_spec& s) {
     int rows_plain = 64;
     int rows_gemm = (s.hist_mode == HIST_PLAIN_F64) ? 0 : gemm_max_splits(p.nodes) * s.block;
     p.part_rows = (s.sum_alg == 2) ? 1 : std::max(rows_plain, rows_gemm);
+    if (s.dims == 1 && s.hist_mode != HIST_PLAIN_F64) p.part_rows += 2;   // rows summed ahead (row_ahead)
     if (lookahead_spec(s)) {
         // the older part's K splits of B rows, then the newer part's single one
         p.part_rows = std::max(p.part_rows, (std::min(gemm_max_splits(p.nodes), kOlderSplits) + 1) * s.block);
@@ -638,6 +639,31 @@ AheadStream ahead_stream(const fpde_solver* s, int n) {
     return h;
 }
 
+// A block of the GEMM forms starts where the levels in memory (t < avail) form
+// a multiple of B: the GEMM cut tc = avail is then group aligned and the near
+// field of step n0+r is at most r+1 levels (1D: avail = n-1, since D[n-1] is
+// made by the step launch itself; 3D: avail = n).
+bool starts_block(const fpde_solver* s, int n, int avail) {
+    const int B = s->spec.block;
+    return s->n0 < 0 || n - s->n0 >= B || (avail > 0 && avail % B == 0 && n > s->n0);
+}
+
+// GEMM forms in per-iteration launches: the history row of step n summed by the
+// launch of step n - 1, as the plain form's, where step n does not start a
+// block (its far rows are there).  The row joins the last two levels in the
+// same order as without (hist_mem).  N = 4000 space-fractional, B = 64: a step
+// launch 9.4 -> 7.1 us, 600 steps 10.4 -> 9.1 ms.
+bool row_ahead(const fpde_solver* s, int n) {
+    const fpde_spec& sp = s->spec;
+    // (levels in memory when step n is prepared: the space-fractional scheme
+    // finishes step n - 1 first)
+    return sp.dims == 1 && sp.hist_mode != HIST_PLAIN_F64 && !s->block_mode && s->w.ser_P == 0 &&
+           !starts_block(s, n, s->w.sp_on ? n : n - 1) && s->tc <= n - 2;
+}
+int64_t row_ahead_off(const fpde_solver* s, int n) {
+    return (int64_t)(s->plan.part_rows - 2 + (n & 1)) * s->plan.ld;       // the last two rows of part, by step parity
+}
+
 // far part of the history for step n (GEMM modes: start a new block when due)
 fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_t* off, int* near_lo) {
     const fpde_spec& sp = s->spec;
@@ -701,11 +727,7 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
         return FPDE_OK;
     }
     int B = sp.block;
-    // A block starts where the levels in memory (t < avail) form a multiple of
-    // B: the GEMM cut tc = avail is then group aligned and the near field of
-    // step n0+r is at most r+1 levels (1D: avail = n-1, since D[n-1] is made by
-    // the step launch itself; 3D: avail = n).
-    if (s->n0 < 0 || n - s->n0 >= B || (avail > 0 && avail % B == 0 && n > s->n0)) {
+    if (starts_block(s, n, avail)) {
         const int tc_prev = s->n0 >= 0 ? s->tc : 0;
         s->n0 = n;
         int tcm = std::max(avail, 0);
@@ -781,6 +803,14 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
             s->stats.history_alg_flops += 2.0 * (tc - t_lo) * (double)p.nodes * B;
         }
     }
+    if (s->ahead_step == n) {                // summed by the previous step's launch, but for the last two levels
+        *nsplit = 1;
+        *stride = (int64_t)B * p.ld;         // (of the far rows, which the next row ahead reads)
+        *off = row_ahead_off(s, n);
+        *near_lo = n - 2;
+        s->omega_cur = s->w.grid ? s->Wnear + (size_t)(n - s->n0) * s->ldwn : s->w.omega;
+        return FPDE_OK;
+    }
     *nsplit = s->gsplits;
     *stride = (int64_t)B * p.ld;
     *off = (int64_t)(n - s->n0) * p.ld;
@@ -816,13 +846,19 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
     a.part_off = off;
     a.near_lo = near_lo;
     a.Sbuf = s->S;
-    if (ahead && plain_ahead(s, n + 1)) {
+    if (ahead && row_ahead(s, n + 1)) {
+        a.ahead_part = s->part + row_ahead_off(s, n + 1);
+        a.ahead_lo = s->tc;
+        a.ahead_rows = s->gsplits;
+        a.ahead_far = s->part + (int64_t)(n + 1 - s->n0) * s->plan.ld;
+        a.ahead_omega = s->w.grid ? s->Wnear + (size_t)(n + 1 - s->n0) * s->ldwn : s->w.omega;
+    } else if (ahead && plain_ahead(s, n + 1)) {
         const AheadStream h = ahead_stream(s, n + 1);
         a.ahead_lo = h.lo;
         a.ahead_hi = h.hi;
         a.ahead_chunk = h.chunk;
         a.ahead_splits = h.splits;
-        a.ahead_part = s->part + h.off;
+        if (h.splits > 0) a.ahead_part = s->part + h.off;
     }
     a.xyz = s->xyz;
     a.red = s->red;
@@ -899,7 +935,8 @@ fpde_status enqueue_1d_step(fpde_solver* s, int n, bool more) {
         s->stats.picard_iters_total++;
     }
     s->ahead_step = -1;
-    if (more && plain_ahead(s, n + 1)) {
+    if (more && row_ahead(s, n + 1)) s->ahead_step = n + 1;
+    else if (more && plain_ahead(s, n + 1)) {
         const AheadStream h = ahead_stream(s, n + 1);
         s->ahead_step = n + 1;
         s->stats.step_alg_bytes += 8.0 * std::max(0, h.hi - h.lo) * (double)s->plan.nodes;

@@ -24,32 +24,29 @@
 
 namespace fpde {
 
-// Far partial sums plus the near levels t in [near_lo, n-2] already in
-// memory, gathered in batches of independent loads (up to 32 partial rows and
-// the first two levels in one memory round trip, a sum over m more levels in
-// ~m/32).  omega is read only at n-t-1 >= 1.
-__device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t part_off,
-                                  const double* __restrict__ omega) {
+// Far partial sums plus the near levels t in [near_lo, t_end) of step n: the
+// partial rows and levels in batches of independent loads (up to 32 partial
+// rows in one memory round trip, a sum over m levels in ~m/32).  omega is read
+// only at n-t-1 >= 1.
+__device__ inline double hist_row(const Step1DArgs& g, int i, int n, int near_lo, int t_end, int nsplit,
+                                  const double* __restrict__ part, const double* __restrict__ omega) {
     constexpr int W = 32;
-    const int t_end = n - 1;   // exclusive: D[n-1] is the newest level, added by the caller
-    double v0 = 0.0, v1 = 0.0, w0 = 0.0, w1 = 0.0;
-    if (g.near_lo < t_end) { v0 = g.D[(int64_t)g.near_lo * g.ld + i]; w0 = omega[n - g.near_lo - 1]; }
-    if (g.near_lo + 1 < t_end) { v1 = g.D[(int64_t)(g.near_lo + 1) * g.ld + i]; w1 = omega[n - g.near_lo - 2]; }
     double far = 0.0;
-    const double* const part = g.part + part_off + i;
+    part += i;
     auto rows = [&](int r0, auto width) {          // (rows past the last: the last again, not added)
         constexpr int V = decltype(width)::value;
         double v[V];
 #pragma unroll
-        for (int j = 0; j < V; j++) v[j] = part[(int64_t)min(r0 + j, g.nsplit - 1) * g.part_stride];
+        for (int j = 0; j < V; j++) v[j] = part[(int64_t)min(r0 + j, nsplit - 1) * g.part_stride];
 #pragma unroll
-        for (int j = 0; j < V; j++) far += r0 + j < g.nsplit ? v[j] : 0.0;
+        for (int j = 0; j < V; j++) far += r0 + j < nsplit ? v[j] : 0.0;
     };
-    if (g.nsplit > 0 && g.nsplit <= 8) rows(0, std::integral_constant<int, 8>{});
+    if (nsplit == 1) far = *part;
+    else if (nsplit > 0 && nsplit <= 8) rows(0, std::integral_constant<int, 8>{});
     else
-        for (int r0 = 0; r0 < g.nsplit; r0 += W) rows(r0, std::integral_constant<int, W>{});
-    double nr0 = w0 * v0, nr1 = w1 * v1;
-    for (int t0 = g.near_lo + 2; t0 < t_end; t0 += W) {
+        for (int r0 = 0; r0 < nsplit; r0 += W) rows(r0, std::integral_constant<int, W>{});
+    double nr0 = 0.0, nr1 = 0.0;
+    for (int t0 = near_lo; t0 < t_end; t0 += W) {
         double v[W], w[W];
 #pragma unroll
         for (int j = 0; j < W; j++) {
@@ -65,6 +62,17 @@ __device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t par
         }
     }
     return far + (nr0 + nr1);
+}
+
+// The history of step n in memory, all levels but the newest (which the caller
+// adds): the row of the levels t < n-2, summed here or ahead by the previous
+// step's launch, and level n-2.
+__device__ inline double hist_mem(const Step1DArgs& g, int i, int n, int64_t part_off,
+                                  const double* __restrict__ omega) {
+    const bool last = g.near_lo <= n - 2;
+    double v = 0.0, w = 0.0;
+    if (last) { v = g.D[(int64_t)(n - 2) * g.ld + i]; w = omega[1]; }
+    return fma(w, v, hist_row(g, i, n, g.near_lo, n - 2, g.nsplit, g.part + part_off, omega));
 }
 
 // The newest level and the two-level corrections of the oldest intervals,
@@ -457,9 +465,15 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
     const int p = 4 * (lane & 15) + (lane >> 4);
     const int c = blockIdx.x;
     const int N = g.N, C = g.C;
+    const int n = g.n;
     if (c >= C) {                         // the next step's history
         __shared__ double wwin[kPlainWin];
         const int b = c - C;
+        if (g.ahead_splits == 0) {
+            const int j = b * T + tid;
+            if (j < N) g.ahead_part[j] = hist_row(g, j, n + 1, g.ahead_lo, n - 1, g.ahead_rows, g.ahead_far, g.ahead_omega);
+            return;
+        }
         plain_stream<T, 16>(g.D + (int64_t)g.ahead_lo * g.ld, g.ld, N, g.n + 1 - g.ahead_lo, g.ahead_hi - g.ahead_lo,
                             g.ahead_chunk, g.omega, g.ahead_part, b % g.ahead_tiles, b / g.ahead_tiles, wwin);
         return;
@@ -468,7 +482,6 @@ __global__ __launch_bounds__(64 * RW) void k_step1d(Step1DArgs g) {
     const int nc = (int)(((int64_t)(c + 1) * N) / C) - s;
     const int i = s + tid;
     const bool act = tid < nc;
-    const int n = g.n;
     const bool first = g.k <= 0;          // first Picard iteration of step n (or finalize)
 
     // ---- 0. loads that do not depend on the pending solve (one round trip) ---
@@ -1307,7 +1320,8 @@ fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st) {
     Step1DArgs arg = a;
     const int T = three ? 192 : 256;
     arg.ahead_tiles = (a.N + 2 * T - 1) / (2 * T);
-    hipLaunchKernelGGL(kern, dim3(a.C + arg.ahead_tiles * a.ahead_splits), dim3(T), 0, st, arg);
+    const int more = a.ahead_splits > 0 ? arg.ahead_tiles * a.ahead_splits : (a.ahead_part ? (a.N + T - 1) / T : 0);
+    hipLaunchKernelGGL(kern, dim3(a.C + more), dim3(T), 0, st, arg);
     return FPDE_OK;
 }
 

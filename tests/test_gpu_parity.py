@@ -1638,6 +1638,32 @@ def test_plain_history_streamed_ahead(fpde, nodes, steps, picard, extra):
     assert err <= TOL_F64
 
 
+@pytest.mark.parametrize("mode,block,picard,extra", [
+    ("mfma_f64", 16, 1, {"gamma": 0.8}), ("split_bf16", 64, 3, {}), ("mfma_f64", 32, 2, {"sum_alg": 1, "sum_param": 1e-2}),
+    ("mfma_f64", 16, 1, {"weight_mode": 0, "fk": 3, "fp": 0.9}), ("split_f16", 128, 1, {"gamma": 0.7})])
+@pytest.mark.parametrize("nodes", [5, 193, 700])
+def test_history_row_summed_ahead(fpde, mode, block, picard, extra, nodes):
+    """GEMM forms in per-iteration launches: a step's history row summed by the
+    previous launch, but where a block starts.  At once, in pieces and as graph
+    replays a solve has the same bits, and it agrees with the plain form."""
+    steps = 150
+    u0 = fpde.init_1d(nodes, 96)
+    kw = dict(alpha=0.7, picard_max=picard, picard_tol=1e-12 if picard > 1 else 0.0, u_top=u0[0], step_mode=1, **extra)
+    spec = fpde.make_spec(nodes, steps, 1e-3, hist_mode=mode, block=block, **kw)
+    whole = fpde.solve(spec, u0)
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b:
+        a.set_initial(u0)
+        b.set_initial(u0)
+        for piece in (1, 1, 13, 2, 16, 33, 0):
+            a.advance(piece)
+        b.advance_graph(0, 7)
+        assert np.array_equal(a.solution(), whole)
+        assert np.array_equal(b.solution(), whole)
+    err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw), u0))
+    print(f"row ahead {mode} B={block} N={nodes} {extra}: rel err {err:.3e}", flush=True)
+    assert err <= (TOL_F64 if mode == "mfma_f64" else TOL_MIXED)
+
+
 @pytest.mark.parametrize("block", [16, 64, 128])
 @pytest.mark.parametrize("picard", [1, 3])
 def test_launches_that_cut_a_block_give_the_same_bits(fpde, block, picard):
