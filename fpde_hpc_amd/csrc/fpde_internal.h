@@ -149,6 +149,7 @@ __host__ __device__ inline void vgm_coefs(double u, double z, double ksat, int m
 // kFoldBatch steps at a time.
 constexpr int kNearGroup = 16;
 constexpr int kFoldBatch = 8;
+
 // one DPP move of a double (both 32-bit halves) inside the rows of 16 lanes
 template <int CTRL>
 __device__ inline double dpp_move(double v) {
