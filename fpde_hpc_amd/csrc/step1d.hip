@@ -1113,14 +1113,14 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         return true;
     };
 
-    // Between the barriers of an iteration (Kh: K at node s-1, `change`: the
-    // lane's share of the chunk's measure): kSolved with the new iterate in
+    // Between the barriers of an iteration (Kh: K at node s-1, `meas`: the
+    // chunk's measure): kSolved with the new iterate in
     // L.u and itn; where `check` asks for it, the decision
     // on the published measures (kCheckMet: U^k met the tolerance -> kMet;
     // kCheckPending: the tentatively ended previous step did not ->
     // kRollback; kDecide: the measure alone is exchanged -> kMet or kNotMet);
     // kTimeout when a wait ran out of time.
-    auto line_solve = [&](int b, int check, double Kh, double Ln, double change, double (&itn)[NV]) -> int {
+    auto line_solve = [&](int b, int check, double Kh, double Ln, double meas, double (&itn)[NV]) -> int {
         double x[R], y[R], z[R];
         const bool decide = check == kDecide;
         int p = pos;
@@ -1128,7 +1128,6 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         const int r0 = R * p;
         if (!decide)
             chunk_line<R>(L.K, L.iC, L.d, N, s, ni, c, p, Kh, Ln, h2inv, x, y, z, L.pub);
-        const double meas = wave_max(change);
         if (lane == 0) L.pub[7] = meas;
         publish(b, decide ? kXchMeasure : 0);
         double largest = 0.0;
@@ -1161,7 +1160,7 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
     };
 
     PicardState ps = picard_state(g);
-    double Ln = 0.0, change = 0.0;
+    double Ln = 0.0, meas = 0.0;                               // meas: the chunk's measure of the last solve
     auto start_step = [&]() {
         Ln = g.Lv ? g.Lv[ps.n] : L0;
         const bool ex = g.extrap && ps.n >= 1;
@@ -1174,17 +1173,18 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         vgm_coefs(it[R + 1], zh, ksat, g.coef_mode, Kh, iCh);
         __syncthreads();                                       // A
         double itn[NV];
-        const int st = __builtin_amdgcn_readfirstlane(line_solve(bk, ps.check, Kh, Ln, change, itn));
+        const int st = __builtin_amdgcn_readfirstlane(line_solve(bk, ps.check, Kh, Ln, meas, itn));
         if (lane == 0) L.status = st;
         __syncthreads();                                       // B
         bk++;
         if (st == kSolved) {
-            change = 0.0;
+            double change = 0.0;
 #pragma unroll
             for (int r = 0; r < NV; r++) {
                 if (r <= R) change = fmax(change, have(r) ? fabs(itn[r] - it[r]) : 0.0);
                 it[r] = itn[r];
             }
+            meas = wave_max(change);                           // (beside the row waves' coefficients)
         }
         const int what = ps.after(st);
         if (what == kGoOn) continue;
