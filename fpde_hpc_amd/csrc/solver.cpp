@@ -1473,6 +1473,8 @@ fpde_status fpde_solver_reset(fpde_solver* s, const double* u0) {
     s->gsplits = 0;
     s->packed_groups = 0;
     s->part_cur = s->part;
+    s->ahead_step = -1;                            // (rows and jobs that a failed call left)
+    s->newer.tc = 0;
     s->la_par = 0;
     if (s->xch) FPDE_HIP_TRY(hipMemsetAsync(s->xch, 0, kXchBytes, s->stream));
     if (s->err) FPDE_HIP_TRY(hipMemsetAsync(s->err, 0, 64, s->stream));
