@@ -259,6 +259,7 @@ enum HistMode : int {
     HIST_SPLIT_BF16X3 = 4 // time-block GEMM, bf16 hi+mid+lo
 };
 
+constexpr int kMaxBlock = 128; // steps of the longest history block
 constexpr int kGroup = 32;     // history levels per packed group (K of one 16x16x32 MFMA)
 
 
@@ -563,7 +564,9 @@ fpde_status launch_gemm_f64_dense(const double* D, int64_t ld, int nodes, int tc
                                   int64_t ldw, double* P, int* splits_out, hipStream_t st,
                                   int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);
 // corr (of the block's first step, with D0 the first two levels): the two-level
-// corrections added to the rows as well.
+// corrections added to the rows as well; read for all `block` rows, also those
+// of steps past the last (corr_entries).
+size_t corr_entries(int steps);
 // W != nullptr: dense weight rows W[r][t] (leading dimension ldw >= tc) of a
 // prescribed grid in place of the Toeplitz vector omega.  afrag / ainv:
 // workspace of split_afrag_bytes(mode, block, tc / 32) bytes and

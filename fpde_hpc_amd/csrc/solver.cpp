@@ -137,6 +137,15 @@ fpde_status validate(const fpde_spec& s) {
 
 constexpr int kOlderSplits = 4;     // K splits of a lookahead solve's older far part
 
+}  // namespace
+
+// Entries of the per-step corrections corr[2 n], corr[2 n + 1]: the GEMM that
+// adds them to a history block's rows reads all rows of the block, and a block
+// that starts at the last step reaches kMaxBlock - 1 steps past it (zero there).
+size_t fpde::corr_entries(int steps) { return 2 * ((size_t)steps + kMaxBlock); }
+
+namespace {
+
 Plan make_plan(const fpde_spec& s) {
     Plan p;
     p.nodes = (s.dims == 1) ? s.nodes : (int64_t)s.nodes * s.nodes * s.nodes;
@@ -169,7 +178,7 @@ size_t footprint_bytes(const fpde_spec& s) {
     if (s.dims == 1 && s.hist_mode != HIST_PLAIN_F64 && s.sum_alg != 2)
         b += sizeof(double) * (size_t)s.block * p.ld;                 // folded near-field groups
     if (s.dims == 3) b += sizeof(double) * (size_t)p.ld * 6;     // V, K, iC, Al, Bt
-    b += sizeof(double) * (size_t)(s.steps + 512) * 3;           // weights
+    b += sizeof(double) * ((size_t)s.steps + 512 + corr_entries(s.steps));   // weights
     if (s.sum_alg == 2) {
         size_t P = (size_t)s.sum_param;
         b += sizeof(double) * P * p.ld;                              // moments
@@ -388,8 +397,9 @@ fpde_status solver_alloc(fpde_solver* s) {
         FPDE_HIP_TRY(hipStreamSynchronize(s->stream));    // the host vector tt goes out of scope
     }
     DALLOC(s->w.omega, sizeof(double) * (size_t)(M + 512));
-    DALLOC(s->w.corr, sizeof(double) * 2 * (size_t)(M + 1));
+    DALLOC(s->w.corr, sizeof(double) * corr_entries(M));
     FPDE_HIP_TRY(hipMemsetAsync(s->w.omega, 0, sizeof(double) * (size_t)(M + 512), s->stream));
+    FPDE_HIP_TRY(hipMemsetAsync(s->w.corr, 0, sizeof(double) * corr_entries(M), s->stream));
     if (sp.sum_alg == 2) {
         int P = (int)sp.sum_param;
         s->w.ser_P = P;

@@ -170,3 +170,15 @@ def test_advance_batch_argument_checks(fpde):
     assert L.fpde_solver_advance_batch(many, 33, 0) == 1
     assert L.fpde_solver_advance_batch(null1, 1, 0) == 1
     assert b"null solver" in L.fpde_last_error()
+
+
+def test_correction_table_holds_every_row_of_the_last_block(fpde):
+    """The history GEMM of a 3D block reads the two corrections of all its
+    rows, also those of steps past the last: the table holds them wherever the
+    last block starts."""
+    entries = fpde.lib()["_ZN4fpde12corr_entriesEi"]
+    entries.argtypes, entries.restype = [ctypes.c_int], ctypes.c_size_t
+    for steps in (1, 63, 64, 65, 70, 1000, 20000):
+        for block in (16, 32, 64, 128):
+            for n0 in (steps - 1, (steps - 1) // block * block):
+                assert entries(steps) > 2 * (n0 + block - 1) + 1, (steps, block, n0)
