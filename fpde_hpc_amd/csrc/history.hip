@@ -862,7 +862,7 @@ fpde_status launch_part_reduce(double* P, int splits, int rows, int64_t ld, int 
 // (~4096 with the node tiles), each streaming >= 32 levels; at most
 // max_splits partial rows.  Returns the number of partial rows.
 int hist_plain_plan(int nodes, int t_hi, int* chunk_out, int max_splits) {
-    if (t_hi <= 0) { if (chunk_out) *chunk_out = 0; return 0; }
+    if (t_hi <= 0 || nodes <= 0) { if (chunk_out) *chunk_out = 0; return 0; }
     int tiles = (nodes + 511) / 512;
     int want = (4096 + tiles - 1) / tiles;
     if (want > max_splits) want = max_splits;
@@ -889,10 +889,10 @@ fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int
 // S[i] = sum_{t < n} omega[n-t-1] D[t][i]; part: kPlainMaxSplits rows of ld.
 fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
                             double* part, hipStream_t st) {
+    if (nodes <= 0) return FPDE_OK;
     if (n <= kShortLevels) {
-        if (nodes > 0)
-            hipLaunchKernelGGL(k_hist_short, dim3((unsigned)((nodes + 127) / 128)), dim3(64 * kShortWaves), 0, st, S, D,
-                               ld, nodes, n, n, omega);
+        hipLaunchKernelGGL(k_hist_short, dim3((unsigned)((nodes + 127) / 128)), dim3(64 * kShortWaves), 0, st, S, D, ld,
+                           nodes, n, n, omega);
         return FPDE_OK;
     }
     int splits = 0;
@@ -908,6 +908,7 @@ fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, i
 // of 8000 x 300 41, 29 and 24 us (fewer partial rows to add), of 500 x 5000
 // 18.5, 18.3 and 19.6 us.
 int ref_sum_splits(int64_t nodes, int64_t intervals) {
+    if (nodes <= 0) return 1;
     const int64_t tiles = (nodes + 511) / 512;
     int64_t s = std::min<int64_t>((2048 + tiles - 1) / tiles, intervals / 64);
     return (int)std::max<int64_t>(1, std::min<int64_t>(s, kPlainMaxSplits));

@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 import subprocess
+import sys
 import tempfile
 
 import numpy as np
@@ -182,3 +183,18 @@ def test_correction_table_holds_every_row_of_the_last_block(fpde):
         for block in (16, 32, 64, 128):
             for n0 in (steps - 1, (steps - 1) // block * block):
                 assert entries(steps) > 2 * (n0 + block - 1) + 1, (steps, block, n0)
+
+
+def test_history_plans_of_no_nodes(fpde):
+    """A sum over no nodes is a call like any other: its plans (which divide
+    the work by tiles of nodes) give one part, no partial row and no crash.  In
+    a process of its own, since a division by zero ends it."""
+    code = ("import ctypes, fpde_hpc_amd as F\n"
+            "L = F.lib()\n"
+            "r, h = L['_ZN4fpde14ref_sum_splitsEll'], L['_ZN4fpde15hist_plain_planEiiPii']\n"
+            "r.argtypes = [ctypes.c_int64] * 2\n"
+            "h.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.POINTER(ctypes.c_int), ctypes.c_int]\n"
+            "c = ctypes.c_int(-1)\n"
+            "assert all(r(0, n) == 1 for n in (-1, 0, 1, 64, 10 ** 6))\n"
+            "assert all(h(0, n, c, 64) == 0 and c.value == 0 for n in (0, 1, 257, 10 ** 6))\n")
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=120)

@@ -1786,3 +1786,22 @@ def test_short_history_sum_edges(fpde, nodes, levels):
             assert (np.abs(S[:nodes] - ref) <= bound).all()
     finally:
         dv.close()
+
+
+@pytest.mark.parametrize("levels", [0, 1, 64, 257, 2000])
+def test_sums_over_no_nodes(fpde, levels):
+    """Calls with no nodes return without an error and write nothing."""
+    L = fpde.lib()
+    dv = Dev(L)
+    try:
+        bS, bD, bw = dv.put(np.full(2, 7.0)), dv.put(np.ones(2 * (levels + 1))), dv.put(np.ones(levels + 1))
+        for fn in (L.fpde_history_sum_f64, L.fpde_history_sum_f64_noalloc):
+            for ld in (0, 2):
+                assert fn(dv.ptr(bS), dv.ptr(bD), levels, 0, ld, dv.ptr(bw)) == 0, L.fpde_last_error()
+        for alg in (0, 1):
+            for os_ in (0, 2):
+                assert L.fpde_reference_sum(dv.ptr(bS), dv.ptr(bD), levels + 1, os_, 0, dv.ptr(bw), dv.ptr(bw), alg,
+                                            0.5) == 0, L.fpde_last_error()
+        assert np.array_equal(dv.get(bS, 2), [7.0, 7.0])
+    finally:
+        dv.close()
