@@ -292,6 +292,7 @@ struct fpde_solver {
     DeviceArena* arena = nullptr;
     bool own_stream = true;
     int64_t wait_ticks = 0;      // grid-barrier bound of the cooperative launches
+    int fail_batch_at = -1;      // tests: a batch fails once before the launch of this step
 };
 
 namespace {
@@ -439,6 +440,8 @@ fpde_status solver_alloc(fpde_solver* s) {
             const long long v = atoll(e);
             if (v > 0) s->wait_ticks = v;
         }
+        // and those of a failed batch one that fails before the launch of this step
+        if (const char* e = getenv("FPDE_TEST_FAIL_BATCH_AT")) s->fail_batch_at = atoi(e);
         // cooperative block launches pay off where a launch covers many steps:
         // the GEMM history forms (one launch per block) and the series form;
         // the plain form needs its history kernel between every two steps
@@ -619,6 +622,19 @@ fpde_status lookahead_drain(fpde_solver* s) {
     if (s->side) FPDE_HIP_TRY(hipStreamSynchronize(s->side));
     s->la_n0 = -1;
     return FPDE_OK;
+}
+
+// After a failed call: launches that the host state counts on may be missing.
+// No block is taken as started, no row as summed ahead and no level as packed;
+// the next step starts a block of its own from the levels in memory.
+void drop_started(fpde_solver* s) {
+    if (s->side) (void)hipStreamSynchronize(s->side);
+    s->la_n0 = -1;
+    s->la_done = nullptr;
+    s->n0 = -1;
+    s->packed_groups = 0;
+    s->ahead_step = -1;
+    s->newer.tc = 0;
 }
 
 // Plain history of 1D step n streamed by the launch of step n - 1, beside its
@@ -1058,6 +1074,7 @@ fpde_status enqueue_1d_blocks(fpde_solver* s, int n, int end) {
         next_block(s, n, end, &n_end, &n0);
         rc = launch_1d_block(s, n, n_end, n0, nsplit, stride, near_lo);
         if (rc != FPDE_OK) return rc;
+        n = s->step = n_end;
         // the block is complete: the next one's older far part starts now,
         // beside this launch
         if (s->la && s->side && s->ev_far && n_end == s->n0 + s->spec.block) {
@@ -1066,8 +1083,6 @@ fpde_status enqueue_1d_blocks(fpde_solver* s, int n, int end) {
             if (rc != FPDE_OK) return rc;
             FPDE_HIP_TRY(hipEventRecord(s->ev_side, s->side));
         }
-        n = n_end;
-        s->step = n;
     }
     return FPDE_OK;
 }
@@ -1328,6 +1343,8 @@ fpde_status advance_3d_batch(fpde_solver* const* v, int count, int nsteps) {
             if (v[j]->stream != bst) hip_ok(hipStreamWaitEvent(v[j]->stream, ev[count], 0));
     for (hipEvent_t e : ev)
         if (e) hipEventDestroy(e);
+    if (rc != FPDE_OK)
+        for (int j = 0; j < count; j++) drop_started(v[j]);
     return rc;
 }
 
@@ -1478,13 +1495,10 @@ fpde_status fpde_solver_reset(fpde_solver* s, const double* u0) {
     s->launches = 0;
     s->last_k = -1;
     s->pending = false;
-    s->n0 = -1;
+    drop_started(s);
     s->tc = 0;
     s->gsplits = 0;
-    s->packed_groups = 0;
     s->part_cur = s->part;
-    s->ahead_step = -1;                            // (rows and jobs that a failed call left)
-    s->newer.tc = 0;
     s->la_par = 0;
     if (s->xch) FPDE_HIP_TRY(hipMemsetAsync(s->xch, 0, kXchBytes, s->stream));
     if (s->err) FPDE_HIP_TRY(hipMemsetAsync(s->err, 0, 64, s->stream));
@@ -1498,20 +1512,19 @@ fpde_status fpde_solver_advance(fpde_solver* s, int nsteps) {
     if (!s->initialized) { set_error("set_initial must be called first"); return FPDE_ERR_STATE; }
     int M = s->spec.steps;
     int end = (nsteps <= 0) ? M : std::min(M, s->step + nsteps);
+    fpde_status rc = FPDE_OK;
     if (s->spec.dims == 1 && s->block_mode) {
-        fpde_status rc = enqueue_1d_blocks(s, s->step, end);
-        if (rc != FPDE_OK) return rc;
-        FPDE_HIP_TRY(hipGetLastError());
-        return FPDE_OK;
+        rc = enqueue_1d_blocks(s, s->step, end);
+    } else {
+        for (int n = s->step; n < end && rc == FPDE_OK; n++) {
+            rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n, n + 1 < end) : enqueue_3d_step(s, n);
+            if (rc == FPDE_OK) s->step = n + 1;
+        }
+        if (rc == FPDE_OK && s->spec.dims == 1 && s->step == M) rc = finalize_1d(s);
     }
-    for (int n = s->step; n < end; n++) {
-        fpde_status rc = (s->spec.dims == 1) ? enqueue_1d_step(s, n, n + 1 < end) : enqueue_3d_step(s, n);
-        if (rc != FPDE_OK) return rc;
-        s->step = n + 1;
-    }
-    if (s->spec.dims == 1 && s->step == M) {
-        fpde_status rc = finalize_1d(s);
-        if (rc != FPDE_OK) return rc;
+    if (rc != FPDE_OK) {
+        drop_started(s);
+        return rc;
     }
     FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
@@ -1630,6 +1643,13 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         if (rc != FPDE_OK) break;
         t.first[B] = first;
         if (first == 0) break;
+        for (fpde_solver* s : blk)
+            if (s->step == s->fail_batch_at) {
+                s->fail_batch_at = -1;
+                set_error("advance_batch: failure forced by FPDE_TEST_FAIL_BATCH_AT");
+                rc = FPDE_ERR_STATE;
+            }
+        if (rc != FPDE_OK) break;
         // the newer far parts of the blocks that start, in one launch per block size
         for (int bs = 16; bs <= 128 && rc == FPDE_OK; bs *= 2) {
             GemmF64Jobs jobs{};
@@ -1645,7 +1665,6 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         if (!hip_ok(hipEventRecord(blk[0]->ev_far, bst))) break;
         rc = launch_step1d_batch(drows, t, bst);
         if (rc != FPDE_OK) break;
-        if (!hip_ok(hipStreamWaitEvent(blk[0]->side, blk[0]->ev_far, 0))) break;
         for (int j = 0; j < B; j++) {
             fpde_solver* s = blk[j];
             if (t.n_end[j] == t.n[j]) continue;
@@ -1654,13 +1673,16 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
             s->stats.step_launches++;
             count_steps(s, t.n[j], t.n_end[j], t.near_lo[j]);
             s->step = t.n_end[j];
+        }
+        if (!hip_ok(hipStreamWaitEvent(blk[0]->side, blk[0]->ev_far, 0))) break;
+        for (int j = 0; j < B && rc == FPDE_OK; j++) {
+            fpde_solver* s = blk[j];
             // the next block's older far parts one after the other on one side
             // stream (on the solves' own six at once they slowed the launch by
             // what they hid: 6 x N = 10^4, 2000 steps, 31.2 ms without work
             // ahead, 32.4 with six side streams, 27.6 with one)
-            if (s->la && t.n_end[j] == s->n0 + s->spec.block)
+            if (s->la && t.n_end[j] != t.n[j] && t.n_end[j] == s->n0 + s->spec.block)
                 rc = lookahead_issue(s, t.n_end[j], blk[0]->side, blk[0]->ev_side);
-            if (rc != FPDE_OK) break;
         }
         if (rc == FPDE_OK) hip_ok(hipEventRecord(blk[0]->ev_side, blk[0]->side));
     }
@@ -1674,7 +1696,10 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
         hipError_t e = hipStreamSynchronize(solvers[i]->stream);
         if (rc == FPDE_OK) hip_ok(e);
     }
-    if (rc != FPDE_OK) return rc;
+    if (rc != FPDE_OK) {
+        for (fpde_solver* s : blk) drop_started(s);
+        return rc;
+    }
     for (fpde_solver* s : blk) {
         rc = check_barrier(s);
         if (rc != FPDE_OK) return rc;

@@ -1805,3 +1805,43 @@ def test_sums_over_no_nodes(fpde, levels):
         assert np.array_equal(dv.get(bS, 2), [7.0, 7.0])
     finally:
         dv.close()
+
+
+@pytest.mark.parametrize("mode,tol", [("mfma_f64", TOL_F64), ("split_bf16", TOL_MIXED)])
+@pytest.mark.parametrize("at", [0, 64, 130])
+def test_solves_go_on_after_a_failed_batch(fpde, monkeypatch, mode, tol, at):
+    """A batch that fails between the far parts of its blocks and their launch
+    (forced from the host before step `at`: the first block's, the next ones'
+    and one that a piece of a batch cut) leaves its solvers where they stood:
+    alone or in a batch they go on to the result of a solve at once.  The far
+    rows of a block begun anew are summed in another form, so the tolerance is
+    the form's."""
+    steps = 300
+    specs, u0s = [], []
+    for k, nodes in enumerate((500, 700, 900)):
+        u0s.append(fpde.init_1d(nodes, 97 + k))
+        specs.append(fpde.make_spec(nodes, steps, 1e-3, alpha=0.6 + 0.1 * k, hist_mode=mode, block=64, picard_max=2,
+                                    picard_tol=1e-12, u_top=u0s[k][0]))
+    whole = [fpde.solve(s, u) for s, u in zip(specs, u0s)]
+    sv = []
+    try:
+        for k in range(3):
+            if k == 1:
+                monkeypatch.setenv("FPDE_TEST_FAIL_BATCH_AT", str(at))
+            sv.append(fpde.Solver(specs[k]))
+            monkeypatch.delenv("FPDE_TEST_FAIL_BATCH_AT", raising=False)
+            sv[k].set_initial(u0s[k])
+        if at == 130:
+            fpde.advance_batch(sv, 130)
+        with pytest.raises(fpde.FpdeError, match="forced"):
+            fpde.advance_batch(sv, 0)
+        sv[0].advance(0)
+        sv[0].sync()
+        fpde.advance_batch(sv[1:], 0)
+        for k in range(3):
+            err = rel_err(sv[k].solution(), whole[k])
+            print(f"after a failed batch at {at} {mode} N={specs[k].nodes}: {err:.3e}", flush=True)
+            assert err <= tol
+    finally:
+        for s in sv:
+            s.close()
