@@ -135,7 +135,7 @@ fpde_status fpde_cl_buf_alloc(fpde_cl_ctx* ctx, size_t bytes, const void* host_i
     if (!ctx || !out) { set_error("null argument"); return FPDE_ERR_ARG; }
     auto* b = new fpde_cl_buf;
     b->bytes = bytes;
-    hipError_t e = hipMalloc(&b->ptr, bytes ? bytes : 8);
+    hipError_t e = device_malloc(&b->ptr, bytes ? bytes : 8);
     if (e != hipSuccess) { delete b; set_error(std::string("hipMalloc: ") + hipGetErrorString(e)); return FPDE_ERR_NOMEM; }
     if (host_init && bytes) {
         e = hipMemcpy(b->ptr, host_init, bytes, hipMemcpyHostToDevice);
@@ -502,7 +502,7 @@ fpde_status fpde_space_sum(double* V, const double* F, int64_t nodes, double h, 
     double *Fp = nullptr, *P = nullptr;
     fpde_status rc = FPDE_OK;
     auto grab = [&](double** p, size_t n) {
-        if (rc == FPDE_OK && hipMalloc(p, sizeof(double) * n) != hipSuccess) {
+        if (rc == FPDE_OK && device_malloc((void**)p, sizeof(double) * n) != hipSuccess) {
             set_error("hipMalloc failed");
             rc = FPDE_ERR_NOMEM;
         }

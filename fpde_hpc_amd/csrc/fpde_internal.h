@@ -709,6 +709,9 @@ private:
     int dev_ = 0;
 };
 bool scratch_shutdown();                // frees what is not leased
+// hipMalloc on the current device; refused, once more after the scratch pool
+// has freed what it keeps there
+hipError_t device_malloc(void** p, size_t bytes);
 
 // A solver whose device buffers come from `arena` and whose launches go to
 // `stream` (both owned by the caller, the request server): destroying it

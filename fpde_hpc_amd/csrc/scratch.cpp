@@ -7,12 +7,15 @@
 // owner gives it back only when the device has finished with it, so a buffer
 // is never shared between threads or streams.  Returned buffers are kept for
 // the next lease on their device up to kPoolBytes in all, the rest is freed;
-// fpde_shutdown frees every buffer that is not leased.
+// an allocation of the library that the device refuses frees what its pool
+// keeps and tries again (device_malloc), and fpde_shutdown frees every buffer
+// that is not leased.
 #include "fpde_internal.h"
 
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <new>
 
 namespace fpde {
 
@@ -25,6 +28,26 @@ struct DevicePool {
 std::mutex g_pool_mu;
 std::map<int, DevicePool> g_pool;
 }  // namespace
+
+// Frees what the pool keeps on the current device; whether that was anything.
+static bool trim_pool() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(g_pool_mu);
+    const auto pool = g_pool.find(dev);
+    if (pool == g_pool.end() || pool->second.free.empty()) return false;
+    for (auto& b : pool->second.free) (void)hipFree(b.second);
+    pool->second.free.clear();
+    pool->second.held = 0;
+    return true;
+}
+
+hipError_t device_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && trim_pool()) e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();     // reported here, not by the next call
+    return e;
+}
 
 fpde_status ScratchLease::take(size_t bytes) {
     give();
@@ -45,7 +68,7 @@ fpde_status ScratchLease::take(size_t bytes) {
         }
     }
     void* q = nullptr;
-    const hipError_t e = hipMalloc(&q, want);
+    const hipError_t e = device_malloc(&q, want);
     if (e != hipSuccess) {
         set_error(std::string("scratch memory: ") + hipGetErrorString(e));
         return FPDE_ERR_NOMEM;
@@ -60,7 +83,7 @@ void ScratchLease::give() {
     if (!ptr_) return;
     void* q = ptr_;
     ptr_ = nullptr;
-    {
+    try {
         std::lock_guard<std::mutex> lock(g_pool_mu);
         DevicePool& p = g_pool[dev_];
         if (p.held + bytes_ <= kPoolBytes) {
@@ -68,6 +91,7 @@ void ScratchLease::give() {
             p.held += bytes_;
             return;
         }
+    } catch (const std::bad_alloc&) {                 // no room for its entry: not kept (destructors come here)
     }
     (void)hipFree(q);
 }

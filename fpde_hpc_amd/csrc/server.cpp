@@ -43,7 +43,7 @@ void* DeviceArena::alloc(size_t bytes) {
     const size_t seg = std::max(seg_bytes_, need);
     if (reserved_ + seg > limit_) return nullptr;
     void* base = nullptr;
-    if (hipMalloc(&base, seg) != hipSuccess) { (void)hipGetLastError(); return nullptr; }
+    if (device_malloc(&base, seg) != hipSuccess) return nullptr;
     const int id = (int)segs_.size();
     segs_.push_back({(char*)base, seg});
     reserved_ += seg;

@@ -303,7 +303,7 @@ fpde_status dalloc(fpde_solver* s, void** p, size_t bytes) {
         *p = s->arena->alloc(bytes);
         if (!*p) { set_error("device arena: no free block of that size within the budget"); return FPDE_ERR_NOMEM; }
     } else {
-        hipError_t e = hipMalloc(p, bytes);
+        hipError_t e = device_malloc(p, bytes);
         if (e != hipSuccess) {
             set_error(std::string("hipMalloc failed: ") + hipGetErrorString(e));
             *p = nullptr;
@@ -1582,7 +1582,7 @@ fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, in
     int dev = 0;
     FPDE_HIP_TRY(hipGetDevice(&dev));
     Step1DArgs*& drows = g_rows_tab[dev];
-    if (!drows) FPDE_HIP_TRY(hipMalloc((void**)&drows, sizeof(Step1DArgs) * kMaxBatch));
+    if (!drows) FPDE_HIP_TRY(device_malloc((void**)&drows, sizeof(Step1DArgs) * kMaxBatch));
     std::vector<Step1DArgs> rows(B);
     for (int j = 0; j < B; j++) rows[j] = block_args(blk[j], blk[j]->step, blk[j]->step, 0, 0, 0, 0);
     for (fpde_solver* s : blk) FPDE_HIP_TRY(hipStreamSynchronize(s->stream));

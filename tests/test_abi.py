@@ -198,3 +198,76 @@ def test_history_plans_of_no_nodes(fpde):
             "assert all(r(0, n) == 1 for n in (-1, 0, 1, 64, 10 ** 6))\n"
             "assert all(h(0, n, c, 64) == 0 and c.value == 0 for n in (0, 1, 257, 10 ** 6))\n")
     subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=120)
+
+
+FAKE_DEVICE = r"""
+#include <stddef.h>
+#include <stdlib.h>
+/* the device calls of the scratch pool on host memory: `budget` bytes per device, two devices */
+static size_t budget, used[2], size_of[64];
+static void *ptr_of[64];
+static int dev_of[64], dev;
+void fake_budget(size_t b) { budget = b; }
+size_t fake_used(int d) { return used[d]; }
+int hipGetDevice(int *d) { *d = dev; return 0; }
+int hipSetDevice(int d) { dev = d; return 0; }
+int hipGetLastError(void) { return 0; }
+int hipMalloc(void **p, size_t n) {
+    if (used[dev] + n > budget) return 2;
+    for (int i = 0; i < 64; i++)
+        if (!ptr_of[i]) {
+            *p = ptr_of[i] = malloc(1);
+            size_of[i] = n; dev_of[i] = dev; used[dev] += n;
+            return 0;
+        }
+    return 2;
+}
+int hipFree(void *p) {
+    for (int i = 0; i < 64; i++)
+        if (p && ptr_of[i] == p) { used[dev_of[i]] -= size_of[i]; free(p); ptr_of[i] = 0; return 0; }
+    return 1;
+}
+"""
+
+SCRATCH_POOL = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1])
+import fpde_hpc_amd as F
+L = F.lib()
+class Lease(ctypes.Structure):
+    _fields_ = [("ptr", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("dev", ctypes.c_int)]
+sz, MB = ctypes.c_size_t, 1 << 20
+fake.fake_budget.argtypes, fake.fake_used.restype = [sz], sz
+take, give = L["_ZN4fpde12ScratchLease4takeEm"], L["_ZN4fpde12ScratchLease4giveEv"]
+take.argtypes, give.argtypes = [ctypes.c_void_p, sz], [ctypes.c_void_p]
+def lease(n):
+    l = Lease()
+    return take(ctypes.byref(l), n), l
+def keep(n):
+    rc, l = lease(n)
+    assert rc == 0
+    give(ctypes.byref(l))
+fake.fake_budget(100 * MB)
+# what the pool keeps gives way to a lease it does not fit and to other allocations
+keep(60 * MB)
+assert fake.fake_used(0) == 60 * MB
+rc, l = lease(80 * MB)
+assert rc == 0 and fake.fake_used(0) == 80 * MB
+assert lease(30 * MB)[0] == 3                     # nothing kept: refused
+give(ctypes.byref(l))
+b = ctypes.c_void_p()
+L.fpde_cl_buf_alloc.argtypes = [ctypes.c_void_p, sz, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+assert L.fpde_cl_buf_alloc(1, 90 * MB, None, ctypes.byref(b)) == 0 and fake.fake_used(0) == 90 * MB
+assert L.fpde_cl_buf_free(b) == 0
+assert L.fpde_shutdown() in (0, 2)                # (its own device calls find no device here)
+"""
+
+
+def test_scratch_pool_gives_way(tmp_path):
+    """The scratch pool on a host stand-in for the device calls it makes: kept
+    buffers are freed when an allocation is refused."""
+    c, so = tmp_path / "fake.c", tmp_path / "fake.so"
+    c.write_text(FAKE_DEVICE)
+    subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(c)])
+    env = dict(os.environ, LD_PRELOAD=" ".join([str(so), os.environ.get("LD_PRELOAD", "")]).strip())
+    subprocess.run([sys.executable, "-c", SCRATCH_POOL, str(so)], cwd=ROOT, env=env, check=True, timeout=120)
