@@ -424,7 +424,7 @@ fpde_status fpde_cl_launch(fpde_cl_ctx* ctx, fpde_cl_kernel* k, int ndims, const
     const size_t need = splits > 1 ? sizeof(double) * (size_t)splits * nodes : 0;
     if (need > ctx->scratch.bytes()) {
         FPDE_HIP_TRY(hipStreamSynchronize(ctx->stream));     // earlier launches are done with what it gives back
-        if ((rc = ctx->scratch.take(need)) != FPDE_OK) return rc;
+        if ((rc = ctx->scratch.take(need, ctx->device, 2 * need)) != FPDE_OK) return rc;
     }
     rc = launch_ref_sum((double*)S->ptr, (const double*)old->ptr, old_size, os, nodes, (const double*)tau->ptr,
                         (const double*)kb->ptr, sum_alg, sum_param, k->prog->bs, (double*)ctx->scratch.ptr(),

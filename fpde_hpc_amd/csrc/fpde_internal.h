@@ -699,7 +699,9 @@ public:
     ScratchLease(const ScratchLease&) = delete;
     ScratchLease& operator=(const ScratchLease&) = delete;
     ~ScratchLease() { give(); }
-    fpde_status take(size_t bytes);     // in place of what it held; on the current device
+    // in place of what it held; on the current device or `device`; a holder that
+    // keeps it for long names the largest buffer it wants for its request
+    fpde_status take(size_t bytes, int device = -1, size_t at_most = ~(size_t)0);
     void give();
     void* ptr() const { return ptr_; }
     size_t bytes() const { return ptr_ ? bytes_ : 0; }

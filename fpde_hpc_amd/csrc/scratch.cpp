@@ -49,16 +49,17 @@ hipError_t device_malloc(void** p, size_t bytes) {
     return e;
 }
 
-fpde_status ScratchLease::take(size_t bytes) {
+fpde_status ScratchLease::take(size_t bytes, int device, size_t at_most) {
     give();
-    int dev = 0;
-    FPDE_HIP_TRY(hipGetDevice(&dev));
+    int cur = 0;
+    FPDE_HIP_TRY(hipGetDevice(&cur));
+    const int dev = device < 0 ? cur : device;
     const size_t want = std::max<size_t>((bytes + 0xfffff) & ~(size_t)0xfffff, (size_t)1 << 20);
     {
         std::lock_guard<std::mutex> lock(g_pool_mu);
         DevicePool& p = g_pool[dev];
         auto it = p.free.lower_bound(want);
-        if (it != p.free.end()) {
+        if (it != p.free.end() && it->first <= std::max(at_most, want)) {
             bytes_ = it->first;
             ptr_ = it->second;
             p.held -= it->first;
@@ -68,7 +69,9 @@ fpde_status ScratchLease::take(size_t bytes) {
         }
     }
     void* q = nullptr;
+    if (dev != cur) FPDE_HIP_TRY(hipSetDevice(dev));
     const hipError_t e = device_malloc(&q, want);
+    if (dev != cur) (void)hipSetDevice(cur);
     if (e != hipSuccess) {
         set_error(std::string("scratch memory: ") + hipGetErrorString(e));
         return FPDE_ERR_NOMEM;

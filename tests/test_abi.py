@@ -236,13 +236,13 @@ import fpde_hpc_amd as F
 L = F.lib()
 class Lease(ctypes.Structure):
     _fields_ = [("ptr", ctypes.c_void_p), ("bytes", ctypes.c_size_t), ("dev", ctypes.c_int)]
-sz, MB = ctypes.c_size_t, 1 << 20
+sz, MB, ANY = ctypes.c_size_t, 1 << 20, ctypes.c_size_t(-1).value
 fake.fake_budget.argtypes, fake.fake_used.restype = [sz], sz
-take, give = L["_ZN4fpde12ScratchLease4takeEm"], L["_ZN4fpde12ScratchLease4giveEv"]
-take.argtypes, give.argtypes = [ctypes.c_void_p, sz], [ctypes.c_void_p]
-def lease(n):
+take, give = L["_ZN4fpde12ScratchLease4takeEmim"], L["_ZN4fpde12ScratchLease4giveEv"]
+take.argtypes, give.argtypes = [ctypes.c_void_p, sz, ctypes.c_int, sz], [ctypes.c_void_p]
+def lease(n, dev=-1, at_most=ANY):
     l = Lease()
-    return take(ctypes.byref(l), n), l
+    return take(ctypes.byref(l), n, dev, at_most), l
 def keep(n):
     rc, l = lease(n)
     assert rc == 0
@@ -259,13 +259,28 @@ b = ctypes.c_void_p()
 L.fpde_cl_buf_alloc.argtypes = [ctypes.c_void_p, sz, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
 assert L.fpde_cl_buf_alloc(1, 90 * MB, None, ctypes.byref(b)) == 0 and fake.fake_used(0) == 90 * MB
 assert L.fpde_cl_buf_free(b) == 0
+# a lease held for long does not take a far larger buffer, a short one does
+keep(60 * MB)
+rc, l = lease(MB, -1, 2 * MB)
+assert rc == 0 and l.bytes == MB and fake.fake_used(0) == 61 * MB
+rc, m = lease(MB)
+assert rc == 0 and m.bytes == 60 * MB
+# memory of another device, the thread's device left as it was
+rc, o = lease(3 * MB, 1)
+assert rc == 0 and o.dev == 1 and fake.fake_used(1) == 3 * MB
+cur = ctypes.c_int(-1)
+fake.hipGetDevice(ctypes.byref(cur))
+assert cur.value == 0
+for x in (l, m, o):
+    give(ctypes.byref(x))
 assert L.fpde_shutdown() in (0, 2)                # (its own device calls find no device here)
 """
 
 
 def test_scratch_pool_gives_way(tmp_path):
     """The scratch pool on a host stand-in for the device calls it makes: kept
-    buffers are freed when an allocation is refused."""
+    buffers are freed when an allocation is refused, a long lease is about as
+    large as its request, and a lease for another device is on that device."""
     c, so = tmp_path / "fake.c", tmp_path / "fake.so"
     c.write_text(FAKE_DEVICE)
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(c)])
