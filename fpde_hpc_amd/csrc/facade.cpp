@@ -473,10 +473,10 @@ fpde_status fpde_history_sum_f64(double* S, const double* D, int64_t n, int64_t 
         return FPDE_OK;
     }
     ScratchLease scratch;
-    fpde_status rc = scratch.take(sizeof(double) * kPlainMaxSplits * (size_t)ld);
-    if (rc != FPDE_OK) return rc;
-    double* part = (double*)scratch.ptr();
-    rc = launch_hist_sum(S, D, ld, (int)nodes, (int)n, omega, part, 0);
+    const int rows = hist_sum_rows((int)nodes, (int)n);
+    fpde_status rc = FPDE_OK;
+    if (rows > 0 && (rc = scratch.take(sizeof(double) * rows * (size_t)ld)) != FPDE_OK) return rc;
+    rc = launch_hist_sum(S, D, ld, (int)nodes, (int)n, omega, (double*)scratch.ptr(), 0);
     hipError_t e = hipDeviceSynchronize();
     if (rc != FPDE_OK) return rc;
     if (e != hipSuccess) { set_error(hipGetErrorString(e)); return FPDE_ERR_HIP; }

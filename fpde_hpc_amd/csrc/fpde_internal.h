@@ -737,6 +737,8 @@ fpde_status launch_space3d(const double* U, const double* K, int n, int axis, do
                            const double* sp_corr, double* E, hipStream_t st);
 fpde_status launch_series3d(double* S, double* H, int P, const double* dnew, const double* ser_c,
                             const double* ser_v, int64_t nodes, int64_t ld, double hscale, hipStream_t st);
+// S[i] = sum_{t < n} omega[n-t-1] D[t][i]; part: hist_sum_rows rows of ld
+int hist_sum_rows(int nodes, int n);
 fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
                             double* part, hipStream_t st);
 // 3D history term of a step, and the folds that go before it

@@ -886,7 +886,9 @@ fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int
     return FPDE_OK;
 }
 
-// S[i] = sum_{t < n} omega[n-t-1] D[t][i]; part: kPlainMaxSplits rows of ld.
+// Partial rows of launch_hist_sum (a short history needs none).
+int hist_sum_rows(int nodes, int n) { return n <= kShortLevels ? 0 : hist_plain_plan(nodes, n, nullptr); }
+
 fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
                             double* part, hipStream_t st) {
     if (nodes <= 0) return FPDE_OK;

@@ -68,7 +68,7 @@ extern "C" fpde_status fpde_history_sum_f64_noalloc(double* S, const double* D, 
     fpde_status rc = scratch_of_current_device(&part);
     if (rc != FPDE_OK) return rc;
     // the same launches as fpde_history_sum_f64 (with no levels, n = 0, S = 0)
-    if (hist_plain_plan((int)nodes, (int)n, nullptr) > kNoAllocRows) {
+    if (hist_sum_rows((int)nodes, (int)n) > kNoAllocRows) {
         set_error("partial rows exceed the scratch array");
         return FPDE_ERR_STATE;
     }

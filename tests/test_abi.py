@@ -211,7 +211,14 @@ void fake_budget(size_t b) { budget = b; }
 size_t fake_used(int d) { return used[d]; }
 int hipGetDevice(int *d) { *d = dev; return 0; }
 int hipSetDevice(int d) { dev = d; return 0; }
-int hipGetLastError(void) { return 0; }
+static int last, launch_error, launches;
+void fake_launch_error(int e) { launch_error = e; }
+int fake_launches(void) { return launches; }
+int hipGetLastError(void) { int e = last; last = 0; return e; }
+int hipLaunchKernel(void) { launches++; return last = launch_error; }
+int __hipPushCallConfiguration(void) { return 0; }
+int __hipPopCallConfiguration(void) { return 0; }
+int hipDeviceSynchronize(void) { return 0; }
 int hipMalloc(void **p, size_t n) {
     if (used[dev] + n > budget) return 2;
     for (int i = 0; i < 64; i++)
@@ -277,12 +284,40 @@ assert L.fpde_shutdown() in (0, 2)                # (its own device calls find n
 """
 
 
-def test_scratch_pool_gives_way(tmp_path):
-    """The scratch pool on a host stand-in for the device calls it makes: kept
-    buffers are freed when an allocation is refused, a long lease is about as
-    large as its request, and a lease for another device is on that device."""
+def _on_fake_device(tmp_path, code):
     c, so = tmp_path / "fake.c", tmp_path / "fake.so"
     c.write_text(FAKE_DEVICE)
     subprocess.check_call(["gcc", "-shared", "-fPIC", "-o", str(so), str(c)])
     env = dict(os.environ, LD_PRELOAD=" ".join([str(so), os.environ.get("LD_PRELOAD", "")]).strip())
-    subprocess.run([sys.executable, "-c", SCRATCH_POOL, str(so)], cwd=ROOT, env=env, check=True, timeout=120)
+    subprocess.run([sys.executable, "-c", code, str(so)], cwd=ROOT, env=env, check=True, timeout=120)
+
+
+def test_scratch_pool_gives_way(tmp_path):
+    """The scratch pool on a host stand-in for the device calls it makes: kept
+    buffers are freed when an allocation is refused, a long lease is about as
+    large as its request, and a lease for another device is on that device."""
+    _on_fake_device(tmp_path, SCRATCH_POOL)
+
+
+HISTORY_SUM_CALLS = r"""
+import ctypes, sys
+fake = ctypes.CDLL(sys.argv[1])
+import fpde_hpc_amd as F
+L = F.lib()
+fake.fake_budget.argtypes, fake.fake_used.restype = [ctypes.c_size_t], ctypes.c_size_t
+def call(levels, nodes):
+    return L.fpde_history_sum_f64(8, 8, levels, nodes, (nodes + 63) // 64 * 64, 8)
+"""
+
+
+def test_history_sum_takes_the_memory_its_form_needs(tmp_path):
+    """A short history's sum is one launch without partial rows; a long one
+    takes as many rows as its plan has parts (fewer than 64 on long lines)."""
+    _on_fake_device(tmp_path, HISTORY_SUM_CALLS + r"""
+fake.fake_budget(0)
+rc = call(64, 20000)
+assert rc == 0 and fake.fake_launches() == 1, (rc, fake.fake_launches(), L.fpde_last_error())
+assert call(2000, 20000) == 3
+fake.fake_budget(24 << 20)
+assert call(300, 3000000) == 0                    # one row of 24 MB
+""")
