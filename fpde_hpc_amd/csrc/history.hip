@@ -39,8 +39,13 @@ __global__ __launch_bounds__(256) void k_hist_plain(const double* __restrict__ D
 // wave's levels in flight together, 8 at a time, the first beside the weights.
 // Whole calls: 64 levels x 1000 nodes 15.9 -> 14.3 us, 256 x 1000 16.6 -> 15.7,
 // 256 x 20000 20.4 -> 18.2; 512 levels 17.0 against 17.9 us (N = 1000), so longer
-// histories keep the split over more workgroups.
-constexpr int kShortLevels = 256, kShortWaves = 16;
+// histories keep the split over more workgroups, and so do longer lines, where
+// the sum is bandwidth again and 16 waves with a few levels each are overhead:
+// 65536 nodes x 16 and 256 levels 16.0 and 32.4 against 15.8 and 33.8 us, 10^5
+// x 16 and 256 19.1 and 43.7 against 15.8 and 47.2, 10^6 x 1 and 16 48 and 70
+// against 21 and 36, 10^7 x 4 432 against 110.
+constexpr int kShortLevels = 256, kShortNodes = 65536, kShortWaves = 16;
+static bool short_sum(int nodes, int n) { return n <= kShortLevels && nodes <= kShortNodes; }
 __global__ __launch_bounds__(64 * kShortWaves) void k_hist_short(double* __restrict__ S, const double* __restrict__ D,
                                                                  int64_t ld, int nodes, int n, int t_hi,
                                                                  const double* __restrict__ omega) {
@@ -887,12 +892,12 @@ fpde_status launch_hist_plain(const double* D, int64_t ld, int nodes, int n, int
 }
 
 // Partial rows of launch_hist_sum (a short history needs none).
-int hist_sum_rows(int nodes, int n) { return n <= kShortLevels ? 0 : hist_plain_plan(nodes, n, nullptr); }
+int hist_sum_rows(int nodes, int n) { return short_sum(nodes, n) ? 0 : hist_plain_plan(nodes, n, nullptr); }
 
 fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, int n, const double* omega,
                             double* part, hipStream_t st) {
     if (nodes <= 0) return FPDE_OK;
-    if (n <= kShortLevels) {
+    if (short_sum(nodes, n)) {
         hipLaunchKernelGGL(k_hist_short, dim3((unsigned)((nodes + 127) / 128)), dim3(64 * kShortWaves), 0, st, S, D, ld,
                            nodes, n, n, omega);
         return FPDE_OK;

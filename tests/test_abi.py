@@ -321,3 +321,14 @@ assert call(2000, 20000) == 3
 fake.fake_budget(24 << 20)
 assert call(300, 3000000) == 0                    # one row of 24 MB
 """)
+
+
+def test_short_history_sums_of_long_lines_are_streamed(tmp_path):
+    """One launch for a short history up to 65536 nodes; beyond, the stream and
+    the sum of its parts."""
+    _on_fake_device(tmp_path, HISTORY_SUM_CALLS + r"""
+fake.fake_budget(1 << 40)
+for nodes, launches in ((65536, 1), (65537, 2), (1 << 29, 2), (1 << 30, 2)):
+    before = fake.fake_launches()
+    assert call(1, nodes) == 0 and fake.fake_launches() - before == launches, nodes
+""")

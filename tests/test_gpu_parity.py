@@ -1845,3 +1845,27 @@ def test_solves_go_on_after_a_failed_batch(fpde, monkeypatch, mode, tol, at):
     finally:
         for s in sv:
             s.close()
+
+
+@pytest.mark.parametrize("nodes", [65535, 65536, 65537, 100001])
+@pytest.mark.parametrize("levels", [0, 1, 5, 256])
+def test_short_history_sum_of_long_lines(fpde, nodes, levels):
+    """The last line length of the one-launch sum and the first past it, against
+    a sum in extended precision, within (levels + 16) roundings of the sum of
+    magnitudes; the call with its own partial rows only where the level fits."""
+    rng = np.random.default_rng(nodes + levels)
+    ld = (nodes + 63) // 64 * 64
+    D, w = rng.uniform(-1.0, 1.0, (max(levels, 1), ld)), rng.uniform(-1.0, 1.0, max(levels, 1))
+    terms = w[::-1, None][:levels] * np.longdouble(D[:levels, :nodes])
+    bound = (levels + 16) * np.finfo(float).eps * np.abs(terms).sum(axis=0)
+    L = fpde.lib()
+    dv = Dev(L)
+    try:
+        bD, bw, bS = dv.put(D), dv.put(w), dv.put(np.full(nodes + 1, 7.0))
+        for fn in (L.fpde_history_sum_f64, L.fpde_history_sum_f64_noalloc)[:2 if ld <= 65536 else 1]:
+            assert fn(dv.ptr(bS), dv.ptr(bD), levels, nodes, ld, dv.ptr(bw)) == 0, L.fpde_last_error()
+            S = dv.get(bS, nodes + 1)
+            assert S[nodes] == 7.0
+            assert (np.abs(S[:nodes] - terms.sum(axis=0)) <= bound).all()
+    finally:
+        dv.close()
