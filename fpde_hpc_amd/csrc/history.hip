@@ -900,13 +900,16 @@ fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, i
     if (short_sum(nodes, n)) {
         hipLaunchKernelGGL(k_hist_short, dim3((unsigned)((nodes + 127) / 128)), dim3(64 * kShortWaves), 0, st, S, D, ld,
                            nodes, n, n, omega);
+        FPDE_HIP_TRY(hipGetLastError());
         return FPDE_OK;
     }
     int splits = 0;
     fpde_status rc = launch_hist_plain(D, ld, nodes, n, n, omega, part, &splits, st);
     if (rc != FPDE_OK) return rc;
     // no near levels, no corrections: the partial rows added
-    return launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, st);
+    rc = launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, st);
+    if (rc == FPDE_OK) FPDE_HIP_TRY(hipGetLastError());
+    return rc;
 }
 
 // Parts of the reference Sum: about 2048 workgroups with the 512-node tiles
@@ -1018,6 +1021,7 @@ fpde_status launch_gemm_f64_jobs(const GemmF64Jobs& b, int count, int block, hip
         case 128: hipLaunchKernelGGL(k_gemm_f64_jobs<128>, grid, dim3(256), 0, st, b); break;
         default: set_error("block must be 16, 32, 64 or 128"); return FPDE_ERR_ARG;
     }
+    FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
 }
 

@@ -332,3 +332,16 @@ for nodes, launches in ((65536, 1), (65537, 2), (1 << 29, 2), (1 << 30, 2)):
     before = fake.fake_launches()
     assert call(1, nodes) == 0 and fake.fake_launches() - before == launches, nodes
 """)
+
+
+def test_history_sum_reports_a_refused_launch(tmp_path):
+    """A launch that the runtime refuses is an error of the call, in the one
+    launch of a short history and in the stream."""
+    _on_fake_device(tmp_path, HISTORY_SUM_CALLS + r"""
+fake.fake_budget(1 << 40)
+for levels in (1, 256, 257, 5000):
+    fake.fake_launch_error(1)
+    assert call(levels, 1000) == 2, levels
+    fake.fake_launch_error(0)
+    assert call(levels, 1000) == 0, levels
+""")
