@@ -498,34 +498,21 @@ fpde_status fpde_space_sum(double* V, const double* F, int64_t nodes, double h, 
     sp.series_eps = series_eps;
     const int64_t ldp = (nodes + kSpTile - 1) / kSpTile * kSpTile;
     const size_t chunks = (size_t)space_chunks((int)(ldp / kSpTile) - 1, ldp);
+    // weights, corrections, F and the partial sums, each from a 64-element boundary
+    const size_t n64 = (size_t)(nodes + 63) / 64 * 64;
+    ScratchLease scratch;
+    fpde_status rc = scratch.take(sizeof(double) * (3 * n64 + (1 + chunks) * (size_t)ldp));
+    if (rc != FPDE_OK) return rc;
     DeviceWeights w;
-    double *Fp = nullptr, *P = nullptr;
-    fpde_status rc = FPDE_OK;
-    auto grab = [&](double** p, size_t n) {
-        if (rc == FPDE_OK && device_malloc((void**)p, sizeof(double) * n) != hipSuccess) {
-            set_error("hipMalloc failed");
-            rc = FPDE_ERR_NOMEM;
-        }
-    };
-    grab(&w.sp_omega, (size_t)nodes);
-    grab(&w.sp_corr, 2 * (size_t)nodes);
-    grab(&Fp, (size_t)ldp);
-    grab(&P, chunks * (size_t)ldp);
-    if (rc == FPDE_OK) {
-        // F on the interior rows, zero elsewhere (calc_v reads F[1..i-1])
-        hipError_t e = hipMemset(Fp, 0, sizeof(double) * ldp);
-        if (e == hipSuccess)
-            e = hipMemcpy(Fp + 1, F + 1, sizeof(double) * (size_t)(nodes - 2), hipMemcpyDeviceToDevice);
-        if (e != hipSuccess) { set_error(hipGetErrorString(e)); rc = FPDE_ERR_HIP; }
-    }
+    w.sp_omega = (double*)scratch.ptr();
+    w.sp_corr = w.sp_omega + n64;
+    double* const Fp = w.sp_corr + 2 * n64;
+    double* const P = Fp + ldp;
+    rc = launch_space_pad(F, (int)nodes, Fp, ldp, 0);
     if (rc == FPDE_OK) rc = launch_space_weights(sp, w, h, 0);
     if (rc == FPDE_OK) rc = launch_space_apply(Fp, (int)nodes, w.sp_omega, P, ldp, 0);
     if (rc == FPDE_OK) rc = launch_space_reduce(V, P, Fp, w.sp_corr, (int)nodes, ldp, 0);
-    hipError_t e = hipDeviceSynchronize();
-    hipFree(w.sp_omega);
-    hipFree(w.sp_corr);
-    hipFree(Fp);
-    hipFree(P);
+    const hipError_t e = hipDeviceSynchronize();             // (before the scratch memory is given back)
     if (rc != FPDE_OK) return rc;
     if (e != hipSuccess) { set_error(hipGetErrorString(e)); return FPDE_ERR_HIP; }
     return FPDE_OK;

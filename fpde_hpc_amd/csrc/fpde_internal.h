@@ -520,6 +520,7 @@ fpde_status launch_weights(const fpde_spec& s, DeviceWeights& w, hipStream_t st)
 fpde_status launch_space_weights(const fpde_spec& s, DeviceWeights& w, double h, hipStream_t st);
 fpde_status launch_space_flux(const double* U, int N, double h, double ksat, int mode, double* F, int64_t ldp,
                               hipStream_t st);
+fpde_status launch_space_pad(const double* F, int N, double* Fp, int64_t ldp, hipStream_t st);
 fpde_status launch_space_apply(const double* F, int N, const double* sp_omega, double* P, int64_t ldp,
                                hipStream_t st);
 fpde_status launch_space_reduce(double* V, const double* P, const double* F, const double* sp_corr, int N,

@@ -32,6 +32,13 @@ __global__ __launch_bounds__(256) void k_space_flux(const double* __restrict__ U
     F[j] = f;
 }
 
+// F of the interior rows as the sums read it, zero elsewhere (calc_v reads
+// F[1..i-1]): the direct call's F is the caller's, whose end rows do not count.
+__global__ __launch_bounds__(256) void k_space_pad(const double* __restrict__ F, int N, double* __restrict__ Fp) {
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    Fp[j] = j >= 1 && j <= N - 2 ? F[j] : 0.0;
+}
+
 // Partial sums of the spatial sum on the matrix cores: one work unit (row
 // tile t, block-diagonal chunk y, space_unit) per workgroup.
 __global__ __launch_bounds__(256) void k_space_apply(const double* __restrict__ F, int N,
@@ -167,6 +174,12 @@ fpde_status launch_space_flux(const double* U, int N, double h, double ksat, int
                               hipStream_t st) {
     if (ldp < N || ldp % kSpTile) { set_error("space flux: bad padded length"); return FPDE_ERR_ARG; }
     hipLaunchKernelGGL(k_space_flux, dim3((unsigned)(ldp / 256)), dim3(256), 0, st, U, N, h, ksat, mode, F, ldp);
+    FPDE_HIP_TRY(hipGetLastError());
+    return FPDE_OK;
+}
+
+fpde_status launch_space_pad(const double* F, int N, double* Fp, int64_t ldp, hipStream_t st) {
+    hipLaunchKernelGGL(k_space_pad, dim3((unsigned)(ldp / 256)), dim3(256), 0, st, F, N, Fp);
     FPDE_HIP_TRY(hipGetLastError());
     return FPDE_OK;
 }
