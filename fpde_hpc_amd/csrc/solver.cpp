@@ -506,13 +506,29 @@ fpde_status gemm_range(fpde_solver* s, int n0, int t_lo, int t_hi, double* P, in
                            s->w.omega, P, splits, st, max_splits);
 }
 
+// K splits of the older part [0, tcA) (0: as many as the GEMM takes).  Up to
+// kOlderSplits the step launch adds them itself, beside its chain: fourteen
+// splits (N = 10^4) and a pass that added them wrote and read 72 MB more per
+// block and solve, 2 to 6 splits measured alike; six solves of N = 10^4, 2000
+// steps, in a batch 38.9 -> 35.3 ms.  On short lines so few splits leave the
+// GEMM on a part of the GPU, and where it takes longer than the step launch it
+// runs beside, the blocks wait for it: there all splits and the pass are the
+// faster way.  FP64 (matrix cores: two workgroups per CU; 4 splits against all,
+// ms): N = 1000, 3 10^4 steps, B = 16 378 / 203, N = 6000 276 / 228, N = 8000
+// 154 / 151, N = 10^4 158 / 163; six N = 1000, 2 10^4 steps 484 / 239.  Split
+// forms (memory, and only long histories): N = 300, 2 10^5 steps, bf16 x3, B =
+// 16 3866 / 1558, N = 1000, 1.5 10^5 1106 / 782 (bf16, B = 64), N = 2000, 6 10^4
+// 319 / 314, N = 3500, 6 10^4 629 / 636 (x3, B = 16), N = 4000 655 / 704; N =
+// 1000 and 4000 steps 38.7 / 39.2.
+int older_splits(const fpde_solver* s, int tcA) {
+    const int64_t wgs = kOlderSplits * ((s->plan.nodes + 63) / 64);
+    const bool all = s->spec.hist_mode == HIST_MFMA_F64 ? wgs < 512 : wgs < 224 && tcA >= 4096;
+    return all ? 0 : kOlderSplits;
+}
+
 // The older part of block n0's far sums, levels [0, tcA), as up to
 // kOlderSplits splits of B rows in P.  The split forms pack the levels it
 // needs first (those not packed yet), on the same stream.
-// The step launch adds the splits itself, beside its chain: fourteen splits
-// (N = 10^4) and a pass that added them wrote and read 72 MB more per block and
-// solve, 2 to 6 splits measured alike; six solves of N = 10^4, 2000 steps, in a
-// batch 38.9 -> 35.3 ms.
 fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t st, int* splits) {
     const fpde_spec& sp = s->spec;
     fpde_status rc = FPDE_OK;
@@ -523,7 +539,11 @@ fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t s
         s->packed_groups = ghi;
         if (rc != FPDE_OK) return rc;
     }
-    rc = gemm_range(s, n0, 0, tcA, P, kOlderSplits, splits, st);
+    rc = gemm_range(s, n0, 0, tcA, P, older_splits(s, tcA), splits, st);
+    if (rc == FPDE_OK && *splits > kOlderSplits) {
+        rc = launch_part_reduce(P, *splits, s->spec.block, s->plan.ld, (int)s->plan.nodes, st);
+        *splits = 1;
+    }
     if (rc == FPDE_OK && tcA > 0) {
         s->stats.history_launches++;
         s->stats.history_alg_bytes += 8.0 * tcA * (double)s->plan.nodes * s->spec.block;

@@ -1869,3 +1869,28 @@ def test_short_history_sum_of_long_lines(fpde, nodes, levels):
             assert (np.abs(S[:nodes] - terms.sum(axis=0)) <= bound).all()
     finally:
         dv.close()
+
+
+@pytest.mark.parametrize("mode,tol,nodes,steps", [
+    ("mfma_f64", TOL_F64, 8128, 300), ("mfma_f64", TOL_F64, 8129, 300), ("mfma_f64", TOL_F64, 130, 700),
+    ("split_bf16", TOL_MIXED, 200, 4500), ("split_f16", TOL_MIXED, 3521, 4300)])
+def test_older_far_parts_in_all_their_splits(fpde, mode, tol, nodes, steps):
+    """The older far part in all its K splits, added by a pass of their own
+    (FP64 on lines up to 8128 nodes, the split forms up to 3520 from 4096 levels
+    on), and in four: a solve at once, in pieces and in a batch gives the same
+    bits, and agrees with the plain history."""
+    u0 = fpde.init_1d(nodes, 98)
+    kw = dict(alpha=0.7, picard_max=2, picard_tol=1e-12, u_top=u0[0])
+    spec = fpde.make_spec(nodes, steps, 1e-3, hist_mode=mode, block=128, **kw)
+    whole = fpde.solve(spec, u0)
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b, fpde.Solver(spec) as c:
+        for s in (a, b, c):
+            s.set_initial(u0)
+        for piece in (1, 130, steps // 2, 0):
+            a.advance(piece)
+        fpde.advance_batch([b, c], 0)
+        for s in (a, b, c):
+            assert np.array_equal(s.solution(), whole)
+    err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw), u0))
+    print(f"older splits {mode} N={nodes} M={steps}: rel err {err:.3e}", flush=True)
+    assert err <= tol
