@@ -314,6 +314,7 @@ struct Step1DArgs {
     const double *ahead_far, *ahead_omega;
     // cooperative block form (k_step1d_block): steps [n, n_end) in one launch
     int n_end;
+    int slim;                 // single launches of long chunks: three waves per workgroup instead of five
     int picard_max;
     int n0;                   // first step of the history block (far partial row = n - n0)
     int blk;                  // rows of the history block (far partial and mid rows)
@@ -587,6 +588,7 @@ fpde_status launch_part_sum(double* P, const double* part, int splits, int rows,
 fpde_status launch_step1d(const Step1DArgs& a, hipStream_t st);
 fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st);
 bool step1d_block_supported(int N, int C);
+bool step1d_block_slim(int N, int C);
 bool step1d_batch_supported(int64_t wgs);
 // History term of a 3D step: S = partial rows + near levels [lo, n) + two-level
 // corrections (corr: of step n; null where the partial rows hold them).

@@ -235,6 +235,7 @@ struct fpde_solver {
     unsigned long long* xch = nullptr;  // grid exchange words of the cooperative 1D block launches
     int* err = nullptr;        // grid-exchange time-out flag, Picard solve count
     bool block_mode = false;   // 1D steps run as cooperative block launches
+    bool slim = false;         // in workgroups that leave room for the far part ahead
     int64_t coop_launches = 0; // cooperative launches so far (the next one's exchange tag)
     int* flags = nullptr;
     // graph-captured step loop: the executable graph of the last captured chunk
@@ -460,6 +461,7 @@ fpde_status solver_alloc(fpde_solver* s) {
         // with helper workgroups for the sum measured no faster)
         s->block_mode = (sp.step_mode == 0) && blocked_history && !space && step1d_block_supported(sp.nodes, s->C);
         s->la = s->block_mode && lookahead_spec(sp);
+        s->slim = s->la && sp.hist_mode == HIST_MFMA_F64 && step1d_block_slim(sp.nodes, s->C);
         if (s->block_mode && s->w.ser_P == 0) DALLOC(s->mid, sizeof(double) * (size_t)sp.block * p.ld);
         DALLOC(s->flags, sizeof(int) * 16);
     } else {
@@ -1011,6 +1013,7 @@ Step1DArgs block_args(fpde_solver* s, int n, int n_end, int n0, int nsplit, int6
     a.coef_mode = sp.coef_mode;
     a.n = n;
     a.n_end = n_end;
+    a.slim = s->slim ? 1 : 0;
     a.n0 = n0;
     a.blk = sp.block;
     a.mid = s->mid;

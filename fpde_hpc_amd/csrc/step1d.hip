@@ -1208,16 +1208,16 @@ __device__ __forceinline__ void solver_steps(const Step1DArgs& g, const int c, S
         __hip_atomic_fetch_add(g.err + 1, ps.solves, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// The body of the single-solve launch and of the batched one: RW row waves,
-// then the solver wave of R rows per lane.  The roles are compiled apart and
+// The body of the single-solve launch and of the batched one: RW row waves of
+// NPT nodes per thread, then the solver wave of RW NPT rows per lane.  The roles are compiled apart and
 // keep their control flow flat: together (one loop with the role inside) their
 // launch constants overflowed the scalar registers, and the reloads and
 // branches between two solves cost 2500 of 15000 cycles.
-template <int RW>
+template <int RW, int NPT>
 __global__ __launch_bounds__(64 * RW + 64) void k_step1d_block(Step1DArgs g) {
     __shared__ Step1DLds L;
-    if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) == RW) solver_steps<RW>(g, (int)blockIdx.x, L);
-    else row_steps<RW, 1>(g, (int)blockIdx.x, L);
+    if (__builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) == RW) solver_steps<RW * NPT>(g, (int)blockIdx.x, L);
+    else row_steps<RW, NPT>(g, (int)blockIdx.x, L);
 }
 
 // Many independent solves in one cooperative launch: workgroups
@@ -1269,14 +1269,34 @@ static bool coop_fits(const void* kern, int threads, int64_t wgs) {
     return (int64_t)per_cu * cus >= wgs;
 }
 
-static const void* block_kernel(int rw) {
-    return rw == 3 ? (const void*)k_step1d_block<3> : (const void*)k_step1d_block<4>;
+// Chunks of up to 192 nodes: three row waves; longer ones four, or two with two
+// nodes per thread (slim).
+struct BlockKernel { const void* fn; int threads; };
+static BlockKernel block_kernel(int N, int C, bool slim) {
+    if (row_waves(N, C) == 3) return {(const void*)k_step1d_block<3, 1>, 256};
+    if (slim) return {(const void*)k_step1d_block<2, 2>, 192};
+    return {(const void*)k_step1d_block<4, 1>, 320};
+}
+
+// Five waves of 247 registers put two on one SIMD of their CU and leave it no
+// room for another kernel's: where the chunks cover most of the GPU, the far
+// part ahead (lookahead) waits for the end of the launch it was to run beside.
+// FP64 takes long enough for that to count; there the launch has the batch's
+// shape, which leaves every SIMD half its registers.  Lagged / Picard, ms, five
+// waves against three: N = 65536, 3000 steps 64 / 44 and 95 / 74 (57 and 101 with
+// the whole workgroup's line solve in four waves), N = 55000, 2000 steps (215
+// chunks) 33 / 26 and 50 / 45; N = 40000 in 157 chunks 21.2 / 21.1 and 36.5 / 38.1.
+// bf16, N = 55000: 20.2 / 21.8 and 38.0 / 40.2.
+bool step1d_block_slim(int N, int C) {
+    int dev = 0, cus = 0;
+    return row_waves(N, C) == 4 && hipGetDevice(&dev) == hipSuccess &&
+           hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && 4 * C > 3 * cus;
 }
 
 // Whether the C workgroups of a cooperative block launch can be co-resident.
 bool step1d_block_supported(int N, int C) {
-    const int rw = row_waves(N, C);
-    return coop_fits(block_kernel(rw), 64 * rw + 64, C);
+    const BlockKernel k = block_kernel(N, C, false);
+    return coop_fits(k.fn, k.threads, C);
 }
 bool step1d_batch_supported(int64_t wgs) { return coop_fits((const void*)k_step1d_batch, kBatchThreads, wgs); }
 
@@ -1302,8 +1322,8 @@ fpde_status launch_step1d_block(const Step1DArgs& a, hipStream_t st) {
     if (a.n_end <= a.n) return FPDE_OK;
     Step1DArgs arg = a;
     void* params[] = {&arg};
-    const int rw = row_waves(a.N, a.C);
-    FPDE_HIP_TRY(hipLaunchCooperativeKernel(block_kernel(rw), dim3(a.C), dim3(64 * rw + 64), params, 0, st));
+    const BlockKernel k = block_kernel(a.N, a.C, a.slim != 0);
+    FPDE_HIP_TRY(hipLaunchCooperativeKernel(k.fn, dim3(a.C), dim3(k.threads), params, 0, st));
     return FPDE_OK;
 }
 

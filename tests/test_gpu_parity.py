@@ -1894,3 +1894,27 @@ def test_older_far_parts_in_all_their_splits(fpde, mode, tol, nodes, steps):
     err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw), u0))
     print(f"older splits {mode} N={nodes} M={steps}: rel err {err:.3e}", flush=True)
     assert err <= tol
+
+
+@pytest.mark.parametrize("nodes", [49153, 50001, 65536])
+@pytest.mark.parametrize("picard", [1, 2])
+def test_long_lines_in_slim_workgroups(fpde, nodes, picard):
+    """FP64 lines whose chunks cover most of the GPU run in workgroups of three
+    waves (two nodes per thread), as a batch does: the same bits alone, in pieces
+    and in a batch, and the plain history's result (193 chunks and 256)."""
+    steps = 70
+    u0 = fpde.init_1d(nodes, 99)
+    kw = dict(alpha=0.7, picard_max=picard, picard_tol=1e-12 if picard > 1 else 0.0, u_top=u0[0])
+    spec = fpde.make_spec(nodes, steps, 1e-3, hist_mode="mfma_f64", block=16, **kw)
+    whole = fpde.solve(spec, u0)
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b:
+        for s in (a, b):
+            s.set_initial(u0)
+        for piece in (1, 20, 0):
+            a.advance(piece)
+        fpde.advance_batch([b], 0)
+        assert np.array_equal(a.solution(), whole)
+        assert np.array_equal(b.solution(), whole)
+    err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw), u0))
+    print(f"slim N={nodes} picard={picard}: rel err {err:.3e}", flush=True)
+    assert err <= TOL_F64
