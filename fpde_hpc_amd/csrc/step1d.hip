@@ -117,7 +117,7 @@ __device__ inline double hist_tail(double om0, double c0, double c1, int n, int 
 // 16 (p mod 4) + p/4 holds position p and a stride of 4 q positions is a DPP
 // row shift by q.  One separator per chunk (not both chunk ends) halves the
 // reduced system, whose couplings fall off with the chunk length: its cyclic
-// reduction ends as soon as none exceeds 2^-60.
+// reduction ends as soon as none exceeds kNoCoupling.
 // Measured (cycles of one iteration at N = 10^4, 53 chunks, phase timers): row
 // waves 2000 from barrier to barrier (coefficients 640); solver wave: rows and
 // line solve 2500, publishing 900, waiting for the other chunks 4700,
@@ -160,7 +160,14 @@ constexpr int kXchMeasure = 14;                                 // first word of
 constexpr int kXchPad = kXchWords + 2;                          // LDS row: 144 B, 16-byte reads spread over the banks
 static_assert(2 * kMaxChunks * kXchWords * 8 == (int)kXchBytes, "exchange buffer size");
 
-constexpr double kNoCoupling = 0x1p-60;                         // below: no effect on a double of its row's size
+// Coupling of two separators (or positions) that is dropped: its part of the one
+// is below rounding, 2^-53, where the other is up to 2^20 times as large, which
+// is the range of heads from 1e-2 to 1e4 m.  (At 2^-60 a dry separator of 1e6
+// beside wet nodes of 1e-2 lost 3e-12 of them.)  Comparing the parts with the
+// values themselves cost 1% of a solve on its dependent chain and 4% of the plain
+// form's, whether the neighbours' values were fetched or bounded over the wave;
+// 2^-86, another level of reduction for 32 orders at N = 4000, 4% of that solve.
+constexpr double kNoCoupling = 0x1p-73;
 
 // ---- one wave's line solve -------------------------------------------------
 // a double moved within the rows of 16 lanes; lanes without a source take fill
@@ -215,7 +222,7 @@ __device__ inline bool coupled(double a, double c, int p) {
 // and UR (right of the last): x_i = x + y UL + z UR.  A position's first R-1
 // rows are eliminated against its last one (Thomas with both couplings as
 // right-hand sides), the last ones reduced cyclically.  With EARLY the
-// reduction stops once no coupling between positions exceeds 2^-60 (the
+// reduction stops once no coupling between positions exceeds kNoCoupling (the
 // boundaries' couplings must be zero: y and z are not formed).
 template <int R, bool EARLY>
 __device__ inline void wave_line(const double (&a)[R], const double (&c)[R], const double (&d)[R], int p,

@@ -1918,3 +1918,44 @@ def test_long_lines_in_slim_workgroups(fpde, nodes, picard):
     err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, hist_mode="plain", **kw), u0))
     print(f"slim N={nodes} picard={picard}: rel err {err:.3e}", flush=True)
     assert err <= TOL_F64
+
+
+@pytest.mark.parametrize("nodes,span,peak,coupling", [(640, 32, 1e6, 64), (2240, 128, 1e9, 64), (640, 32, 1.5e4, 74),
+                                                      (2240, 128, 6e4, 74)])
+@pytest.mark.parametrize("step_mode", [0, 1])
+def test_separators_of_very_different_size(fpde, nodes, span, peak, coupling, step_mode):
+    """A separator of 1e6 (1e9) among nodes of 1e-2, with a coupling to the next
+    one (to the next lane's, with four separators per lane) of 2^-64: its part
+    there is 3e-12 (9e-10) of the value, and each node is compared by itself.
+    At 2^-74 the coupling may be dropped: up to 10^6 times as large, the part is
+    below 2^-54.  One step with K = C = 1 against the same rows solved in extended precision;
+    every product is of one sign, so a node's error is at most about six
+    roundings per row of the `span` rows eliminated between the two."""
+    lam = 2.0 ** (-coupling / span)
+    h = 1.0 / (nodes - 1)
+    tau = h * h / (lam + 1.0 / lam - 2.0)                  # alpha = 1: L = 1 / tau
+    u0 = np.full(nodes, 1e-2)
+    at = 32 * (10 if span == 32 else 43)                   # a chunk's first node, the last of its lane
+    u0[at] = peak
+    spec = fpde.make_spec(nodes, 1, tau, alpha=1.0, coef_mode=1, ksat=1.0, hist_mode="mfma_f64", block=16,
+                          u_top=u0[0], chunk_rows=32, step_mode=step_mode)
+    with fpde.Solver(spec) as s:
+        s.set_initial(u0)
+        L = np.longdouble(s.weights()[0])
+        s.advance()
+        u = s.solution()
+    g = 1.0 / np.longdouble(spec.length / (nodes - 1)) ** 2
+    q, d = np.zeros(nodes, np.longdouble), np.zeros(nodes, np.longdouble)
+    d[0] = u0[0]
+    for i in range(1, nodes - 1):
+        piv = 2.0 * g + L - g * q[i - 1]
+        q[i] = g / piv
+        d[i] = (L * np.longdouble(u0[i]) + g * d[i - 1]) / piv
+    ref = np.zeros(nodes, np.longdouble)
+    ref[-1] = d[-2] / (1.0 - q[-2])
+    for i in range(nodes - 2, -1, -1):
+        ref[i] = q[i] * ref[i + 1] + d[i]
+    err = float(np.max(np.abs(u - ref) / np.abs(ref)))
+    print(f"separators N={nodes} step_mode={step_mode} L h^2={float(L / g):.4f}: per-node rel err {err:.3e}", flush=True)
+    assert abs(float(L) * tau - 1.0) < 1e-12
+    assert err <= 6 * span * np.finfo(float).eps
