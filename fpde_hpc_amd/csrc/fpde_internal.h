@@ -294,7 +294,6 @@ struct Step1DArgs {
     double* xyz;              // [3][ld] chunk factors
     double* red;              // [2][C][8] the chunks' values of the separators' system, by launch parity
     double* Uit;              // Picard iterate (for the convergence test)
-    int* flags;               // unused
     double tol;
     int64_t omega_stride;     // per-step weight rows (prescribed grid): omega + (n - n0) * stride
     const double* Lv;         // per-step local coefficient (prescribed grid), else L

@@ -237,7 +237,6 @@ struct fpde_solver {
     bool block_mode = false;   // 1D steps run as cooperative block launches
     bool slim = false;         // in workgroups that leave room for the far part ahead
     int64_t coop_launches = 0; // cooperative launches so far (the next one's exchange tag)
-    int* flags = nullptr;
     // graph-captured step loop: the executable graph of the last captured chunk
     hipGraphExec_t gexec = nullptr;
     int64_t graph_launches = 0, graph_instantiations = 0;
@@ -463,7 +462,6 @@ fpde_status solver_alloc(fpde_solver* s) {
         s->la = s->block_mode && lookahead_spec(sp);
         s->slim = s->la && sp.hist_mode == HIST_MFMA_F64 && step1d_block_slim(sp.nodes, s->C);
         if (s->block_mode && s->w.ser_P == 0) DALLOC(s->mid, sizeof(double) * (size_t)sp.block * p.ld);
-        DALLOC(s->flags, sizeof(int) * 16);
     } else {
         int n = sp.nodes;
         if (sp.gamma > 0.0 && sp.gamma < 1.0) {
@@ -911,7 +909,6 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
     a.xyz = s->xyz;
     a.red = s->red;
     a.Uit = s->Uit;
-    a.flags = s->flags;
     a.tol = sp.picard_tol;
     a.prev_k = s->last_k;
     a.extrap = sp.picard_max > 1 ? 1 : 0;

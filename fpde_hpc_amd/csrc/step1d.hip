@@ -784,7 +784,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
     // most 17; near_lo is n0 or up to 31 levels before it).  The schedule
     // depends on the step alone: launches may end anywhere in a block.
     auto ready = [&](int j) { return max(g.n0, g.near_lo + kNearGroup * j + kNearGroup + 1); };    // s_j
-    auto groups = [&](int m) { return g.mid && m - 2 >= g.n0 ? (m - 3 - g.near_lo) / kNearGroup : 0; };
+    auto groups = [&](int m) { return m - 2 >= g.n0 ? (m - 3 - g.near_lo) / kNearGroup : 0; };
     int fold_done = n_first - 1;                               // (a step done again does not fold again)
     PicardState ps = picard_state(g);
     // of a tentatively ended step, what its last iteration still needs
@@ -846,7 +846,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
                 n0 = fma(wl[max(m - 2 - lo - j, 0)], v[j], n0);
                 n1 = fma(wl[max(m - 3 - lo - j, 0)], v[j + 1], n1);
             }
-            // levels past the first 16 (a 17th, or a block without g.mid)
+            // levels past the first 16: a 17th, and those before a block's first two steps
             for (int t = lo + W; t < m - 1; t++) n0 = fma(om[m - 1 - t], Dc[(int64_t)t * g.ld + col], n0);
             h[q] = far + (n0 + n1);
         }
@@ -926,7 +926,7 @@ __device__ __forceinline__ void row_steps(const Step1DArgs& g, const int c, Step
         }
         __syncthreads();                                       // A
         if (fresh && !series) {
-            if (g.mid && ps.n > fold_done) {
+            if (ps.n > fold_done) {
                 fold_done = ps.n;
                 for (int j = 0; j < groups(ps.n + 2); j++) {
                     const int p0 = ready(j) + 2 + kFoldBatch * (ps.n - ready(j)), end = g.n0 + g.blk;
