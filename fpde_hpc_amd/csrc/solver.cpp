@@ -665,15 +665,14 @@ void drop_started(fpde_solver* s) {
 // rounds alike.  At most 32 partial rows, which the chain reads in one memory
 // trip.  N = 3001: 11.6 -> 7.2 us per step over 1500 steps; N = 10^4: 26.7 ->
 // 20.0 over 3000 steps, 44.6 -> 41.6 over 6000, 89 -> 85 over 12000: 5 to 7 us
-// a step at any length.  A history beyond kAheadBytes streams for over 90 us,
-// of which that is 5%: it keeps its own launch (64 partial rows), which the
-// profile's history class times.
+// a step at any length.  Where a history exceeds 512 MB, a launch of its own
+// and 64 partial rows are still the slower way: N = 6000, 12000 steps 600.6 ->
+// 594.9 ms, N = 10^4, 16000 steps 1864 -> 1817, N = 30000, 3000 steps 204 ->
+// 194, N = 65536, 1500 steps 115.3 -> 109.8, N = 1500, 45000 steps 2380 -> 2325.
 constexpr int kAheadSplits = 32;
-constexpr double kAheadBytes = 512e6;
-bool plain_ahead(const fpde_solver* s, int n) {
+bool plain_ahead(const fpde_solver* s) {
     const fpde_spec& sp = s->spec;
-    return sp.dims == 1 && sp.hist_mode == HIST_PLAIN_F64 && sp.sum_alg != 2 && !s->w.grid &&
-           8.0 * n * (double)s->plan.nodes <= kAheadBytes;
+    return sp.dims == 1 && sp.hist_mode == HIST_PLAIN_F64 && sp.sum_alg != 2 && !s->w.grid;
 }
 struct AheadStream { int lo, hi, chunk, splits; int64_t off; };
 AheadStream ahead_stream(const fpde_solver* s, int n) {
@@ -723,7 +722,7 @@ fpde_status far_part(fpde_solver* s, int n, int* nsplit, int64_t* stride, int64_
     }
     // levels available in memory: t < avail
     int avail = s->pending ? n - 1 : n;
-    if (sp.hist_mode == HIST_PLAIN_F64 && plain_ahead(s, n)) {
+    if (sp.hist_mode == HIST_PLAIN_F64 && plain_ahead(s)) {
         const AheadStream h = ahead_stream(s, n);
         if (s->ahead_step != n && h.splits > 0) {
             size_t slot = 0;
@@ -898,7 +897,7 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
         a.ahead_rows = s->gsplits;
         a.ahead_far = s->part + (int64_t)(n + 1 - s->n0) * s->plan.ld;
         a.ahead_omega = s->w.grid ? s->Wnear + (size_t)(n + 1 - s->n0) * s->ldwn : s->w.omega;
-    } else if (ahead && plain_ahead(s, n + 1)) {
+    } else if (ahead && plain_ahead(s)) {
         const AheadStream h = ahead_stream(s, n + 1);
         a.ahead_lo = h.lo;
         a.ahead_hi = h.hi;
@@ -981,7 +980,7 @@ fpde_status enqueue_1d_step(fpde_solver* s, int n, bool more) {
     }
     s->ahead_step = -1;
     if (more && row_ahead(s, n + 1)) s->ahead_step = n + 1;
-    else if (more && plain_ahead(s, n + 1)) {
+    else if (more && plain_ahead(s)) {
         const AheadStream h = ahead_stream(s, n + 1);
         s->ahead_step = n + 1;
         s->stats.step_alg_bytes += 8.0 * std::max(0, h.hi - h.lo) * (double)s->plan.nodes;

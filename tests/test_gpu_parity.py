@@ -1959,3 +1959,26 @@ def test_separators_of_very_different_size(fpde, nodes, span, peak, coupling, st
     print(f"separators N={nodes} step_mode={step_mode} L h^2={float(L / g):.4f}: per-node rel err {err:.3e}", flush=True)
     assert abs(float(L) * tau - 1.0) < 1e-12
     assert err <= 6 * span * np.finfo(float).eps
+
+
+def test_plain_history_over_512_mb_streamed_ahead(fpde):
+    """A plain history is streamed by the previous step's launch at any length:
+    from 977 levels of 65536 nodes (512 MB) on no launch of its own, the same
+    bits in pieces (whose first step streams by itself), and the FP64 block
+    GEMM's result."""
+    nodes, steps = 65536, 1000
+    u0 = fpde.init_1d(nodes, 5)
+    spec = fpde.make_spec(nodes, steps, 1e-3, alpha=0.7, hist_mode="plain", u_top=u0[0])
+    with fpde.Solver(spec) as a, fpde.Solver(spec) as b:
+        for s in (a, b):
+            s.set_initial(u0)
+        a.advance(0)
+        for piece in (979, 2, 0):
+            b.advance(piece)
+        whole = a.solution()
+        assert np.array_equal(b.solution(), whole)
+        launches = [s.stats()["history_launches"] for s in (a, b)]
+    err = rel_err(whole, fpde.solve(fpde.make_spec(nodes, steps, 1e-3, alpha=0.7, hist_mode="mfma_f64", u_top=u0[0]), u0))
+    print(f"plain ahead N={nodes} M={steps}: history launches {launches}, rel err {err:.3e}", flush=True)
+    assert launches == [0, 2]
+    assert err <= TOL_F64
