@@ -802,8 +802,8 @@ __global__ __launch_bounds__(256) void k_gemm_split_direct(const double* __restr
     }
 }
 
-// P[r][i] = the K splits' partial rows added in split order (as the 3D history
-// combine adds them), for every row of a block at once.
+// P[r][i] = the K splits' partial rows added in split order, for every row of a
+// block at once (one row: the parts of a streamed history sum).
 __global__ __launch_bounds__(256) void k_part_sum(double* __restrict__ P, const double* __restrict__ part, int splits,
                                                   int rows, int64_t ld, int nodes) {
     constexpr int W = 16;
@@ -906,10 +906,10 @@ fpde_status launch_hist_sum(double* S, const double* D, int64_t ld, int nodes, i
     int splits = 0;
     fpde_status rc = launch_hist_plain(D, ld, nodes, n, n, omega, part, &splits, st);
     if (rc != FPDE_OK) return rc;
-    // no near levels, no corrections: the partial rows added
-    rc = launch_hist_combine(S, Hist3D{part, ld, splits, D, ld, 0, 0, omega, nullptr}, nodes, 1.0, st);
-    if (rc == FPDE_OK) FPDE_HIP_TRY(hipGetLastError());
-    return rc;
+    // 16 rows to a memory trip: with the 3D history combine, which takes 8 (16
+    // cost it 1 to 3% of a 3D solve), whole calls took 19.6 us at 300 nodes x
+    // 2000 levels (19.0 so) and 25.4 at 1000 x 4000 (24.6)
+    return launch_part_sum(S, part, splits, 1, ld, nodes, st);
 }
 
 // Parts of the reference Sum: about 2048 workgroups with the 512-node tiles
