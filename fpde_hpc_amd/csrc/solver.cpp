@@ -674,6 +674,9 @@ bool plain_ahead(const fpde_solver* s) {
     const fpde_spec& sp = s->spec;
     return sp.dims == 1 && sp.hist_mode == HIST_PLAIN_F64 && sp.sum_alg != 2 && !s->w.grid;
 }
+// (a profile of the history kernels times the stream in launches of its own:
+// the same split, the same bits)
+bool streams_ahead(const fpde_solver* s) { return plain_ahead(s) && !(s->prof & 1); }
 struct AheadStream { int lo, hi, chunk, splits; int64_t off; };
 AheadStream ahead_stream(const fpde_solver* s, int n) {
     AheadStream h{};
@@ -897,7 +900,7 @@ fpde_status launch_1d(fpde_solver* s, int n, int k, int nsplit, int64_t stride, 
         a.ahead_rows = s->gsplits;
         a.ahead_far = s->part + (int64_t)(n + 1 - s->n0) * s->plan.ld;
         a.ahead_omega = s->w.grid ? s->Wnear + (size_t)(n + 1 - s->n0) * s->ldwn : s->w.omega;
-    } else if (ahead && plain_ahead(s)) {
+    } else if (ahead && streams_ahead(s)) {
         const AheadStream h = ahead_stream(s, n + 1);
         a.ahead_lo = h.lo;
         a.ahead_hi = h.hi;
@@ -980,7 +983,7 @@ fpde_status enqueue_1d_step(fpde_solver* s, int n, bool more) {
     }
     s->ahead_step = -1;
     if (more && row_ahead(s, n + 1)) s->ahead_step = n + 1;
-    else if (more && plain_ahead(s)) {
+    else if (more && streams_ahead(s)) {
         const AheadStream h = ahead_stream(s, n + 1);
         s->ahead_step = n + 1;
         s->stats.step_alg_bytes += 8.0 * std::max(0, h.hi - h.lo) * (double)s->plan.nodes;

@@ -335,7 +335,9 @@ fpde_status fpde_solver_write_results(fpde_solver *s, const char *path_txt, cons
 /* Effective weights (local, omega[M], corr[2M]) the solver uses (host copies). */
 fpde_status fpde_solver_get_weights(fpde_solver *s, double *local, double *omega, double *corr);
 /* Per-kernel timing with hipEvents on the solver's stream: bit 0 = history
- * kernels (plain stream / pack+GEMM / combine), bit 1 = step kernels. */
+ * kernels (plain stream / pack+GEMM / combine), bit 1 = step kernels.  With bit
+ * 0 the plain 1D stream, which otherwise runs inside the step's launch, has
+ * launches of its own; results are the same bits. */
 fpde_status fpde_solver_set_profiling(fpde_solver *s, int mask);
 fpde_status fpde_solver_get_stats(fpde_solver *s, fpde_stats *out);
 

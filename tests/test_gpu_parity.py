@@ -1982,3 +1982,25 @@ def test_plain_history_over_512_mb_streamed_ahead(fpde):
     print(f"plain ahead N={nodes} M={steps}: history launches {launches}, rel err {err:.3e}", flush=True)
     assert launches == [0, 2]
     assert err <= TOL_F64
+
+
+@pytest.mark.parametrize("nodes,steps,extra", [(700, 90, {}), (1537, 60, {"sum_alg": 1, "sum_param": 1e-2}),
+                                               (300, 40, {"picard_max": 3, "picard_tol": 1e-12})])
+def test_profile_times_the_plain_history(fpde, nodes, steps, extra):
+    """A profile of the history kernels times the plain stream of every step that
+    has one (from the fourth on: the step's launch adds the last two levels),
+    and the solve has the same bits as without."""
+    u0 = fpde.init_1d(nodes, 6)
+    with fpde.Solver(fpde.make_spec(nodes, steps, 1e-3, alpha=0.7, hist_mode="plain", u_top=u0[0], **extra)) as s:
+        s.set_initial(u0)
+        s.advance(0)
+        whole = s.solution()
+        assert s.stats()["history_launches"] == 0
+        for mask in (1, 3):
+            s.reset(u0)
+            s.set_profiling(mask)
+            s.advance(0)
+            assert np.array_equal(s.solution(), whole)
+            st = s.stats()
+            assert st["history_launches"] == steps - 3
+            assert st["ms_history"] > 0.0 and (st["ms_step"] > 0.0) == (mask == 3)
