@@ -618,8 +618,9 @@ def main():
         out["speedup_vs_plain_fp64"] = variants["plain"]["ms_per_solve"] / (t_mean * 1e3)
         pv = variants["plain"]
         out["speedup_note"] = (
-            f"plain runs its FP64 history stream between every two steps, so its steps launch per Picard "
-            f"iteration ({pv['step_launches']} step launches, {pv['step_ms']:.0f} ms of step time); the "
+            f"plain streams its whole FP64 history once per step, beside the step's launch, so its steps launch "
+            f"per Picard iteration ({pv['step_launches']} step launches, {pv['step_ms']:.0f} ms of step time, and "
+            f"{pv['history_ms']:.0f} ms of streams when profiled apart); the "
             f"{args.headline} form runs one cooperative launch per history block "
             f"({variants[args.headline]['step_launches']} launches, {variants[args.headline]['step_ms']:.0f} ms)")
         if ref_u is not None:

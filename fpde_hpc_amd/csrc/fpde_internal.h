@@ -360,7 +360,12 @@ struct BatchTick {
 // d < 16 (t + 1) and space_chunks(t, ldp) partial rows.  Chunks of 64 leave a
 // short line on few workgroups (N = 4000: 40, whose waves each do 64 FP64 MFMA
 // one after the other), of 16 make as many rows of partial sums as tiles; up to
-// 8192 rows these are 32 rows at most.
+// 8192 rows these are 32 rows at most.  Chunks of 16 against 64 on both sides of
+// that line: solves of 300 steps, ms: N = 4000 4.42 / 4.92, 6144 4.83 / 4.93,
+// 7168 5.15 / 4.96, 8192 5.27 / 4.98, 8193 5.12 / 5.54, 9472 5.65 / 5.59, 12288
+// 6.28 / 6.35, 16000 8.01 / 7.40, 32768 16.4 / 12.6; direct sums, us: 4096 32.1
+// / 34.9, 8192 34.9 / 35.5, 8193 34.7 / 37.3, 12288 38.5 / 39.8, 16000 44.9 /
+// 42.9, 65536 165 / 130: between 6000 and 14000 rows either way within 8%.
 constexpr int kSpTile = 256;
 constexpr int kSpDiag = 64;
 __host__ __device__ inline int space_diag(int64_t ldp) { return ldp <= 8192 ? 16 : kSpDiag; }
@@ -543,8 +548,9 @@ fpde_status launch_ref_series(double* S, const double* old, int64_t old_size, in
                               double gt, double alpha, hipStream_t st);
 // The GEMM launchers write K-split partial rows P[ks][r][i], ks < *splits_out
 // (at most max_splits when that is > 0); the readers add them in split order:
-// the 3D history combine itself, the 1D step kernels after launch_part_reduce
-// has folded them into P[0].
+// the 3D history combine, the 1D cooperative launches whose far part is
+// computed ahead (at most four of the older part and the newer one), and
+// launch_part_reduce, which folds them into P[0], for the other 1D forms.
 fpde_status launch_gemm_f64(const double* D, int64_t ld, int nodes, int n0, int tc, int block,
                             const double* omega, double* P, int* splits_out, hipStream_t st,
                             int max_splits = 0, const double* corr = nullptr, const double* D0 = nullptr);

@@ -54,12 +54,16 @@ bool lookahead_spec(const fpde_spec& s) {
 }
 
 // Chunks of a 1D line (one workgroup each in the partitioned solve).  The
-// automatic size is 192 nodes: with three waves of rows per workgroup the
-// chunk PCR levels and the near-field history loads cost less per workgroup,
-// and the reduced system (2C rows) stays within seven PCR levels up to
-// N = 12288; the headline solve (N = 10^4) measured 0.387 s at 160-192
-// nodes against 0.409 s at 256.  Where 192-node chunks would number more
-// than 256, 256-node ones are taken.
+// automatic size is 192 nodes, three rows per lane of the wave that solves a
+// chunk's line; up to 64 chunks (N = 12288) that wave holds one separator per
+// lane, beyond four.  ms with chunks of 192 / 256 nodes, split bf16, Picard:
+// N = 10^4, 2 10^4 steps 199.6 / 207.2 (160 nodes 201.2, 128 269.5), N = 1000,
+// 4000 steps 39.8 / 42.7, N = 12288, 2000 steps 19.7 / 21.0, N = 24000, 1500
+// steps 20.3 / 20.9.  It is not the best size for every line: where 256-node
+// chunks stay within 64 and 192-node ones do not (N up to 16384) they are
+// faster, N = 14000, 2000 steps 26.5 / 21.0, and so are they for the longest
+// lines, N = 40000, 1000 steps 18.3 / 16.5 (chunk_rows sets them).  Where
+// 192-node chunks would number more than 256, 256-node ones are taken.
 int chunk_count(const fpde_spec& s) {
     if (s.chunk_rows > 0) return (s.nodes + s.chunk_rows - 1) / s.chunk_rows;
     const int c = (s.nodes + 191) / 192;
@@ -442,9 +446,9 @@ fpde_status solver_alloc(fpde_solver* s) {
         }
         // and those of a failed batch one that fails before the launch of this step
         if (const char* e = getenv("FPDE_TEST_FAIL_BATCH_AT")) s->fail_batch_at = atoi(e);
-        // cooperative block launches pay off where a launch covers many steps:
-        // the GEMM history forms (one launch per block) and the series form;
-        // the plain form needs its history kernel between every two steps
+        // cooperative block launches cover many steps: the GEMM history forms
+        // (one launch per block) and the series form; the plain form streams
+        // its whole history once per step, beside the step's own launch
         bool blocked_history = sp.hist_mode != HIST_PLAIN_F64 || sp.sum_alg == 2;
         const bool space = sp.gamma > 0.0 && sp.gamma < 1.0;
         if (space) {
@@ -527,7 +531,7 @@ int older_splits(const fpde_solver* s, int tcA) {
 }
 
 // The older part of block n0's far sums, levels [0, tcA), as up to
-// kOlderSplits splits of B rows in P.  The split forms pack the levels it
+// kOlderSplits splits of B rows in P (more are added up into one).  The split forms pack the levels it
 // needs first (those not packed yet), on the same stream.
 fpde_status older_part(fpde_solver* s, int n0, int tcA, double* P, hipStream_t st, int* splits) {
     const fpde_spec& sp = s->spec;
@@ -1552,11 +1556,12 @@ fpde_status fpde_solver_advance(fpde_solver* s, int nsteps) {
     return FPDE_OK;
 }
 
-// Many solvers advanced together.  Per history block: the far part of each
-// 1D block-mode solver on its own stream (they overlap), then one cooperative
-// launch of k_step1d_batch that runs the block's steps of all of them.  The
-// other solvers advance on their own streams meanwhile.  Returns when every
-// solver has reached its end step.
+// Many solvers advanced together.  Per history block of the 1D block-mode
+// solvers, on the first one's stream: their newer far parts in one launch, then
+// one cooperative launch of k_step1d_batch that runs the block's steps of all of
+// them; the older far parts of the next blocks run beside it, one after the
+// other, on that solver's side stream.  The other solvers advance on their own
+// streams meanwhile.  Returns when every solver has reached its end step.
 fpde_status fpde_solver_advance_batch(fpde_solver* const* solvers, int count, int nsteps) {
     if (!solvers || count < 1 || count > kMaxBatch) { set_error("advance_batch: 1 to 32 solvers"); return FPDE_ERR_ARG; }
     for (int i = 0; i < count; i++) {

@@ -122,10 +122,11 @@ __device__ inline double hist_tail(double om0, double c0, double c1, int n, int 
 // waves 2000 from barrier to barrier (coefficients 640); solver wave: rows and
 // line solve 2500, publishing 900, waiting for the other chunks 4700,
 // decision 150, separators 1100, U to LDS 500.  Headline solve (N = 10^4, M =
-// 2 10^4) 374 -> 206 ms, N = 1000 35.7 -> 21.5 ms, six solves in a batch 59.0
-// -> 38.9 ms against the whole workgroup's cyclic reduction over LDS with both
-// chunk ends as separators (five words per row and level, a workgroup barrier
-// per level) and coefficients by square roots and divisions (1700 cycles).
+// 2 10^4) 200 ms, N = 1000, M = 2000 19.7 ms, six N = 10^4, M = 2000 in a batch
+// 25.3 ms; 374, 34.2 and 57.8 ms with the whole workgroup's cyclic reduction over
+// LDS, both chunk ends as separators (five words per row and level, a workgroup
+// barrier per level), coefficients by square roots and divisions (1700 cycles)
+// and the far parts' K splits added between the launches.
 //
 // The arithmetic is written with explicit fma and contraction off: single
 // and batched launches round alike in every instantiation.
